@@ -1,0 +1,232 @@
+"""The workloads this library is timed on.
+
+A case is one pass of what a program that serves or trains a Mixture-of-Experts model asks of the library: a prefill
+layer (front end, block build, ``moe_cte``), a decode layer (``moe_tkg``) or the router.  ``listed()`` are the sizes of
+the repository's configurations, tests and benchmark; ``draw()`` gives further cases of the same ranges.
+
+Keys of a case: ``path`` (``cte`` | ``tkg`` | ``router``), ``kind`` (element types, see ``prepare``), T tokens, H hidden
+size, I intermediate size, E experts, k experts per token, B block size; the options ``act``, ``bias``, ``clamps``,
+``skip_token``, ``skew`` (standard deviation of a per-expert router bias: popular and unpopular experts), ``ckpt``.
+"""
+
+import math
+import os
+import sys
+
+import torch
+
+_PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nki-library_amd")
+if _PKG not in sys.path:
+    sys.path.insert(0, _PKG)
+
+from nkilib import synthetic as syn  # noqa: E402
+from nkilib.core.moe.moe_cte import (  # noqa: E402
+    MoECTEImplementation, MoECTESpec, QuantizationConfig, ShardOnIConfig, SkipMode, build_token_blocks, get_n_blocks,
+    moe_cte)
+from nkilib.core.moe.moe_tkg import moe_tkg  # noqa: E402
+from nkilib.core.rmsnorm import RmsNormQuantKernelArgs, rmsnorm_quant_kernel  # noqa: E402
+from nkilib.core.router_topk import route_for_moe  # noqa: E402
+from nkilib.core.subkernels.rmsnorm_mx_quantize_tkg import rmsnorm_mx_quantize  # noqa: E402
+from nkilib.core.utils.common_types import ActFnType, ExpertAffinityScaleMode, RouterActFnType  # noqa: E402
+
+_DEFAULTS = dict(path="cte", B=128, act="silu", bias=False, clamps=False, skip_token=False, skew=0.0, ckpt=False)
+_ACT = {"silu": ActFnType.SiLU, "swish": ActFnType.Swish}
+# gate <= 7, -7 <= up <= 7: the clamp triple of the models that clamp
+_CLAMPS = dict(gate_clamp_upper_limit=7.0, up_clamp_upper_limit=7.0, up_clamp_lower_limit=-7.0)
+
+
+def _case(name, **kw):
+    return dict(_DEFAULTS, name=name, **kw)
+
+
+def listed():
+    return [
+        # one token through the DeepSeek-V3-shaped MXFP8 experts: the latency of a single decode stream
+        _case("decode_mxfp8_1", path="tkg", kind="mxfp8", T=1, H=7168, I=2048, E=256, k=8),
+        # the same experts under a small decode batch: the expert weights are streamed once
+        _case("decode_mxfp8_32", path="tkg", kind="mxfp8", T=32, H=7168, I=2048, E=256, k=8),
+        # a decode batch over Qwen3-MoE-shaped bf16 experts
+        _case("decode_bf16_20", path="tkg", kind="bf16", T=20, H=2048, I=768, E=128, k=8),
+        # the DeepSeek-V3-shaped prefill layer that the benchmark reports
+        _case("prefill_mxfp8_8192", kind="mxfp8", T=8192, H=7168, I=2048, E=256, k=8),
+        # the Qwen3-MoE-shaped prefill layer with popular and unpopular experts
+        _case("prefill_mxfp8_skewed_8192", kind="mxfp8", T=8192, H=2048, I=768, E=128, k=8, skew=0.5),
+        # a short prompt of odd length over 4-bit experts with biases and clamped activations, hidden states in bf16
+        # (quantised inside the call)
+        _case("prefill_mxfp4_1999", kind="mxfp4", T=1999, H=3072, I=1536, E=32, k=4, B=256, act="swish", bias=True,
+              clamps=True),
+        # the Mixtral-shaped layer with fp8 weights (scales per channel) and fp8 activations (scales per row)
+        _case("prefill_fp8row_4096", kind="fp8row", T=4096, H=4096, I=14336, E=8, k=2),
+        # a bf16 layer of few large experts
+        _case("prefill_bf16_4096", kind="bf16", T=4096, H=2048, I=4096, E=8, k=2),
+        # the smallest prefill: a 256-token prompt over small bf16 experts
+        _case("prefill_bf16_256", kind="bf16", T=256, H=512, I=1024, E=8, k=2),
+        # many experts cut narrow by tensor parallelism (I = 192), a long prompt, biases and clamps
+        _case("prefill_bf16_narrow_10240", kind="bf16", T=10240, H=3072, I=192, E=128, k=4, B=256, act="swish", bias=True,
+              clamps=True, skip_token=True),
+        # the forward pass of a training step: gate/up and down activations are kept for the backward pass
+        _case("train_bf16_1024", kind="bf16", T=1024, H=3072, I=2048, E=8, k=4, B=512, act="swish", bias=True, ckpt=True),
+        # the router of the DeepSeek-V3-shaped layer
+        _case("router_8192", path="router", kind="bf16", T=8192, H=7168, I=0, E=256, k=8),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    """Half prefill, a third decode, the rest router; hidden and intermediate sizes over the range of the listed ones in
+    the steps their layouts allow (the intermediate size may end in a short tile), token and expert counts at will."""
+    path = rng.choice(("cte", "cte", "cte", "tkg", "tkg", "router"))
+    if path == "router":
+        return dict(_DEFAULTS, path=path, kind="bf16", T=_log_int(rng, 1, 8192), H=128 * rng.randint(4, 56), I=0,
+                    E=rng.choice((8, 16, 60, 64, 96, 128, 160, 256)), k=rng.randint(1, 8))
+    kind = rng.choice(("mxfp8", "mxfp8", "mxfp4", "fp8row", "bf16", "bf16_w8"))
+    if path == "tkg" and kind == "fp8row":
+        kind = "bf16_w8"  # (decode takes bf16 hidden states)
+    while True:
+        c = dict(_DEFAULTS, path=path, kind=kind)
+        c["T"] = _log_int(rng, 1, 128) if path == "tkg" else _log_int(rng, 100, 8192)
+        c["H"] = 512 * rng.randint(1, 14)
+        c["E"] = rng.choice((4, 8, 16, 32, 60, 64, 128, 256))
+        c["k"] = rng.randint(1, min(8, c["E"]))
+        c["B"] = 128 if path == "tkg" else rng.choice((128, 128, 256, 512))
+        # most intermediate sizes are multiples of 128, tensor parallelism leaves multiples of 64 or 32
+        step = rng.choice((128, 128, 128, 64, 32))
+        c["I"] = step * max(1, _log_int(rng, 192, 8192) // step)
+        c["act"] = rng.choice(("silu", "silu", "swish"))
+        c["bias"] = rng.random() < 0.3
+        c["clamps"] = c["act"] == "swish"
+        c["skip_token"] = path == "tkg" or rng.random() < 0.3
+        c["skew"] = rng.choice((0.0, 0.0, 0.5))
+        c["ckpt"] = path == "cte" and kind in ("bf16", "bf16_w8") and rng.random() < 0.3
+        if _weight_bytes(c) > 8e9:
+            continue
+        flops = 6.0 * c["T"] * c["k"] * c["H"] * c["I"]
+        if flops > (1.2e12 if kind.startswith("bf16") else 2.8e12):
+            continue
+        if get_n_blocks(c["T"], c["k"], c["E"], c["B"]) < 1 or _slots(c) * max(c["H"], c["I"]) > 6e8:
+            continue
+        return c
+
+
+def _slots(c):
+    return get_n_blocks(c["T"], c["k"], c["E"], c["B"]) * c["B"]
+
+
+def _weight_bytes(c):
+    per = {"mxfp8": 33 / 32, "mxfp4": 0.5 + 1 / 32, "fp8row": 1, "bf16": 2, "bf16_w8": 1}[c["kind"]]
+    return c["E"] * 3 * c["H"] * c["I"] * per
+
+
+def _gen(seed, salt):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed * 16 + salt)
+    return g
+
+
+def _bf16(g, shape, std):
+    return (torch.randn(shape, generator=g, device="cuda") * std).to(torch.bfloat16)
+
+
+def prepare(case, seed):
+    """Hidden states ~N(0, 1) with the zero padding row where the path takes one, weights ~N(0, 0.02) in the layout of
+    their kind, the router's expert ids and affinities."""
+    c = dict(_DEFAULTS, **case)
+    dev = torch.device("cuda:0")
+    T, H, I, E, k = c["T"], c["H"], c["I"], c["E"], c["k"]
+    st = {"case": c}
+    x = syn.hidden_states(T, H, dev, seed=seed)
+    if c["path"] == "router":
+        st["x"] = x
+        st["w"] = _bf16(_gen(seed, 1), (H, E), H ** -0.5)
+        return st
+    st["ids"], aff = syn.route(T, E, k, dev, seed=seed, mode="softmax" if c["skew"] else "sigmoid", expert_bias_std=c["skew"])
+    padded = not (c["skip_token"] or c["path"] == "tkg")  # tables with the padding token's row
+    st["x"] = x if padded else x[:T].contiguous()
+    st["aff"] = aff if padded else aff[:T].contiguous()
+    st["gamma"] = torch.ones((1, H), dtype=torch.bfloat16, device=dev)
+    kind = c["kind"]
+    st["gu_s"] = st["d_s"] = None
+    if kind == "mxfp8":
+        st["gu"], st["gu_s"], st["d"], st["d_s"] = syn.mx_expert_weights(E, H, I, 0.02, dev, seed=seed)
+    elif kind == "mxfp4":
+        st["gu"], st["gu_s"], st["d"], st["d_s"] = syn.mx4_expert_weights(E, H, I, dev, seed=seed)
+        if I > 512 and I % 512:
+            st["d"][:, I % 512 // 4:, I // 512] = 0  # the padding of a short last intermediate tile
+    elif kind == "bf16":
+        st["gu"] = _bf16(_gen(seed, 2), (E, H, 2, I), 0.02)
+        st["d"] = _bf16(_gen(seed, 3), (E, I, H), 0.02)
+    else:
+        gu, st["gu_s"], d, st["d_s"] = syn.fp8_channel_weights(E, H, I, 0.02, dev, seed=seed)
+        st["gu"], st["d"] = gu.view(torch.float8_e4m3fn), d.view(torch.float8_e4m3fn)
+        if c["path"] == "tkg":  # decode takes the same scales as [E, 2, I] and [E, H]
+            st["gu_s"], st["d_s"] = st["gu_s"].view(E, 2, I), st["d_s"].view(E, H)
+    st["gu_b"] = st["d_b"] = None
+    if c["bias"]:
+        if kind.startswith("mx"):
+            shape = (E, 128 if I > 512 else I // 4, 2, math.ceil(I / 512), 4)
+        else:
+            shape = (E, 2, I)
+        st["gu_b"] = _bf16(_gen(seed, 4), shape, 0.5)
+        st["d_b"] = _bf16(_gen(seed, 5), (E, H), 0.5)
+    st["N"] = get_n_blocks(T, k, E, c["B"])
+    return st
+
+
+def run(state):
+    """One pass; the outputs are what the entry points return."""
+    c = state["case"]
+    if c["path"] == "router":
+        return route_for_moe(state["x"], state["w"], None, c["k"], RouterActFnType.SIGMOID, norm_topk_prob=True)
+    clamps = _CLAMPS if c["clamps"] else {}
+    if c["path"] == "tkg":
+        return moe_tkg(state["x"], state["gu"], state["d"], state["aff"], state["ids"], False,
+                       expert_gate_up_bias=state["gu_b"], expert_down_bias=state["d_b"],
+                       expert_gate_up_weights_scale=state["gu_s"], expert_down_weights_scale=state["d_s"],
+                       expert_affinities_scaling_mode=ExpertAffinityScaleMode.POST_SCALE, activation_fn=_ACT[c["act"]],
+                       **clamps)
+    x, kw = state["x"], dict(clamps)
+    if c["kind"] == "mxfp8":
+        x, kw["hidden_states_scale"] = rmsnorm_mx_quantize(x, state["gamma"])
+    elif c["kind"] == "fp8row":
+        x = rmsnorm_quant_kernel(x, state["gamma"], RmsNormQuantKernelArgs())
+    if state["gu_s"] is not None:
+        kw["quantization_config"] = QuantizationConfig(state["gu_s"], state["d_s"])
+    tp2id, b2e, _ = build_token_blocks(state["ids"], c["E"], c["B"], state["N"], skip_token=c["skip_token"])
+    if c["kind"].startswith("mx"):
+        spec = MoECTESpec(implementation=MoECTEImplementation.shard_on_block_mx)
+    elif c["ckpt"]:
+        spec = MoECTESpec(implementation=MoECTEImplementation.shard_on_i,
+                          shard_on_I=ShardOnIConfig(checkpoint_activation=True, expert_affinity_multiply_on_I=False))
+    else:
+        spec = MoECTESpec(implementation=MoECTEImplementation.shard_on_block)
+    return moe_cte(x, state["aff"].reshape(-1, 1), state["gu"], state["d"], tp2id, b2e, c["B"], spec,
+                   gate_and_up_proj_bias=state["gu_b"], down_proj_bias=state["d_b"], activation_function=_ACT[c["act"]],
+                   skip_dma=SkipMode(c["skip_token"], False), **kw)
+
+
+def work(case):
+    """The experts that at least one token is routed to (their expected number, routing taken as uniform), hidden
+    states and affinities in; one row per token, and the activations that are kept, out."""
+    c = dict(_DEFAULTS, **case)
+    T, H, I, E, k = c["T"], c["H"], c["I"], c["E"], c["k"]
+    if c["path"] == "router":
+        return {"bytes": 2.0 * T * H + 2.0 * H * E + 4.0 * T * k + 2.0 * T * E, "flops": 2.0 * T * H * E}
+    hit = 1.0 - (1.0 - k / E) ** T
+    # (decode and the plain variants return [T, H], the prefill variants a second plane of zeros beside it)
+    planes = 1 if c["path"] == "tkg" or c["ckpt"] else 2
+    byts = _weight_bytes(c) * hit + 2.0 * T * H + 2.0 * T * k + 4.0 * T * k + 2.0 * planes * T * H
+    if c["ckpt"]:
+        byts += _slots(c) * (2 * I + H) * 2.0
+    return {"bytes": byts, "flops": 6.0 * T * k * H * I}
+
+
+def tolerance(case):
+    # Another order of the sums moves results by roundings of bf16 (contributions and outputs are bf16) and, for the
+    # quantised kinds, by steps of a few re-quantised intermediate values.  Against the same computation with its sums
+    # in another order: 0.003 .. 0.0044 (bf16), 0.002 (MX), 0.0017 (router affinities, against 64 bits).
+    if case["path"] == "router":
+        return {"rel": 7e-3, "differ": 2e-4}  # (two experts whose logits tie within the rounding of the sums may swap)
+    return {"rel": 8e-3} if case["kind"].startswith("mx") else {"rel": 1e-2}
