@@ -15,7 +15,7 @@ import sys
 
 import torch
 
-_PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nki-library_amd")
+_PKG = os.path.abspath("nki-library_amd")  # (run from the repository's root)
 if _PKG not in sys.path:
     sys.path.insert(0, _PKG)
 
