@@ -18,7 +18,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ_DIR = os.path.join(HERE, "build")
 OUT_DIR = os.path.join(HERE, "nkilib", "_lib")
 OUT = os.path.join(OUT_DIR, "libmoe_gfx950.so")
-SOURCES = ["rmsnorm_quant.hip", "build_blocks.hip", "combine.hip", "bwmm.hip", "bwmm_mx.hip", "router_topk.hip", "index_ops.hip", "capi.hip"]
+SOURCES = ["rmsnorm_quant.hip", "build_blocks.hip", "combine.hip", "bwmm.hip", "bwmm_mx.hip", "bwmm_rows.hip", "router_topk.hip", "index_ops.hip", "capi.hip"]
 # (stage, weight format) instances of the large-tile MX GEMM; formats as MX_WFMT_* in csrc/bwmm.hpp
 MX_INSTANCES = [(1, 0), (2, 0), (1, 1), (2, 1), (1, 2), (2, 2), (1, 3), (2, 3), (1, 4), (2, 4)]
 FLAGS = [
@@ -33,7 +33,7 @@ FLAGS = [
 # csrc/router_topk.hip) draw one inline-asm diagnostic per such load, thousands of times; every other translation
 # unit keeps the diagnostic on
 MX_FLAGS = ["-Wno-inline-asm"]
-M0_CLOBBER_SOURCES = ("bwmm_mx.hip", "router_topk.hip")
+M0_CLOBBER_SOURCES = ("bwmm_mx.hip", "bwmm_rows.hip", "router_topk.hip")
 NOISE = "is not a recognized feature for this target"
 
 

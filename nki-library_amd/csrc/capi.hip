@@ -304,10 +304,10 @@ extern "C" int moe_prepare_kmajor_weights(const moe_bwmm_args* a, void* gate_up_
     if (!mx_packable(a, 0)) return MOE_E_UNSUPPORTED;
     const int fp4 = a->weight_dtype == MOE_DT_FP4_E2M1;
     if (!gate_up_kmajor || (((uintptr_t)gate_up_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
-    rc = launch_mx_pack_weights(1, fp4, a->gate_up_proj_weight, gate_up_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
+    rc = launch_mx_pack_weights(1, fp4, a->gate_up_proj_weight, a->gate_up_proj_scale, gate_up_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
     if (rc != MOE_OK || !mx_packable(a, 1)) return rc;
     if (!down_kmajor || (((uintptr_t)down_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
-    return launch_mx_pack_weights(2, fp4, a->down_proj_weight, down_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
+    return launch_mx_pack_weights(2, fp4, a->down_proj_weight, a->down_proj_scale, down_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
   }
   if (!gate_up_kmajor || !down_kmajor) return MOE_E_BAD_ARG;
   if ((((uintptr_t)gate_up_kmajor) & 255) != 0 || (((uintptr_t)down_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
@@ -490,6 +490,14 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
     }
   }
   const unsigned gyc = (unsigned)bk.max_chunks;
+  // few rows per expert: the kernel of bwmm_rows.hip (a table lists a token at most once per expert, so a chunk holds at
+  // most n_real rows; a table of N blocks is made for about (N - (E - 1)) * B routed rows); the activation checkpoints
+  // are written by the large-tile kernels' epilogues
+  const int64_t avg_rows = a->N > a->E - 1 ? (a->N - (a->E - 1)) * a->B / a->E : 0;
+  auto few_rows = [&](int stage, unsigned gx) {
+    return !a->gate_up_activations_T && !a->down_activations &&
+           mx_rows_fits(stage, m.wfmt, n_real, avg_rows, (int64_t)gx * bk.max_chunks);
+  };
   mark(2);
   // checkpoints of blocks that never run stay zero
   if (a->gate_up_activations_T && (stages & MOE_STAGE_GATE_UP)) {
@@ -509,6 +517,7 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m1.bias = a->gate_and_up_proj_bias;
       if (mx_packable(a, 0) && a->gate_up_proj_weight_kmajor) {
         m1.W = (const uint32_t*)a->gate_up_proj_weight_kmajor;
+        m1.W_scale = (const uint8_t*)m1.W + mx_packed_scales_offset(1, m1.wfmt == MX_WFMT_E2M1, a->E, a->H, a->I);
         m1.w_packed = 1;
       }
       if (r8_fast) {
@@ -526,7 +535,8 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m1.clk = a->gemm_clocks;
 
       // column tiles of 32 partitions x 4 q, gate and up: 4 per full intermediate tile + those of a short last one
-      rc = launch_mx_gemm(1, m1, (unsigned)((a->I / 512) * 4 + (a->I % 512) / 128), gyc, s);
+      const unsigned gx = (unsigned)((m1.I / 512) * 4 + (m1.I % 512) / 128);
+      rc = few_rows(1, gx) ? launch_mx_rows(1, m1, gx, bk.max_chunks, n_real, s) : launch_mx_gemm(1, m1, gx, gyc, s);
     } else {
       rc = launch_gemm_stage(a->kind, 1, g1, gx1, gy, s);
     }
@@ -547,6 +557,7 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m2.bias = a->down_proj_bias;
       if (mx_packable(a, 1) && a->down_proj_weight_kmajor) {
         m2.W = (const uint32_t*)a->down_proj_weight_kmajor;
+        m2.W_scale = (const uint8_t*)m2.W + mx_packed_scales_offset(2, m2.wfmt == MX_WFMT_E2M1, a->E, a->H, a->I);
         m2.w_packed = 1;
       }
       if (r8_fast) {
@@ -566,7 +577,8 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       }
       m2.clk = a->gemm_clocks ? a->gemm_clocks + 2 : nullptr;
 
-      rc = launch_mx_gemm(2, m2, (unsigned)(a->H / 256), gyc, s);
+      const unsigned gx = (unsigned)(a->H / 256);
+      rc = few_rows(2, gx) ? launch_mx_rows(2, m2, gx, bk.max_chunks, n_real, s) : launch_mx_gemm(2, m2, gx, gyc, s);
     } else {
       rc = launch_gemm_stage(a->kind, 2, g2, gx2, gy, s);
     }

@@ -58,23 +58,25 @@ def clear_kmajor_weight_cache():
 
 
 def _bytes_of(t):
-    """Where a weight tensor's bytes are: (address of its storage, byte offset, byte length).  Views and casts of one
-    allocation (``w.view(torch.int32)`` made anew for every call, say) name the same bytes."""
-    return (t.untyped_storage().data_ptr(), t.storage_offset() * t.element_size(), t.numel() * t.element_size())
+    """Where a weight tensor's bytes are: (address of its storage, byte offset, byte length; the strides of a tensor that
+    is not contiguous).  Views and casts of one allocation (``w.view(torch.int32)`` made anew for every call, say) name
+    the same bytes."""
+    return (t.untyped_storage().data_ptr(), t.storage_offset() * t.element_size(), t.numel() * t.element_size(),
+            None if t.is_contiguous() else t.stride())
 
 
-def _kmajor_weights(L, a, guw, dw, dev):
-    """``guw`` / ``dw``: the weight tensors as the caller of the operator passed them.  An entry is found through the
-    bytes the tensors name and how the call reads them (kind, weight type, expert shape), so a fresh view of the same
-    allocation hits; it is valid while both allocations are alive (weak references to the storages: an address that
-    was freed and handed out again is a different storage) and unchanged (torch's version counters, which views
-    share with their base)."""
-    st0, st1 = guw.untyped_storage(), dw.untyped_storage()
-    key = (_bytes_of(guw), _bytes_of(dw), int(a.kind), int(a.weight_dtype), int(a.E), int(a.H), int(a.I), int(a.I_pad))
-    sig = (guw._version, dw._version)
+def _kmajor_weights(L, a, tensors, dev):
+    """``tensors``: what the copies are made of, as the caller of the operator passed it (the gate/up and down weights;
+    the MX formats' copies hold the block scales as well).  An entry is found through the bytes the tensors name and how
+    the call reads them (kind, weight type, expert shape), so a fresh view of the same allocation hits; it is valid while
+    all the allocations are alive (weak references to the storages: an address that was freed and handed out again is a
+    different storage) and unchanged (torch's version counters, which views share with their base)."""
+    storages = [t.untyped_storage() for t in tensors]
+    key = (*map(_bytes_of, tensors), int(a.kind), int(a.weight_dtype), int(a.E), int(a.H), int(a.I), int(a.I_pad))
+    sig = tuple(t._version for t in tensors)
     ent = _kmajor.get(key)
-    if ent is not None and ent[0]() is st0 and ent[1]() is st1 and ent[2] == sig:
-        return ent[3], ent[4]
+    if ent is not None and ent[1] == sig and all(r() is st for r, st in zip(ent[0], storages)):
+        return ent[3], ent[2]
     n0 = L.moe_kmajor_weights_bytes(ctypes.byref(a), 0)
     n1 = L.moe_kmajor_weights_bytes(ctypes.byref(a), 1)
     if n0 == 0:
@@ -87,7 +89,7 @@ def _kmajor_weights(L, a, guw, dw, dev):
     if len(_kmajor) >= _KMAJOR_MAX_ENTRIES:
         _kmajor.pop(next(iter(_kmajor)))
     drop = lambda _ref, key=key: _kmajor.pop(key, None)
-    _kmajor[key] = (weakref.ref(st0, drop), weakref.ref(st1, drop), sig, k0, k1)
+    _kmajor[key] = ([weakref.ref(st, drop) for st in storages], sig, k1, k0)
     return k0, k1
 
 
@@ -239,7 +241,7 @@ def run_blockwise(
     if (kmajor_weight_cache and kind in (nv.KIND_BF16, nv.KIND_FP8_ROW)) or (mx_weight_copies and kind == nv.KIND_MXFP8):
         # (weight_objects: the caller's own tensor objects where the operator had to make views of them)
         wo = weight_objects or (gate_up_proj_weight, down_proj_weight)
-        kmajor = _kmajor_weights(L, a, wo[0], wo[1], dev)
+        kmajor = _kmajor_weights(L, a, wo, dev)
         a.gate_up_proj_weight_kmajor = nv.ptr(kmajor[0])
         a.down_proj_weight_kmajor = nv.ptr(kmajor[1])
 

@@ -1,0 +1,102 @@
+"""GPU parity of the few-rows expert kernel (csrc/bwmm_rows.hip) against the oracle at the edges of its instances: one,
+two and four row tiles (16 / 17, 32 / 33, 64 / 65 tokens), passes over more rows than an instance multiplies, K loops
+shorter than the waves that split them, short last intermediate tiles, both column groupings (few and many 64-column
+groups), every weight format and the options of the epilogues.  Tolerances are those of test_gpu_moe.py."""
+
+import numpy as np
+import pytest
+
+from helpers import dense_case, from_bf16_tensor, mx_case
+from oracle import moe as omoe
+from test_gpu_moe import (REF_MX_CLAMPS, _check, _golden_dense, _golden_mx_options, _run_dense, _run_fp8_row,
+                          _run_mx_options)
+
+pytestmark = pytest.mark.gpu
+
+CL = dict(gate_clamp_upper_limit=0.8, gate_clamp_lower_limit=-0.7, up_clamp_upper_limit=0.9, up_clamp_lower_limit=-0.5)
+
+
+@pytest.mark.parametrize("T,H,I,E,k,act,mode,bias,skip,fp8w", [
+    (1, 256, 128, 4, 2, 0, 1, False, False, False),     # four K slices for four waves; one slice each in the down stage
+    (16, 512, 384, 8, 2, 0, 1, True, True, False),      # one full row tile; a short last intermediate tile (768 bytes of K)
+    (17, 512, 128, 4, 4, 3, 2, True, False, False),     # two row tiles; Swish, PRE_SCALE; two K slices for four waves
+    (33, 2560, 1152, 16, 4, 0, 1, False, False, True),  # four row tiles; 128-column workgroups in both stages; fp8 weights
+    (64, 512, 256, 3, 2, 1, 0, True, True, False),      # GELU, NO_SCALE
+    (65, 512, 128, 8, 2, 0, 1, False, False, False),    # more tokens than a pass has rows
+    (256, 512, 256, 8, 2, 2, 1, True, False, False),    # experts of more than 64 rows: a second pass
+])
+def test_rows_dense(T, H, I, E, k, act, mode, bias, skip, fp8w):
+    c = dense_case(T, H, I, E, k, 128, seed=31, skip_token=skip, bias=bias, quant=fp8w, hidden_std=1.0)
+    o = from_bf16_tensor(_run_dense(c, act=act, mode=mode, clamps=CL, fp8_weights=fp8w))[:, 0]
+    g = _golden_dense(c, act=act, mode=mode, clamps=CL, fp8_weights=fp8w)
+    _check(o[:T], g[:T], f"few rows bf16 T={T} H={H} I={I}")
+
+
+@pytest.mark.parametrize("T,H,I,E,k,mode", [(5, 512, 512, 4, 2, 2), (24, 2560, 1152, 16, 2, 1), (50, 512, 640, 2, 2, 1)])
+def test_rows_fp8_row(T, H, I, E, k, mode):
+    c = dense_case(T, H, I, E, k, 128, seed=32, quant=True, bias=True, hidden_std=1.0)
+    rec, out = _run_fp8_row(c, np.ones((1, H), np.float32), mode=mode, clamps=CL, act=3)
+    import torch
+
+    raw = rec.view(torch.uint8).cpu().numpy()
+    g = omoe.moe_blockwise_fp8_row_ref(raw[:, :H], raw[:, H:].copy().view(np.float32).reshape(-1), c["aff"], c["gate_up_q"],
+                                       c["down_q"], c["gate_up_scale"], c["down_scale"], c["tp2id"], c["b2e"], c["B"],
+                                       gate_up_proj_bias=c["gate_up_bias"], down_proj_bias=c["down_bias"],
+                                       activation_function=3, expert_affinities_scaling_mode=mode, **CL)
+    _check(from_bf16_tensor(out)[:T, 0], g[:T], f"few rows fp8 row T={T}")
+
+
+@pytest.mark.parametrize("T,H,I,E,k,fmt,skip", [
+    (1, 512, 128, 8, 4, "e4m3", False),
+    (16, 1024, 640, 4, 2, "e4m3", True),     # a short last intermediate tile
+    (17, 512, 512, 2, 2, "e4m3", False),
+    (32, 2560, 1152, 16, 4, "e5m2", False),  # 128-column workgroups in the down stage
+    (8, 512, 384, 4, 2, "e2m1", True),       # 4-bit weights: both stages
+    (60, 1024, 512, 2, 2, "e2m1", False),    # ... the down stage alone, four row tiles
+])
+@pytest.mark.parametrize("copies", [True, False])
+def test_rows_mx(T, H, I, E, k, fmt, skip, copies):
+    """With the weights' copies in read order and from the reference layout in place."""
+    from nkilib.core.moe.moe_cte import _launch
+
+    c = mx_case(T, H, I, E, k, 128, seed=33, skip_token=skip, bias=True, weight_format=fmt, random_codes=True)
+    was = _launch.mx_weight_copies
+    try:
+        _launch.mx_weight_copies = copies
+        o = from_bf16_tensor(_run_mx_options(c, 3, REF_MX_CLAMPS, False))
+    finally:
+        _launch.mx_weight_copies = was
+    _check(o[0, :T], _golden_mx_options(c, 3, REF_MX_CLAMPS)[:T], f"few rows mx {fmt} T={T} H={H} I={I} copies={copies}")
+
+
+def test_mx_copies_follow_the_block_scales():
+    """The kept copy of MX gate/up weights holds their block scales: a scale changed in place, or another scale tensor with
+    the same weights, must reach the result."""
+    import torch
+    from nkilib import synthetic as syn
+    from nkilib.core.moe.moe_cte import _launch
+    from nkilib.core.moe.moe_tkg import moe_tkg
+    from nkilib.core.utils.common_types import ExpertAffinityScaleMode
+
+    dev = torch.device("cuda:0")
+    T, H, I, E, k = 4, 512, 256, 4, 2
+    gu, gs, d, ds = syn.mx_expert_weights(E, H, I, 0.05, dev, seed=5)
+    ids, aff = syn.route(T, E, k, dev, seed=5)
+    x = syn.hidden_states(T, H, dev, seed=5)[:T].contiguous()
+
+    def layer(scale):
+        return moe_tkg(x, gu, d, aff[:T].contiguous(), ids, False, expert_gate_up_weights_scale=scale,
+                       expert_down_weights_scale=ds, expert_affinities_scaling_mode=ExpertAffinityScaleMode.POST_SCALE)
+
+    def plain(scale):
+        _launch.mx_weight_copies = False
+        try:
+            return layer(scale)
+        finally:
+            _launch.mx_weight_copies = True
+
+    assert torch.equal(layer(gs), plain(gs))
+    other = gs + 1
+    assert torch.equal(layer(other), plain(other)) and not torch.equal(layer(other), layer(gs))
+    gs.add_(1)
+    assert torch.equal(layer(gs), layer(other))
