@@ -279,7 +279,7 @@ typedef struct moe_bwmm_args {
   /* Optional K-contiguous copies of the bf16 / fp8 weights of the BF16 and FP8_ROW kinds, made once by
    * moe_prepare_kmajor_weights (they depend on the weights only).  Both NULL: every call makes its own copies
    * in the workspace.  (What a copy holds depends on the kind, the weight type and the shape only -- for bf16
-   * weights with H % 256 == 0 and I % 128 == 0, and fp8-row weights with H % 512 == 0 and I % 128 == 0, the order
+   * weights with H % 256 == 0, and fp8-row weights with H % 512 == 0, the order
    * the large-tile kernels read, otherwise K-contiguous rows -- so one pair serves every call with those weights;
    * a bf16 call on such a shape that asks for activation checkpoints runs the general kernel and makes its own
    * K-contiguous copies regardless.)  MXFP8 kind: the x4 layouts are K-major already and are read in place when both are NULL;

@@ -5,7 +5,8 @@
 //            per-channel weight scales applied to the fp32 accumulators
 //   MXFP8    v_mfma_scale_f32_16x16x128_f8f6f4, E8M0 block scales of both operands applied by
 //            the matrix core
-// This file holds the general tiled kernel: a 256-thread workgroup owns 128 rows of one block
+// This file holds the general tiled kernel, for the shapes the large-tile kernels (bwmm_mx.hip) do not take (H % 256,
+// % 512 for the fp8 kinds; I % 128 for MXFP8): a 256-thread workgroup owns 128 rows of one block
 // (one expert) and 128 output columns (256 in stage 1: gate and up), stages one 128-byte
 // K-slice of both operands in LDS in K-contiguous order and lets each of the four waves run
 // 2 x (8|16) MFMA tiles over it.  Rows are gathered through token_position_to_id while the A
@@ -532,15 +533,15 @@ __global__ __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(KIND == MOE_
 __global__ __launch_bounds__(256) void row_requant_kernel(const float* __restrict__ Y, uint8_t* __restrict__ Yq,
                                                           float* __restrict__ ys, const int32_t* __restrict__ n_active,
                                                           const int32_t* __restrict__ valid_rows, int64_t B, int64_t I,
-                                                          int64_t Iw) {
+                                                          int64_t y_stride, int64_t Iw) {
   __shared__ float red[16];
   const int64_t slot = blockIdx.x;
   const int64_t b = slot / B, r = slot % B;
   if (b >= *n_active || r >= valid_rows[b]) return;
-  const float* y = Y + slot * I;
+  const float* y = Y + slot * y_stride;
   uint8_t* q = Yq + slot * Iw;
   constexpr int MAXV = 16;  // float4 per thread kept in registers: rows of up to 16384 values are read once
-  if (I % 4 == 0 && I <= (int64_t)MAXV * 4 * 256) {
+  if (I % 4 == 0 && y_stride % 4 == 0 && I <= (int64_t)MAXV * 4 * 256) {
     float4 v[MAXV];
     float am = 0.f;
 #pragma unroll
@@ -692,7 +693,7 @@ int launch_transpose_fp8(const uint8_t* src, uint8_t* dst, int64_t R, int64_t C,
 }
 
 // One thread per four adjacent output columns: four 4-byte reads (the four K rows of the x4 elements), a 4 x 4 byte
-// transpose, one 16-byte write.  I % 4 == 0 and H % 4 == 0 on this path.
+// transpose, one 16-byte write.
 __device__ __forceinline__ uint4 bytes_4x4_transposed(const uint32_t (&r)[4]) {
   uint32_t o[4];
 #pragma unroll
@@ -701,22 +702,33 @@ __device__ __forceinline__ uint4 bytes_4x4_transposed(const uint32_t (&r)[4]) {
            (((r[3] >> (8 * c)) & 0xffu) << 24);
   return make_uint4(o[0], o[1], o[2], o[3]);
 }
+// Four neighbouring bytes; byte by byte where fewer than four exist (n < 4: zeros behind them) or the matrix or its rows
+// are not 4-byte aligned.
+__device__ __forceinline__ uint32_t four_bytes(const uint8_t* p, int64_t n, bool aligned) {
+  if (aligned && n >= 4) return *(const uint32_t*)p;
+  uint32_t v = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if (k < n) v |= (uint32_t)p[k] << (8 * k);
+  return v;
+}
+// Ic >= I, a multiple of 128: columns of the copy; those from I on are zero.
 __global__ __launch_bounds__(256) void relayout_gu_x4_kernel(const uint8_t* __restrict__ W, uint32_t* __restrict__ X,
-                                                             int64_t H, int64_t I, int64_t total4) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, 128, 2, nH, I / 4]
+                                                             int64_t H, int64_t I, int64_t Ic, bool aligned, int64_t total4) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, 128, 2, nH, Ic / 4]
   if (idx >= total4) return;
-  const int64_t nH = H / 512, I4 = I / 4;
+  const int64_t nH = H / 512, I4 = Ic / 4;
   const int64_t i = (idx % I4) * 4, t = (idx / I4) % nH, gu = (idx / (I4 * nH)) % 2, p = (idx / (I4 * nH * 2)) % 128,
                 e = idx / (I4 * nH * 2 * 128);
   const int64_t h = t * 512 + p * 4;
   uint32_t r[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) r[q] = *(const uint32_t*)(W + ((e * H + h + q) * 2 + gu) * I + i);
+  for (int q = 0; q < 4; ++q) r[q] = four_bytes(W + ((e * H + h + q) * 2 + gu) * I + i, I - i, aligned);
   *(uint4*)(X + idx * 4) = bytes_4x4_transposed(r);
 }
 __global__ __launch_bounds__(256) void relayout_down_x4_kernel(const uint8_t* __restrict__ W, uint32_t* __restrict__ X,
                                                                int64_t H, int64_t I, int64_t I_pad, int64_t pI,
-                                                               int64_t nI, int64_t total4) {
+                                                               int64_t nI, bool aligned, int64_t total4) {
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, pI, nI, H / 4]
   if (idx >= total4) return;
   const int64_t H4 = H / 4;
@@ -724,7 +736,7 @@ __global__ __launch_bounds__(256) void relayout_down_x4_kernel(const uint8_t* __
   const int64_t i0 = t * 512 + p * 4;
   uint32_t r[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) r[q] = (i0 + q < I) ? *(const uint32_t*)(W + (e * I_pad + i0 + q) * H + h) : 0u;
+  for (int q = 0; q < 4; ++q) r[q] = (i0 + q < I) ? four_bytes(W + (e * I_pad + i0 + q) * H + h, 4, aligned) : 0u;
   *(uint4*)(X + idx * 4) = bytes_4x4_transposed(r);
 }
 __global__ __launch_bounds__(256) void fill_bytes_kernel(uint32_t* __restrict__ p, int64_t words, uint32_t v) {
@@ -744,19 +756,18 @@ int launch_fill_bytes(void* p, size_t bytes, uint8_t value, hipStream_t s) {
 
 int launch_relayout_x4(const uint8_t* gate_up, const uint8_t* down, uint8_t* dst, int which, int64_t E, int64_t H,
                        int64_t I, int64_t I_pad, hipStream_t s) {
-  if ((((uintptr_t)dst) & 15) != 0 || (((uintptr_t)gate_up) & 3) != 0 || (((uintptr_t)down) & 3) != 0)
-    return MOE_E_BAD_ARG;
+  if ((((uintptr_t)dst) & 15) != 0) return MOE_E_BAD_ARG;
   if (which == 0) {
-    const int64_t total = E * 128 * 2 * (H / 512) * (I / 4);
+    const int64_t Ic = dense_cols(I), total = E * 128 * 2 * (H / 512) * (Ic / 4);
     if ((total + 255) / 256 >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
     hipLaunchKernelGGL(relayout_gu_x4_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, gate_up,
-                       (uint32_t*)dst, H, I, total);
+                       (uint32_t*)dst, H, I, Ic, I % 4 == 0 && ((uintptr_t)gate_up & 3) == 0, total);
   } else {
-    const int64_t nI = (I + 511) / 512, pI = I > 512 ? 128 : I / 4;
+    const int64_t Kb = dense_k_bytes(I, false), nI = (Kb + 511) / 512, pI = Kb > 512 ? 128 : Kb / 4;
     const int64_t total = E * pI * nI * (H / 4);
     if ((total + 255) / 256 >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
     hipLaunchKernelGGL(relayout_down_x4_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, down,
-                       (uint32_t*)dst, H, I, I_pad, pI, nI, total);
+                       (uint32_t*)dst, H, I, I_pad, pI, nI, ((uintptr_t)down & 3) == 0, total);
   }
   MOE_CHECK_LAUNCH();
   return MOE_OK;
@@ -764,16 +775,22 @@ int launch_relayout_x4(const uint8_t* gate_up, const uint8_t* down, uint8_t* dst
 
 // bf16 weights (W8: fp8-e4m3 weights widened to bf16 on the way, exactly): one thread per four adjacent output
 // columns, two 8-byte (4-byte) reads (the two K rows of the x4 elements), one 16-byte write.
+// (n < 4 elements exist, zeros behind them; aligned: rows and matrix are aligned to four elements)
 template <bool W8>
-__device__ __forceinline__ uint2 four_as_bf16(const void* W, int64_t elem) {
+__device__ __forceinline__ uint2 four_as_bf16(const void* W, int64_t elem, int64_t n, bool aligned) {
   if constexpr (W8) {
-    const uint32_t raw = *(const uint32_t*)((const uint8_t*)W + elem);
+    const uint32_t raw = four_bytes((const uint8_t*)W + elem, n, aligned);
     uint32_t v[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) v[q] = f32_to_bf16_bits(e4m3_to_f32((raw >> (8 * q)) & 0xffu));
     return make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
   } else {
-    return *(const uint2*)((const uint16_t*)W + elem);
+    const uint16_t* p = (const uint16_t*)W + elem;
+    if (aligned && n >= 4) return *(const uint2*)p;
+    uint32_t v[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = (q < n) ? p[q] : 0u;
+    return make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
   }
 }
 __device__ __forceinline__ uint4 pairs_of_4(const uint2& r0, const uint2& r1) {
@@ -782,57 +799,57 @@ __device__ __forceinline__ uint4 pairs_of_4(const uint2& r0, const uint2& r1) {
 }
 template <bool W8>
 __global__ __launch_bounds__(256) void relayout_gu_x4_bf16_kernel(const void* __restrict__ W, uint32_t* __restrict__ X,
-                                                                  int64_t H, int64_t I, int64_t total4) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, 128, 2, 2H / 512, I / 4]
+                                                                  int64_t H, int64_t I, int64_t Ic, bool aligned,
+                                                                  int64_t total4) {
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, 128, 2, 2H / 512, Ic / 4]
   if (idx >= total4) return;
-  const int64_t nH = H / 256, I4 = I / 4;
+  const int64_t nH = H / 256, I4 = Ic / 4;
   const int64_t i = (idx % I4) * 4, t = (idx / I4) % nH, gu = (idx / (I4 * nH)) % 2, p = (idx / (I4 * nH * 2)) % 128,
                 e = idx / (I4 * nH * 2 * 128);
   const int64_t h = t * 256 + p * 2;
-  const uint2 r0 = four_as_bf16<W8>(W, ((e * H + h) * 2 + gu) * I + i);
-  const uint2 r1 = four_as_bf16<W8>(W, ((e * H + h + 1) * 2 + gu) * I + i);
+  const uint2 r0 = four_as_bf16<W8>(W, ((e * H + h) * 2 + gu) * I + i, I - i, aligned);
+  const uint2 r1 = four_as_bf16<W8>(W, ((e * H + h + 1) * 2 + gu) * I + i, I - i, aligned);
   *(uint4*)(X + idx * 4) = pairs_of_4(r0, r1);
 }
 template <bool W8>
 __global__ __launch_bounds__(256) void relayout_down_x4_bf16_kernel(const void* __restrict__ W,
                                                                     uint32_t* __restrict__ X, int64_t H, int64_t I,
-                                                                    int64_t I_pad, int64_t pI, int64_t nI,
+                                                                    int64_t I_pad, int64_t pI, int64_t nI, bool aligned,
                                                                     int64_t total4) {
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, pI, nI, H / 4], pI and nI those of 2I bytes
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;  // over [E, pI, nI, H / 4], pI and nI those of the K bytes
   if (idx >= total4) return;
   const int64_t H4 = H / 4;
   const int64_t h = (idx % H4) * 4, t = (idx / H4) % nI, p = (idx / (H4 * nI)) % pI, e = idx / (H4 * nI * pI);
   const int64_t i0 = t * 256 + p * 2;
   const uint2 zero = make_uint2(0u, 0u);
-  const uint2 r0 = (i0 < I) ? four_as_bf16<W8>(W, (e * I_pad + i0) * H + h) : zero;
-  const uint2 r1 = (i0 + 1 < I) ? four_as_bf16<W8>(W, (e * I_pad + i0 + 1) * H + h) : zero;
+  const uint2 r0 = (i0 < I) ? four_as_bf16<W8>(W, (e * I_pad + i0) * H + h, 4, aligned) : zero;
+  const uint2 r1 = (i0 + 1 < I) ? four_as_bf16<W8>(W, (e * I_pad + i0 + 1) * H + h, 4, aligned) : zero;
   *(uint4*)(X + idx * 4) = pairs_of_4(r0, r1);
 }
 int launch_relayout_x4_bf16(const void* gate_up, const void* down, int w8, uint8_t* dst, int which, int64_t E, int64_t H,
                             int64_t I, int64_t I_pad, hipStream_t s) {
   const uintptr_t src_align = w8 ? 3 : 7;
-  if ((((uintptr_t)dst) & 15) != 0 || (((uintptr_t)gate_up) & src_align) != 0 || (((uintptr_t)down) & src_align) != 0 ||
-      H % 256 != 0 || I % 4 != 0)
-    return MOE_E_BAD_ARG;
+  if ((((uintptr_t)dst) & 15) != 0 || H % 256 != 0) return MOE_E_BAD_ARG;
+  const bool aligned = which == 0 ? I % 4 == 0 && ((uintptr_t)gate_up & src_align) == 0 : ((uintptr_t)down & src_align) == 0;
   if (which == 0) {
-    const int64_t total = E * 128 * 2 * (H / 256) * (I / 4);
+    const int64_t Ic = dense_cols(I), total = E * 128 * 2 * (H / 256) * (Ic / 4);
     if ((total + 255) / 256 >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
     if (w8)
       hipLaunchKernelGGL(relayout_gu_x4_bf16_kernel<true>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, gate_up,
-                         (uint32_t*)dst, H, I, total);
+                         (uint32_t*)dst, H, I, Ic, aligned, total);
     else
       hipLaunchKernelGGL(relayout_gu_x4_bf16_kernel<false>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, gate_up,
-                         (uint32_t*)dst, H, I, total);
+                         (uint32_t*)dst, H, I, Ic, aligned, total);
   } else {
-    const int64_t Ib = 2 * I, nI = (Ib + 511) / 512, pI = Ib > 512 ? 128 : Ib / 4;
+    const int64_t Ib = dense_k_bytes(I, true), nI = (Ib + 511) / 512, pI = Ib > 512 ? 128 : Ib / 4;
     const int64_t total = E * pI * nI * (H / 4);
     if ((total + 255) / 256 >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
     if (w8)
       hipLaunchKernelGGL(relayout_down_x4_bf16_kernel<true>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, down,
-                         (uint32_t*)dst, H, I, I_pad, pI, nI, total);
+                         (uint32_t*)dst, H, I, I_pad, pI, nI, aligned, total);
     else
       hipLaunchKernelGGL(relayout_down_x4_bf16_kernel<false>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, down,
-                         (uint32_t*)dst, H, I, I_pad, pI, nI, total);
+                         (uint32_t*)dst, H, I, I_pad, pI, nI, aligned, total);
   }
   MOE_CHECK_LAUNCH();
   return MOE_OK;
@@ -854,9 +871,9 @@ int launch_gemm_stage(int kind, int stage, const GemmArgs& g, unsigned gx, unsig
 }
 
 int launch_row_requant(const float* Y, uint8_t* Yq, float* ys, const Bookkeeping& k, int64_t N, int64_t B, int64_t I,
-                       int64_t Iw, hipStream_t s) {
+                       int64_t y_stride, int64_t Iw, hipStream_t s) {
   hipLaunchKernelGGL(row_requant_kernel, dim3((unsigned)(N * B)), dim3(256), 0, s, Y, Yq, ys, k.n_active, k.valid_rows,
-                     B, I, Iw);
+                     B, I, y_stride, Iw);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

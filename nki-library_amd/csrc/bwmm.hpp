@@ -64,6 +64,7 @@ struct MxArgs {
   int64_t y_stride, ys_stride;
   uint16_t* D;             // stage 2 output, bf16 [N*B, H]
   int64_t H, I, E, n_real;
+  int64_t I_tab;           // MX_WFMT_ROW8 / BF16: columns of the gate/up bias and channel-scale tables (I without padding)
   int32_t pI, nI;
   int32_t act_fn, scaling_mode, clamp_mask;
   float clamp[4];
@@ -93,7 +94,15 @@ struct MxArgs {
 
 constexpr int MX_WFMT_E4M3 = 0, MX_WFMT_E5M2 = 1, MX_WFMT_E2M1 = 2, MX_WFMT_ROW8 = 3, MX_WFMT_BF16 = 4;
 
-// True when the large-tile kernels cover the shape: every intermediate tile holds a multiple
+// The dense kinds run on copies of their weights, which are padded with zeros to what the large-tile kernels take: gate/up
+// columns to a multiple of 128 (whole column tiles), the down stage's K to whole 128-byte slices.  Results of the padded
+// columns are act(0) * 0 = 0 (their bias counts as 0, their scale as 1).  Measured at T = 10240 over 128 bf16 experts of
+// H = 3072, I = 192 (a third more gate/up columns than needed): gate/up + down 281 + 358 us on the general kernel, whose
+// two-byte stores and three-step K loops are what the down stage waits for, 223 + 164 us here.
+inline int64_t dense_cols(int64_t I) { return (I + 127) / 128 * 128; }
+inline int64_t dense_k_bytes(int64_t I, bool bf16) { return bf16 ? (I + 63) / 64 * 128 : (I + 127) / 128 * 128; }
+
+// MX kinds: true when the large-tile kernels cover the shape: every intermediate tile holds a multiple
 // of 32 partitions (I % 128 == 0); other shapes run the general kernel.
 inline bool mx_fast_path_ok(int64_t H, int64_t I) { return H % 512 == 0 && I % 128 == 0; }
 int launch_mx_gemm(int stage, const MxArgs& m, unsigned gx, unsigned gy, hipStream_t s);
@@ -127,7 +136,7 @@ int launch_transpose_w16(const void* src, int w8, uint16_t* dst, int64_t R, int6
 int launch_transpose_fp8(const uint8_t* src, uint8_t* dst, int64_t R, int64_t C, int64_t src_row_stride, int64_t Kp,
                          int64_t nb0, int nb1, int64_t src_bs0, int64_t src_bs1, hipStream_t s);
 // The fp8-row kind's weights in the x4 order the large-tile kernels read, K in natural order: gate/up
-// [E, H, 2, I] -> [E, 128 (p), 2, H/512 (t), I, 4 (q)] with h = t*512 + p*4 + q; down [E, I_pad, H] ->
+// [E, H, 2, I] -> [E, 128 (p), 2, H/512 (t), dense_cols(I), 4 (q)] with h = t*512 + p*4 + q; down [E, I_pad, H] ->
 // [E, pI, nI, H, 4] with i = t*512 + p*4 + q (zeros past I).
 int launch_relayout_x4(const uint8_t* gate_up, const uint8_t* down, uint8_t* dst, int which, int64_t E, int64_t H,
                        int64_t I, int64_t I_pad, hipStream_t s);
@@ -138,6 +147,6 @@ int launch_relayout_x4_bf16(const void* gate_up, const void* down, int w8, uint8
                             int64_t I, int64_t I_pad, hipStream_t s);
 int launch_fill_bytes(void* p, size_t bytes, uint8_t value, hipStream_t s);
 int launch_row_requant(const float* Y, uint8_t* Yq, float* ys, const Bookkeeping& k, int64_t N, int64_t B, int64_t I,
-                       int64_t Iw, hipStream_t s);
+                       int64_t y_stride, int64_t Iw, hipStream_t s);
 
 }  // namespace moe

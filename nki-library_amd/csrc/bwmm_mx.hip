@@ -426,13 +426,19 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const int hcol = (STAGE == 1) ? (c >> 3) : 0, cl = (STAGE == 1) ? (c & 7) : c;
   // the natural column of the thread's table entry: gate/up (gu = tid/128, q = tid/32 % 4, pl = tid % 32) ->
   // gu * I + tile*512 + q*Pt + p0 + pl; down -> h0 + tid
+  // (columns that only pad the weights have no entry: natural_live is false, and natural_col the last real column's)
+  auto tile_col = [&](const Tile& t) {
+    return (uint32_t)tile_tI(t) * 512u + (uint32_t)((tid >> 5) & 3) * (uint32_t)tile_Pt(t) + (uint32_t)(tile_p0(t) + (tid & 31));
+  };
+  auto natural_live = [&](const Tile& t) { return STAGE != 1 || tile_col(t) < (uint32_t)a.I_tab; };
   auto natural_col = [&](const Tile& t) {
-    if (STAGE == 1)
-      return (uint32_t)(tid >> 7) * (uint32_t)a.I + (uint32_t)tile_tI(t) * 512u +
-             (uint32_t)((tid >> 5) & 3) * (uint32_t)tile_Pt(t) + (uint32_t)(tile_p0(t) + (tid & 31));
+    if (STAGE == 1) {
+      const uint32_t col = tile_col(t);
+      return (uint32_t)(tid >> 7) * (uint32_t)a.I_tab + (col < (uint32_t)a.I_tab ? col : (uint32_t)a.I_tab - 1u);
+    }
     return (uint32_t)tile_h0(t) + (uint32_t)tid;
   };
-  const uint32_t ncols = (STAGE == 1) ? 2u * (uint32_t)a.I : (uint32_t)a.H;  // table entries per expert
+  const uint32_t ncols = (STAGE == 1) ? 2u * (uint32_t)a.I_tab : (uint32_t)a.H;  // table entries per expert
   auto bias_index = [&](const Tile& t) {
     if (ROW8) return (uint32_t)t.e * ncols + natural_col(t);
     if (STAGE == 1) {
@@ -447,7 +453,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     ld_b32(raw, a.bias ? elem_offset(bias_index(t), a.bias_dtype == MOE_DT_BF16) : 0u, rd, 0);
   };
   auto bias_put = [&](const Tile& t, int buf, int raw) {
-    s_bias[buf][tid] = a.bias ? elem_value(raw, bias_index(t), a.bias_dtype == MOE_DT_BF16) : 0.f;
+    s_bias[buf][tid] = (a.bias && (!ROW8 || natural_live(t))) ? elem_value(raw, bias_index(t), a.bias_dtype == MOE_DT_BF16) : 0.f;
   };
   // ROW8: the weights' per-channel scale of the thread's column (fp32), and the activation rows' scales: gate/up,
   // the fp32 behind the H codes of the token's record, times the affinity under PRE_SCALE (the affinity scales
@@ -458,8 +464,8 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       ld_b32(raw, a.w_cscale ? ((a.cscale_experts > 1 ? (uint32_t)t.e * ncols : 0u) + natural_col(t)) << 2 : 0u, rd, 0);
     }
   };
-  auto wsc_put = [&](int buf, int raw) {
-    if constexpr (ROW8) s_wsc[buf][tid] = a.w_cscale ? __builtin_bit_cast(float, raw) : 1.f;
+  auto wsc_put = [&](const Tile& t, int buf, int raw) {
+    if constexpr (ROW8) s_wsc[buf][tid] = (a.w_cscale && natural_live(t)) ? __builtin_bit_cast(float, raw) : 1.f;
   };
   auto rs_raw = [&](const Tile& t, int buf, int (&raw)[2]) {
     if constexpr (ROW8) {
@@ -865,7 +871,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
   ids_put(0, cur.nrows, ids_nn);
   bias_put(cur, 0, bias_n);
-  wsc_put(0, wsc_n);
+  wsc_put(cur, 0, wsc_n);
   __syncthreads();
   if (AFF_ROWS) {
     aff_raw(cur, 0, aff_n);
@@ -1076,6 +1082,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
               uint16_t* ck1 = a.ckpt + (((int64_t)n1 * 2) * a.ckpt_I + col) * a.ckpt_B + r1;
 #pragma unroll
               for (int t = 0; t < 4; ++t) {
+                if (col + t >= a.ckpt_I) continue;  // (a column that only pads the weights)
                 const uint32_t gp = pack2_bf16(ckg[t][0], ckg[t][1]), up = pack2_bf16(cku[t][0], cku[t][1]);
                 if (pair) {
                   *(uint32_t*)(ck + (int64_t)t * a.ckpt_B) = gp;
@@ -1248,7 +1255,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   if (STAGE == 2) aff_put(nxt.e, buf ^ 1, aff_n);
   rs_put(nxt.e, buf ^ 1, rs_n, aff_n);
   bias_put(nxt, buf ^ 1, bias_n);
-  wsc_put(buf ^ 1, wsc_n);
+  wsc_put(nxt, buf ^ 1, wsc_n);
   if (have_nn) ids_put(buf, nn.nrows, ids_nn);  // the table of the tile that has just ended
   cur = nxt;
   L = Ln;

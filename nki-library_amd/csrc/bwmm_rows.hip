@@ -329,16 +329,17 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
           for (int k = 0; k < 2; ++k) {
             float gv = part(r, qq * 64 + j + k), uv = part(r, qq * 64 + 32 + j + k);
             float sg = 1.f, su = 1.f;
-            if (a.w_cscale) {
-              const float* ws = a.w_cscale + (a.cscale_experts > 1 ? (int64_t)e * 2 * a.I : 0);
+            const bool live = col + k < a.I_tab;  // (columns that only pad the weights: act(0) * 0)
+            if (a.w_cscale && live) {
+              const float* ws = a.w_cscale + (a.cscale_experts > 1 ? (int64_t)e * 2 * a.I_tab : 0);
               sg = ws[col + k];
-              su = ws[a.I + col + k];
+              su = ws[a.I_tab + col + k];
             }
             gv = (gv * sg) * rs;
             uv = (uv * su) * rs;
-            if (a.bias) {
-              gv += bias_at((int64_t)e * 2 * a.I + col + k);
-              uv += bias_at((int64_t)e * 2 * a.I + a.I + col + k);
+            if (a.bias && live) {
+              gv += bias_at((int64_t)e * 2 * a.I_tab + col + k);
+              uv += bias_at((int64_t)e * 2 * a.I_tab + a.I_tab + col + k);
             }
             y[k] = gate_up(gv, uv);
           }

@@ -131,17 +131,19 @@ int validate(const moe_bwmm_args* a) {
 // A call runs there when both hold (activation checkpoints of the bf16 kind included: those epilogues write them).
 // A call on such a shape that cannot run there uses the general kernel on K-contiguous copies of its own, made per
 // call in the workspace: kept copies are in the other order and are ignored (*_kept_usable).
+// (I of any size: the copies are padded with zeros, see dense_cols / dense_k_bytes)
 bool row8_shape(const moe_bwmm_args* a) {
-  if (a->kind != MOE_KIND_FP8_ROW || !mx_fast_path_ok(a->H, a->I)) return false;
+  if (a->kind != MOE_KIND_FP8_ROW || a->H % 512 != 0) return false;
   const int64_t lim32 = (int64_t)1 << 32, lim31 = (int64_t)1 << 31;
-  const int64_t pI = a->I > 512 ? 128 : a->I / 4, nI = (a->I + 511) / 512;
-  if (2 * a->H * a->I >= lim31 || pI * nI * a->H * 4 >= lim31) return false;
-  if (a->E * 2 * a->I * 4 >= lim32 || a->E * a->H * 4 >= lim32) return false;
+  const int64_t Ic = dense_cols(a->I), Kb = dense_k_bytes(a->I, false);
+  const int64_t pI = Kb > 512 ? 128 : Kb / 4, nI = (Kb + 511) / 512;
+  if (2 * a->H * Ic >= lim31 || pI * nI * a->H * 4 >= lim31) return false;
+  if (a->E * 2 * Ic * 4 >= lim32 || a->E * a->H * 4 >= lim32) return false;
   return true;
 }
 bool row8_call_fits(const moe_bwmm_args* a) {
   const int64_t lim32 = (int64_t)1 << 32;
-  const int64_t slots = a->N * a->B, Iw = (a->I + 127) / 128 * 128;
+  const int64_t slots = a->N * a->B, Iw = dense_cols(a->I);
   return a->T1 * (a->H + 4) < lim32 && slots * Iw < lim32 && slots * 4 < lim32 && a->T1 * a->E * 4 < lim32;
 }
 bool row8_fast(const moe_bwmm_args* a) { return row8_shape(a) && row8_call_fits(a); }
@@ -149,18 +151,18 @@ bool row8_kept_usable(const moe_bwmm_args* a) { return row8_fast(a) || !row8_sha
 // (bf16 weights, or fp8 weights widened to bf16 in the copy; K extents in bytes: 2H, 2I)
 bool bf16_fast_shape(const moe_bwmm_args* a) {
   if (a->kind != MOE_KIND_BF16 || (a->weight_dtype != MOE_DT_BF16 && a->weight_dtype != MOE_DT_FP8_E4M3)) return false;
-  if (a->H % 256 != 0 || a->I % 128 != 0) return false;
+  if (a->H % 256 != 0) return false;
   const int64_t lim32 = (int64_t)1 << 32, lim31 = (int64_t)1 << 31;
-  const int64_t Ib = 2 * a->I, Hb = 2 * a->H;
-  const int64_t pI = Ib > 512 ? 128 : Ib / 4, nI = (Ib + 511) / 512;
-  if (2 * Hb * a->I >= lim31 || pI * nI * a->H * 4 >= lim31) return false;
-  if (a->E * 2 * a->I * 4 >= lim32 || a->E * a->H * 4 >= lim32) return false;
+  const int64_t Ic = dense_cols(a->I), Kb = dense_k_bytes(a->I, true), Hb = 2 * a->H;
+  const int64_t pI = Kb > 512 ? 128 : Kb / 4, nI = (Kb + 511) / 512;
+  if (2 * Hb * Ic >= lim31 || pI * nI * a->H * 4 >= lim31) return false;
+  if (a->E * 2 * Ic * 4 >= lim32 || a->E * a->H * 4 >= lim32) return false;
   return true;
 }
 bool bf16_call_fits(const moe_bwmm_args* a) {
   const int64_t lim32 = (int64_t)1 << 32;
   const int64_t slots = a->N * a->B;
-  return a->T1 * 2 * a->H < lim32 && slots * 2 * a->I < lim32 && slots * 4 < lim32 && a->T1 * a->E * 4 < lim32;
+  return a->T1 * 2 * a->H < lim32 && slots * 2 * dense_cols(a->I) < lim32 && slots * 4 < lim32 && a->T1 * a->E * 4 < lim32;
 }
 bool bf16_fast(const moe_bwmm_args* a) { return bf16_fast_shape(a) && bf16_call_fits(a); }
 bool bf16_kept_usable(const moe_bwmm_args* a) { return bf16_fast(a) || !bf16_fast_shape(a); }
@@ -174,11 +176,11 @@ struct Row8Copy {
 Row8Copy row8_copy(const moe_bwmm_args* a, int which) {
   auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
   const size_t es = a->kind == MOE_KIND_BF16 ? 2 : 1;
-  const size_t Hb = (size_t)a->H * es, Ib = (size_t)a->I * es;
+  const size_t Hb = (size_t)a->H * es, Ic = (size_t)dense_cols(a->I), Ib = (size_t)dense_k_bytes(a->I, es == 2);
   const size_t nH = Hb / 512, nI = (Ib + 511) / 512, pI = Ib > 512 ? 128 : Ib / 4;
   Row8Copy c;
-  const size_t w = which == 0 ? (size_t)a->E * 2 * Hb * a->I : (size_t)a->E * pI * nI * a->H * 4;
-  const size_t ws = which == 0 ? 16 * 2 * nH * (size_t)a->I : ((pI + 7) / 8) * nI * (size_t)a->H;
+  const size_t w = which == 0 ? (size_t)a->E * 2 * Hb * Ic : (size_t)a->E * pI * nI * a->H * 4;
+  const size_t ws = which == 0 ? 16 * 2 * nH * Ic : ((pI + 7) / 8) * nI * (size_t)a->H;
   c.w_scale = al(w);
   c.a_scale = c.w_scale + al(ws);
   c.a_scale_bytes = al(which == 0 ? Hb / 32 : nI * 16);
@@ -203,14 +205,15 @@ Plan make_plan(const moe_bwmm_args* a) {
     p.yq = off; off += al256(slots * (size_t)p.Iw);
     p.ys = off; off += al256(slots * (size_t)(p.Iw / 32));
   } else if (a->kind == MOE_KIND_BF16) {
-    p.Iw = (a->I + 63) / 64 * 64;
+    const bool bf = bf16_fast(a);
+    p.Iw = bf ? dense_cols(a->I) : (a->I + 63) / 64 * 64;
     p.y = off; off += al256(slots * (size_t)p.Iw * 2);
     // K-contiguous bf16 copies of the weights: [E, 2, I, Hk] and [E, H, Iw]
     p.Hk = (a->H + 63) / 64 * 64;
-    const bool bf = bf16_fast(a);
-    if (bf) {  // the x4 geometry of the down weights over 2I bytes of K
-      p.nI = (2 * a->I + 511) / 512;
-      p.pI = 2 * a->I > 512 ? 128 : a->I / 2;
+    if (bf) {  // the x4 geometry of the down weights over the bytes of K
+      const int64_t Kb = dense_k_bytes(a->I, true);
+      p.nI = (Kb + 511) / 512;
+      p.pI = Kb > 512 ? 128 : Kb / 4;
     }
     const bool kept = bf16_kept_usable(a);
     if (!(a->gate_up_proj_weight_kmajor && kept)) {
@@ -221,15 +224,16 @@ Plan make_plan(const moe_bwmm_args* a) {
     }
   } else {
     p.Iw = (a->I + 127) / 128 * 128;
-    p.y = off; off += al256(slots * (size_t)a->I * 4);
+    p.y = off; off += al256(slots * (size_t)(row8_fast(a) ? dense_cols(a->I) : a->I) * 4);
     p.yq = off; off += al256(slots * (size_t)p.Iw);
     p.ys = off; off += al256(slots * 4);
     // K-contiguous copies of the fp8 weights: [E, 2, I, Hk] and [E, H, Iw]
     p.Hk = (a->H + 127) / 128 * 128;
     const bool r8 = row8_fast(a);
     if (r8) {  // the x4 geometry of the down weights, as for the MXFP8 kind
-      p.nI = (a->I + 511) / 512;
-      p.pI = a->I > 512 ? 128 : a->I / 4;
+      const int64_t Kb = dense_k_bytes(a->I, false);
+      p.nI = (Kb + 511) / 512;
+      p.pI = Kb > 512 ? 128 : Kb / 4;
     }
     const bool kept = row8_kept_usable(a);
     if (!(a->gate_up_proj_weight_kmajor && kept)) {
@@ -480,7 +484,9 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m.cscale_experts = a->scale_experts;
       m.w_scale_shared = 1;
       m.Y32 = (float*)(ws + p.y);
-      m.y32_stride = a->I;
+      m.y32_stride = dense_cols(a->I);
+      m.I = dense_cols(a->I);
+      m.I_tab = a->I;
     }
     if (bf_fast) {
       m.wfmt = MX_WFMT_BF16;
@@ -544,7 +550,7 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
   }
   mark(3);
   if (a->kind == MOE_KIND_FP8_ROW && (stages & MOE_STAGE_REQUANT)) {
-    rc = launch_row_requant((const float*)(ws + p.y), ws + p.yq, (float*)(ws + p.ys), bk, a->N, a->B, a->I, p.Iw, s);
+    rc = launch_row_requant((const float*)(ws + p.y), ws + p.yq, (float*)(ws + p.ys), bk, a->N, a->B, a->I, r8_fast ? dense_cols(a->I) : a->I, p.Iw, s);
     if (rc != MOE_OK) return rc;
   }
   mark(4);
@@ -567,10 +573,10 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
         m2.A_scale = g2.W + c.a_scale; m2.a_scale_stride = 0; m2.a_scale_bytes = (int64_t)c.a_scale_bytes;
         m2.w_cscale = (const float*)a->down_proj_scale;
         m2.a_rscale = (const float*)(ws + p.ys);
+        m2.I = dense_k_bytes(a->I, bf_fast);  // K in bytes
       }
       if (bf_fast) {
         m2.A = ws + p.y; m2.a_stride = p.Iw * 2;
-        m2.I = 2 * a->I;  // K in bytes
         m2.a_rscale = nullptr;
         m2.ckpt = (uint16_t*)a->down_activations;
         m2.ckpt_B = a->B; m2.ckpt_I = a->I;

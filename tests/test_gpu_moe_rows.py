@@ -100,3 +100,28 @@ def test_mx_copies_follow_the_block_scales():
     assert torch.equal(layer(other), plain(other)) and not torch.equal(layer(other), layer(gs))
     gs.add_(1)
     assert torch.equal(layer(gs), layer(other))
+
+
+@pytest.mark.parametrize("T", [20, 150])  # the few-rows and the large-tile kernels
+@pytest.mark.parametrize("I,fp8w", [(36, False), (130, False), (202, True), (264, False)])
+def test_padded_intermediate_dense(T, I, fp8w):
+    """Intermediate sizes that fill neither a column tile of 128 nor a K slice of 64 (and rows of weights that are not
+    aligned to four elements): the padding columns must add nothing, biases and scales keep their columns."""
+    c = dense_case(T, 512, I, 4, 2, 128, seed=34, bias=True, quant=fp8w, hidden_std=1.0)
+    o = from_bf16_tensor(_run_dense(c, act=1, mode=1, clamps=CL, fp8_weights=fp8w))[:, 0]
+    _check(o[:T], _golden_dense(c, act=1, mode=1, clamps=CL, fp8_weights=fp8w)[:T], f"padded bf16 T={T} I={I}")
+
+
+@pytest.mark.parametrize("T", [20, 150])
+@pytest.mark.parametrize("I", [36, 264])
+def test_padded_intermediate_fp8_row(T, I):
+    c = dense_case(T, 512, I, 4, 2, 128, seed=35, quant=True, bias=True, hidden_std=1.0)
+    rec, out = _run_fp8_row(c, np.ones((1, 512), np.float32), clamps=CL, act=3)
+    import torch
+
+    raw = rec.view(torch.uint8).cpu().numpy()
+    g = omoe.moe_blockwise_fp8_row_ref(raw[:, :512], raw[:, 512:].copy().view(np.float32).reshape(-1), c["aff"],
+                                       c["gate_up_q"], c["down_q"], c["gate_up_scale"], c["down_scale"], c["tp2id"],
+                                       c["b2e"], c["B"], gate_up_proj_bias=c["gate_up_bias"], down_proj_bias=c["down_bias"],
+                                       activation_function=3, **CL)
+    _check(from_bf16_tensor(out)[:T, 0], g[:T], f"padded fp8 row T={T} I={I}")
