@@ -42,6 +42,7 @@ EXPORTED_SYMBOLS = (
     "moe_indexed_flatten",
     "moe_cumsum",
     "moe_router_topk_workspace_bytes",
+    "moe_router_topk_workspace_bytes_for",
     "moe_router_topk",
     "moe_blockwise_workspace_bytes",
     "moe_blockwise",
@@ -164,6 +165,8 @@ def lib():
     L.moe_cumsum.argtypes = [c_void_p, c_void_p, c_int, c_int64, c_int64, c_void_p]
     L.moe_router_topk_workspace_bytes.restype = c_size_t
     L.moe_router_topk_workspace_bytes.argtypes = [c_int64, c_int64]
+    L.moe_router_topk_workspace_bytes_for.restype = c_size_t
+    L.moe_router_topk_workspace_bytes_for.argtypes = [c_int64, c_int64, c_int64]
     L.moe_router_topk.restype = c_int
     L.moe_router_topk.argtypes = [c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int, c_int, c_int,
                                   c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p, c_void_p,

@@ -58,8 +58,8 @@ def _router_topk(x, w, w_bias, router_logits, expert_affinities, expert_index, a
                       "expert_index must be a contiguous 32-bit integer tensor")
     topk_aff = torch.empty((T, int(k)), dtype=torch.float32, device=dev) if return_eager_affi else None
     L = nv.lib()
-    wsb = L.moe_router_topk_workspace_bytes(H, E)
-    ws = nv.workspace(dev, wsb)
+    # (its size follows T: from the caching allocator, which knows the stream, not from the scratch that only grows)
+    ws = torch.empty(L.moe_router_topk_workspace_bytes_for(T, H, E), dtype=torch.uint8, device=dev)
     rc = L.moe_router_topk(
         nv.ptr(x), nv.ptr(w), nv.ptr(bias), nv.dtype_code(bias, "w_bias") if bias is not None else 0, T, H, E, int(k),
         act.value, int(bool(router_pre_norm)), int(bool(norm_topk_prob)), int(bool(_mask_to_topk)), int(bool(_pad_row)),

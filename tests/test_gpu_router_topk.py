@@ -69,6 +69,56 @@ def test_router_topk_matches_oracle(T, H, E, k, act, pre, norm, bias, layout):
     assert np.abs(ta[safe] - want[safe]).max() <= 1e-5 + 1e-4 * np.abs(want).max()
 
 
+@pytest.mark.parametrize(
+    "T,H,E,k",
+    [
+        (1, 128, 8, 2),       # one token, a single part of K
+        (64, 7168, 256, 8),   # the last size of the 64-token tiles, K in 16 parts
+        (65, 7168, 256, 8),   # the first of the 128-token tiles, one row in the second half
+        (129, 1024, 128, 6),  # a second tile of one token, experts in one group of 128
+        (40, 1088, 100, 4),   # K steps that the parts do not share out evenly, padded experts
+        (700, 896, 65, 3),    # one expert past the group of 64
+        (33000, 192, 60, 2),  # more tiles than CUs: one part
+        (200, 640, 260, 8),   # two groups of 256
+    ],
+)
+def test_router_split_over_k_matches_the_unsplit_kernel(T, H, E, k):
+    """The C entry with the small workspace (one workgroup per token tile) and with the one for K split over workgroups:
+    the logits differ by the order of fp32 sums: H roundings of independent sign, each at most 2^-24 * sum |x w|, so
+    sqrt(H) of these is a deviation of either side's sum, taken four times for both sides.  Where the logits around the
+    selected ones are further apart than that the selections are equal."""
+    import torch
+    from nkilib import _native as nv
+
+    dev = torch.device("cuda:0")
+    L = nv.lib()
+    g = torch.Generator(device=dev).manual_seed(T)
+    x = torch.randn((T, H), generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn((H, E), generator=g, device=dev) * H ** -0.5).to(torch.bfloat16)
+    b = torch.randn((E,), generator=g, device=dev)
+    res = []
+    for size in (L.moe_router_topk_workspace_bytes(H, E), L.moe_router_topk_workspace_bytes_for(T, H, E)):
+        ws = torch.full((size,), 255, dtype=torch.uint8, device=dev)
+        lg = torch.empty((T, E), device=dev)
+        idx = torch.empty((T, k), dtype=torch.int32, device=dev)
+        aff = torch.full((T + 1, E), 7.0, device=dev)
+        nv.check(L.moe_router_topk(nv.ptr(x), nv.ptr(w), nv.ptr(b), nv.DT_FP32, T, H, E, k, 0, 1, 1, 1, 1, nv.ptr(lg),
+                                   nv.DT_FP32, nv.ptr(idx), nv.ptr(aff), nv.DT_FP32, None, nv.ptr(ws), size,
+                                   nv.stream_ptr(dev)), "router")
+        torch.cuda.synchronize()
+        res.append((lg, idx, aff))
+    (l0, i0, a0), (l1, i1, a1) = res
+    bound = 8 * H ** 0.5 * 2.0 ** -24 * (x.abs().float() @ w.abs().float()) + 1e-6
+    assert ((l0 - l1).abs() <= bound).all()
+    assert not a0[T].any() and not a1[T].any()
+    srt = l0.sort(dim=1, descending=True).values
+    gaps = (srt[:, :k] - srt[:, 1:k + 1]).min(dim=1).values if k < E else (srt[:, :k - 1] - srt[:, 1:k]).min(dim=1).values
+    safe = gaps > bound.max()
+    assert safe.float().mean() > 0.5
+    assert torch.equal(i0[safe], i1[safe])
+    assert (a0[:T][safe] - a1[:T][safe]).abs().max() <= 2 * bound.max()
+
+
 def test_route_for_moe_feeds_the_block_build():
     """Masked table + ids from hidden states: zero outside the top-k, zero padding row, ids usable as they are."""
     import torch
