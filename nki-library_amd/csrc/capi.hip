@@ -341,17 +341,28 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
   uint8_t* ws = (uint8_t*)a->workspace;
   const int64_t n_real = a->skip_token ? a->T1 : a->T1 - 1;
   // The chunk / slot bookkeeping: derived here from token_position_to_id, or taken as the block build left it
-  // (moe_build_blocks_plan).  Activation checkpoints cover whole blocks, which a plan's chunks do not: the plan is
-  // then left aside.
+  // (moe_build_blocks_plan).  With activation checkpoints the large-tile kernels' chunks hold one padding row per expert
+  // more than the plan's: they are cut anew from the plan's valid rows, the rest of the plan is used as it is.
   // (measurement hook: HIP events of the caller's, recorded on the stream between the stages)
   auto mark = [&](int i) {
     if (a->stage_events && a->stage_events[i]) (void)hipEventRecord((hipEvent_t)a->stage_events[i], s);
   };
   mark(0);
-  const bool planned = a->block_plan != nullptr && !a->gate_up_activations_T && !a->down_activations;
-  if (planned && (a->block_plan_bytes < bookkeeping_bytes(a->T1, a->N, a->B) || ((uintptr_t)a->block_plan & 255) != 0))
-    return MOE_E_BAD_ARG;
-  const Bookkeeping bk = carve_bookkeeping(planned ? (void*)a->block_plan : (void*)(ws + p.book), a->T1, a->N, a->B);
+  const bool ckpt = a->gate_up_activations_T || a->down_activations;
+  const bool plan_ok = a->block_plan_bytes >= bookkeeping_bytes(a->T1, a->N, a->B) && ((uintptr_t)a->block_plan & 255) == 0;
+  if (a->block_plan && !ckpt && !plan_ok) return MOE_E_BAD_ARG;
+  const bool planned = a->block_plan != nullptr && plan_ok && (!ckpt || ((stages & MOE_STAGE_CHECKPOINT_PLAN) && bf16_fast(a)));
+  Bookkeeping bk = carve_bookkeeping(planned ? (void*)a->block_plan : (void*)(ws + p.book), a->T1, a->N, a->B);
+  if (planned && ckpt) {
+    const Bookkeeping own = carve_bookkeeping(ws + p.book, a->T1, a->N, a->B);
+    bk.n_chunks = own.n_chunks; bk.chunk_slot = own.chunk_slot; bk.chunk_rows = own.chunk_rows;
+    bk.chunk_expert = own.chunk_expert; bk.chunk_xcd = own.chunk_xcd; bk.q_chunk = own.q_chunk; bk.q_off = own.q_off;
+    if (stages & MOE_STAGE_PREP) {
+      rc = launch_plan_chunks(bk, a->block_to_expert, a->N, a->B, a->E, s, own.n_active, a->conditions == nullptr);
+      if (rc != MOE_OK) return rc;
+    }
+    bk.n_active = own.n_active;
+  }
   if ((stages & MOE_STAGE_PREP) && !planned) {
     rc = launch_prep(bk, a, n_real, s);
     if (rc != MOE_OK) return rc;
@@ -505,12 +516,13 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
            mx_rows_fits(stage, m.wfmt, n_real, avg_rows, (int64_t)gx * bk.max_chunks);
   };
   mark(2);
-  // checkpoints of blocks that never run stay zero
-  if (a->gate_up_activations_T && (stages & MOE_STAGE_GATE_UP)) {
+  // Checkpoints of blocks that never run stay zero: cleared ahead for the general kernel; behind the large-tile kernels
+  // launch_ckpt_pad clears them with the copies of the padding rows.
+  if (!mx_fast && a->gate_up_activations_T && (stages & MOE_STAGE_GATE_UP)) {
     rc = launch_fill_zero_bytes(a->gate_up_activations_T, (size_t)a->N * 2 * a->I * a->B * 2, s);
     if (rc != MOE_OK) return rc;
   }
-  if (a->down_activations && (stages & MOE_STAGE_DOWN)) {
+  if (!mx_fast && a->down_activations && (stages & MOE_STAGE_DOWN)) {
     rc = launch_fill_zero_bytes(a->down_activations, (size_t)a->N * a->B * a->H * 2, s);
     if (rc != MOE_OK) return rc;
   }
@@ -547,6 +559,10 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       rc = launch_gemm_stage(a->kind, 1, g1, gx1, gy, s);
     }
     if (rc != MOE_OK) return rc;
+    if (mx_fast && a->gate_up_activations_T) {
+      rc = launch_ckpt_pad(1, (uint16_t*)a->gate_up_activations_T, bk, a, s);
+      if (rc != MOE_OK) return rc;
+    }
   }
   mark(3);
   if (a->kind == MOE_KIND_FP8_ROW && (stages & MOE_STAGE_REQUANT)) {
@@ -589,6 +605,10 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       rc = launch_gemm_stage(a->kind, 2, g2, gx2, gy, s);
     }
     if (rc != MOE_OK) return rc;
+    if (mx_fast && a->down_activations) {
+      rc = launch_ckpt_pad(2, (uint16_t*)a->down_activations, bk, a, s);
+      if (rc != MOE_OK) return rc;
+    }
   }
   mark(5);
   if (stages & MOE_STAGE_COMBINE) {

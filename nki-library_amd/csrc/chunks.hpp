@@ -17,7 +17,7 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
                                              int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert,
                                              int32_t* __restrict__ chunk_xcd, int32_t* __restrict__ q_chunk,
                                              int32_t* __restrict__ q_off, int64_t max_chunks, int* s_ws,
-                                             bool whole_blocks) {
+                                             bool pad_row) {
   const int64_t na = *n_active;
   // The walk along a run below is a chain of dependent reads, one block after the other: from LDS when the active
   // blocks fit there (a global read per step made the run length the pace of this kernel).
@@ -48,12 +48,15 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
       e = expert_of(b);
       const bool start = (b == 0) || (expert_of(b - 1) != e);
       if (start && e >= 0 && e < E) {
-        // (whole_blocks: activation checkpoints hold every row of every executed block, padding rows included, so
-        // a run's chunks then cover its blocks to the end)
-        for (int64_t j = b; j < na && expert_of(j) == e; ++j) {
-          const int v = whole_blocks ? (int)B : valid_of(j);
+        int64_t j = b;
+        for (; j < na && expert_of(j) == e; ++j) {
+          const int v = valid_of(j);
           if (v > 0) last_end = j * B + v;
         }
+        // (pad_row: activation checkpoints hold every row of every executed block, padding rows included.  Those behind
+        // the last token are all alike, so the chunks take one of them along, which ckpt_pad_gate_up_kernel /
+        // ckpt_pad_down_kernel then copy to the others)
+        if (pad_row) last_end = last_end < 0 ? b * B + 1 : last_end < j * B ? last_end + 1 : last_end;
         // chunks of CHUNK_ROWS rows; the last one absorbs a remainder of up to CHUNK_ROWS_MAX - CHUNK_ROWS
         // rows, which saves the pass over the expert's weights that a small chunk of its own would cost
         const int64_t len = last_end - b * B;

@@ -92,24 +92,138 @@ __global__ __launch_bounds__(1024) void chunks_and_offsets_kernel(
     int64_t N, int64_t B, int64_t E, int32_t* __restrict__ n_chunks, int32_t* __restrict__ chunk_slot,
     int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert, int32_t* __restrict__ chunk_xcd,
     int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks,
-    const int32_t* __restrict__ cnt, int32_t* __restrict__ off, int64_t n_real, bool whole_blocks) {
+    const int32_t* __restrict__ cnt, int32_t* __restrict__ off, int64_t n_real, bool pad_row) {
   __shared__ int s_ws[16];
   if (blockIdx.x == 0)
     build_chunks(b2e, n_active, valid_rows, N, B, E, n_chunks, chunk_slot, chunk_rows, chunk_expert, chunk_xcd, q_chunk,
-                 q_off, max_chunks, s_ws, whole_blocks);
+                 q_off, max_chunks, s_ws, pad_row);
   else
     inv_scan(cnt, off, n_real, s_ws);
 }
 
-// One workgroup: chunks and work queues from a block build's own valid rows (moe_build_blocks_plan).
+// One workgroup: chunks and work queues from a block build's own valid rows (moe_build_blocks_plan).  With n_active_out
+// the chunks are those of a call with activation checkpoints, whose executed blocks are the build's or, without
+// conditions, all of them; their number goes there.
 __global__ __launch_bounds__(1024) void plan_chunks_kernel(
-    const int32_t* __restrict__ b2e, const int32_t* __restrict__ n_active, const int32_t* __restrict__ valid_rows,
+    const int32_t* __restrict__ b2e, const int32_t* n_active, const int32_t* __restrict__ valid_rows,
     int64_t N, int64_t B, int64_t E, int32_t* __restrict__ n_chunks, int32_t* __restrict__ chunk_slot,
     int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert, int32_t* __restrict__ chunk_xcd,
-    int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks) {
+    int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks, int32_t* n_active_out, bool all_blocks) {
   __shared__ int s_ws[16];
+  if (n_active_out) {
+    if (threadIdx.x == 0) *n_active_out = all_blocks ? (int32_t)N : *n_active;
+    __threadfence_block();
+    __syncthreads();
+    n_active = n_active_out;
+  }
   build_chunks(b2e, n_active, valid_rows, N, B, E, n_chunks, chunk_slot, chunk_rows, chunk_expert, chunk_xcd, q_chunk,
-               q_off, max_chunks, s_ws, false);
+               q_off, max_chunks, s_ws, n_active_out != nullptr);
+}
+
+// ---- activation checkpoints: the rows behind the last token -------------------------------------------------
+//
+// The gate_up checkpoint [N, 2, I, B] and the down checkpoint [N, B, H] hold every row of every executed block; blocks
+// that do not run stay zero.  Behind an expert's last token all rows are padding, i.e. a zero hidden row each, with the
+// same results: the GEMMs compute the first of them (see build_chunks), and these kernels copy it to the rest of the
+// expert's blocks and clear the blocks that do not run.  A training-shaped call has as many padding rows as tokens:
+// T = 1024, top-4 of 8 experts of H = 3072, I = 2048, B = 512 lists 7680 rows for 4096 routed ones: the GEMMs over all of them
+// took 205 + 134 us and clearing both checkpoints beforehand 33; over the routed ones 125 + 82, and 15 + 9 for these copies.
+
+// A block's run (the executed blocks of its expert around it): the slot of the row to copy, and the block's first row
+// behind it; rows 0 .. B of a block that does not run are to be cleared (src = -1).  Every thread of the workgroup gets it.
+struct CkptPad {
+  int64_t src;
+  int first;
+};
+__device__ __forceinline__ CkptPad ckpt_pad_of(int64_t b, const int32_t* __restrict__ b2e, const int32_t* __restrict__ n_active,
+                                               const int32_t* __restrict__ valid_rows, int64_t B, int64_t E, int* s_w) {
+  const int na = *n_active, e = b2e[b];
+  if (b >= na || e < 0 || e >= E) return CkptPad{-1, 0};  // (the same for the whole workgroup)
+  if (threadIdx.x == 0) {
+    s_w[0] = 0;   // first block of the run
+    s_w[1] = na;  // the one behind it
+    s_w[2] = -1;  // its last block that holds a token
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < na; j += blockDim.x)
+    if (b2e[j] != e) {
+      if (j < b) atomicMax(&s_w[0], j + 1);
+      else atomicMin(&s_w[1], j);
+    }
+  __syncthreads();
+  const int j0 = s_w[0], j1 = s_w[1];
+  for (int j = j0 + (int)threadIdx.x; j < j1; j += blockDim.x)
+    if (valid_rows[j] > 0) atomicMax(&s_w[2], j);
+  __syncthreads();
+  const int last = s_w[2];
+  const int64_t src = last < 0 ? j0 * B : last * B + valid_rows[last];  // (its block may be the next one, or past the run)
+  const int64_t first = src + 1 - b * B;
+  return CkptPad{src, (int)(first < 0 ? 0 : first > B ? B : first)};
+}
+
+constexpr int CKPT_COLS = 64;  // columns of the gate_up checkpoint per workgroup
+__global__ __launch_bounds__(256) void ckpt_pad_gate_up_kernel(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
+                                                               const int32_t* __restrict__ n_active,
+                                                               const int32_t* __restrict__ valid_rows, int64_t B, int64_t E,
+                                                               int64_t cols) {
+  __shared__ int s_w[3];
+  __shared__ uint16_t s_v[CKPT_COLS];
+  const int64_t b = blockIdx.x;
+  const CkptPad p = ckpt_pad_of(b, b2e, n_active, valid_rows, B, E, s_w);
+  if (p.first >= B) return;
+  for (int64_t c0 = (int64_t)blockIdx.y * CKPT_COLS; c0 < cols; c0 += (int64_t)gridDim.y * CKPT_COLS) {
+    __syncthreads();  // (s_v of the pass before)
+    const int nc = (int)(cols - c0 < CKPT_COLS ? cols - c0 : CKPT_COLS);
+    if ((int)threadIdx.x < nc) {
+      uint16_t v = 0;
+      if (p.src >= 0) v = ck[(p.src / B * cols + c0 + threadIdx.x) * B + p.src % B];
+      s_v[threadIdx.x] = v;
+    }
+    __syncthreads();
+    uint16_t* base = ck + (b * cols + c0) * B;
+    if (B % 8 == 0 && ((uintptr_t)ck & 15) == 0) {
+      // pieces of eight rows, 2^lw threads side by side along a column; the first piece may begin with rows to keep
+      const int g0 = p.first / 8, g1 = (int)(B / 8), lw = g1 >= 64 ? 6 : g1 >= 32 ? 5 : g1 >= 16 ? 4 : 3;
+      for (int col = (int)threadIdx.x >> lw; col < nc; col += 256 >> lw) {
+        const uint32_t v = s_v[col], w = v | (v << 16);
+        for (int gr = g0 + ((int)threadIdx.x & ((1 << lw) - 1)); gr < g1; gr += 1 << lw) {
+          uint16_t* q = base + (int64_t)col * B + gr * 8;
+          if (gr * 8 >= p.first) *(uint4*)q = make_uint4(w, w, w, w);
+          else
+            for (int r = p.first - gr * 8; r < 8; ++r) q[r] = (uint16_t)v;
+        }
+      }
+    } else {
+      const int nr = (int)B - p.first;
+      for (int64_t i = threadIdx.x; i < (int64_t)nc * nr; i += 256) base[i / nr * B + p.first + i % nr] = s_v[i / nr];
+    }
+  }
+}
+
+constexpr int CKPT_ROWS = 16;  // rows of the down checkpoint per workgroup
+__global__ __launch_bounds__(256) void ckpt_pad_down_kernel(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
+                                                            const int32_t* __restrict__ n_active,
+                                                            const int32_t* __restrict__ valid_rows, int64_t B, int64_t E,
+                                                            int64_t H) {
+  __shared__ int s_w[3];
+  const int64_t b = blockIdx.x;
+  const CkptPad p = ckpt_pad_of(b, b2e, n_active, valid_rows, B, E, s_w);
+  for (int64_t rb = (int64_t)blockIdx.y * CKPT_ROWS; rb < B; rb += (int64_t)gridDim.y * CKPT_ROWS) {
+    const int64_t r0 = rb < p.first ? p.first : rb, r1 = rb + CKPT_ROWS < B ? rb + CKPT_ROWS : B;
+    if (r0 >= r1) continue;
+    if (H % 8 == 0 && ((uintptr_t)ck & 15) == 0) {
+      for (int64_t h = threadIdx.x; h < H / 8; h += 256) {
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (p.src >= 0) v = *(const uint4*)(ck + p.src * H + h * 8);
+        for (int64_t r = r0; r < r1; ++r) *(uint4*)(ck + (b * B + r) * H + h * 8) = v;
+      }
+    } else {
+      for (int64_t h = threadIdx.x; h < H; h += 256) {
+        const uint16_t v = p.src >= 0 ? ck[p.src * H + h] : (uint16_t)0;
+        for (int64_t r = r0; r < r1; ++r) ck[(b * B + r) * H + h] = v;
+      }
+    }
+  }
 }
 
 // The whole bookkeeping of a small problem (decode-sized: a few ten thousand slots) by ONE workgroup of 1024
@@ -123,7 +237,7 @@ __global__ __launch_bounds__(1024) void prep_small_kernel(
     int32_t* __restrict__ valid_rows, int32_t* __restrict__ cnt, int64_t clear_words, int32_t* __restrict__ n_chunks,
     int32_t* __restrict__ chunk_slot, int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert,
     int32_t* __restrict__ chunk_xcd, int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks,
-    int32_t* __restrict__ off, int32_t* __restrict__ cursor, int32_t* __restrict__ list, bool whole_blocks) {
+    int32_t* __restrict__ off, int32_t* __restrict__ cursor, int32_t* __restrict__ list, bool pad_row) {
   __shared__ int s_ws[16];
   __shared__ int s_first_zero;
   for (int64_t i = threadIdx.x; i < clear_words; i += blockDim.x) cnt[i] = 0;  // cnt and cursor are adjacent
@@ -183,7 +297,7 @@ __global__ __launch_bounds__(1024) void prep_small_kernel(
   __threadfence_block();
   __syncthreads();
   build_chunks(b2e, n_active, valid_rows, N, B, E, n_chunks, chunk_slot, chunk_rows, chunk_expert, chunk_xcd, q_chunk,
-               q_off, max_chunks, s_ws, whole_blocks);
+               q_off, max_chunks, s_ws, pad_row);
   __syncthreads();
   inv_scan(cnt, off, n_real, s_ws);
   __threadfence_block();
@@ -326,7 +440,7 @@ Bookkeeping carve_bookkeeping(void* base, int64_t T1, int64_t N, int64_t B) {
 constexpr int64_t PREP_SMALL_SLOTS = 40960, PREP_SMALL_TOKENS = 4096;
 
 int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hipStream_t s) {
-  const bool whole_blocks = a->gate_up_activations_T != nullptr || a->down_activations != nullptr;
+  const bool pad_row = a->gate_up_activations_T != nullptr || a->down_activations != nullptr;
   // cnt and cursor are adjacent: one clear covers both.  A fill kernel rather than a memset
   // node, so that the sequence stays safe to record into a HIP graph.
   const int64_t clear_words = (int64_t)((uint8_t*)k.off - (uint8_t*)k.cnt) / 4;
@@ -334,7 +448,7 @@ int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hi
     hipLaunchKernelGGL(prep_small_kernel, dim3(1), dim3(1024), 0, s, a->token_position_to_id, a->block_to_expert,
                        a->conditions, a->n_conditions, a->N, a->B, a->E, n_real, k.n_active, k.valid_rows, k.cnt,
                        clear_words, k.n_chunks, k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk,
-                       k.q_off, k.max_chunks, k.off, k.cursor, k.list, whole_blocks);
+                       k.q_off, k.max_chunks, k.off, k.cursor, k.list, pad_row);
     MOE_CHECK_LAUNCH();
     return MOE_OK;
   }
@@ -347,7 +461,7 @@ int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hi
   MOE_CHECK_LAUNCH();
   hipLaunchKernelGGL(chunks_and_offsets_kernel, dim3(2), dim3(1024), 0, s, a->block_to_expert, k.n_active, k.valid_rows,
                      a->N, a->B, a->E, k.n_chunks, k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk, k.q_off,
-                     k.max_chunks, k.cnt, k.off, n_real, whole_blocks);
+                     k.max_chunks, k.cnt, k.off, n_real, pad_row);
   MOE_CHECK_LAUNCH();
   const int64_t slots = a->N * a->B;
   const unsigned gs = (unsigned)((slots + 255) / 256);
@@ -358,10 +472,24 @@ int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hi
 }
 
 int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int64_t N, int64_t B, int64_t E,
-                       hipStream_t s) {
+                       hipStream_t s, int32_t* n_active_out, bool all_blocks) {
   hipLaunchKernelGGL(plan_chunks_kernel, dim3(1), dim3(1024), 0, s, block_to_expert, k.n_active, k.valid_rows, N, B, E,
                      k.n_chunks, k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk, k.q_off,
-                     k.max_chunks);
+                     k.max_chunks, n_active_out, all_blocks);
+  MOE_CHECK_LAUNCH();
+  return MOE_OK;
+}
+
+int launch_ckpt_pad(int stage, uint16_t* ck, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s) {
+  const int64_t cols = 2 * a->I;
+  const int64_t gy = stage == 1 ? (cols + CKPT_COLS - 1) / CKPT_COLS : (a->B + CKPT_ROWS - 1) / CKPT_ROWS;
+  const dim3 grid((unsigned)a->N, (unsigned)(gy < 65535 ? gy : 65535));
+  if (stage == 1)
+    hipLaunchKernelGGL(ckpt_pad_gate_up_kernel, grid, dim3(256), 0, s, ck, a->block_to_expert, k.n_active, k.valid_rows, a->B,
+                       a->E, cols);
+  else
+    hipLaunchKernelGGL(ckpt_pad_down_kernel, grid, dim3(256), 0, s, ck, a->block_to_expert, k.n_active, k.valid_rows, a->B,
+                       a->E, a->H);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
