@@ -9,9 +9,13 @@
 //                      token_position_to_id with the pad id.
 //   2. layout_kernel   one workgroup: per expert the sum of the slabs' counts; blocks per expert, padding blocks to the last
 //                      expert (or split), exclusive scan -> first slot of every expert, block_to_expert, conditions
-//   3. scatter_kernel  per slab, the same bitmaps again: a token's rank among the tokens of its expert is the
+//   3. scatter_kernel  (with a plan one more workgroup, which cuts the chunks) per slab, the same bitmaps again: a token's rank among the tokens of its expert is the
 //                      number of set bits below its own, plus the slab's offset; writes the token ids
-// The work is latency bound (a few hundred KB of int32), so each step is a single small launch.
+// The work is latency bound (a few hundred KB of int32): small launches, and inside each a chain of round trips, which is
+// what was shortened where it could be (counts handed on in LDS, ids kept in registers, scans without LDS shuffles, the
+// chunks cut beside the scatter).  Block build with plan, us: T = 8192, top-8 of 256 experts 37 -> 23; T = 1999, top-4 of
+// 32 experts 25 -> 17; one launch: T = 1, top-8 of 256 experts 14 -> 12, T = 256, top-2 of 8 12 -> 9.5, T = 1024, top-4 of 8
+// 33 -> 25.
 #include <mutex>
 
 #include "chunks.hpp"
@@ -35,26 +39,35 @@ struct BlockPlanOut {
   int32_t* valid_rows;  // [N]   rows of a block that hold tokens (they are packed from the block's first row)
   int32_t* off;         // [T+1] first list entry of token t: t * k
   int32_t* list;        // [T*k] slot of (t, j), or -1 (id outside [0, E), an id listed before in the row, no room)
-  // The layout step's workgroup goes on to cut the expert chunks and fill the work queues (build_chunks) when
-  // chunks_inline is set: the tables that takes (all of the blockwise layer's Bookkeeping).
+  // The layout step of the single launch goes on to cut the expert chunks and fill the work queues (build_chunks) when
+  // chunks_inline is set; otherwise the scatter launch does.  The tables that takes: all of the layer's Bookkeeping.
   int chunks_inline;
   Bookkeeping k;
 };
 
 // The bitmaps of 256 tokens: bit (tid & 31) of word bm[(tid >> 5) * E + e] says that token t0 + tid selected
 // expert e.  Ids outside [0, E) are ignored; an id listed twice sets its bit once.
+// Up to 8 ids per token are held in my (-1 past the k-th): requested together, and kept for the second use.
 __device__ __forceinline__ void bb_mark(const int32_t* __restrict__ ids, int64_t t, bool live, int64_t k, int64_t E,
                                         uint32_t* bm, int my[8]) {
   const uint32_t bit = 1u << (threadIdx.x & 31);
   uint32_t* row = bm + (threadIdx.x >> 5) * E;
-  if (k == 8) {  // two 16-byte loads
-    int4 a = make_int4(-1, -1, -1, -1), b = a;
-    if (live) {
-      a = ((const int4*)(ids + t * 8))[0];
-      b = ((const int4*)(ids + t * 8))[1];
+  if (k <= 8) {
+    if (k == 8 && ((uintptr_t)ids & 15) == 0) {  // two 16-byte loads
+      int4 a = make_int4(-1, -1, -1, -1), b = a;
+      if (live) {
+        a = ((const int4*)(ids + t * 8))[0];
+        b = ((const int4*)(ids + t * 8))[1];
+      }
+      my[0] = a.x; my[1] = a.y; my[2] = a.z; my[3] = a.w;
+      my[4] = b.x; my[5] = b.y; my[6] = b.z; my[7] = b.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        my[j] = -1;
+        if (live && j < k) my[j] = ids[t * k + j];
+      }
     }
-    my[0] = a.x; my[1] = a.y; my[2] = a.z; my[3] = a.w;
-    my[4] = b.x; my[5] = b.y; my[6] = b.z; my[7] = b.w;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       if (my[j] >= 0 && my[j] < E) atomicOr(&row[my[j]], bit);
@@ -87,11 +100,12 @@ __device__ __forceinline__ void bb_fill_pad(int32_t* __restrict__ tp2id, int64_t
 // Workgroup = slab of slab_tokens tokens (a multiple of 256).  slab_counts[slab][e] = tokens of the slab that
 // selected e.  All workgroups together also fill token_position_to_id with the pad id, which the scatter
 // overwrites where tokens sit.
-// (slab = this workgroup's slab, n_wg = workgroups that share the pad fill; bb_lds = 9 E words of LDS)
+// (slab = this workgroup's slab, n_wg = workgroups that share the pad fill; bb_lds = 9 E words of LDS, which keep the
+// bitmaps of the last 256 tokens and, behind them, the slab's counts; my: this thread's ids of the last pass)
 __device__ __forceinline__ void bb_count_body(const int32_t* __restrict__ ids, int64_t T, int64_t k, int64_t E,
                                               int64_t slab_tokens, int32_t* __restrict__ slab_counts,
                                               int32_t* __restrict__ tp2id, int64_t NB, int pad_id, int64_t slab,
-                                              int64_t n_wg, uint32_t* bb_lds) {
+                                              int64_t n_wg, uint32_t* bb_lds, int my[8]) {
   uint32_t* bm = bb_lds;            // [8][E]
   int* run = (int*)(bb_lds + 8 * E);  // [E]
   for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) run[e] = 0;
@@ -100,13 +114,13 @@ __device__ __forceinline__ void bb_count_body(const int32_t* __restrict__ ids, i
     for (int64_t i = threadIdx.x; i < 8 * E; i += BB_THREADS) bm[i] = 0;
     __syncthreads();
     const int64_t t = t_begin + sub + threadIdx.x;
-    int my[8];
     bb_mark(ids, t, t < T, k, E, bm, my);
     __syncthreads();
     for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) run[e] += bb_bits(bm, E, e);
     __syncthreads();
   }
-  for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) slab_counts[slab * E + e] = run[e];
+  if (slab_counts)
+    for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) slab_counts[slab * E + e] = run[e];
   bb_fill_pad(tp2id, NB, pad_id, slab, n_wg);
 }
 
@@ -115,7 +129,8 @@ __global__ __launch_bounds__(BB_THREADS) void bb_count_kernel(const int32_t* __r
                                                              int32_t* __restrict__ slab_counts,
                                                              int32_t* __restrict__ tp2id, int64_t NB, int pad_id) {
   extern __shared__ uint32_t bb_lds[];
-  bb_count_body(ids, T, k, E, slab_tokens, slab_counts, tp2id, NB, pad_id, blockIdx.x, gridDim.x, bb_lds);
+  int my[8];
+  bb_count_body(ids, T, k, E, slab_tokens, slab_counts, tp2id, NB, pad_id, blockIdx.x, gridDim.x, bb_lds, my);
 }
 
 // ws layout: first_slot[E] | slab_counts[BB_SLABS_MAX][E]
@@ -126,7 +141,9 @@ __device__ __forceinline__ void bb_layout_body(const int32_t* __restrict__ slab_
                                                int32_t* __restrict__ first_slot, int32_t* __restrict__ block_to_expert,
                                                int32_t* __restrict__ conditions, int64_t n_conditions, int64_t E,
                                                int64_t B, int64_t N, int use_split_padding,
-                                               int32_t* __restrict__ status, int* s_nb, const BlockPlanOut plan) {
+                                               int32_t* __restrict__ status, int* s_nb, const BlockPlanOut plan,
+                                               const int* lds_counts = nullptr) {
+  // lds_counts: the counts of the only slab, where this workgroup has taken them itself (first_slot may then be null)
   // s_nb: [E] blocks per expert, then [E] first block of every expert, then [E] tokens of every expert
   int* s_first = s_nb + E;
   int* s_count = s_nb + 2 * E;
@@ -135,10 +152,24 @@ __device__ __forceinline__ void bb_layout_body(const int32_t* __restrict__ slab_
   __shared__ int s_ws[16];
   // blocks per expert and their sum
   int mine = 0;
-  for (int64_t e = threadIdx.x; e < E; e += nthr) {
-    int64_t count = 0;
+  if (!lds_counts) {
+    // four threads share an expert's slabs (a sum by one thread was eight round trips to the L2 at 64 slabs)
+    constexpr int PARTS = 4;
+    const int64_t per = (n_slabs + PARTS - 1) / PARTS;
+    for (int64_t e = threadIdx.x; e < E; e += nthr) s_count[e] = 0;
+    __syncthreads();
+    for (int64_t i = threadIdx.x; i < PARTS * E; i += nthr) {
+      const int64_t part = i / E, e = i - part * E;
+      const int64_t end = (part + 1) * per < n_slabs ? (part + 1) * per : n_slabs;
+      int count = 0;
 #pragma unroll 8
-    for (int64_t sl = 0; sl < n_slabs; ++sl) count += slab_counts[sl * E + e];
+      for (int64_t sl = part * per; sl < end; ++sl) count += slab_counts[sl * E + e];
+      atomicAdd(&s_count[e], count);
+    }
+    __syncthreads();
+  }
+  for (int64_t e = threadIdx.x; e < E; e += nthr) {
+    const int64_t count = lds_counts ? lds_counts[e] : s_count[e];
     const int nb = (int)((count + B - 1) / B);
     s_count[e] = (int)count;
     s_nb[e] = nb;
@@ -170,7 +201,8 @@ __device__ __forceinline__ void bb_layout_body(const int32_t* __restrict__ slab_
     carry += total;
   }
   __syncthreads();
-  for (int64_t e = threadIdx.x; e < E; e += nthr) first_slot[e] = (int32_t)((int64_t)s_first[e] * B);
+  if (first_slot)
+    for (int64_t e = threadIdx.x; e < E; e += nthr) first_slot[e] = (int32_t)((int64_t)s_first[e] * B);
   // A block's expert is the last one whose first block is not beyond it (experts without blocks share their first
   // block with the next expert, so the last of equals is the one that owns the block).  A search per block: the
   // padding blocks of a small batch all belong to one expert, and a loop per expert would write them one by one.
@@ -221,11 +253,15 @@ __global__ __launch_bounds__(1024) void bb_layout_kernel(const int32_t* __restri
 __device__ __forceinline__ void bb_scatter_body(const int32_t* __restrict__ ids, int64_t T, int64_t k, int64_t E,
                                                 int64_t slab_tokens, const int32_t* __restrict__ slab_counts,
                                                 const int32_t* __restrict__ first_slot, int32_t* __restrict__ tp2id,
-                                                int64_t NB, int64_t slab, uint32_t* bb_lds, const BlockPlanOut plan) {
+                                                int64_t NB, int64_t slab, uint32_t* bb_lds, const BlockPlanOut plan,
+                                                const int* lds_first = nullptr, int64_t B = 0, bool marked = false,
+                                                const int* marked_ids = nullptr) {
+  // lds_first: every expert's first block in LDS, in place of first_slot; marked: the bitmaps in LDS and marked_ids are
+  // those of the only 256 tokens
   uint32_t* bm = bb_lds;
   int* run = (int*)(bb_lds + 8 * E);
   for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) {
-    int before = first_slot[e];
+    int before = lds_first ? (int)(lds_first[e] * B) : first_slot[e];
 #pragma unroll 8
     for (int64_t sl = 0; sl < slab; ++sl) before += slab_counts[sl * E + e];
     run[e] = before;
@@ -234,37 +270,48 @@ __device__ __forceinline__ void bb_scatter_body(const int32_t* __restrict__ ids,
   const int wd = threadIdx.x >> 5;
   const uint32_t below = (1u << (threadIdx.x & 31)) - 1u;
   for (int64_t sub = 0; sub < slab_tokens && t_begin + sub < T; sub += BB_THREADS) {
-    for (int64_t i = threadIdx.x; i < 8 * E; i += BB_THREADS) bm[i] = 0;
-    __syncthreads();
     const int64_t t = t_begin + sub + threadIdx.x;
     const bool live = t < T;
     int my[8];
-    bb_mark(ids, t, live, k, E, bm, my);
+    if (marked) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) my[j] = marked_ids[j];
+    } else {
+      for (int64_t i = threadIdx.x; i < 8 * E; i += BB_THREADS) bm[i] = 0;
+      __syncthreads();
+      bb_mark(ids, t, live, k, E, bm, my);
+    }
     __syncthreads();
     if (live) {
       // the slot of token t under expert e: the expert's first free slot + the tokens of e before t in this pass
       auto place = [&](int e) -> int32_t {
         if (e < 0 || e >= E) return -1;
-        int r = __popc(bm[wd * E + e] & below);
-        for (int w = 0; w < wd; ++w) r += __popc(bm[w * E + e]);
+        // (all eight words, requested together: a walk to the token's own is up to seven LDS round trips)
+        int r = 0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) r += __popc(bm[w * E + e] & (w < wd ? ~0u : w == wd ? below : 0u));
         const int64_t pos = (int64_t)run[e] + r;
         if (pos >= NB) return -1;
         tp2id[pos] = (int32_t)t;
         return (int32_t)pos;
       };
       // (for the plan: an id that the row lists twice owns one slot, the second mention adds nothing)
-      if (k == 8) {
+      if (k <= 8) {
         int32_t slot[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          slot[j] = place(my[j]);
+          slot[j] = j < k ? place(my[j]) : -1;
 #pragma unroll
           for (int j2 = 0; j2 < j; ++j2)
             if (my[j2] == my[j]) slot[j] = -1;
         }
-        if (plan.list) {  // two 16-byte stores (the plan is 256-byte aligned)
+        if (plan.list && k == 8) {  // two 16-byte stores (the plan is 256-byte aligned)
           ((int4*)(plan.list + t * 8))[0] = make_int4(slot[0], slot[1], slot[2], slot[3]);
           ((int4*)(plan.list + t * 8))[1] = make_int4(slot[4], slot[5], slot[6], slot[7]);
+        } else if (plan.list) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (j < k) plan.list[t * k + j] = slot[j];
         }
       } else {
         for (int64_t j = 0; j < k; ++j) {
@@ -282,37 +329,59 @@ __device__ __forceinline__ void bb_scatter_body(const int32_t* __restrict__ ids,
         if (t == T - 1) plan.off[T] = (int32_t)(T * k);
       }
     }
+    if (sub + BB_THREADS >= slab_tokens || t_begin + sub + BB_THREADS >= T) break;  // (the last pass)
     __syncthreads();
     for (int64_t e = threadIdx.x; e < E; e += BB_THREADS) run[e] += bb_bits(bm, E, e);
     __syncthreads();  // the bitmaps are cleared next
   }
 }
 
-__global__ __launch_bounds__(BB_THREADS) void bb_scatter_kernel(const int32_t* __restrict__ ids, int64_t T, int64_t k,
+// PLANNED: workgroups of 1024 threads, of which the scattering ones use 256.
+template <bool PLANNED>
+__global__ __launch_bounds__(PLANNED ? 1024 : BB_THREADS) void bb_scatter_kernel(const int32_t* __restrict__ ids, int64_t T, int64_t k,
                                                                int64_t E, int64_t slab_tokens,
                                                                const int32_t* __restrict__ slab_counts,
                                                                const int32_t* __restrict__ first_slot,
                                                                int32_t* __restrict__ tp2id, int64_t NB,
-                                                               const BlockPlanOut plan) {
+                                                               const BlockPlanOut plan,
+                                                               const int32_t* __restrict__ block_to_expert, int64_t N,
+                                                               int64_t B) {
   extern __shared__ uint32_t bb_lds[];
-  bb_scatter_body(ids, T, k, E, slab_tokens, slab_counts, first_slot, tp2id, NB, blockIdx.x, bb_lds, plan);
+  int64_t slab = blockIdx.x;
+  // With a plan the first workgroup cuts the chunks while the others scatter: both wait for the layout alone.
+  if constexpr (PLANNED) {
+    __shared__ int s_ws[16];
+    if (slab == 0) {
+      build_chunks(block_to_expert, plan.n_active, plan.valid_rows, N, B, E, plan.k.n_chunks, plan.k.chunk_slot,
+                   plan.k.chunk_rows, plan.k.chunk_expert, plan.k.chunk_xcd, plan.k.q_chunk, plan.k.q_off,
+                   plan.k.max_chunks, s_ws, false);
+      return;
+    }
+    --slab;
+    if (threadIdx.x >= BB_THREADS) return;  // (whole waves: a barrier counts the waves that have not ended)
+  }
+  bb_scatter_body(ids, T, k, E, slab_tokens, slab_counts, first_slot, tp2id, NB, slab, bb_lds, plan);
 }
 
-// Few tokens (one slab): the three steps in one launch by one workgroup.  What one step leaves in global memory
-// (the slab's counts, the first slots, the pad ids under the tokens' slots) the next reads or overwrites after a
-// workgroup barrier: all of it goes through this CU's L1.
+// Few tokens (one slab): the three steps in one launch by one workgroup, which hand the counts and the first blocks on in
+// LDS (and up to 256 tokens their bitmaps and ids).  The pad ids under the tokens' slots are overwritten after a workgroup
+// barrier, through this CU's L1.
 __global__ __launch_bounds__(BB_THREADS) void bb_single_slab_kernel(
-    const int32_t* __restrict__ ids, int64_t T, int64_t k, int64_t E, int64_t slab_tokens,
-    int32_t* __restrict__ slab_counts, int32_t* __restrict__ first_slot, int32_t* __restrict__ tp2id, int64_t NB,
-    int pad_id, int32_t* __restrict__ block_to_expert, int32_t* __restrict__ conditions, int64_t n_conditions, int64_t B,
-    int64_t N, int use_split_padding, int32_t* __restrict__ status, const BlockPlanOut plan) {
+    const int32_t* __restrict__ ids, int64_t T, int64_t k, int64_t E, int64_t slab_tokens, int32_t* __restrict__ tp2id,
+    int64_t NB, int pad_id, int32_t* __restrict__ block_to_expert, int32_t* __restrict__ conditions, int64_t n_conditions,
+    int64_t B, int64_t N, int use_split_padding, int32_t* __restrict__ status, const BlockPlanOut plan) {
   extern __shared__ uint32_t bb_lds[];  // 9 E words of the count / scatter steps, then 3 E of the layout step
-  bb_count_body(ids, T, k, E, slab_tokens, slab_counts, tp2id, NB, pad_id, 0, 1, bb_lds);
+  int my[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) my[j] = -1;
+  bb_count_body(ids, T, k, E, slab_tokens, nullptr, tp2id, NB, pad_id, 0, 1, bb_lds, my);
   __syncthreads();
-  bb_layout_body(slab_counts, 1, first_slot, block_to_expert, conditions, n_conditions, E, B, N, use_split_padding,
-                 status, (int*)(bb_lds + 9 * E), plan);
+  int* s_nb = (int*)(bb_lds + 9 * E);
+  bb_layout_body(nullptr, 1, nullptr, block_to_expert, conditions, n_conditions, E, B, N, use_split_padding, status, s_nb,
+                 plan, (const int*)(bb_lds + 8 * E));
   __syncthreads();
-  bb_scatter_body(ids, T, k, E, slab_tokens, slab_counts, first_slot, tp2id, NB, 0, bb_lds, plan);
+  bb_scatter_body(ids, T, k, E, slab_tokens, nullptr, nullptr, tp2id, NB, 0, bb_lds, plan, s_nb + E, B,
+                  T <= BB_THREADS && k <= 8, my);
 }
 
 }  // namespace moe
@@ -349,7 +418,7 @@ int build_blocks_launch(const int32_t* topk_ids, int64_t T, int64_t k, int64_t E
     // (the chunk builder's tables are static LDS of the kernel: it runs in this launch while both fit in 64 KB)
     plan.chunks_inline = planned && lds + 3 * E * sizeof(int32_t) + BB_CHUNKS_STATIC_LDS <= 65536;
     hipLaunchKernelGGL(bb_single_slab_kernel, dim3(1), dim3(BB_THREADS), lds + 3 * E * sizeof(int32_t), s, topk_ids, T,
-                       k, E, slab_tokens, slab_counts, first_slot, token_position_to_id, N * B,
+                       k, E, slab_tokens, token_position_to_id, N * B,
                        skip_token ? -1 : (int)T, block_to_expert, conditions, n_conditions, B, N, use_split_padding,
                        status_out, plan);
     MOE_CHECK_LAUNCH();
@@ -359,13 +428,18 @@ int build_blocks_launch(const int32_t* topk_ids, int64_t T, int64_t k, int64_t E
   hipLaunchKernelGGL(bb_count_kernel, dim3((unsigned)n_slabs), dim3(BB_THREADS), lds, s, topk_ids, T, k, E, slab_tokens,
                      slab_counts, token_position_to_id, N * B, skip_token ? -1 : (int)T);
   MOE_CHECK_LAUNCH();
-  plan.chunks_inline = planned;  // (3 E words of dynamic LDS beside the chunk builder's tables: E <= 1024 fits)
-  hipLaunchKernelGGL(bb_layout_kernel, dim3(1), dim3(planned ? 1024 : BB_THREADS), 3 * E * sizeof(int), s, slab_counts, n_slabs,
+  hipLaunchKernelGGL(bb_layout_kernel, dim3(1), dim3(1024), 3 * E * sizeof(int), s, slab_counts, n_slabs,
                      first_slot, block_to_expert, conditions, n_conditions, E, B, N, use_split_padding, status_out,
                      plan);
   MOE_CHECK_LAUNCH();
-  hipLaunchKernelGGL(bb_scatter_kernel, dim3((unsigned)n_slabs), dim3(BB_THREADS), lds, s, topk_ids, T, k, E,
-                     slab_tokens, slab_counts, first_slot, token_position_to_id, N * B, plan);
+  // (9 E words of dynamic LDS beside the chunk builder's tables: a plan exists up to E = 512, just under 64 KB in all)
+  const dim3 grid((unsigned)(n_slabs + (planned ? 1 : 0)));
+  if (planned)
+    hipLaunchKernelGGL(bb_scatter_kernel<true>, grid, dim3(1024), lds, s, topk_ids, T, k, E, slab_tokens, slab_counts,
+                       first_slot, token_position_to_id, N * B, plan, block_to_expert, N, B);
+  else
+    hipLaunchKernelGGL(bb_scatter_kernel<false>, grid, dim3(BB_THREADS), lds, s, topk_ids, T, k, E, slab_tokens, slab_counts,
+                       first_slot, token_position_to_id, N * B, plan, block_to_expert, N, B);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

@@ -90,7 +90,10 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
   if (threadIdx.x == 0) s_runs = 0;
   __threadfence_block();
   __syncthreads();
-  if (runs > 0) atomicAdd(&s_runs, runs);
+  // (one addition per wave: at decode sizes every expert is a run, and 256 of them on one word took 2 us)
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) runs += __shfl_xor(runs, o, 64);
+  if ((threadIdx.x & 63) == 0 && runs > 0) atomicAdd(&s_runs, runs);
   __syncthreads();
   // How many chunks of one expert the large-tile GEMMs work on side by side (the kernels read it behind q_off).
   // While experts hold fewer than three chunks on average: 1, i.e. a round of an XCD's workgroups covers the column

@@ -141,24 +141,25 @@ __device__ __forceinline__ float block_max(float v, float* red) {
 // Exclusive prefix sum of v over the workgroup (blockDim.x a multiple of 64, at most 1024): shuffles
 // inside a wave, one exchange of the wave totals through `ws` (16 ints).  *total = sum over the workgroup.
 __device__ __forceinline__ int block_excl_scan(int v, int* ws, int* total) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  int inc = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int t = __shfl_up(inc, o, 64);
-    if (lane >= o) inc += t;
-  }
+  // (moves between lanes with DPP: a shuffle goes through LDS, and six of them in a row were most of a scan, which the
+  // block build and the chunk builder are chains of)
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), nw = blockDim.x >> 6;
+  auto row_scan = [](int x) {  // inclusive over each 16 lanes: row_shr by 1, 2, 4, 8, zeros shifted in
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    return x;
+  };
+  int inc = row_scan(v);
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  inc += __builtin_amdgcn_update_dpp(0, inc, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
   __syncthreads();  // `ws` may still be read from a previous call
   if (lane == 63) ws[w] = inc;
   __syncthreads();
-  int base = 0, tot = 0;
-  for (int i = 0; i < nw; ++i) {
-    const int t = ws[i];
-    base += (i < w) ? t : 0;
-    tot += t;
-  }
-  *total = tot;
-  return base + inc - v;
+  const int t = row_scan(lane < nw ? ws[lane] : 0);  // (at most 16 waves)
+  *total = __builtin_amdgcn_readlane(t, 15);
+  return (w > 0 ? __builtin_amdgcn_readlane(t, w > 0 ? w - 1 : 0) : 0) + inc - v;
 }
 
 // ---- activation functions (ActFnType, common_types.py:32-36) ---------------------------

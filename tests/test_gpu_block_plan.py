@@ -155,6 +155,12 @@ def test_plan_says_what_the_tables_say(T, k, E, B, skip, split, alpha, spoil):
     assert 1 <= int(p["q_off"][8 * (CLASSES + 1)]) <= 8
 
 
+@pytest.mark.parametrize("T,k,E,B,spoil", [
+    (256, 3, 16, 128, True), (257, 7, 16, 128, False), (1025, 9, 512, 128, True), (2000, 4, 512, 64, False)])
+def test_plan_edges(T, k, E, B, spoil):
+    test_plan_says_what_the_tables_say(T, k, E, B, False, False, None, spoil)
+
+
 def test_plan_refusals():
     import torch
     from nkilib import _native as nv

@@ -45,3 +45,15 @@ def test_build_blocks_bit_exact(T, k, E, B, skip, split, alpha):
     _, _, cond2 = build_token_blocks(i32_tensor(router, dev), E, B, N, skip_token=skip, use_split_padding=split,
                                      n_conditions=N + 2)
     assert np.array_equal(cond2.cpu().numpy(), g_cond2)
+
+
+@pytest.mark.parametrize("T,k,E,B", [
+    (256, 3, 16, 128),    # one pass of 256 tokens: the bitmaps are kept between the two uses
+    (257, 7, 16, 128),    # two passes
+    (256, 9, 20, 64),     # more ids per token than are held in registers
+    (1025, 5, 40, 128),   # the first size of the launches in several workgroups
+    (1500, 2, 1024, 64),  # the largest number of experts
+    (16385, 4, 24, 512),  # slabs of more than one pass, the slabs not a multiple of the parts they are summed in
+])
+def test_build_blocks_edges(T, k, E, B):
+    test_build_blocks_bit_exact(T, k, E, B, False, False, None)
