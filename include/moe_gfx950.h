@@ -284,9 +284,8 @@ typedef struct moe_bwmm_args {
    * moe_prepare_kmajor_weights (they depend on the weights only).  Both NULL: every call makes its own copies
    * in the workspace.  (What a copy holds depends on the kind, the weight type and the shape only -- for bf16
    * weights with H % 256 == 0, and fp8-row weights with H % 512 == 0, the order
-   * the large-tile kernels read, otherwise K-contiguous rows -- so one pair serves every call with those weights;
-   * a bf16 call on such a shape that asks for activation checkpoints runs the general kernel and makes its own
-   * K-contiguous copies regardless.)  MXFP8 kind: the x4 layouts are K-major already and are read in place when both are NULL;
+   * the large-tile kernels read, otherwise K-contiguous rows -- so one pair serves every call with those weights,
+   * activation checkpoints included.)  MXFP8 kind: the x4 layouts are K-major already and are read in place when both are NULL;
    * on shapes with H % 512 == 0 and I % 128 == 0 the same two calls make a copy of the gate/up weights in the
    * order the kernel reads them (each workgroup then reads its weights as contiguous 32 KB runs: the gate/up GEMM
    * is 5 % faster at H = 7168, I = 2048 with 8-bit weights, for a second copy of those weights in memory); used
@@ -309,7 +308,8 @@ typedef struct moe_bwmm_args {
   /* Nullable, no counterpart in the reference: the bookkeeping that moe_build_blocks_plan wrote for exactly these
    * token_position_to_id / block_to_expert tables (see there for the conditions under which it may be passed).
    * With it moe_blockwise launches no bookkeeping kernels of its own.  Ignored when activation checkpoints are
-   * requested, unless the call goes through moe_blockwise_stages with MOE_STAGE_CHECKPOINT_PLAN.  The plan is read only; it may be passed to any number of calls. */
+   * requested, unless the call goes through moe_blockwise_stages with MOE_STAGE_CHECKPOINT_PLAN.  The plan is read
+   * only; it may be passed to any number of calls. */
   const void* block_plan;
   size_t block_plan_bytes;
   /* Nullable, no counterpart in the reference: seven hipEvent_t of the caller's (null entries are skipped).  The

@@ -9,8 +9,9 @@
 //                      token_position_to_id with the pad id.
 //   2. layout_kernel   one workgroup: per expert the sum of the slabs' counts; blocks per expert, padding blocks to the last
 //                      expert (or split), exclusive scan -> first slot of every expert, block_to_expert, conditions
-//   3. scatter_kernel  (with a plan one more workgroup, which cuts the chunks) per slab, the same bitmaps again: a token's rank among the tokens of its expert is the
-//                      number of set bits below its own, plus the slab's offset; writes the token ids
+//   3. scatter_kernel  per slab, the same bitmaps again: a token's rank among the tokens of its expert is the
+//                      number of set bits below its own, plus the slab's offset; writes the token ids.  With a plan
+//                      one more workgroup cuts the chunks
 // The work is latency bound (a few hundred KB of int32): small launches, and inside each a chain of round trips, which is
 // what was shortened where it could be (counts handed on in LDS, ids kept in registers, scans without LDS shuffles, the
 // chunks cut beside the scatter).  Block build with plan, us: T = 8192, top-8 of 256 experts 37 -> 23; T = 1999, top-4 of

@@ -73,9 +73,11 @@ def test_router_topk_matches_oracle(T, H, E, k, act, pre, norm, bias, layout):
     "T,H,E,k",
     [
         (1, 128, 8, 2),       # one token, a single part of K
-        (64, 7168, 256, 8),   # the last size of the 64-token tiles, K in 16 parts
-        (65, 7168, 256, 8),   # the first of the 128-token tiles, one row in the second half
-        (129, 1024, 128, 6),  # a second tile of one token, experts in one group of 128
+        (64, 7168, 256, 8),   # a full tile of 64 tokens, K in 16 parts
+        (65, 7168, 256, 8),   # a second tile of one token
+        (4097, 256, 200, 4),  # the first of the 128-token tiles of a group of 256, one token in the last tile
+        (8193, 192, 100, 3),  # the same of a group of 128
+        (129, 1024, 128, 6),  # a third tile of one token, experts in one group of 128
         (40, 1088, 100, 4),   # K steps that the parts do not share out evenly, padded experts
         (700, 896, 65, 3),    # one expert past the group of 64
         (33000, 192, 60, 2),  # more tiles than CUs: one part
