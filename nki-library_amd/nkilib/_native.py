@@ -5,6 +5,7 @@ Loading is lazy and loud: if the shared library has not been built
 ``NativeLibraryError``.  There is no fallback path.
 """
 
+import contextlib
 import ctypes
 import os
 from ctypes import POINTER, c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
@@ -193,12 +194,23 @@ def check(rc, what):
         kernel_assert(False, f"{what}: {msg} (code {rc})")
 
 
+# A layer over few tokens is bound by the host side of its calls: addresses and streams are handed over as plain
+# integers (every function and field that takes one is declared c_void_p), no Stream object is made to be asked for
+# its handle, and the device is changed only where it is another one.
 def ptr(t):
-    return None if t is None else c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def stream_ptr(device):
-    return c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device):
+    """Context in which ``device`` is the current one."""
+    return _SAME_DEVICE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 _DT = {torch.bfloat16: DT_BF16, torch.float16: DT_FP16, torch.float32: DT_FP32}

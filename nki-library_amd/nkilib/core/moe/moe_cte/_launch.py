@@ -57,11 +57,11 @@ def clear_kmajor_weight_cache():
     _kmajor.clear()
 
 
-def _bytes_of(t):
+def _bytes_of(t, storage):
     """Where a weight tensor's bytes are: (address of its storage, byte offset, byte length; the strides of a tensor that
     is not contiguous).  Views and casts of one allocation (``w.view(torch.int32)`` made anew for every call, say) name
     the same bytes."""
-    return (t.untyped_storage().data_ptr(), t.storage_offset() * t.element_size(), t.numel() * t.element_size(),
+    return (storage.data_ptr(), t.storage_offset() * t.element_size(), t.numel() * t.element_size(),
             None if t.is_contiguous() else t.stride())
 
 
@@ -72,7 +72,7 @@ def _kmajor_weights(L, a, tensors, dev):
     all the allocations are alive (weak references to the storages: an address that was freed and handed out again is a
     different storage) and unchanged (torch's version counters, which views share with their base)."""
     storages = [t.untyped_storage() for t in tensors]
-    key = (*map(_bytes_of, tensors), int(a.kind), int(a.weight_dtype), int(a.E), int(a.H), int(a.I), int(a.I_pad))
+    key = (*map(_bytes_of, tensors, storages), int(a.kind), int(a.weight_dtype), int(a.E), int(a.H), int(a.I), int(a.I_pad))
     sig = tuple(t._version for t in tensors)
     ent = _kmajor.get(key)
     if ent is not None and ent[1] == sig and all(r() is st for r, st in zip(ent[0], storages)):
@@ -83,7 +83,7 @@ def _kmajor_weights(L, a, tensors, dev):
         return None, None
     k0 = torch.empty(n0, dtype=torch.uint8, device=dev)
     k1 = torch.empty(n1, dtype=torch.uint8, device=dev) if n1 else None  # (MXFP8: gate/up only)
-    with torch.cuda.device(dev):
+    with nv.on_device(dev):
         nv.check(L.moe_prepare_kmajor_weights(ctypes.byref(a), nv.ptr(k0), nv.ptr(k1), nv.stream_ptr(dev)),
                  "moe_cte (K-contiguous weight copies)")
     if len(_kmajor) >= _KMAJOR_MAX_ENTRIES:
@@ -260,7 +260,7 @@ def run_blockwise(
     a.workspace_bytes = ws.numel()
     # (the plan counts with activation checkpoints too: it is known to be that of these tables)
     plan_bit = nv.STAGE_CHECKPOINT_PLAN if plan is not None and (checkpoint_gate_up or checkpoint_down) else 0
-    with torch.cuda.device(dev):
+    with nv.on_device(dev):
         if stage_callback is None:
             rc = L.moe_blockwise_stages(ctypes.byref(a), nv.STAGE_ALL | plan_bit, nv.stream_ptr(dev))
         else:

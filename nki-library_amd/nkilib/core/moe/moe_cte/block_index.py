@@ -71,20 +71,23 @@ def build_token_blocks(topk_ids: torch.Tensor, E: int, B: int, N: int = None, sk
     if block_plans and not use_split_padding and T >= 1 and T * k <= N * B and E <= 512:
         plan_words = L.moe_block_plan_bytes(T, B, N, 1 if skip_token else 0) // 4  # (a multiple of 256 bytes)
     buf = torch.empty(plan_words + N * B + N + n_conditions + 1 + ws_words, dtype=torch.int32, device=dev)
-    plan, tp2id, b2e, cond, status, ws = torch.split(buf, [plan_words, N * B, N, n_conditions, 1, ws_words])
-    with torch.cuda.device(dev):
+    _, tp2id, b2e, cond, rest = torch.split(buf, [plan_words, N * B, N, n_conditions, 1 + ws_words])
+    plan_ptr, tp2id_ptr, b2e_ptr, cond_ptr = buf.data_ptr(), tp2id.data_ptr(), b2e.data_ptr(), cond.data_ptr()
+    status_ptr = rest.data_ptr()
+    ws_ptr = status_ptr + 4
+    with nv.on_device(dev):
         if plan_words:
             rc = L.moe_build_blocks_plan(nv.ptr(ids), T, k, E, B, N, 1 if skip_token else 0,
-                                         1 if use_split_padding else 0, nv.ptr(tp2id), nv.ptr(b2e), nv.ptr(cond),
-                                         n_conditions, nv.ptr(ws), ws.numel() * 4, nv.ptr(status), nv.ptr(plan),
-                                         plan.numel() * 4, nv.stream_ptr(dev))
+                                         1 if use_split_padding else 0, tp2id_ptr, b2e_ptr, cond_ptr,
+                                         n_conditions, ws_ptr, ws_words * 4, status_ptr, plan_ptr, plan_words * 4,
+                                         nv.stream_ptr(dev))
         else:
             rc = L.moe_build_blocks(nv.ptr(ids), T, k, E, B, N, 1 if skip_token else 0, 1 if use_split_padding else 0,
-                                    nv.ptr(tp2id), nv.ptr(b2e), nv.ptr(cond), n_conditions, nv.ptr(ws), ws.numel() * 4,
-                                    nv.ptr(status), nv.stream_ptr(dev))
+                                    tp2id_ptr, b2e_ptr, cond_ptr, n_conditions, ws_ptr, ws_words * 4, status_ptr,
+                                    nv.stream_ptr(dev))
     nv.check(rc, "build_token_blocks")
     if check:
-        kernel_assert(int(status.item()) == 0, f"N={N} blocks cannot hold this routing")
+        kernel_assert(int(rest[0].item()) == 0, f"N={N} blocks cannot hold this routing")
     if plan_words:
         st = buf.untyped_storage()
         key = st.data_ptr()
@@ -92,6 +95,6 @@ def build_token_blocks(topk_ids: torch.Tensor, E: int, B: int, N: int = None, sk
             _plans.pop(next(iter(_plans)))
         # (no reference to the allocation is kept: the entry goes when the caller drops the tables)
         _plans[key] = (weakref.ref(st, lambda _ref, key=key: _plans.pop(key, None)), buf._version,
-                       (tp2id.data_ptr(), b2e.data_ptr(), cond.data_ptr(), cond.numel()),
-                       (B, N, T if skip_token else T + 1), (plan.data_ptr(), plan.numel() * 4))
+                       (tp2id_ptr, b2e_ptr, cond_ptr, n_conditions),
+                       (B, N, T if skip_token else T + 1), (plan_ptr, plan_words * 4))
     return tp2id, b2e, cond

@@ -106,7 +106,7 @@ def _rmsnorm_quant_kernel(
     x_dt = nv.dtype_code(hidden, "hidden")
     g_dt = nv.dtype_code(gamma, "ln_w") if gamma is not None else nv.DT_BF16
     stream = nv.stream_ptr(hidden.device)
-    with torch.cuda.device(hidden.device):
+    with nv.on_device(hidden.device):
         if kargs.is_row_quant():
             out = torch.empty((*hidden.shape[:-1], H + DEQUANT_SCALE_SIZE), dtype=torch.uint8, device=hidden.device)
             lb = float(kargs.lower_bound) if kargs.has_lower_bound() else 0.0

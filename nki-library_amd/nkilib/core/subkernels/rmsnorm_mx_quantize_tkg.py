@@ -73,7 +73,7 @@ def rmsnorm_mx_quantize_tkg(
                  (output_residual, "output_residual")):
         if t is not None:
             kernel_assert(t.is_cuda and t.is_contiguous(), f"{n} must be a contiguous device tensor")
-    with torch.cuda.device(x.device):
+    with nv.on_device(x.device):
         rc = L.moe_rmsnorm_quant_mxfp8(nv.ptr(x), nv.dtype_code(x, "input"), nv.ptr(r), nv.ptr(output_residual), nv.ptr(g),
                                        nv.dtype_code(g, "gamma"), nv.ptr(output_quant), nv.ptr(output_scale),
                                        nv.ptr(output), BxS, H, float(eps), int(hidden_actual or H), 1, layout,
@@ -106,7 +106,7 @@ def rmsnorm_mx_quantize(hidden: torch.Tensor, gamma: Optional[torch.Tensor], eps
         r = nv.require_device_tensor(residual, "residual")
         kernel_assert(tuple(r.shape) == (T, H) and r.dtype == x.dtype, "residual must match hidden in shape and dtype")
         out_r = torch.empty_like(x)
-    with torch.cuda.device(x.device):
+    with nv.on_device(x.device):
         rc = L.moe_rmsnorm_quant_mxfp8(nv.ptr(x), nv.dtype_code(x, "hidden"), nv.ptr(r), nv.ptr(out_r), nv.ptr(g),
                                        nv.dtype_code(g, "gamma") if g is not None else nv.DT_BF16, nv.ptr(q), nv.ptr(s),
                                        None, T, H, float(eps), H, 1 if do_norm else 0, nv.MX_TOKEN_MAJOR,
