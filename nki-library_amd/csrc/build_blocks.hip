@@ -15,8 +15,8 @@
 // The work is latency bound (a few hundred KB of int32): small launches, and inside each a chain of round trips, which is
 // what was shortened where it could be (counts handed on in LDS, ids kept in registers, scans without LDS shuffles, the
 // chunks cut beside the scatter).  Block build with plan, us: T = 8192, top-8 of 256 experts 37 -> 23; T = 1999, top-4 of
-// 32 experts 25 -> 17; one launch: T = 1, top-8 of 256 experts 14 -> 12, T = 256, top-2 of 8 12 -> 9.5, T = 1024, top-4 of 8
-// 33 -> 25.
+// 32 experts 25 -> 17; one launch: T = 1, top-8 of 256 experts 14 -> 12, T = 256, top-2 of 8 12 -> 9.5; T = 1024,
+// top-4 of 8, in three launches instead of one 33 -> 14.
 #include <mutex>
 
 #include "chunks.hpp"
@@ -28,7 +28,11 @@ namespace moe {
 constexpr int BB_THREADS = 256;
 
 constexpr int BB_SLABS_MAX = 64;
-constexpr int64_t BB_SINGLE_MAX_TOKENS = 1024;  // up to this many tokens form one slab, built by a single launch
+// Up to this many tokens form one slab, built by a single launch.  Its workgroup takes 256 tokens per pass, the slabs of the
+// three launches take theirs side by side.  Block build with plan, single | three launches, us (without the host, whose two
+// more launches cost what the second pass does): top-8 of 256 experts 17.4 | 13.3 at 257 tokens, 21.2 | 13.3 at 513,
+// 25.5 | 13.4 at 1024; top-2 of 8 experts 12.6 | 11.6, 15.6 | 11.8, 18.7 | 12.1.
+constexpr int64_t BB_SINGLE_MAX_TOKENS = 512;
 constexpr int64_t BB_SINGLE_MAX_SLOTS = 1 << 17;  // one workgroup fills the pad ids of up to this many slots itself
 constexpr int BB_E_MAX = 1024;  // bitmaps and running counts of all experts in LDS: 36 bytes per expert
 constexpr size_t BB_CHUNKS_STATIC_LDS = 46 * 1024;  // static LDS of build_chunks (csrc/chunks.hpp), rounded up

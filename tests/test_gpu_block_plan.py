@@ -156,7 +156,8 @@ def test_plan_says_what_the_tables_say(T, k, E, B, skip, split, alpha, spoil):
 
 
 @pytest.mark.parametrize("T,k,E,B,spoil", [
-    (256, 3, 16, 128, True), (257, 7, 16, 128, False), (1025, 9, 512, 128, True), (2000, 4, 512, 64, False)])
+    (256, 3, 16, 128, True), (257, 7, 16, 128, False), (512, 4, 16, 128, True), (513, 8, 256, 128, True),
+    (1025, 9, 512, 128, True), (2000, 4, 512, 64, False)])
 def test_plan_edges(T, k, E, B, spoil):
     test_plan_says_what_the_tables_say(T, k, E, B, False, False, None, spoil)
 
