@@ -289,9 +289,8 @@ typedef struct moe_bwmm_args {
    * on shapes with H % 512 == 0 and I % 128 == 0 the same two calls make a copy of the gate/up weights in the
    * order the kernel reads them (each workgroup then reads its weights as contiguous 32 KB runs: the gate/up GEMM
    * is 5 % faster at H = 7168, I = 2048 with 8-bit weights, for a second copy of those weights in memory); used
-   * when gate_up_proj_weight_kmajor is set.  The copy holds the block scales of those weights as well (a wave's 64 scale
-   * dwords of a K slice side by side: 12 % of the gate/up time of a decode batch), so it is made again when either
-   * changes; gate_up_proj_scale is then not read by the GEMM.  A copy of the down weights exists for 4-bit weights only
+   * when gate_up_proj_weight_kmajor is set.  The block scales are no part of a copy: every call reads the tables it
+   * passes in gate_up_proj_scale / down_proj_scale.  A copy of the down weights exists for 4-bit weights only
    * (moe_kmajor_weights_bytes(args, 1) is 0 otherwise and the pointer is ignored). */
   const void* gate_up_proj_weight_kmajor;
   const void* down_proj_weight_kmajor;
@@ -350,7 +349,7 @@ int moe_blockwise_stages(const moe_bwmm_args* args, unsigned stages, void* strea
 /* No counterpart in the reference, whose dense weights are consumed N-contiguous ([E, H, 2, I], [E, I_pad, H]):
  * the MFMA operands of the BF16 and FP8_ROW kinds are read along K, so the GEMMs run on K-contiguous copies
  * ([E, 2, I, Hk] and [E, H, Ik]; bf16 for the BF16 kind, fp8 weights widened; fp8 for FP8_ROW; tails zero).
- * A caller whose weights (MXFP8: and block scales) do not change (inference) makes the copies once and passes them in
+ * A caller whose weights do not change (inference) makes the copies once and passes them in
  * moe_bwmm_args.*_kmajor.  moe_kmajor_weights_bytes: bytes of the gate/up (which == 0) or down (which == 1)
  * copy for these args, 0 if the kind has none.  moe_prepare_kmajor_weights fills both (256-byte aligned). */
 size_t moe_kmajor_weights_bytes(const moe_bwmm_args* args, int which);

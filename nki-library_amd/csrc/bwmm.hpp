@@ -111,14 +111,12 @@ int launch_mx_gemm(int stage, const MxArgs& m, unsigned gx, unsigned gy, hipStre
 // mx_rows_fits says whether that kernel is the faster one.
 bool mx_rows_fits(int stage, int wfmt, int64_t rows, int64_t avg_rows, int64_t tiles);
 int launch_mx_rows(int stage, const MxArgs& m, unsigned gx, int64_t max_chunks, int64_t rows, hipStream_t s);
-// Copy of the x4 weights of one stage (1 gate/up, 2 down) and of their block scales in the order the large-tile kernel
-// reads them: for expert e, column tile xt, K slice ks, wave q, load i, lane l the 16 bytes (4-bit weights: 8) that the
-// lane's i-th load of that slice fetches, at ((((e * col_tiles + xt) * nks + ks) * 4 + q) * 8 + i) * 64 + mx_pack_lane(l)
-// such pieces (down stage: + l); behind them (at mx_packed_scales_offset) the dword of scale bytes that the lane loads
-// with the slice, at (((e * col_tiles + xt) * nks + ks) * 4 + q) * 64 + mx_pack_lane(l) dwords.
-int launch_mx_pack_weights(int stage, int fp4, const void* W, const void* W_scale, void* dst, int64_t E, int64_t H, int64_t I,
-                           hipStream_t s);
-size_t mx_packed_scales_offset(int stage, int fp4, int64_t E, int64_t H, int64_t I);
+// Copy of the x4 weights of one stage (1 gate/up, 2 down) in the order the large-tile kernel reads them: for expert
+// e, column tile xt, K slice ks, wave q, load i, lane l the 16 bytes (4-bit weights: 8) that the lane's i-th load of
+// that slice fetches, at ((((e * col_tiles + xt) * nks + ks) * 4 + q) * 8 + i) * 64 + mx_pack_lane(l) such pieces (down
+// stage: + l).  The block scales are no part of it: a copy follows from the weights alone, and the kernels read the
+// scales that the call passes.
+int launch_mx_pack_weights(int stage, int fp4, const void* W, void* dst, int64_t E, int64_t H, int64_t I, hipStream_t s);
 // Place of a lane's piece within a gate/up load.  Lane g * 16 + c holds gate (c < 8) or up columns of partitions
 // 4 (c & 7) ..: the first 16 partitions of gate and up come first, then the last 16, so that the two halves of a column
 // tile that bwmm_rows.hip gives to two workgroups are whole 128-byte lines.

@@ -576,9 +576,8 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const uint32_t w_voff = (uint32_t)pk * (uint32_t)(pk_lane * PK_LANE) +
                           (uint32_t)npk * ((STAGE == 1) ? (uint32_t)((GROWS * g * w_pstride + hcol * nH * a.I + 4 * cl) * ES)
                                                         : (uint32_t)((GROWS * g * w_pstride + 4 * c) * ES));
-  const uint32_t s_voff = (uint32_t)pk * (uint32_t)(pk_lane * 4) +
-                          (uint32_t)npk * ((STAGE == 1) ? (uint32_t)(g * w_pstride + hcol * nH * a.I + 4 * cl)
-                                                        : (uint32_t)(g * w_pstride + 4 * c));
+  const uint32_t s_voff = (STAGE == 1) ? (uint32_t)(g * w_pstride + hcol * nH * a.I + 4 * cl)
+                                       : (uint32_t)(g * w_pstride + 4 * c);
   // bytes of one expert's weights: the reference layout's, or col_tiles x nks runs of 32 KB
   const int64_t w_expert_bytes = pk * ((int64_t)a.col_tiles * nks * PK_SLICE) +
                                  npk * ((STAGE == 1) ? 128 * w_pstride * ES : (int64_t)a.pI * w_pstride * ES);
@@ -647,13 +646,12 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     if (STAGE == 1) {
       colu = (int64_t)tile_tI(t) * 512 + (int64_t)q * tile_Pt(t) + tile_p0(t);
       rw_ = make_rsrc(Wb + (int64_t)t.e * w_expert_bytes, (uint32_t)w_expert_bytes);
-      const int64_t sb = pk * ((int64_t)a.col_tiles * nks * 1024) + npk * (16 * w_pstride);
-      rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * sb, (uint32_t)sb);
+      rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * 16 * w_pstride, (uint32_t)(16 * w_pstride));
     } else {
       colu = tile_h0(t) + 64 * q;
-      const int64_t sb = pk * ((int64_t)a.col_tiles * nks * 1024) + npk * ((int64_t)((a.pI + 7) / 8) * w_pstride);
+      const int64_t sp = (a.pI + 7) / 8;
       rw_ = make_rsrc(Wb + (int64_t)t.e * w_expert_bytes, (uint32_t)w_expert_bytes);
-      rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * sb, (uint32_t)sb);
+      rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * sp * w_pstride, (uint32_t)(sp * w_pstride));
     }
     rw_rec = rw_[2];
     rs_rec = rs_[2];
@@ -662,7 +660,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       const int pr = FP4 ? i : ((i < 4) ? i : (16 + i - 4));
       w_soff[i] = uni(pk * (((t.xt * nks) * 4 + q) * PK_WAVE + i * PK_LOAD) + npk * (int)(((int64_t)pr * w_pstride + colu) * ES));
     }
-    s_soff = uni(pk * (((t.xt * nks) * 4 + q) * 256) + npk * (int)colu);
+    s_soff = uni(colu);
   };
   // Everything a slice's loads share: descriptors (of zero records past the end: such a load is out
   // of range, fetches nothing and returns zeros, so the K loop needs no conditions around its loads)
@@ -687,7 +685,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     r.a_off = ks * 128;
     r.as_off = ks * 4;
     r.w_off = uni(pk * (ks * PK_SLICE) + npk * (int)(((int64_t)(pb * 32) * w_pstride + (int64_t)kt * w_tstride) * ES));
-    r.s_off = uni(pk * (ks * 1024) + npk * (int)((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride));
+    r.s_off = uni((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride);
     return r;
   };
   auto issue_load = [&](auto idx_, const SliceAddr& sa, BRaw& b, ScaleRegs& sc0, ScaleRegs& sc1, auto with_scales_) {
@@ -1371,8 +1369,7 @@ int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT)(const MxArgs& m, u
 // (w_voff + w_soff[i] + w_off).
 template <int LB>
 __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const uint8_t* __restrict__ W,
-                                                              const uint8_t* __restrict__ W_scale, uint8_t* __restrict__ dst,
-                                                              uint32_t* __restrict__ dst_scale, int64_t H, int64_t I,
+                                                              uint8_t* __restrict__ dst, int64_t H, int64_t I,
                                                               int64_t col_tiles, int64_t nks, int64_t pieces) {
   constexpr bool FP4 = LB == 8;
   constexpr int ES = FP4 ? 2 : 4, GROWS = FP4 ? 8 : 4;
@@ -1382,7 +1379,7 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
   const int64_t ks = (d >> 11) % nks, xt = ((d >> 11) / nks) % col_tiles, e = (d >> 11) / (nks * col_tiles);
   const int g = lane >> 4, c = lane & 15;
   const int64_t pr = FP4 ? i : ((i < 4) ? i : (16 + i - 4)), kt = ks >> 2, pb = ks & 3;
-  int64_t elem, expert_elems, selem, expert_scales;  // (selem: the first byte of the lane's scale dword, load 0's thread moves it)
+  int64_t elem, expert_elems;
   if (stage == 1) {
     const int64_t nH = H / 512, pstride = 2 * nH * I;
     const int64_t tI = xt >> 2, p0 = (xt & 3) * 32;
@@ -1390,25 +1387,15 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
     const int64_t colu = tI * 512 + q * (rows_t / 4) + p0;
     elem = (GROWS * g + pr + pb * 32) * pstride + (c >> 3) * nH * I + 4 * (c & 7) + colu + kt * I;
     expert_elems = 128 * pstride;
-    selem = (g + pb * 4) * pstride + (c >> 3) * nH * I + 4 * (c & 7) + colu + kt * I;
-    expert_scales = 16 * pstride;
   } else {
     const int64_t nI = (I + 511) / 512, pI = I > 512 ? 128 : I / 4, pstride = nI * H;
     elem = (GROWS * g + pr + pb * 32) * pstride + 4 * c + xt * 256 + 64 * q + kt * H;
     expert_elems = pI * pstride;
-    selem = (g + pb * 4) * pstride + 4 * c + xt * 256 + 64 * q + kt * H;
-    expert_scales = (pI + 7) / 8 * pstride;
   }
   const uint8_t* src = W + (e * expert_elems + elem) * ES;
   const int64_t o = (d & ~(int64_t)63) + (stage == 1 ? mx_pack_lane(lane) : lane);
   if constexpr (FP4) *(uint2*)(dst + o * LB) = *(const uint2*)src;
   else *(uint4*)(dst + o * LB) = *(const uint4*)src;
-  if (i == 0) {
-    const uint8_t* ss = W_scale + e * expert_scales + selem;
-    uint32_t* const ds = dst_scale + ((o >> 9) << 6) + (o & 63);
-    if (((uintptr_t)W_scale & 3) == 0) *ds = *(const uint32_t*)ss;  // (selem and expert_scales are multiples of 4)
-    else *ds = (uint32_t)ss[0] | (uint32_t)ss[1] << 8 | (uint32_t)ss[2] << 16 | (uint32_t)ss[3] << 24;
-  }
 }
 
 static void mx_pack_geometry(int stage, int64_t H, int64_t I, int64_t* col_tiles, int64_t* nks) {
@@ -1416,32 +1403,25 @@ static void mx_pack_geometry(int stage, int64_t H, int64_t I, int64_t* col_tiles
   *col_tiles = stage == 1 ? over_i : H / 256;
   *nks = stage == 1 ? H / 128 : over_i;
 }
-size_t mx_packed_scales_offset(int stage, int fp4, int64_t E, int64_t H, int64_t I) {
+size_t mx_packed_weights_bytes(int stage, int fp4, int64_t E, int64_t H, int64_t I) {
   int64_t ct, nks;
   mx_pack_geometry(stage, H, I, &ct, &nks);
   return (size_t)E * ct * nks * (fp4 ? 16384 : 32768);
 }
-size_t mx_packed_weights_bytes(int stage, int fp4, int64_t E, int64_t H, int64_t I) {
-  int64_t ct, nks;
-  mx_pack_geometry(stage, H, I, &ct, &nks);
-  return mx_packed_scales_offset(stage, fp4, E, H, I) + (size_t)E * ct * nks * 1024;
-}
-int launch_mx_pack_weights(int stage, int fp4, const void* W, const void* W_scale, void* dst, int64_t E, int64_t H, int64_t I,
+int launch_mx_pack_weights(int stage, int fp4, const void* W, void* dst, int64_t E, int64_t H, int64_t I,
                            hipStream_t s) {
-  if (!mx_fast_path_ok(H, I) || (((uintptr_t)W) & 15) != 0 || (((uintptr_t)dst) & 15) != 0)
-    return MOE_E_BAD_ARG;
-  uint32_t* dst_scale = (uint32_t*)((uint8_t*)dst + mx_packed_scales_offset(stage, fp4, E, H, I));
+  if (!mx_fast_path_ok(H, I) || (((uintptr_t)W) & 15) != 0 || (((uintptr_t)dst) & 15) != 0) return MOE_E_BAD_ARG;
   int64_t ct, nks;
   mx_pack_geometry(stage, H, I, &ct, &nks);
   const int64_t pieces = E * ct * nks * 2048;
   if ((pieces + 255) / 256 >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
   const dim3 grid((unsigned)((pieces + 255) / 256));
   if (fp4)
-    hipLaunchKernelGGL(mx_pack_weights_kernel<8>, grid, dim3(256), 0, s, stage, (const uint8_t*)W,
-                       (const uint8_t*)W_scale, (uint8_t*)dst, dst_scale, H, I, ct, nks, pieces);
+    hipLaunchKernelGGL(mx_pack_weights_kernel<8>, grid, dim3(256), 0, s, stage, (const uint8_t*)W, (uint8_t*)dst, H, I,
+                       ct, nks, pieces);
   else
-    hipLaunchKernelGGL(mx_pack_weights_kernel<16>, grid, dim3(256), 0, s, stage, (const uint8_t*)W,
-                       (const uint8_t*)W_scale, (uint8_t*)dst, dst_scale, H, I, ct, nks, pieces);
+    hipLaunchKernelGGL(mx_pack_weights_kernel<16>, grid, dim3(256), 0, s, stage, (const uint8_t*)W, (uint8_t*)dst, H, I,
+                       ct, nks, pieces);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

@@ -16,7 +16,7 @@
 // A wave is held to 256 registers: with 128 the K loop's two slices of weights spill, and the launch is slower than the
 // large-tile kernel's.
 // Measured (gate/up + down, large-tile kernel -> this one): one token, 8 MXFP8 experts of H = 7168, I = 2048:
-// 56 + 27 -> 42 + 23 us (5.8 TB/s over both; a plain stream of as many bytes by 256 workgroups takes 36 us for gate/up);
+// 58 + 29 -> 49 + 24 us (363 MB in all: 4.9 and 5.0 TB/s);
 // 20 tokens, 128 bf16 experts of H = 2048, I = 768: 117 + 54 -> 91 + 48 us (6.2 TB/s); 256 tokens, 8 bf16 experts of
 // H = 512, I = 1024: 21 + 23 -> 15 + 17 us.
 // A chunk with more rows than the instance multiplies at once (MT row tiles of 16) is walked in passes that stream the
@@ -90,8 +90,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   constexpr int PK_LANE = FP4 ? 8 : 16, PK_LOAD = 64 * PK_LANE, PK_WAVE = 8 * PK_LOAD, PK_SLICE = 4 * PK_WAVE;
   const int64_t w_expert_bytes = pk ? (int64_t)a.col_tiles * nks * PK_SLICE
                                     : (STAGE == 1) ? 128 * w_pstride * ES : (int64_t)a.pI * w_pstride * ES;
-  const int64_t ws_expert = pk ? (int64_t)a.col_tiles * nks * 1024
-                               : (STAGE == 1) ? 16 * w_pstride : (int64_t)((a.pI + 7) / 8) * w_pstride;
+  const int64_t ws_expert = (STAGE == 1) ? 16 * w_pstride : (int64_t)((a.pI + 7) / 8) * w_pstride;
 
   typedef typename std::conditional<FP4, v2i, v4i>::type RawLoad;
   struct Slice {  // a slice's weights as loaded, with their scale bytes
@@ -119,11 +118,11 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
     // packed copies: the lane's place within a load (see mx_pack_lane) and, HALF, its quarter's block
     const int pl = HALF ? g * 16 + sub * 8 + gu * 4 + cl : (STAGE == 1) ? mx_pack_lane(lane) : lane;
     const uint32_t w_voff = pk ? (uint32_t)((HALF ? q * PK_WAVE : 0) + pl * PK_LANE) : (uint32_t)((GROWS * g * w_pstride + lane_col) * ES);
-    const uint32_t s_voff = pk ? (uint32_t)((HALF ? q * 256 : 0) + pl * 4) : (uint32_t)(g * w_pstride + lane_col);
+    const uint32_t s_voff = (uint32_t)(g * w_pstride + lane_col);
     // scalar byte offset of load i: one base and one step (the loads' partition rows are 0..3 and 16..19; 0..7 for
     // 4-bit weights), so that no table of offsets occupies scalar registers
     const int w_base = uni32(pk ? (xt * nks) * PK_SLICE + (HALF ? 0 : q * PK_WAVE) : (int)(colu * ES));
-    const int s_base = uni32(pk ? (xt * nks) * 1024 + (HALF ? 0 : q * 256) : (int)colu);
+    const int s_base = uni32((int)colu);
     const int w_step = uni32(pk ? PK_LOAD : (int)(w_pstride * ES)), w_jump = uni32(pk ? 4 : 16);
     const uint8_t* Wp = (const uint8_t*)a.W + (int64_t)e * w_expert_bytes;
     const uint8_t* Sp = a.W_scale + (int64_t)e * ws_expert;
@@ -191,7 +190,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
         }
         if constexpr (SCALED) {
           const rsrc_t rs = rsrc_of(Sp, live ? (uint32_t)ws_expert : 0u);
-          s.bs = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, s_voff, s_base + uni32(pk ? ks * 1024 : (int)((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride)), 0);
+          s.bs = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, s_voff, s_base + uni32((int)((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride)), 0);
         }
       };
       auto load_a = [&](ASlice& s, int ks) {

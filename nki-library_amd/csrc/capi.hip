@@ -308,10 +308,10 @@ extern "C" int moe_prepare_kmajor_weights(const moe_bwmm_args* a, void* gate_up_
     if (!mx_packable(a, 0)) return MOE_E_UNSUPPORTED;
     const int fp4 = a->weight_dtype == MOE_DT_FP4_E2M1;
     if (!gate_up_kmajor || (((uintptr_t)gate_up_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
-    rc = launch_mx_pack_weights(1, fp4, a->gate_up_proj_weight, a->gate_up_proj_scale, gate_up_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
+    rc = launch_mx_pack_weights(1, fp4, a->gate_up_proj_weight, gate_up_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
     if (rc != MOE_OK || !mx_packable(a, 1)) return rc;
     if (!down_kmajor || (((uintptr_t)down_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
-    return launch_mx_pack_weights(2, fp4, a->down_proj_weight, a->down_proj_scale, down_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
+    return launch_mx_pack_weights(2, fp4, a->down_proj_weight, down_kmajor, a->E, a->H, a->I, (hipStream_t)stream);
   }
   if (!gate_up_kmajor || !down_kmajor) return MOE_E_BAD_ARG;
   if ((((uintptr_t)gate_up_kmajor) & 255) != 0 || (((uintptr_t)down_kmajor) & 255) != 0) return MOE_E_BAD_ARG;
@@ -535,7 +535,6 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m1.bias = a->gate_and_up_proj_bias;
       if (mx_packable(a, 0) && a->gate_up_proj_weight_kmajor) {
         m1.W = (const uint32_t*)a->gate_up_proj_weight_kmajor;
-        m1.W_scale = (const uint8_t*)m1.W + mx_packed_scales_offset(1, m1.wfmt == MX_WFMT_E2M1, a->E, a->H, a->I);
         m1.w_packed = 1;
       }
       if (r8_fast) {
@@ -579,7 +578,6 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m2.bias = a->down_proj_bias;
       if (mx_packable(a, 1) && a->down_proj_weight_kmajor) {
         m2.W = (const uint32_t*)a->down_proj_weight_kmajor;
-        m2.W_scale = (const uint8_t*)m2.W + mx_packed_scales_offset(2, m2.wfmt == MX_WFMT_E2M1, a->E, a->H, a->I);
         m2.w_packed = 1;
       }
       if (r8_fast) {

@@ -66,10 +66,10 @@ def _bytes_of(t, storage):
 
 
 def _kmajor_weights(L, a, tensors, dev):
-    """``tensors``: what the copies are made of, as the caller of the operator passed it (the gate/up and down weights;
-    the MX formats' copies hold the block scales as well).  An entry is found through the bytes the tensors name and how
-    the call reads them (kind, weight type, expert shape), so a fresh view of the same allocation hits; it is valid while
-    all the allocations are alive (weak references to the storages: an address that was freed and handed out again is a
+    """``tensors``: what the copies are made of, as the caller of the operator passed it (the gate/up and down weights:
+    scales are no part of a copy).  An entry is found through the bytes the tensors name and how the call reads them
+    (kind, weight type, expert shape), so a fresh view of the same allocation hits; it is valid while both allocations
+    are alive (weak references to the storages: an address that was freed and handed out again is a
     different storage) and unchanged (torch's version counters, which views share with their base)."""
     storages = [t.untyped_storage() for t in tensors]
     key = (*map(_bytes_of, tensors, storages), int(a.kind), int(a.weight_dtype), int(a.E), int(a.H), int(a.I), int(a.I_pad))

@@ -70,8 +70,7 @@ def test_rows_mx(T, H, I, E, k, fmt, skip, copies):
 
 
 def test_mx_copies_follow_the_block_scales():
-    """The kept copy of MX gate/up weights holds their block scales: a scale changed in place, or another scale tensor with
-    the same weights, must reach the result."""
+    """A scale changed in place, or another scale tensor with the same weights, must reach the result."""
     import torch
     from nkilib import synthetic as syn
     from nkilib.core.moe.moe_cte import _launch
@@ -100,6 +99,59 @@ def test_mx_copies_follow_the_block_scales():
     assert torch.equal(layer(other), plain(other)) and not torch.equal(layer(other), layer(gs))
     gs.add_(1)
     assert torch.equal(layer(gs), layer(other))
+
+
+@pytest.mark.parametrize("T", [4, 150])  # the few-rows and the large-tile kernels
+@pytest.mark.parametrize("fp4", [False, True])
+def test_mx_scales_are_read_by_every_call(T, fp4):
+    """The kept copies hold weights alone: scales written past torch's version counter, scale tensors that did not exist
+    when the copies were made, and scales updated between the replays of a recorded graph all reach the result, and none
+    of them makes the copies anew."""
+    import torch
+    from nkilib import synthetic as syn
+    from nkilib.core.moe.moe_cte import _launch
+    from nkilib.core.moe.moe_tkg import moe_tkg
+    from nkilib.core.utils.common_types import ExpertAffinityScaleMode
+
+    dev = torch.device("cuda:0")
+    H, I, E, k = 512, 256, 4, 2
+    gu, gs, d, ds = syn.mx4_expert_weights(E, H, I, dev, seed=6) if fp4 else syn.mx_expert_weights(E, H, I, 0.05, dev, seed=6)
+    ids, aff = syn.route(T, E, k, dev, seed=6)
+    x = syn.hidden_states(T, H, dev, seed=6)[:T].contiguous()
+    aff = aff[:T].contiguous()
+
+    def layer(gs, ds):
+        return moe_tkg(x, gu, d, aff, ids, False, expert_gate_up_weights_scale=gs, expert_down_weights_scale=ds,
+                       expert_affinities_scaling_mode=ExpertAffinityScaleMode.POST_SCALE)
+
+    def plain(gs, ds):
+        _launch.mx_weight_copies = False
+        try:
+            return layer(gs, ds)
+        finally:
+            _launch.mx_weight_copies = True
+
+    _launch.clear_kmajor_weight_cache()
+    gs0, ds0 = torch.zeros_like(gs), torch.zeros_like(ds)
+    layer(gs0, ds0)  # (the copies are made here, before the scales are there)
+    (copies,) = _launch._kmajor.values()
+    first = layer(gs, ds)
+    assert first.abs().sum() > 0 and torch.equal(first, plain(gs, ds))
+    gs.data.add_(1)
+    ds.data.sub_(1)
+    assert torch.equal(layer(gs, ds), plain(gs, ds)) and not torch.equal(layer(gs, ds), first)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(gs, ds)
+    for step in range(3):
+        if step:
+            gs.add_(1)
+            ds.add_(1)
+        want = plain(gs, ds)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), step
+    assert list(_launch._kmajor.values()) == [copies]
 
 
 @pytest.mark.parametrize("T", [20, 150])  # the few-rows and the large-tile kernels
