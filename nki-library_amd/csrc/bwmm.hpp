@@ -109,7 +109,11 @@ int launch_mx_gemm(int stage, const MxArgs& m, unsigned gx, unsigned gy, hipStre
 // The same stage for launches with few rows per expert (bwmm_rows.hip): `rows` = rows that a chunk holds at most in a
 // well-formed table (longer chunks are walked in passes), max_chunks = upper bound on the number of chunks.
 // mx_rows_fits says whether that kernel is the faster one.
-bool mx_rows_fits(int stage, int wfmt, int64_t rows, int64_t avg_rows, int64_t tiles);
+struct RowsCall {
+  int64_t rows, H, E, N, B;  // H: hidden size (elements); N blocks of B rows in the table
+  int64_t col_tiles, max_chunks;
+};
+bool mx_rows_fits(int stage, int wfmt, const RowsCall& c);
 int launch_mx_rows(int stage, const MxArgs& m, unsigned gx, int64_t max_chunks, int64_t rows, hipStream_t s);
 // Copy of the x4 weights of one stage (1 gate/up, 2 down) in the order the large-tile kernel reads them: for expert
 // e, column tile xt, K slice ks, wave q, load i, lane l the 16 bytes (4-bit weights: 8) that the lane's i-th load of

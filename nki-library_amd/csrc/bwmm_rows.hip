@@ -409,22 +409,54 @@ static int launch_rows(const MxArgs& m, int64_t rows, int64_t max_chunks, int cu
   if (rows <= 16) return launch_mt<STAGE, WFMT, 1>(m, max_chunks, cus, s);
   if constexpr (ROWS_MT4<STAGE, WFMT>)
     if (rows > 32) return launch_mt<STAGE, WFMT, 4>(m, max_chunks, cus, s);
-  return launch_mt<STAGE, WFMT, 2>(m, max_chunks, cus, s);
+  if constexpr (STAGE == 1 && WFMT == MX_WFMT_E2M1) return MOE_E_BAD_ARG;  // (mx_rows_fits: up to 8 rows)
+  else return launch_mt<STAGE, WFMT, 2>(m, max_chunks, cus, s);
 }
 
-// `rows`: most rows a chunk can hold; `avg_rows`: rows an expert holds on average when the block table is as large as the
-// routing makes it; `tiles`: column tiles x chunks of the large-tile kernel's launch.
-//   up to 32 rows: everything but the 4-bit gate/up stage beyond 8 (its 8-byte loads: 52 us here, 43 us on the large-tile
-//     kernel at 16 tokens of 32 experts of H = 3072, I = 1536; 37 and 42 us at 8 tokens);
-//   up to 64: the kinds whose four row tiles fit the registers, but not the fp8-row gate/up stage (54 and 52 us);
-//     MXFP8 at 48 tokens of 32 experts of H = 7168, I = 2048: 284 + 140 us with spills, 155 + 92 us on the large-tile kernel;
-//   up to 256, one pass of 64 on average: bf16 launches that give the large-tile kernel a tile for half of the CUs or less
-//     (256 tokens, two of 8 experts each, of H = 512, I = 1024: 15 + 17 and 21 + 24 us; with a tile for every CU,
-//     H = 2048, I = 4096: gate/up 92 and 58 us).
-bool mx_rows_fits(int stage, int wfmt, int64_t rows, int64_t avg_rows, int64_t tiles) {
-  if (rows <= 32) return !(stage == 1 && wfmt == MX_WFMT_E2M1 && rows > 8);
-  if (rows <= 64) return wfmt == MX_WFMT_BF16 || (stage == 2 && (wfmt == MX_WFMT_ROW8 || wfmt == MX_WFMT_E2M1));
-  return rows <= 256 && avg_rows <= 64 && wfmt == MX_WFMT_BF16 && tiles <= 128;
+// How many rows a launch holds is known from the number of tokens, how many experts they hit is not (it stands in the
+// table, on the device): a table of N >= E blocks is taken to hit all E, a shorter one E / 4 per token, 2 at least and 8
+// at most.  Times below are us between two events on the stream, large-tile
+// kernel | this one.
+//   MX gate/up.  A half column tile per CU and round: one round (128 tiles) beats the large-tile kernel's, from then on
+//     both are bound by the stream, where the large tiles' longer runs are the better ones (8-bit weights), or the 8-byte
+//     loads of this kernel's 4-bit weights by far the worse.  Up to four experts always: the large-tile kernel gives an
+//     expert's tiles to one XCD.  8-bit, experts hit of H, I: 8 of 7168, 2048: 58 | 49; 16: 86 | 90; 57: 280 | 317; 8 of
+//     5120, 1536: 51 | 31; 14: 52 | 57; 2 of 4096, 14336: 126 | 51; 8: 167 | 174; 8 of 1024, 512: 20 | 11.  4-bit: 8 of
+//     7168, 2048: 47 | 50; 16: 52 | 90; 8 of 3072, 1536: 26 | 21; 15: 29 | 40; 3 of 4096, 14336: 94 | 73; 6: 100 | 139.
+//     (Between one round and two an estimate of 8 experts per token is as often 4, hence the 256 of 8-bit weights.)
+//   Dense gate/up: up to 16 rows, up to 32 where K is not long or the tiles are few, up to 64 where they are fewer still.
+//     bf16, 16 rows: 58 experts of 7168, 2048: 667 | 695; 41 of 5120, 1536: 277 | 239; 32 rows: 64 of 7168, 2048: 702 |
+//     754; 104 of 2048, 768: 127 | 113; 64 rows: 64 of 4096, 2048: 374 | 386; 8 of 3072, 4096: 82 | 86; 59 of 1024, 768:
+//     51 | 41; 8 of 4096, 1024: 65 | 34.  fp8-row, 16 rows: 41 of 4096, 2048: 134 | 139; 58 of 4096, 768: 85 | 64.
+//   Down: up to 32 rows (MXFP8, 32 rows: 159 experts of 7168, 2048: 376 | 362; 32 of 3072, 1536: 42 | 31), up to 64 for
+//     the kinds whose four row tiles fit the registers (bf16, 64 rows: 64 of 7168, 2048: 303 | 308; 128 of 2048, 768:
+//     80 | 70); 4-bit ones there while the tiles are few (48 rows: 119 of 4096, 2048: 115 | 131; 32 of 3072, 1536: 31 | 28).
+//   bf16 beyond 64 rows, one pass of 64 on average, while the large-tile kernel has a tile for half of the CUs or less: 256
+//     tokens over 8 experts, two of them each, of H = 512, I = 1024: gate/up 23 | 17, down 27 | 18; of H = 4096, I = 1024:
+//     72 | 61 and 28 | 33; 384 tokens of the former: 23 | 20 and 27 | 21, not taken: a pass more per expert and falling.
+bool mx_rows_fits(int stage, int wfmt, const RowsCall& c) {
+  const bool fp4 = wfmt == MX_WFMT_E2M1, bf16 = wfmt == MX_WFMT_BF16, mx = !bf16 && wfmt != MX_WFMT_ROW8;
+  const int64_t all = (c.N < c.E ? c.N : c.E) * c.col_tiles;  // tiles when every expert is hit
+  if (stage == 1 && mx) {
+    if (c.rows > (fp4 ? 8 : 32)) return false;
+    int64_t per_token = c.E / 4 < 2 ? 2 : c.E / 4 > 8 ? 8 : c.E / 4, hit = c.rows * per_token;
+    const bool some = c.N < c.E && hit < c.E;
+    if (!some) hit = c.E;
+    const int64_t tiles = hit * c.col_tiles;
+    return hit <= 4 || (fp4 ? tiles < 128 : tiles <= 128 || (some && tiles < 256));
+  }
+  if (c.rows <= 16) return true;
+  if (stage == 1) {
+    if (c.rows <= 32 && (c.H <= 4096 || all <= 256)) return true;
+    if (!bf16) return false;
+    if (c.rows <= 64 && c.H <= 1024) return true;
+  } else {
+    if (c.rows <= 32) return true;
+    if (c.rows <= 64 && (bf16 || wfmt == MX_WFMT_ROW8 || (fp4 && all <= 512))) return true;
+  }
+  // (a table of N blocks is made for about (N - (E - 1)) * B routed rows)
+  const int64_t avg_rows = c.N > c.E - 1 ? (c.N - (c.E - 1)) * c.B / c.E : 0;
+  return bf16 && c.rows <= 256 && avg_rows <= 64 && c.col_tiles * c.max_chunks <= 128;
 }
 
 int launch_mx_rows(int stage, const MxArgs& m0, unsigned gx, int64_t max_chunks, int64_t rows, hipStream_t s) {

@@ -508,12 +508,10 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
   }
   const unsigned gyc = (unsigned)bk.max_chunks;
   // few rows per expert: the kernel of bwmm_rows.hip (a table lists a token at most once per expert, so a chunk holds at
-  // most n_real rows; a table of N blocks is made for about (N - (E - 1)) * B routed rows); the activation checkpoints
-  // are written by the large-tile kernels' epilogues
-  const int64_t avg_rows = a->N > a->E - 1 ? (a->N - (a->E - 1)) * a->B / a->E : 0;
+  // most n_real rows); the activation checkpoints are written by the large-tile kernels' epilogues
   auto few_rows = [&](int stage, unsigned gx) {
     return !a->gate_up_activations_T && !a->down_activations &&
-           mx_rows_fits(stage, m.wfmt, n_real, avg_rows, (int64_t)gx * bk.max_chunks);
+           mx_rows_fits(stage, m.wfmt, RowsCall{n_real, a->H, a->E, a->N, a->B, (int64_t)gx, bk.max_chunks});
   };
   mark(2);
   // Checkpoints of blocks that never run stay zero: cleared ahead for the general kernel; behind the large-tile kernels

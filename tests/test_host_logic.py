@@ -136,3 +136,48 @@ def test_bench_refuses_more_than_one_gpu():
                          timeout=120)
     assert res.returncode != 0
     assert "one GPU" in res.stderr and res.stdout.strip() == ""
+
+
+@pytest.mark.parametrize("stage,fmt,H,I,E,k,T,few", [
+    # MX gate/up: up to four experts, one round of half tiles, the start of the second with 8-bit weights
+    (1, "e4m3", 7168, 2048, 256, 8, 1, True), (1, "e4m3", 7168, 2048, 256, 8, 2, False),
+    (1, "e4m3", 7168, 2048, 256, 8, 32, False), (1, "e5m2", 5120, 1536, 64, 4, 2, True),
+    (1, "e4m3", 4096, 14336, 8, 2, 2, True), (1, "e4m3", 4096, 14336, 8, 2, 8, False),
+    (1, "e4m3", 7168, 2048, 8, 2, 32, True), (1, "e4m3", 7168, 2048, 8, 2, 33, False),
+    # 4-bit weights: these had been sent to the kernel that takes up to twice as long
+    (1, "e2m1", 7168, 2048, 256, 8, 1, False), (1, "e2m1", 7168, 2048, 256, 8, 4, False),
+    (1, "e2m1", 4096, 2048, 128, 8, 8, False), (1, "e2m1", 3072, 1536, 32, 4, 1, True),
+    (1, "e2m1", 4096, 14336, 8, 2, 2, True), (1, "e2m1", 4096, 14336, 8, 2, 4, False),
+    (1, "e2m1", 512, 512, 8, 2, 8, True), (1, "e2m1", 512, 512, 8, 2, 9, False),
+    (2, "e2m1", 4096, 2048, 128, 8, 32, True), (2, "e2m1", 4096, 2048, 128, 8, 48, False),
+    (2, "e2m1", 3072, 1536, 32, 4, 64, True), (2, "e2m1", 3072, 1536, 32, 4, 65, False),
+    (2, "e4m3", 7168, 2048, 256, 8, 32, True), (2, "e4m3", 7168, 2048, 256, 8, 33, False),
+    # dense kinds
+    (1, "bf16", 7168, 2048, 64, 8, 16, True), (1, "bf16", 7168, 2048, 64, 8, 32, False),
+    (1, "bf16", 4096, 2048, 64, 4, 32, True), (1, "bf16", 4096, 2048, 64, 4, 64, False),
+    (1, "bf16", 1024, 768, 60, 4, 64, True), (2, "bf16", 7168, 2048, 64, 8, 64, True),
+    (1, "row8", 4096, 2048, 64, 4, 32, True), (1, "row8", 512, 512, 8, 2, 33, False),
+    (2, "row8", 7168, 2048, 32, 4, 64, True), (2, "row8", 7168, 2048, 32, 4, 65, False),
+    (1, "bf16", 512, 1024, 8, 2, 256, True), (1, "bf16", 512, 1024, 8, 2, 257, False),
+    (2, "bf16", 4096, 1024, 8, 2, 256, False),
+])
+def test_few_rows_rule(stage, fmt, H, I, E, k, T, few):
+    """mx_rows_fits (csrc/bwmm_rows.hip) at sizes where both kernels were timed."""
+    from nkilib.core.moe.moe_cte import get_n_blocks
+
+    assert _rows_fit(stage, fmt, H, I, E, get_n_blocks(T, k, E, 128), 128, T) is few
+
+
+def _rows_fit(stage, fmt, H, I, E, N, B, rows):
+    import ctypes
+
+    from nkilib import _native as nv
+
+    class RowsCall(ctypes.Structure):  # (csrc/bwmm.hpp)
+        _fields_ = [(n, ctypes.c_int64) for n in ("rows", "H", "E", "N", "B", "col_tiles", "max_chunks")]
+
+    f = getattr(nv.lib(), "_ZN3moe12mx_rows_fitsEiiRKNS_8RowsCallE")
+    f.restype, f.argtypes = ctypes.c_bool, [ctypes.c_int, ctypes.c_int, ctypes.POINTER(RowsCall)]
+    tiles = (I + 127) // 128 if stage == 1 else H // 256
+    c = RowsCall(rows, H, E, N, B, tiles, N * ((B + 255) // 256))
+    return bool(f(stage, ("e4m3", "e5m2", "e2m1", "row8", "bf16").index(fmt), ctypes.byref(c)))
