@@ -454,9 +454,13 @@ bool mx_rows_fits(int stage, int wfmt, const RowsCall& c) {
     if (c.rows <= 32) return true;
     if (c.rows <= 64 && (bf16 || wfmt == MX_WFMT_ROW8 || (fp4 && all <= 512))) return true;
   }
-  // (a table of N blocks is made for about (N - (E - 1)) * B routed rows)
-  const int64_t avg_rows = c.N > c.E - 1 ? (c.N - (c.E - 1)) * c.B / c.E : 0;
-  return bf16 && c.rows <= 256 && avg_rows <= 64 && c.col_tiles * c.max_chunks <= 128;
+  if (!bf16 || c.rows > 256 || c.col_tiles * c.max_chunks > 128) return false;
+  // A table of N blocks is made for about (N - (E - 1)) * B routed rows.  One with fewer blocks than experts was cut by the
+  // caller to what it holds, which may be whole blocks: several passes, worth it while the large-tile kernel has a chunk
+  // for an XCD or less (gate/up, 7 blocks of 128 rows over H = 2048, I = 1024: 76 | 44; 4 of 256: 114 | 74; 16 of 256 over
+  // H = 4096: 112 | 275).
+  if (c.N < c.E) return c.max_chunks <= 8 || (c.B < c.rows ? c.B : c.rows) <= 64;
+  return (c.N - (c.E - 1)) * c.B / c.E <= 64;
 }
 
 int launch_mx_rows(int stage, const MxArgs& m0, unsigned gx, int64_t max_chunks, int64_t rows, hipStream_t s) {

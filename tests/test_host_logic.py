@@ -168,6 +168,15 @@ def test_few_rows_rule(stage, fmt, H, I, E, k, T, few):
     assert _rows_fit(stage, fmt, H, I, E, get_n_blocks(T, k, E, 128), 128, T) is few
 
 
+@pytest.mark.parametrize("H,I,E,N,B,few", [
+    (512, 1024, 8, 1, 256, True), (2048, 1024, 8, 7, 128, True), (2048, 1024, 8, 4, 256, True),
+    (1024, 1024, 32, 16, 256, False), (4096, 512, 32, 31, 256, False), (512, 512, 32, 31, 64, True),
+])
+def test_few_rows_rule_of_a_table_with_fewer_blocks_than_experts(H, I, E, N, B, few):
+    """Such a table may hold whole blocks: many chunks of 256 rows are no launch of few rows."""
+    assert _rows_fit(1, "bf16", H, I, E, N, B, 256) is few
+
+
 def _rows_fit(stage, fmt, H, I, E, N, B, rows):
     import ctypes
 
