@@ -282,11 +282,17 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
         for (int k = 0; k < KP; ++k) v += s_part[((size_t)k * ROWS + r) * PITCH + col];
         return v;
       };
+      auto limit = [&](int bit, float v, float none) { return (a.clamp_mask & bit) ? v : none; };
+      const float inf = __builtin_inff();
+      const float g_hi = limit(MOE_CLAMP_GATE_HI, a.clamp[0], inf), g_lo = limit(MOE_CLAMP_GATE_LO, fminf(a.clamp[1], g_hi), -inf);
+      const float u_hi = limit(MOE_CLAMP_UP_HI, a.clamp[2], inf), u_lo = limit(MOE_CLAMP_UP_LO, fminf(a.clamp[3], u_hi), -inf);
       auto gate_up = [&](float gv, float uv) {
-        if (a.clamp_mask & MOE_CLAMP_GATE_LO) gv = fmaxf(gv, a.clamp[1]);
-        if (a.clamp_mask & MOE_CLAMP_GATE_HI) gv = fminf(gv, a.clamp[0]);
-        if (a.clamp_mask & MOE_CLAMP_UP_LO) uv = fmaxf(uv, a.clamp[3]);
-        if (a.clamp_mask & MOE_CLAMP_UP_HI) uv = fminf(uv, a.clamp[2]);
+        // (the medians of the large-tile kernels' epilogue, not minima and maxima: these would turn a NaN under an upper
+        // clamp alone into that clamp; without clamps the values go through as they are)
+        if (a.clamp_mask) {
+          gv = __builtin_amdgcn_fmed3f(gv, g_lo, g_hi);
+          uv = __builtin_amdgcn_fmed3f(uv, u_lo, u_hi);
+        }
         return act_apply(gv, a.act_fn) * uv;
       };
       const int live_rows = (nrows - row0 < ROWS) ? nrows - row0 : ROWS;

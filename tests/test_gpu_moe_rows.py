@@ -155,6 +155,20 @@ def test_mx_scales_are_read_by_every_call(T, fp4):
     assert list(_launch._kmajor.values()) == [copies]
 
 
+@pytest.mark.parametrize("T", [1, 20, 150])  # the few-rows and the large-tile kernels
+@pytest.mark.parametrize("act", [0, 3])
+def test_nan_rows_stay_nan_under_an_upper_gate_clamp(T, act):
+    """The clamps of the models that clamp (gate from above, up from both sides): a token that is not a number must not
+    come out as one, and no other token may be touched by it."""
+    c = dense_case(T, 512, 256, 4, 2, 128, seed=36, bias=True, hidden_std=1.0)
+    clamps = dict(gate_clamp_upper_limit=0.8, up_clamp_upper_limit=0.9, up_clamp_lower_limit=-0.5)
+    want = from_bf16_tensor(_run_dense(c, act=act, mode=1, clamps=clamps))[:T, 0]
+    c["hidden"][0] = np.nan
+    o = from_bf16_tensor(_run_dense(c, act=act, mode=1, clamps=clamps))[:T, 0]
+    assert np.isnan(o[0]).all()
+    assert np.array_equal(o[1:], want[1:])
+
+
 @pytest.mark.parametrize("T", [20, 150])  # the few-rows and the large-tile kernels
 @pytest.mark.parametrize("I,fp8w", [(36, False), (130, False), (202, True), (264, False)])
 def test_padded_intermediate_dense(T, I, fp8w):
