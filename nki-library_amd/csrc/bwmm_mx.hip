@@ -1016,6 +1016,14 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
                               ROW8 ? (uint32_t)(cur.nrows * y_rowb) : 0u);
     const uint32_t y_voff = (uint32_t)((4 * g_e + 2 * hcol_e) * y_rowb) +
                             (uint32_t)(tile_tI(cur) * 512 + q * tile_Pt(cur) + tile_p0(cur) + pl0) * (BF16 ? 2u : 4u);
+    // bf16 kind: columns that only pad the weights go out as zeros whatever they hold (an infinity in a row times their
+    // zero weights is not a number, and neither is that times the zero rows of the down weights)
+    int y_live[2] = {-1, -1};
+    if constexpr (BF16) {
+      const int n = (int)a.I_tab - (tile_tI(cur) * 512 + q * tile_Pt(cur) + tile_p0(cur) + pl0);
+      y_live[0] = n >= 2 ? -1 : n == 1 ? 0xffff : 0;
+      y_live[1] = n >= 4 ? -1 : n == 3 ? 0xffff : 0;
+    }
     auto passes = [&](auto act_, auto plain_) {
     constexpr int ACT = decltype(act_)::value;
     constexpr bool PLAIN = decltype(plain_)::value;
@@ -1102,8 +1110,8 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
               typedef __bf16 v2bf_ __attribute__((ext_vector_type(2)));
               typedef float v2f_ __attribute__((ext_vector_type(2)));
               const v2f_ p0 = {y[k][0], y[k][1]}, p1 = {y[k][2], y[k][3]};
-              const v2i o = {__builtin_bit_cast(int, __builtin_convertvector(p0, v2bf_)),
-                             __builtin_bit_cast(int, __builtin_convertvector(p1, v2bf_))};
+              const v2i o = {__builtin_bit_cast(int, __builtin_convertvector(p0, v2bf_)) & y_live[0],
+                             __builtin_bit_cast(int, __builtin_convertvector(p1, v2bf_)) & y_live[1]};
               st_b64(o, y_voff, rdy, (ps * 64 + ml * 16 + k) * y_rowb);
             } else if constexpr (ROW8) {
               const v4i o = {__builtin_bit_cast(int, y[k][0]), __builtin_bit_cast(int, y[k][1]),

@@ -334,7 +334,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
           for (int k = 0; k < 2; ++k) {
             float gv = part(r, qq * 64 + j + k), uv = part(r, qq * 64 + 32 + j + k);
             float sg = 1.f, su = 1.f;
-            const bool live = col + k < a.I_tab;  // (columns that only pad the weights: act(0) * 0)
+            const bool live = col + k < a.I_tab;  // (a column that only pads the weights is zero, also for a row with an infinity)
             if (a.w_cscale && live) {
               const float* ws = a.w_cscale + (a.cscale_experts > 1 ? (int64_t)e * 2 * a.I_tab : 0);
               sg = ws[col + k];
@@ -346,7 +346,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
               gv += bias_at((int64_t)e * 2 * a.I_tab + col + k);
               uv += bias_at((int64_t)e * 2 * a.I_tab + a.I_tab + col + k);
             }
-            y[k] = gate_up(gv, uv);
+            y[k] = live ? gate_up(gv, uv) : 0.f;
           }
           const int64_t slot = slot0 + row0 + r;
           if constexpr (BF16) *(uint32_t*)((uint16_t*)a.Yq + slot * a.y_stride + col) = pack2_bf16(y[0], y[1]);

@@ -180,6 +180,21 @@ def test_padded_intermediate_dense(T, I, fp8w):
 
 
 @pytest.mark.parametrize("T", [20, 150])
+@pytest.mark.parametrize("I", [36, 130, 203, 256])
+def test_infinite_rows_with_a_padded_intermediate(T, I):
+    """An infinity times weights that are all positive is an infinity in every output: the columns that pad the weights,
+    zeros, must not make it something else (256 fills its tiles: no padding)."""
+    c = dense_case(T, 512, I, 4, 2, 128, seed=37, hidden_std=1.0)
+    c["gate_up_w"], c["down_w"] = np.abs(c["gate_up_w"]) + 2.0 ** -7, np.abs(c["down_w"]) + 2.0 ** -7
+    want = from_bf16_tensor(_run_dense(c, act=0, mode=1))[:T, 0]
+    c["hidden"][0] = np.abs(c["hidden"][0])
+    c["hidden"][0, 5] = np.inf
+    o = from_bf16_tensor(_run_dense(c, act=0, mode=1))[:T, 0]
+    assert np.isposinf(o[0]).all()
+    assert np.array_equal(o[1:], want[1:])
+
+
+@pytest.mark.parametrize("T", [20, 150])
 @pytest.mark.parametrize("I", [36, 264])
 def test_padded_intermediate_fp8_row(T, I):
     c = dense_case(T, 512, I, 4, 2, 128, seed=35, quant=True, bias=True, hidden_std=1.0)
