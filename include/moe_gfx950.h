@@ -299,10 +299,11 @@ typedef struct moe_bwmm_args {
    * output_shard1 + t*out_row_stride elements and the combine pass writes it as zeros along with row t of
    * `output`, so the caller needs no separate clear. */
   void* output_shard1;
-  /* Nullable, no counterpart in the reference: device int64 [4].  Workgroup 0 of the large-tile gate/up GEMM writes
-   * [0] = shader clock cycles and [1] = ticks of the constant 100 MHz counter between its first and last
-   * instruction, the down GEMM the same into [2], [3]: cycles / ticks x 0.1 is the shader clock in GHz that the
-   * part held under that launch (it is set by power management, not by the data sheet).  Read by bench.py. */
+  /* Nullable, no counterpart in the reference: device int64 [4].  Workgroup 0 of the gate/up GEMM writes [0] =
+   * shader clock cycles and [1] = ticks of the constant 100 MHz counter between its first and last instruction, the
+   * down GEMM the same into [2], [3]: cycles / ticks x 0.1 is the shader clock in GHz that the part held under that
+   * launch (it is set by power management, not by the data sheet).  The general kernel writes nothing.  Read by
+   * bench.py. */
   int64_t* gemm_clocks;
   /* Nullable, no counterpart in the reference: the bookkeeping that moe_build_blocks_plan wrote for exactly these
    * token_position_to_id / block_to_expert tables (see there for the conditions under which it may be passed).

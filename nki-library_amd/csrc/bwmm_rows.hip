@@ -67,7 +67,12 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   __shared__ int s_tok[ROWS];
   __shared__ float s_aff[ROWS], s_rs[ROWS];
 
+  __shared__ long long s_clk[2];  // (start of the launch, see MxArgs::clk; the K loop has no scalar registers to spare)
   const int tid = threadIdx.x, lane = tid & 63;
+  if (a.clk && blockIdx.x == 0 && tid == 0) {
+    s_clk[0] = clock64();
+    s_clk[1] = wall_clock64();
+  }
   const int w = uni32(tid >> 6);
   const int cg = w % CG, kp = w / CG;
   const int c = lane & 15, g = lane >> 4;
@@ -372,6 +377,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
         }
       }
     }
+  }
+  if (a.clk && blockIdx.x == 0 && tid == 0) {
+    a.clk[0] = clock64() - s_clk[0];
+    a.clk[1] = wall_clock64() - s_clk[1];
   }
 }
 

@@ -42,7 +42,7 @@ kmajor_weight_cache = True
 # copy of the gate/up weights in HBM, made on the first call with a weight tensor pair; ``mx_weight_copies =
 # False`` reads the reference layout in place.
 mx_weight_copies = True
-# Measurement hook: an int64 device tensor of 4 elements that the large-tile GEMMs fill with the shader cycles and
+# Measurement hook: an int64 device tensor of 4 elements that the GEMMs (not the general kernel) fill with the shader cycles and
 # the 100 MHz ticks of their workgroup 0 (gate/up, then down): cycles / ticks * 0.1 = the clock in GHz under load.
 gemm_clock_probe = None
 # Measurement hook: seven ``torch.cuda.Event(enable_timing=True)`` (each recorded at least once before, so that its

@@ -70,6 +70,26 @@ def test_rows_mx(T, H, I, E, k, fmt, skip, copies):
     _check(o[0, :T], _golden_mx_options(c, 3, REF_MX_CLAMPS)[:T], f"few rows mx {fmt} T={T} H={H} I={I} copies={copies}")
 
 
+@pytest.mark.parametrize("kind,T", [("bf16", 20), ("bf16", 200), ("mx", 1), ("mx", 150)])
+def test_clock_probe_is_filled(kind, T):
+    """The gate/up and the down GEMM each store their workgroup 0's cycles and 100 MHz ticks, whichever kernel they are."""
+    import torch
+    from nkilib.core.moe.moe_cte import _launch
+
+    probe = torch.full((4,), -1, dtype=torch.int64, device="cuda:0")
+    _launch.gemm_clock_probe = probe
+    try:
+        if kind == "mx":
+            _run_mx_options(mx_case(T, 512, 512, 4, 2, 128, seed=38, bias=True, random_codes=True), 3, REF_MX_CLAMPS, False)
+        else:
+            _run_dense(dense_case(T, 512, 256, 4, 2, 128, seed=38, hidden_std=1.0))
+        torch.cuda.synchronize()
+    finally:
+        _launch.gemm_clock_probe = None
+    cycles, ticks = probe[0::2].tolist(), probe[1::2].tolist()
+    assert all(t > 0 for t in ticks) and all(c > 0 for c in cycles), probe.tolist()
+
+
 def test_mx_copies_follow_the_block_scales():
     """A scale changed in place, or another scale tensor with the same weights, must reach the result."""
     import torch
