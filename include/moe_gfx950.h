@@ -308,8 +308,7 @@ typedef struct moe_bwmm_args {
   /* Nullable, no counterpart in the reference: the bookkeeping that moe_build_blocks_plan wrote for exactly these
    * token_position_to_id / block_to_expert tables (see there for the conditions under which it may be passed).
    * With it moe_blockwise launches no bookkeeping kernels of its own.  Ignored when activation checkpoints are
-   * requested, unless the call goes through moe_blockwise_stages with MOE_STAGE_CHECKPOINT_PLAN.  The plan is read
-   * only; it may be passed to any number of calls. */
+   * requested (their chunks hold padding rows too).  The plan is read only; it may be passed to any number of calls. */
   const void* block_plan;
   size_t block_plan_bytes;
   /* Nullable, no counterpart in the reference: seven hipEvent_t of the caller's (null entries are skipped).  The
@@ -342,9 +341,6 @@ int moe_blockwise(const moe_bwmm_args* args, void* stream);
 #define MOE_STAGE_DOWN 16u     /* down GEMM + bias + affinity                                        */
 #define MOE_STAGE_COMBINE 32u  /* per-token accumulation of the contributions into the output        */
 #define MOE_STAGE_ALL 63u
-/* Beside stages: block_plan is that of the call's tables also when activation checkpoints are requested (they need one
- * small launch then, not the whole bookkeeping); pass it with every stage of a split call. */
-#define MOE_STAGE_CHECKPOINT_PLAN 64u
 int moe_blockwise_stages(const moe_bwmm_args* args, unsigned stages, void* stream);
 
 /* No counterpart in the reference, whose dense weights are consumed N-contiguous ([E, H, 2, I], [E, I_pad, H]):

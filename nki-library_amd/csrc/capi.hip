@@ -341,28 +341,17 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
   uint8_t* ws = (uint8_t*)a->workspace;
   const int64_t n_real = a->skip_token ? a->T1 : a->T1 - 1;
   // The chunk / slot bookkeeping: derived here from token_position_to_id, or taken as the block build left it
-  // (moe_build_blocks_plan).  With activation checkpoints the large-tile kernels' chunks hold one padding row per expert
-  // more than the plan's: they are cut anew from the plan's valid rows, the rest of the plan is used as it is.
+  // (moe_build_blocks_plan).  With activation checkpoints the chunks hold one padding row per expert more than a plan's:
+  // the plan is then left aside.
   // (measurement hook: HIP events of the caller's, recorded on the stream between the stages)
   auto mark = [&](int i) {
     if (a->stage_events && a->stage_events[i]) (void)hipEventRecord((hipEvent_t)a->stage_events[i], s);
   };
   mark(0);
-  const bool ckpt = a->gate_up_activations_T || a->down_activations;
-  const bool plan_ok = a->block_plan_bytes >= bookkeeping_bytes(a->T1, a->N, a->B) && ((uintptr_t)a->block_plan & 255) == 0;
-  if (a->block_plan && !ckpt && !plan_ok) return MOE_E_BAD_ARG;
-  const bool planned = a->block_plan != nullptr && plan_ok && (!ckpt || ((stages & MOE_STAGE_CHECKPOINT_PLAN) && bf16_fast(a)));
-  Bookkeeping bk = carve_bookkeeping(planned ? (void*)a->block_plan : (void*)(ws + p.book), a->T1, a->N, a->B);
-  if (planned && ckpt) {
-    const Bookkeeping own = carve_bookkeeping(ws + p.book, a->T1, a->N, a->B);
-    bk.n_chunks = own.n_chunks; bk.chunk_slot = own.chunk_slot; bk.chunk_rows = own.chunk_rows;
-    bk.chunk_expert = own.chunk_expert; bk.chunk_xcd = own.chunk_xcd; bk.q_chunk = own.q_chunk; bk.q_off = own.q_off;
-    if (stages & MOE_STAGE_PREP) {
-      rc = launch_plan_chunks(bk, a->block_to_expert, a->N, a->B, a->E, s, own.n_active, a->conditions == nullptr);
-      if (rc != MOE_OK) return rc;
-    }
-    bk.n_active = own.n_active;
-  }
+  const bool planned = a->block_plan != nullptr && !a->gate_up_activations_T && !a->down_activations;
+  if (planned && (a->block_plan_bytes < bookkeeping_bytes(a->T1, a->N, a->B) || ((uintptr_t)a->block_plan & 255) != 0))
+    return MOE_E_BAD_ARG;
+  const Bookkeeping bk = carve_bookkeeping(planned ? (void*)a->block_plan : (void*)(ws + p.book), a->T1, a->N, a->B);
   if ((stages & MOE_STAGE_PREP) && !planned) {
     rc = launch_prep(bk, a, n_real, s);
     if (rc != MOE_OK) return rc;

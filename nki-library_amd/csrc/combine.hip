@@ -101,23 +101,15 @@ __global__ __launch_bounds__(1024) void chunks_and_offsets_kernel(
     inv_scan(cnt, off, n_real, s_ws);
 }
 
-// One workgroup: chunks and work queues from a block build's own valid rows (moe_build_blocks_plan).  With n_active_out
-// the chunks are those of a call with activation checkpoints, whose executed blocks are the build's or, without
-// conditions, all of them; their number goes there.
+// One workgroup: chunks and work queues from a block build's own valid rows (moe_build_blocks_plan).
 __global__ __launch_bounds__(1024) void plan_chunks_kernel(
-    const int32_t* __restrict__ b2e, const int32_t* n_active, const int32_t* __restrict__ valid_rows,
+    const int32_t* __restrict__ b2e, const int32_t* __restrict__ n_active, const int32_t* __restrict__ valid_rows,
     int64_t N, int64_t B, int64_t E, int32_t* __restrict__ n_chunks, int32_t* __restrict__ chunk_slot,
     int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert, int32_t* __restrict__ chunk_xcd,
-    int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks, int32_t* n_active_out, bool all_blocks) {
+    int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks) {
   __shared__ int s_ws[16];
-  if (n_active_out) {
-    if (threadIdx.x == 0) *n_active_out = all_blocks ? (int32_t)N : *n_active;
-    __threadfence_block();
-    __syncthreads();
-    n_active = n_active_out;
-  }
   build_chunks(b2e, n_active, valid_rows, N, B, E, n_chunks, chunk_slot, chunk_rows, chunk_expert, chunk_xcd, q_chunk,
-               q_off, max_chunks, s_ws, n_active_out != nullptr);
+               q_off, max_chunks, s_ws, false);
 }
 
 // ---- activation checkpoints: the rows behind the last token -------------------------------------------------
@@ -472,10 +464,10 @@ int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hi
 }
 
 int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int64_t N, int64_t B, int64_t E,
-                       hipStream_t s, int32_t* n_active_out, bool all_blocks) {
+                       hipStream_t s) {
   hipLaunchKernelGGL(plan_chunks_kernel, dim3(1), dim3(1024), 0, s, block_to_expert, k.n_active, k.valid_rows, N, B, E,
                      k.n_chunks, k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk, k.q_off,
-                     k.max_chunks, n_active_out, all_blocks);
+                     k.max_chunks);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

@@ -62,9 +62,8 @@ Bookkeeping carve_bookkeeping(void* base, int64_t T1, int64_t N, int64_t B);
 int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hipStream_t s);
 // The chunk list and the work queues alone, from valid_rows / n_active that the caller has filled in (the block
 // build's hand-over, see moe_build_blocks_plan).
-// n_active_out: for a call with activation checkpoints, see plan_chunks_kernel.
 int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int64_t N, int64_t B, int64_t E,
-                       hipStream_t s, int32_t* n_active_out = nullptr, bool all_blocks = false);
+                       hipStream_t s);
 // The padding rows and the blocks that do not run of the gate/up (stage 1) or down (2) checkpoint, after the large-tile
 // GEMM that wrote the other rows.
 int launch_ckpt_pad(int stage, uint16_t* ck, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s);

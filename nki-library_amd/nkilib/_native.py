@@ -25,7 +25,6 @@ MX_TOKEN_MAJOR, MX_REF_DENSE, MX_REF_STRIDED = 0, 1, 2
 CLAMP_GATE_HI, CLAMP_GATE_LO, CLAMP_UP_HI, CLAMP_UP_LO = 1, 2, 4, 8
 # MOE_STAGE_*
 STAGE_PREP, STAGE_ACT_QUANT, STAGE_GATE_UP, STAGE_REQUANT, STAGE_DOWN, STAGE_COMBINE, STAGE_ALL = 1, 2, 4, 8, 16, 32, 63
-STAGE_CHECKPOINT_PLAN = 64
 
 EXPORTED_SYMBOLS = (
     "moe_error_string",

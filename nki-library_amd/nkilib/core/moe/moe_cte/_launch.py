@@ -226,11 +226,13 @@ def run_blockwise(
         ck_down = torch.empty((N, B, H), dtype=torch.bfloat16, device=dev)
         a.down_activations = nv.ptr(ck_down)
 
-    from . import block_index
+    # (the bookkeeping of a call with activation checkpoints is derived from its tables, whatever became of them)
+    if not (checkpoint_gate_up or checkpoint_down):
+        from . import block_index
 
-    plan = block_index.plan_for(tp2id, b2e, cond, B, N, T1)
-    if plan is not None:
-        a.block_plan, a.block_plan_bytes = plan
+        plan = block_index.plan_for(tp2id, b2e, cond, B, N, T1)
+        if plan is not None:
+            a.block_plan, a.block_plan_bytes = plan
     if gemm_clock_probe is not None:
         kernel_assert(gemm_clock_probe.dtype == torch.int64 and gemm_clock_probe.numel() >= 4 and gemm_clock_probe.is_cuda,
                       "gemm_clock_probe must be a device int64 tensor of 4 elements")
@@ -258,11 +260,9 @@ def run_blockwise(
     ws = nv.workspace(dev, need)
     a.workspace = nv.ptr(ws)
     a.workspace_bytes = ws.numel()
-    # (the plan counts with activation checkpoints too: it is known to be that of these tables)
-    plan_bit = nv.STAGE_CHECKPOINT_PLAN if plan is not None and (checkpoint_gate_up or checkpoint_down) else 0
     with nv.on_device(dev):
         if stage_callback is None:
-            rc = L.moe_blockwise_stages(ctypes.byref(a), nv.STAGE_ALL | plan_bit, nv.stream_ptr(dev))
+            rc = L.moe_blockwise(ctypes.byref(a), nv.stream_ptr(dev))
         else:
             rc = 0
             for name, bit in _STAGES:
@@ -270,7 +270,7 @@ def run_blockwise(
                     continue
                 if name == "requant" and kind != nv.KIND_FP8_ROW:
                     continue
-                rc = L.moe_blockwise_stages(ctypes.byref(a), bit | plan_bit, nv.stream_ptr(dev))
+                rc = L.moe_blockwise_stages(ctypes.byref(a), bit, nv.stream_ptr(dev))
                 if rc != 0:
                     break
                 stage_callback(name)

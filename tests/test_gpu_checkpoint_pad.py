@@ -1,5 +1,6 @@
 """Activation checkpoints behind an expert's last token and in blocks that do not run (ckpt_pad_*_kernel): every row against
-the oracle's without a plan, and the same bits with the block build's plan.  Tolerances are those of test_gpu_moe.py."""
+the oracle's, and the same bits whether the tables are the block build's own or copies of them; calls with checkpoints
+follow tables that change.  Tolerances are those of test_gpu_moe.py."""
 
 import numpy as np
 import pytest
@@ -53,3 +54,47 @@ def test_checkpoint_padding(T, H, I, E, k, B, skip, cond):
         _check(from_bf16_tensor(d), g_d, "down_activations")
     for x, y in zip(*outs):
         assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+
+
+def test_checkpoints_follow_the_tables():
+    """Tables of the block build that are overwritten past torch's version counter, or between the replays of a recorded
+    graph: nothing that was derived from what they held before counts."""
+    import torch
+    from nkilib.core.moe.moe_cte import SkipMode, build_token_blocks
+    from nkilib.core.moe.moe_cte.bwmm_shard_on_block import run_dense_variant
+
+    dev = torch.device("cuda:0")
+    T, H, I, E, k, B = 300, 512, 256, 4, 2, 128
+    c = dense_case(T, H, I, E, k, B, seed=42, hidden_std=1.0)
+    aff = torch.rand((T + 1, E), device=dev).to(torch.bfloat16).reshape(-1, 1)
+    args = (bf16_tensor(c["hidden"], dev), aff, bf16_tensor(c["gate_up_w"], dev), bf16_tensor(c["down_w"], dev))
+    rng = np.random.default_rng(42)
+    # three routings, of other experts' loads each: the first two, two of the first three, and any
+    ids = [i32_tensor(np.stack([rng.permutation(m)[:k] for _ in range(T)]).astype(np.int32), dev) for m in (2, 3, 4)]
+
+    def layer(tp, b2e):
+        return run_dense_variant(*args, B, tp, b2e, "TH", skip_dma=SkipMode(False, False), checkpoint_gate_up=True,
+                                 checkpoint_down=True)
+
+    tables = [[t.clone() for t in build_token_blocks(i, E, B, c["N"])[:2]] for i in ids]
+    want = [layer(*t) for t in tables]
+    assert not torch.equal(want[0][0], want[1][0]) and not torch.equal(want[1][0], want[2][0])
+    tp, b2e, _ = build_token_blocks(ids[0], E, B, c["N"])
+
+    def same(outs, n):
+        return all(torch.equal(x.view(torch.int16), y.view(torch.int16)) for x, y in zip(outs, want[n]))
+
+    assert same(layer(tp, b2e), 0)
+    tp.data.copy_(tables[1][0])
+    b2e.data.copy_(tables[1][1])
+    assert same(layer(tp, b2e), 1)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = layer(tp, b2e)
+    for n in (1, 2, 0):
+        tp.copy_(tables[n][0])
+        b2e.copy_(tables[n][1])
+        layer(*tables[0])  # (eager work between the replays)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert same(outs, n), n
