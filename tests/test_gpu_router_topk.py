@@ -69,6 +69,69 @@ def test_router_topk_matches_oracle(T, H, E, k, act, pre, norm, bias, layout):
     assert np.abs(ta[safe] - want[safe]).max() <= 1e-5 + 1e-4 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("small_ws,unaligned", [(True, False), (False, False), (False, True)])
+@pytest.mark.parametrize("aff_bf16", [False, True])
+@pytest.mark.parametrize(
+    "T,H,E,k,act,pre,norm,mask,bias",
+    [
+        (70, 512, 64, 2, 1, 1, 0, 0, True),     # softmax over all experts, unmasked
+        (70, 512, 64, 2, 0, 1, 0, 0, False),    # sigmoid, unmasked
+        (65, 1024, 200, 8, 1, 1, 0, 1, False),  # softmax, zeros outside the selected
+        (130, 448, 256, 4, 0, 1, 1, 0, True),   # sigmoid, renormalised
+        (33, 512, 100, 3, 1, 1, 1, 1, True),    # softmax, renormalised
+        (129, 640, 300, 4, 1, 0, 0, 0, True),   # activation after the selection; more than 256 experts
+        (1, 128, 17, 8, 0, 0, 0, 0, False),
+    ],
+)
+def test_router_c_entry_matches_oracle(T, H, E, k, act, pre, norm, mask, bias, aff_bf16, small_ws, unaligned):
+    """Every form through the C entry on both of its paths: with the small workspace, and for tokens that are not 16-byte
+    aligned whatever the workspace, one launch walks K and selects; otherwise K is split over workgroups."""
+    import torch
+    from nkilib import _native as nv
+
+    dev = torch.device("cuda:0")
+    L = nv.lib()
+    g = torch.Generator(device=dev).manual_seed(T + E)
+    buf = torch.empty((T * H + 1,), dtype=torch.bfloat16, device=dev).uniform_(-1, 1, generator=g)
+    x = (buf[1:] if unaligned else buf[:-1]).view(T, H)
+    assert (x.data_ptr() % 16 != 0) == unaligned
+    w = torch.empty((H, E), device=dev).uniform_(-0.1, 0.1, generator=g).to(torch.bfloat16)
+    b = torch.empty((E,), device=dev).uniform_(-0.5, 0.5, generator=g) if bias else None
+    size = L.moe_router_topk_workspace_bytes(H, E) if small_ws else L.moe_router_topk_workspace_bytes_for(T, H, E)
+    ws = torch.full((size,), 255, dtype=torch.uint8, device=dev)
+    logits = torch.empty((T, E), device=dev)
+    idx = torch.empty((T, k), dtype=torch.int32, device=dev)
+    aff = torch.full((T + 1, E), 7.0, dtype=torch.bfloat16 if aff_bf16 else torch.float32, device=dev)
+    topk = torch.empty((T, k), device=dev)
+    nv.check(L.moe_router_topk(nv.ptr(x), nv.ptr(w), nv.ptr(b), nv.DT_FP32, T, H, E, k, act, pre, norm, mask, 1,
+                               nv.ptr(logits), nv.DT_FP32, nv.ptr(idx), nv.ptr(aff),
+                               nv.DT_BF16 if aff_bf16 else nv.DT_FP32, nv.ptr(topk), nv.ptr(ws), size,
+                               nv.stream_ptr(dev)), "router")
+    torch.cuda.synchronize()
+    r = orr.router_topk_ref(_np(x), _np(w), None if b is None else b.cpu().numpy(), act, k, router_pre_norm=bool(pre),
+                            norm_topk_prob=bool(norm))
+    # (the bound on the logits is that of the next test)
+    bound = 8 * H ** 0.5 * 2.0 ** -24 * (np.abs(_np(x)) @ np.abs(_np(w)) + 0.5) + 1e-6
+    assert (np.abs(_np(logits) - r["router_logits"]) <= bound).all()
+    srt = -np.sort(-r["router_logits"], axis=1)
+    safe = (srt[:, :k] - srt[:, 1:k + 1]).min(axis=1) > 2 * bound.max()
+    assert safe.mean() > 0.5
+    gi = idx.cpu().numpy()
+    assert np.array_equal(gi[safe], r["expert_index"][safe])
+    want = r["expert_affinities"].copy()
+    if mask:  # (the oracle has no such option: zeros outside the selected experts)
+        keep = np.zeros_like(want, dtype=bool)
+        np.put_along_axis(keep, r["expert_index"].astype(np.int64), True, axis=1)
+        want[~keep] = 0
+    # both activations follow the logits with a relative slope of at most 1, quotients with twice that, and once more where
+    # they are renormalised; exponents of up to 16 are rounded by 2^-20 on either side; bf16 rounds by 2^-8 of the value
+    rel = 4 * bound.max() + 2.0 ** -18
+    assert (np.abs(_np(aff)[:T] - want)[safe] <= (rel + (2.0 ** -8 if aff_bf16 else 0)) * np.abs(want)[safe]).all()
+    assert not _np(aff)[T].any()
+    sel = np.take_along_axis(want, gi.astype(np.int64), axis=1)
+    assert (np.abs(topk.cpu().numpy() - sel)[safe] <= rel * np.abs(sel)[safe]).all()
+
+
 @pytest.mark.parametrize(
     "T,H,E,k",
     [
