@@ -51,7 +51,9 @@ def test_build_blocks_bit_exact(T, k, E, B, skip, split, alpha):
     (256, 3, 16, 128),    # one pass of 256 tokens: the bitmaps are kept between the two uses
     (257, 7, 16, 128),    # two passes
     (256, 9, 20, 64),     # more ids per token than are held in registers
-    (1025, 5, 40, 128),   # the first size of the launches in several workgroups
+    (512, 4, 40, 128),    # the last size of the single launch
+    (513, 5, 40, 128),    # the first of the launches in several workgroups
+    (1025, 5, 40, 128),   # a fifth slab of one token
     (1500, 2, 1024, 64),  # the largest number of experts
     (16385, 4, 24, 512),  # slabs of more than one pass, the slabs not a multiple of the parts they are summed in
 ])
