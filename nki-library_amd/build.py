@@ -33,7 +33,7 @@ FLAGS = [
 # csrc/router_topk.hip) draw one inline-asm diagnostic per such load, thousands of times; every other translation
 # unit keeps the diagnostic on
 MX_FLAGS = ["-Wno-inline-asm"]
-M0_CLOBBER_SOURCES = ("bwmm_mx.hip", "bwmm_rows.hip", "router_topk.hip")
+M0_CLOBBER_SOURCES = ("bwmm_mx.hip", "router_topk.hip")
 NOISE = "is not a recognized feature for this target"
 
 

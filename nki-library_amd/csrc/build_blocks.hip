@@ -29,9 +29,11 @@ constexpr int BB_THREADS = 256;
 
 constexpr int BB_SLABS_MAX = 64;
 // Up to this many tokens form one slab, built by a single launch.  Its workgroup takes 256 tokens per pass, the slabs of the
-// three launches take theirs side by side.  Block build with plan, single | three launches, us (without the host, whose two
-// more launches cost what the second pass does): top-8 of 256 experts 17.4 | 13.3 at 257 tokens, 21.2 | 13.3 at 513,
-// 25.5 | 13.4 at 1024; top-2 of 8 experts 12.6 | 11.6, 15.6 | 11.8, 18.7 | 12.1.
+// three launches take theirs side by side.  Block build with plan, single | three launches, us on the GPU: top-8 of 256
+// experts 17.4 | 13.3 at 257 tokens, 21.2 | 13.3 at 513, 25.5 | 13.4 at 1024; top-2 of 8 experts 12.6 | 11.6, 15.6 | 11.8,
+// 18.7 | 12.1.  On the host two more launches cost about 4 us, what the second pass of 256 tokens does: hence 512 for
+// eager calls, whose layers are host bound at these sizes; a recorded graph has no such cost and would gain the difference
+// from 257 on, but one line has to serve both.
 constexpr int64_t BB_SINGLE_MAX_TOKENS = 512;
 constexpr int64_t BB_SINGLE_MAX_SLOTS = 1 << 17;  // one workgroup fills the pad ids of up to this many slots itself
 constexpr int BB_E_MAX = 1024;  // bitmaps and running counts of all experts in LDS: 36 bytes per expert

@@ -64,7 +64,6 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   constexpr bool BF16 = Cfg::BF16, ROW8 = Cfg::ROW8, FP4 = Cfg::FP4, SCALED = !ROW8;
   constexpr int CG = Cfg::CG, NTHR = 64 * Cfg::NW, ROWS = Cfg::ROWS, PITCH = Cfg::PITCH;
   extern __shared__ __attribute__((aligned(16))) float s_part[];  // [KP][ROWS][PITCH]
-  __shared__ int s_tok[ROWS];
   __shared__ float s_aff[ROWS], s_rs[ROWS];
 
   __shared__ long long s_clk[2];  // (start of the launch, see MxArgs::clk; the K loop has no scalar registers to spare)
@@ -133,7 +132,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
     const uint8_t* Sp = a.W_scale + (int64_t)e * ws_expert;
 
     for (int row0 = 0; row0 < nrows; row0 += ROWS) {
-      // rows of this pass: token ids, affinities, row scales (read behind the barrier that ends the K loop)
+      // rows of this pass: affinities, row scales (read behind the barrier that ends the K loop)
       __syncthreads();  // (the results of the pass before have been read)
       for (int r = tid; r < ROWS; r += NTHR) {
         const int row = row0 + r, slot = slot0 + row;
@@ -143,7 +142,6 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
         if (a.aff && id >= 0)
           af = a.aff_dtype == MOE_DT_BF16 ? bf16_bits_to_f32(((const uint16_t*)a.aff)[(int64_t)id * a.E + e])
                                           : ((const float*)a.aff)[(int64_t)id * a.E + e];
-        s_tok[r] = id;
         s_aff[r] = af;
         if constexpr (ROW8) {
           float v = 1.f;
