@@ -426,46 +426,44 @@ static int launch_rows(const MxArgs& m, int64_t rows, int64_t max_chunks, int cu
   else return launch_mt<STAGE, WFMT, 2>(m, max_chunks, cus, s);
 }
 
-// How many rows a launch holds is known from the number of tokens, how many experts they hit is not (it stands in the
-// table, on the device): a table of N >= E blocks is taken to hit all E, a shorter one E / 4 per token, 2 at least and 8
-// at most.  Times below are us between two events on the stream, large-tile
-// kernel | this one.
+// How many rows a launch holds is known from the number of tokens; how many experts they hit stands in the table, on the
+// device: one of N >= E blocks is taken to hit all E, a shorter one so many per token as models of E experts route to.
+// Times below are us between two events on the stream, large-tile kernel | this one.
 //   MX gate/up.  A half column tile per CU and round: one round (128 tiles) beats the large-tile kernel's, from then on
-//     both are bound by the stream, where the large tiles' longer runs are the better ones (8-bit weights), or the 8-byte
+//     both are bound by the stream, where the large tiles' longer runs are the better ones (8-bit weights) or the 8-byte
 //     loads of this kernel's 4-bit weights by far the worse.  Up to four experts always: the large-tile kernel gives an
 //     expert's tiles to one XCD.  8-bit, experts hit of H, I: 8 of 7168, 2048: 58 | 49; 16: 86 | 90; 57: 280 | 317; 8 of
-//     5120, 1536: 51 | 31; 14: 52 | 57; 2 of 4096, 14336: 126 | 51; 8: 167 | 174; 8 of 1024, 512: 20 | 11.  4-bit: 8 of
-//     7168, 2048: 47 | 50; 16: 52 | 90; 8 of 3072, 1536: 26 | 21; 15: 29 | 40; 3 of 4096, 14336: 94 | 73; 6: 100 | 139.
-//     (Between one round and two an estimate of 8 experts per token is as often 4, hence the 256 of 8-bit weights.)
-//   Dense gate/up: up to 16 rows, up to 32 where K is not long or the tiles are few, up to 64 where they are fewer still.
-//     bf16, 16 rows: 58 experts of 7168, 2048: 667 | 695; 41 of 5120, 1536: 277 | 239; 32 rows: 64 of 7168, 2048: 702 |
-//     754; 104 of 2048, 768: 127 | 113; 64 rows: 64 of 4096, 2048: 374 | 386; 8 of 3072, 4096: 82 | 86; 59 of 1024, 768:
-//     51 | 41; 8 of 4096, 1024: 65 | 34.  fp8-row, 16 rows: 41 of 4096, 2048: 134 | 139; 58 of 4096, 768: 85 | 64.
+//     5120, 1536: 51 | 31; 14: 52 | 57; 2 of 4096, 14336: 126 | 51; 8: 167 | 174.  4-bit: 8 of 7168, 2048: 47 | 50;
+//     16: 52 | 90; 57: 166 | 314; 8 of 3072, 1536: 26 | 21; 15: 29 | 40; 3 of 4096, 14336: 94 | 73; 6: 100 | 139.  Between
+//     one round and two the estimate decides (a low one for 8-bit weights, where a wrong choice costs 10 % at most, a high
+//     one for 4-bit): over random shapes up to 32 (8) tokens the stage then takes 1.034 (1.012) times the better kernel's
+//     time, the large-tile kernel 1.41 (1.29), this one 1.017 (1.12) with losses up to 1.29 (1.9).
+//   Dense gate/up: up to 32 rows (fp8-row) or 64 (bf16), except a long K over many tiles (bf16, 64 experts of 7168, 2048,
+//     16 rows: 667 | 695, 32: 702 | 754, 64: 706 | 775; of 5120, 1536, 16 rows: 277 | 239, 32: 307 | 329; 104 of 2048, 768,
+//     32 rows: 127 | 113; 59 of 1024, 768, 64: 51 | 41; 8 of 4096, 1024, 64: 65 | 34.  fp8-row, 58 of 4096, 768, 16 rows:
+//     85 | 64; 56 of 4096, 2048, 32: 177 | 185, 64: 192 | 215).
 //   Down: up to 32 rows (MXFP8, 32 rows: 159 experts of 7168, 2048: 376 | 362; 32 of 3072, 1536: 42 | 31), up to 64 for
 //     the kinds whose four row tiles fit the registers (bf16, 64 rows: 64 of 7168, 2048: 303 | 308; 128 of 2048, 768:
-//     80 | 70); 4-bit ones there while the tiles are few (48 rows: 119 of 4096, 2048: 115 | 131; 32 of 3072, 1536: 31 | 28).
+//     80 | 70); 4-bit ones there while the tiles are few (48 rows: 119 of 4096, 2048: 115 | 131; 59 of 2048, 6400: 81 | 104;
+//     32 of 3072, 1536: 31 | 28).
 //   bf16 beyond 64 rows, one pass of 64 on average, while the large-tile kernel has a tile for half of the CUs or less: 256
 //     tokens over 8 experts, two of them each, of H = 512, I = 1024: gate/up 23 | 17, down 27 | 18; of H = 4096, I = 1024:
 //     72 | 61 and 28 | 33; 384 tokens of the former: 23 | 20 and 27 | 21, not taken: a pass more per expert and falling.
 bool mx_rows_fits(int stage, int wfmt, const RowsCall& c) {
   const bool fp4 = wfmt == MX_WFMT_E2M1, bf16 = wfmt == MX_WFMT_BF16, mx = !bf16 && wfmt != MX_WFMT_ROW8;
-  const int64_t all = (c.N < c.E ? c.N : c.E) * c.col_tiles;  // tiles when every expert is hit
   if (stage == 1 && mx) {
     if (c.rows > (fp4 ? 8 : 32)) return false;
-    int64_t per_token = c.E / 4 < 2 ? 2 : c.E / 4 > 8 ? 8 : c.E / 4, hit = c.rows * per_token;
+    const int64_t per = c.E / (fp4 ? 4 : 16), hit = c.rows * (per < 1 ? 1 : per > 8 ? 8 : per);
     const bool some = c.N < c.E && hit < c.E;
-    if (!some) hit = c.E;
-    const int64_t tiles = hit * c.col_tiles;
-    return hit <= 4 || (fp4 ? tiles < 128 : tiles <= 128 || (some && tiles < 256));
+    const int64_t experts = some ? hit : c.E, tiles = experts * c.col_tiles;
+    return experts <= 4 || tiles <= 128 || (some && tiles < (fp4 ? 192 : 256));
   }
   if (c.rows <= 16) return true;
   if (stage == 1) {
-    if (c.rows <= 32 && (c.H <= 4096 || all <= 256)) return true;
-    if (!bf16) return false;
-    if (c.rows <= 64 && c.H <= 1024) return true;
+    if (c.rows <= (bf16 ? 64 : 32)) return !(c.N >= c.E && c.H > 5120 && c.E * c.col_tiles > 512);
   } else {
     if (c.rows <= 32) return true;
-    if (c.rows <= 64 && (bf16 || wfmt == MX_WFMT_ROW8 || (fp4 && all <= 512))) return true;
+    if (c.rows <= 64) return bf16 || wfmt == MX_WFMT_ROW8 || (fp4 && (c.N < c.E ? c.N : c.E) * c.col_tiles <= 384);
   }
   if (!bf16 || c.rows > 256 || c.col_tiles * c.max_chunks > 128) return false;
   // A table of N blocks is made for about (N - (E - 1)) * B routed rows.  One with fewer blocks than experts was cut by the

@@ -20,8 +20,8 @@ CL = dict(gate_clamp_upper_limit=0.8, gate_clamp_lower_limit=-0.7, up_clamp_uppe
     (1, 256, 128, 4, 2, 0, 1, False, False, False),     # four K slices for four waves; one slice each in the down stage
     (16, 512, 384, 8, 2, 0, 1, True, True, False),      # one full row tile; a short last intermediate tile (768 bytes of K)
     (17, 512, 128, 4, 4, 3, 2, True, False, False),     # two row tiles; Swish, PRE_SCALE; two K slices for four waves
-    (33, 2560, 1152, 16, 4, 0, 1, False, False, True),  # down: four row tiles, 128-column workgroups; fp8 weights
-    (40, 512, 1152, 16, 4, 0, 1, True, True, False),    # gate/up: the same
+    (33, 2560, 1152, 16, 4, 0, 1, False, False, True),  # four row tiles; 128-column workgroups in both stages; fp8 weights
+    (40, 512, 1152, 16, 4, 0, 1, True, True, False),    # the same from a short K, bf16 weights
     (64, 512, 256, 3, 2, 1, 0, True, True, False),      # GELU, NO_SCALE
     (65, 512, 128, 8, 2, 0, 1, False, False, False),    # more tokens than a pass has rows
     (256, 512, 256, 8, 2, 2, 1, True, False, False),    # experts of more than 64 rows: a second pass
