@@ -8,8 +8,10 @@ parallel into ``nki-library_amd/build/`` and linked; the MXFP8 large-tile GEMM
 """
 
 import os
+import re
 import subprocess
 import sys
+import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -45,6 +47,35 @@ def _run(cmd):
     return err
 
 
+LLVM = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
+
+
+def check_tile_code(obj):
+    """What the tile loops of the large-tile GEMMs rely on and the compiler does not know of, read from the compiled code:
+    it keeps nothing of its own in the accumulation registers (their contents are named in inline instructions alone),
+    and no vector instruction writes a scalar register within the five wait states ahead of a load that carries only
+    the wait for M0 (``s_nop 0``)."""
+    with tempfile.TemporaryDirectory() as tmp:
+        fat, co = os.path.join(tmp, "fat"), os.path.join(tmp, "co")
+        _run([os.path.join(LLVM, "llvm-objcopy"), f"--dump-section=.hip_fatbin={fat}", obj, os.path.join(tmp, "o")])
+        _run([os.path.join(LLVM, "clang-offload-bundler"), "--unbundle", "--type=o", f"--input={fat}", f"--output={co}",
+              "--targets=hipv4-amdgcn-amd-amdhsa--gfx950"])
+        dis = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--no-show-raw-insn", "--no-leading-addr", co],
+                             capture_output=True, text=True, check=True).stdout
+    code = [t for t in (line.split("//")[0].strip() for line in dis.splitlines()) if t]
+    loads = 0
+    for i, t in enumerate(code):
+        if re.match(r"v_accvgpr_(write|mov)_b32 a\S+, [va]", t):
+            raise RuntimeError(f"{obj}: the compiler uses an accumulation register: {t}")
+        if t.startswith("buffer_load") and t.endswith("lds") and code[i - 1] == "s_nop 0":
+            loads += 1
+            for u in code[max(0, i - 7):i]:
+                if u.startswith(("v_readlane", "v_readfirstlane", "v_cmp")):
+                    raise RuntimeError(f"{obj}: {u} too close to a load of the K loop")
+    if loads == 0:
+        raise RuntimeError(f"{obj}: no K loop found in the compiled code")
+
+
 def build(verbose=True, jobs=None):
     os.makedirs(OUT_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -63,6 +94,8 @@ def build(verbose=True, jobs=None):
     jobs = jobs or min(len(cmds), os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         errs = list(ex.map(_run, cmds))
+        # (4-bit weights run on the other tile loop, all of whose loads carry the longer wait)
+        list(ex.map(check_tile_code, [u[0] for u, (_, fmt) in zip(units, MX_INSTANCES) if fmt != 2]))
     link = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *[u[0] for u in units], "-o", OUT]
     if verbose:
         print(" ".join(link), flush=True)

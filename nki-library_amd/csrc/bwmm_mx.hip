@@ -1,4 +1,5 @@
-// MX (MXFP8 / MXFP4 weights, MXFP8 activations) blockwise expert GEMMs for gfx950, large-tile version.
+// Blockwise expert GEMMs for gfx950, large-tile version: the launch, and the tile loop of 4-bit weights and of tiles of up
+// to 64 rows (all others: mx_wide.hpp, both operands through LDS).
 //
 // A 256-thread workgroup (4 waves, one per SIMD) owns an "expert chunk" of up to 320 consecutive
 // slots of one expert and 256 output columns:
@@ -38,18 +39,11 @@
 //
 // Reference semantics: test/integration/nkilib/core/mlp/test_mlp_common.py:550-682 (layouts,
 // re-quantisation), test/integration/nkilib/core/moe/moe_cte/test_utils.py:474-735 (block loop).
-#include <type_traits>
-
-#include "bwmm.hpp"
+#include "mx_wide.hpp"
 
 namespace moe {
 
-constexpr int MXT = 256;                       // threads
-constexpr int MX_ROWS_MAX = CHUNK_ROWS_MAX;    // rows of the largest chunk (320)
-constexpr int MXROW = 128;                     // LDS pitch of one staged row; 16-byte chunk ch of row r sits in
-                                               // slot ch ^ (r & 7), which makes the fragment reads (16 rows x 4
-                                               // chunks per instruction) and the staging writes conflict free
-constexpr int MX_EP = 128 + 8;                 // epilogue exchange: floats per row ([q][32 partitions] + pad)
+constexpr int MX_EP = 128 + 8;  // epilogue exchange: floats per row ([q][32 partitions] + pad)
 // Per variant (NMT row tiles): how many slices the loads run ahead, the ring of activation stages, and
 // the bytes of one stage.  Chunks of up to 256 rows: 3 slices ahead, 4 stages of 256 rows.  Chunks of
 // 257..320 rows (an expert's usual load plus a small excess, which would otherwise cost a second pass
@@ -69,13 +63,6 @@ constexpr int MX_LDS_LOOP = MxCfg<16>::LDS > MxCfg<20>::LDS ? MxCfg<16>::LDS : M
 constexpr int MX_LDS_EPI = 64 * MX_EP * 4;
 constexpr int MX_LDS = MX_LDS_EPI > MX_LDS_LOOP ? MX_LDS_EPI : MX_LDS_LOOP;
 
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    static_for<I + 1, N>(f);
-  }
-}
 
 template <class Operand>
 struct BFrag {
@@ -92,28 +79,6 @@ __device__ __forceinline__ v8i frag_from_lds(const uint8_t* plo, const uint8_t* 
   return r;
 }
 
-// The accumulators live in fixed accumulation registers that only the statements below name: tile
-// (mt, nt) of a wave's 16 x 4 tiles is a[16 mt + 4 nt .. + 3].  They are not C++ values, so the
-// compiler never moves, copies or spills them (it would do so without the wait that a read of an
-// MFMA result needs: it does not know these statements as MFMAs).  Every accumulation register is
-// declared clobbered at both ends of each K slice, so the compiler keeps nothing of its own there.
-#define MX_A10(p) "a" #p "0", "a" #p "1", "a" #p "2", "a" #p "3", "a" #p "4", "a" #p "5", "a" #p "6", "a" #p "7", "a" #p "8", "a" #p "9"
-#define MX_ALL_ACC                                                                                               \
-  "a0", "a1", "a2", "a3", "a4", "a5", "a6", "a7", "a8", "a9", MX_A10(1), MX_A10(2), MX_A10(3), MX_A10(4),        \
-      MX_A10(5), MX_A10(6), MX_A10(7), MX_A10(8), MX_A10(9), MX_A10(10), MX_A10(11), MX_A10(12), MX_A10(13),     \
-      MX_A10(14), MX_A10(15), MX_A10(16), MX_A10(17), MX_A10(18), MX_A10(19), MX_A10(20), MX_A10(21), MX_A10(22), \
-      MX_A10(23), MX_A10(24), "a250", "a251", "a252", "a253", "a254", "a255"
-__device__ __forceinline__ void acc_fence() { asm volatile("" ::: MX_ALL_ACC); }
-template <int I>
-__device__ __forceinline__ void acc_zero() {
-  asm volatile("v_accvgpr_write_b32 a[%0], 0" : : "n"(I));
-}
-template <int I>
-__device__ __forceinline__ float acc_get() {
-  float x;
-  asm volatile("v_accvgpr_read_b32 %0, a[%1]" : "=v"(x) : "n"(I));
-  return x;
-}
 // One MFMA of row-tile fragment `af` (scale byte OA of `sa`) with column tile NT of `b`, written as
 // an instruction: statements of this kind keep their order, so what the source puts between two
 // MFMAs (a load, an LDS read) is issued between them and runs in the shadow of the first -- with one
@@ -200,83 +165,6 @@ __device__ __forceinline__ void mfma_asm_v(v4f& c, const v8i& af, const BOp& bf,
 #undef MX_MFMA_CASE
 #undef MX_MFMA_ASM
 
-// A vector memory instruction that reads a scalar register (descriptor, scalar offset) needs five wait states
-// after a vector ALU instruction that wrote that register (v_readfirstlane, v_readlane: the compiler reloads
-// spilled scalars with the latter right where they are used).  The compiler keeps that distance for instructions
-// of its own; for the instructions written out in this file it cannot (it does not see which operands an inline
-// statement reads when), so each of them carries the wait states itself.  They are issue slots in the shadow of
-// the MFMAs between which the loads sit.
-#define MX_SGPR_WAIT "s_nop 4\n\t"
-
-// Raw buffer descriptor over [p, p + bytes): loads take a per-lane 32-bit byte offset (VGPR) plus a
-// wave-uniform 32-bit byte offset (SGPR), which is exactly the shape of every address in this
-// kernel, so no 64-bit per-lane pointer is ever formed.
-// (The descriptor and the uniform offsets are passed through readfirstlane: 64-bit address
-// arithmetic on uniform values is done by the vector ALU, and without the hint the compiler wraps
-// every load in a loop that checks whether all lanes agree on the descriptor.)
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ int uni(int64_t v) { return __builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ v4i make_rsrc(const void* p, uint32_t bytes) {
-  const uint64_t addr = (uint64_t)p;
-  v4i d;
-  d[0] = uni((int)(uint32_t)addr);
-  d[1] = uni((int)(uint32_t)(addr >> 32)) & 0xffff;  // stride 0: raw buffer
-  d[2] = uni((int)bytes);
-  d[3] = 0x00020000;
-  return d;
-}
-// The K loop's loads are written as instructions, not builtins: the compiler orders the results of
-// its own loads with a counter that completes in order, and places those waits as if every load it
-// can see on any path had just been issued -- which with two alternating weight sets means waiting
-// for the set that was only just requested.  Loads the compiler cannot see get no waits from it;
-// the waits are placed by hand where the data is first used (vm_wait).  The destination is an
-// in/out operand so that the load updates the variable's register in place.
-// NT: non-temporal, for data that nobody will ask the L2 for again.
-template <bool NT>
-__device__ __forceinline__ void ld_b128(v4i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  if constexpr (NT)
-    asm volatile(MX_SGPR_WAIT "buffer_load_dwordx4 %0, %1, %2, %3 offen nt" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-  else
-    asm volatile(MX_SGPR_WAIT "buffer_load_dwordx4 %0, %1, %2, %3 offen" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void st_b64(const v2i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "buffer_store_dwordx2 %0, %1, %2, %3 offen nt" : : "v"(d), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void st_b128(const v4i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "buffer_store_dwordx4 %0, %1, %2, %3 offen nt" : : "v"(d), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-// 16 bytes per lane straight into LDS at lds + 16 * lane (no destination registers).  The instruction takes its
-// LDS base from M0, which is set in the same statement.  M0 is declared clobbered: the compiler warns that it
-// does not save reserved registers around a statement, which is what is wanted here -- on this target it never
-// carries a value in M0 from one instruction to the next (it writes M0 itself immediately before each instruction
-// of its own that reads it), so there is nothing to save.
-__device__ __forceinline__ void ld_lds_b128(uint32_t lds, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               : : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff) : "memory", "m0");
-}
-template <bool NT>
-__device__ __forceinline__ void ld_b64(v2i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  if constexpr (NT)
-    asm volatile(MX_SGPR_WAIT "buffer_load_dwordx2 %0, %1, %2, %3 offen nt" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-  else
-    asm volatile(MX_SGPR_WAIT "buffer_load_dwordx2 %0, %1, %2, %3 offen" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-typedef int v3i __attribute__((ext_vector_type(3)));
-__device__ __forceinline__ void ld_dwords(v3i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "buffer_load_dwordx3 %0, %1, %2, %3 offen" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void ld_dwords(v2i& d, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "buffer_load_dwordx2 %0, %1, %2, %3 offen" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-__device__ __forceinline__ void ld_b32(int& d, uint32_t voff, const v4i& rsrc, int soff) {
-  asm volatile(MX_SGPR_WAIT "buffer_load_dword %0, %1, %2, %3 offen" : "+v"(d) : "v"(voff), "s"(rsrc), "s"(soff) : "memory");
-}
-
-// A workgroup barrier that orders LDS traffic only.  (__syncthreads also makes the workgroup's global stores
-// visible, for which the compiler waits until every vector memory operation has completed -- the loads in flight
-// for the next tile included.)
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 // NMT = number of 16-row tiles this instantiation multiplies (the chunks it takes have at most NMT*16 rows).
 // Keeping it a compile-time constant keeps the K loop free of branches around the MFMAs.
 // LASTUSE: the chunks are the last ones of their experts, so their weights are streamed past the L2 (which
@@ -320,196 +208,10 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const int64_t nH = a.H / 512;
   const int q = w;
 
-  // ---- tiles ------------------------------------------------------------------------------------
-  // Everything that says which tile: uniform values, kept in scalar registers.  A tile's queue entry (two words)
-  // is read through the scalar cache where it is needed, with an instruction of this file's own: a plain load is a
-  // vector load to the compiler (it cannot know that no store aliases the queue), and a vector load in the wrong
-  // place waits for every load in flight.
-  struct Tile {
-    int nrows, e, slot0, xt;
-  };
-  typedef int v2i_t __attribute__((ext_vector_type(2)));
-  // Item l of the class -> (chunk position, column tile).  G = `interleave` chunks at a time (chosen with the queues): within a
-  // group of G queue positions the chunk varies fastest, so that workgroups with neighbouring items work on the
-  // same column tile of different chunks (of one expert: they share the weight tile); G = 1 is column tiles
-  // innermost.  The last group of a class may hold fewer than G chunks.
-  // (items are numbered through the XCD's whole queue; the class's own run from startL to endL)
-  const int pos0 = startL / a.col_tiles, npos = (endL - startL) / a.col_tiles;
-  auto tile_at = [&](int l) {
-    int pos, xt;
-    if (interleave == 1) {
-      pos = l / a.col_tiles;
-      xt = l - pos * a.col_tiles;
-    } else {
-      const int per_group = interleave * a.col_tiles;
-      const int lr = l - startL;
-      const int grp = lr / per_group, j = lr - grp * per_group;
-      const int base = grp * interleave;
-      const int G = (npos - base < interleave) ? npos - base : interleave;
-      xt = j / G;
-      pos = pos0 + base + (j - xt * G);
-    }
-    v2i_t raw;
-    asm volatile(MX_SGPR_WAIT "s_load_dwordx2 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
-                 : "=s"(raw) : "s"(a.q_chunk), "s"((qbase + pos) * 8) : "memory");
-    Tile t;
-    t.xt = xt;
-    t.slot0 = raw[0];
-    t.nrows = raw[1] & 0xffff;
-    t.e = raw[1] >> 16;
-    return t;
-  };
-  // gate/up: column tiles are numbered over the existing ones, 4 per full intermediate tile, then those of a
-  // short last tile (whose partitions per q are a multiple of 32 on this path): intermediate tile, first
-  // partition, partitions per q.  down: first hidden column.
-  auto tile_tI = [&](const Tile& t) { return t.xt >> 2; };
-  auto tile_p0 = [&](const Tile& t) { return (t.xt & 3) * 32; };
-  auto tile_Pt = [&](const Tile& t) {
-    const int64_t rows_t = (a.I - (int64_t)(t.xt >> 2) * 512 < 512) ? (a.I - (int64_t)(t.xt >> 2) * 512) : 512;
-    return (int)(rows_t / 4);
-  };
-  auto tile_h0 = [&](const Tile& t) { return (int64_t)t.xt * 256; };
-  // Rows: a thread looks after rows tid and 256 + tid of the chunk (token id, affinity), and after one of the
-  // tile's 256 bias values.  Each of these is fetched in two steps: `*_raw` issues loads (always from a valid
-  // address, no branch), `*_put` turns what arrived into the value and stores it in LDS.  Between the two lies an
-  // epilogue with a tile's first loads in flight.  The loads are instructions of this file's own, like those of
-  // the K loop: the compiler waits for a load of its own wherever it first touches the result or reuses the
-  // register, and such a wait would hold the epilogue until everything issued before it has arrived.
-  constexpr bool ROWS2 = NMT * 16 > 256;
-  auto ids_raw = [&](const Tile& t, int (&raw)[2]) {
-    const v4i rd = make_rsrc(a.tp2id, 0xffffffffu);
-#pragma unroll
-    for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-      const int r = tid + 256 * j;
-      ld_b32(raw[j], (uint32_t)(t.slot0 + ((r < t.nrows) ? r : t.nrows - 1)) * 4u, rd, 0);
-    }
-  };
-  auto ids_put = [&](int buf, int nrows, const int (&raw)[2]) {
-#pragma unroll
-    for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-      const int r = tid + 256 * j;
-      if (r < Cfg::ROWS) s_tok[buf][r] = (r < nrows && raw[j] >= 0 && raw[j] < a.n_real) ? raw[j] : -1;
-    }
-  };
-  // (No branch may surround such a load: where two paths that load into the same variable meet, the compiler
-  // copies the register right behind the load instruction, i.e. before the data has arrived.  So there is one
-  // load instruction for both element types -- the aligned word that holds the element, the half picked later --
-  // and a table that is absent is replaced by an address that is valid.)
-  auto elem_offset = [&](uint32_t idx, bool two_byte) { return two_byte ? ((idx << 1) & ~3u) : (idx << 2); };
-  auto elem_value = [&](int word, uint32_t idx, bool two_byte) {
-    return two_byte ? bf16_bits_to_f32((uint16_t)((uint32_t)word >> ((idx & 1u) * 16u))) : __builtin_bit_cast(float, word);
-  };
-  auto aff_index = [&](int e, int buf, int r) {
-    const int id = s_tok[buf][(r < NMT * 16) ? r : 0];
-    return (uint32_t)((id >= 0) ? id : 0) * (uint32_t)a.E + (uint32_t)e;
-  };
-  auto aff_raw = [&](const Tile& t, int buf, int (&raw)[2]) {
-    const v4i rd = make_rsrc(a.aff ? a.aff : (const void*)a.tp2id, 0xffffffffu);
-#pragma unroll
-    for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-      const uint32_t off = a.aff ? elem_offset(aff_index(t.e, buf, tid + 256 * j), a.aff_dtype == MOE_DT_BF16) : 0u;
-      ld_b32(raw[j], off, rd, 0);
-    }
-  };
-  auto aff_put = [&](int e, int buf, const int (&raw)[2]) {
-#pragma unroll
-    for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-      const int r = tid + 256 * j;
-      if (r < NMT * 16) {
-        float v = 0.f;
-        if (a.aff && s_tok[buf][r] >= 0) v = elem_value(raw[j], aff_index(e, buf, r), a.aff_dtype == MOE_DT_BF16);
-        s_aff[buf][r] = v;
-      }
-    }
-  };
-  // gate/up: bias value (gu*4 + q)*32 + pl belongs to partition p0 + pl; down: value j to column h0 + j.
+  typedef MxTileWalk<STAGE, NMT, WFMT> TW;
+  const TW tw{a, s_tok, s_aff, s_bias, s_rs, s_wsc, tid, startL, qbase, interleave, startL / a.col_tiles,
+              (endL - startL) / a.col_tiles};
   const int hcol = (STAGE == 1) ? (c >> 3) : 0, cl = (STAGE == 1) ? (c & 7) : c;
-  // the natural column of the thread's table entry: gate/up (gu = tid/128, q = tid/32 % 4, pl = tid % 32) ->
-  // gu * I + tile*512 + q*Pt + p0 + pl; down -> h0 + tid
-  // (columns that only pad the weights have no entry: natural_live is false, and natural_col the last real column's)
-  auto tile_col = [&](const Tile& t) {
-    return (uint32_t)tile_tI(t) * 512u + (uint32_t)((tid >> 5) & 3) * (uint32_t)tile_Pt(t) + (uint32_t)(tile_p0(t) + (tid & 31));
-  };
-  auto natural_live = [&](const Tile& t) { return STAGE != 1 || tile_col(t) < (uint32_t)a.I_tab; };
-  auto natural_col = [&](const Tile& t) {
-    if (STAGE == 1) {
-      const uint32_t col = tile_col(t);
-      return (uint32_t)(tid >> 7) * (uint32_t)a.I_tab + (col < (uint32_t)a.I_tab ? col : (uint32_t)a.I_tab - 1u);
-    }
-    return (uint32_t)tile_h0(t) + (uint32_t)tid;
-  };
-  const uint32_t ncols = (STAGE == 1) ? 2u * (uint32_t)a.I_tab : (uint32_t)a.H;  // table entries per expert
-  auto bias_index = [&](const Tile& t) {
-    if (ROW8) return (uint32_t)t.e * ncols + natural_col(t);
-    if (STAGE == 1) {
-      const uint32_t p = (uint32_t)(tile_p0(t) + (tid & 31));
-      return ((((uint32_t)t.e * (uint32_t)a.pI + p) * 2u + (uint32_t)(tid >> 7)) * (uint32_t)a.nI + (uint32_t)tile_tI(t)) * 4u +
-             (uint32_t)((tid >> 5) & 3);
-    }
-    return (uint32_t)t.e * (uint32_t)a.H + (uint32_t)tile_h0(t) + (uint32_t)tid;
-  };
-  auto bias_raw = [&](const Tile& t, int& raw) {
-    const v4i rd = make_rsrc(a.bias ? a.bias : (const void*)a.tp2id, 0xffffffffu);
-    ld_b32(raw, a.bias ? elem_offset(bias_index(t), a.bias_dtype == MOE_DT_BF16) : 0u, rd, 0);
-  };
-  auto bias_put = [&](const Tile& t, int buf, int raw) {
-    s_bias[buf][tid] = (a.bias && (!ROW8 || natural_live(t))) ? elem_value(raw, bias_index(t), a.bias_dtype == MOE_DT_BF16) : 0.f;
-  };
-  // ROW8: the weights' per-channel scale of the thread's column (fp32), and the activation rows' scales: gate/up,
-  // the fp32 behind the H codes of the token's record, times the affinity under PRE_SCALE (the affinity scales
-  // the token's row, i.e. its dequantisation scale); down, the scale of the re-quantised intermediate row.
-  auto wsc_raw = [&](const Tile& t, int& raw) {
-    if constexpr (ROW8) {
-      const v4i rd = make_rsrc(a.w_cscale ? (const void*)a.w_cscale : (const void*)a.tp2id, 0xffffffffu);
-      ld_b32(raw, a.w_cscale ? ((a.cscale_experts > 1 ? (uint32_t)t.e * ncols : 0u) + natural_col(t)) << 2 : 0u, rd, 0);
-    }
-  };
-  auto wsc_put = [&](const Tile& t, int buf, int raw) {
-    if constexpr (ROW8) s_wsc[buf][tid] = (a.w_cscale && natural_live(t)) ? __builtin_bit_cast(float, raw) : 1.f;
-  };
-  auto rs_raw = [&](const Tile& t, int buf, int (&raw)[2]) {
-    if constexpr (ROW8) {
-      // (bf16: nothing to fetch; the load stays, from an address that is valid, so that every format issues the
-      // same loads)
-      const v4i rd = make_rsrc((STAGE == 1 || BF16) ? (const void*)a.A : (const void*)a.a_rscale, 0xffffffffu);
-#pragma unroll
-      for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-        const int r = tid + 256 * j;
-        uint32_t off;
-        if (STAGE == 1) {
-          const int id = s_tok[buf][(r < NMT * 16) ? r : 0];
-          off = (uint32_t)((id >= 0) ? id : 0) * (uint32_t)a.a_stride + (BF16 ? 0u : (uint32_t)a.H);
-        } else {
-          off = (uint32_t)(t.slot0 + ((r < t.nrows) ? r : t.nrows - 1)) << 2;
-        }
-        ld_b32(raw[j], off, rd, 0);
-      }
-    }
-  };
-  // (gate/up under PRE_SCALE: `aff` holds what aff_raw fetched for the same rows)
-  auto rs_put = [&](int e, int buf, const int (&raw)[2], const int (&aff)[2]) {
-    if constexpr (ROW8) {
-      const bool pre = STAGE == 1 && (a.scaling_mode == MOE_SCALE_PRE || a.scaling_mode == MOE_SCALE_PRE_DELAYED);
-#pragma unroll
-      for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
-        const int r = tid + 256 * j;
-        if (r < NMT * 16) {
-          float v = BF16 ? 1.f : __builtin_bit_cast(float, raw[j]);
-          if (STAGE == 1 && s_tok[buf][r] < 0) v = 0.f;
-          if (pre && a.aff && s_tok[buf][r] >= 0) v *= elem_value(aff[j], aff_index(e, buf, r), a.aff_dtype == MOE_DT_BF16);
-          s_rs[buf][r] = v;
-        }
-      }
-    }
-  };
-  // which stages fetch the affinities: down always; gate/up of the fp8-row kind, for PRE_SCALE
-  constexpr bool AFF_ROWS = STAGE == 2 || ROW8;
-  // what has been requested with the *_raw functions above may be used once this has passed
-  auto all_loads_landed = [&](int (&x)[2], int (&y)[2], int& z, int (&u)[2], int& v) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(y[0]), "+v"(y[1]), "+v"(z));
-    if constexpr (ROW8) asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(v));
-  };
 
   // A staging: thread covers rows (tid>>3) + 32 j; its load goes straight to LDS slot tid&7 of that
   // row and fetches the 16-byte chunk (tid&7) ^ (row&7) that belongs there
@@ -617,7 +319,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   int w_soff[NBL];
   int s_soff = 0;
   // Point the loads at a tile: rows (token ids of the tile sit in s_tok[buf]), expert, columns.
-  auto aim_loads_at = [&](const Tile& t, int buf) {
+  auto aim_loads_at = [&](const MxTile& t, int buf) {
 #pragma unroll
     for (int j = 0; j < NAV; ++j) {
       const int row = arow0 + 32 * j;
@@ -644,11 +346,11 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     as_voff2 = BIG ? scale_row_off(256 + (tid & 63)) : 0u;
     int64_t colu;
     if (STAGE == 1) {
-      colu = (int64_t)tile_tI(t) * 512 + (int64_t)q * tile_Pt(t) + tile_p0(t);
+      colu = (int64_t)tw.tile_tI(t) * 512 + (int64_t)q * tw.tile_Pt(t) + tw.tile_p0(t);
       rw_ = make_rsrc(Wb + (int64_t)t.e * w_expert_bytes, (uint32_t)w_expert_bytes);
       rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * 16 * w_pstride, (uint32_t)(16 * w_pstride));
     } else {
-      colu = tile_h0(t) + 64 * q;
+      colu = tw.tile_h0(t) + 64 * q;
       const int64_t sp = (a.pI + 7) / 8;
       rw_ = make_rsrc(Wb + (int64_t)t.e * w_expert_bytes, (uint32_t)w_expert_bytes);
       rs_ = make_rsrc(a.W_scale + (int64_t)(a.w_scale_shared ? 0 : t.e) * sp * w_pstride, (uint32_t)(sp * w_pstride));
@@ -860,23 +562,23 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   auto request_first_slices = [&]() { request_first(std::integral_constant<int, 0>{}, std::integral_constant<int, NFIRST>{}); };
 
   // ---- first tile: nothing is in flight yet, so plain loads and waits do ----------------------------------
-  Tile cur = tile_at(L);
+  MxTile cur = tw.tile_at(L);
   int ids_nn[2] = {0, 0}, aff_n[2] = {0, 0}, bias_n = 0;  // requested ahead of an epilogue, put in place after it
   int rs_n[2] = {0, 0}, wsc_n = 0;                          // (fp8-row kind only)
-  ids_raw(cur, ids_nn);
-  bias_raw(cur, bias_n);
-  wsc_raw(cur, wsc_n);
-  all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-  ids_put(0, cur.nrows, ids_nn);
-  bias_put(cur, 0, bias_n);
-  wsc_put(cur, 0, wsc_n);
+  tw.ids_raw(cur, ids_nn);
+  tw.bias_raw(cur, bias_n);
+  tw.wsc_raw(cur, wsc_n);
+  tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  tw.ids_put(0, cur.nrows, ids_nn);
+  tw.bias_put(cur, 0, bias_n);
+  tw.wsc_put(cur, 0, wsc_n);
   __syncthreads();
-  if (AFF_ROWS) {
-    aff_raw(cur, 0, aff_n);
-    rs_raw(cur, 0, rs_n);
-    all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-    if (STAGE == 2) aff_put(cur.e, 0, aff_n);
-    rs_put(cur.e, 0, rs_n, aff_n);
+  if (TW::AFF_ROWS) {
+    tw.aff_raw(cur, 0, aff_n);
+    tw.rs_raw(cur, 0, rs_n);
+    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+    if (STAGE == 2) tw.aff_put(cur.e, 0, aff_n);
+    tw.rs_put(cur.e, 0, rs_n, aff_n);
   }
   aim_loads_at(cur, 0);
   request_first_slices();
@@ -884,10 +586,10 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   bool have_next = Ln < endL;
   {
     // (the wait in here also waits for the first slices: once per workgroup and class)
-    const Tile nx = tile_at(have_next ? Ln : L);
-    ids_raw(nx, ids_nn);
-    all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-    if (have_next) ids_put(1, nx.nrows, ids_nn);  // published by the barrier below
+    const MxTile nx = tw.tile_at(have_next ? Ln : L);
+    tw.ids_raw(nx, ids_nn);
+    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+    if (have_next) tw.ids_put(1, nx.nrows, ids_nn);  // published by the barrier below
   }
   int buf = 0;  // which of the two row tables (s_tok, s_aff, s_bias) belongs to the current tile
 
@@ -942,8 +644,8 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   // same, the slices through descriptors of zero records (no traffic), the rest from the addresses of the last
   // tile.
   const bool have_nn = Ln + Lstep < endL;
-  const Tile nxt = tile_at(have_next ? Ln : L);
-  const Tile nn = tile_at(have_nn ? Ln + Lstep : L);
+  const MxTile nxt = tw.tile_at(have_next ? Ln : L);
+  const MxTile nn = tw.tile_at(have_nn ? Ln + Lstep : L);
   const int nbuf = have_next ? buf ^ 1 : buf;  // (behind the last tile: its own row table, which holds valid ids)
   tile_live = have_next ? -1 : 0;
   aim_loads_at(nxt, nbuf);
@@ -952,11 +654,11 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   // down launch at decode sizes)
   constexpr bool SPREAD_FIRST = STAGE == 2 && NMT >= 8;
   if constexpr (!SPREAD_FIRST) request_first_slices();
-  if (AFF_ROWS) aff_raw(nxt, nbuf, aff_n);
-  rs_raw(nxt, nbuf, rs_n);
-  bias_raw(nxt, bias_n);
-  wsc_raw(nxt, wsc_n);
-  ids_raw(nn, ids_nn);
+  if (TW::AFF_ROWS) tw.aff_raw(nxt, nbuf, aff_n);
+  tw.rs_raw(nxt, nbuf, rs_n);
+  tw.bias_raw(nxt, bias_n);
+  tw.wsc_raw(nxt, wsc_n);
+  tw.ids_raw(nn, ids_nn);
 
   // ---- epilogue ---------------------------------------------------------------------------------------------
   // What the epilogue derives from the thread index it derives again here, from a copy the compiler cannot see
@@ -1015,12 +717,12 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
                                    : (const void*)((const uint8_t*)a.Y32 + (int64_t)cur.slot0 * y_rowb),
                               ROW8 ? (uint32_t)(cur.nrows * y_rowb) : 0u);
     const uint32_t y_voff = (uint32_t)((4 * g_e + 2 * hcol_e) * y_rowb) +
-                            (uint32_t)(tile_tI(cur) * 512 + q * tile_Pt(cur) + tile_p0(cur) + pl0) * (BF16 ? 2u : 4u);
+                            (uint32_t)(tw.tile_tI(cur) * 512 + q * tw.tile_Pt(cur) + tw.tile_p0(cur) + pl0) * (BF16 ? 2u : 4u);
     // bf16 kind: columns that only pad the weights go out as zeros whatever they hold (an infinity in a row times their
     // zero weights is not a number, and neither is that times the zero rows of the down weights)
     int y_live[2] = {-1, -1};
     if constexpr (BF16) {
-      const int n = (int)a.I_tab - (tile_tI(cur) * 512 + q * tile_Pt(cur) + tile_p0(cur) + pl0);
+      const int n = (int)a.I_tab - (tw.tile_tI(cur) * 512 + q * tw.tile_Pt(cur) + tw.tile_p0(cur) + pl0);
       y_live[0] = n >= 2 ? -1 : n == 1 ? 0xffff : 0;
       y_live[1] = n >= 4 ? -1 : n == 3 ? 0xffff : 0;
     }
@@ -1080,7 +782,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
             if (a.ckpt != nullptr && row < cur.nrows) {
               const uint32_t slot = (uint32_t)(cur.slot0 + row);
               const uint32_t n = slot / (uint32_t)a.ckpt_B, r = slot - n * (uint32_t)a.ckpt_B;
-              const int64_t col = (int64_t)tile_tI(cur) * 512 + (int64_t)q * tile_Pt(cur) + tile_p0(cur) + pl0;
+              const int64_t col = (int64_t)tw.tile_tI(cur) * 512 + (int64_t)q * tw.tile_Pt(cur) + tw.tile_p0(cur) + pl0;
               uint16_t* ck = a.ckpt + (((int64_t)n * 2) * a.ckpt_I + col) * a.ckpt_B + r;
               // (an even block size keeps the pair inside one block and the store aligned; otherwise row by row)
               const bool pair = (a.ckpt_B & 1) == 0;
@@ -1148,11 +850,11 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
           for (int k = 0; k < 8; ++k)
             d[k] = pack4_e4m3(clip448(yv[0][k] * is), clip448(yv[1][k] * is), clip448(yv[2][k] * is), clip448(yv[3][k] * is));
           const int64_t slot = cur.slot0 + row;
-          const int pw = tile_p0(cur) + 8 * j;  // first partition of the block within the intermediate tile
-          uint4* o = (uint4*)(a.Yq + slot * a.y_stride + tile_tI(cur) * 512 + pw * 4);
+          const int pw = tw.tile_p0(cur) + 8 * j;  // first partition of the block within the intermediate tile
+          uint4* o = (uint4*)(a.Yq + slot * a.y_stride + tw.tile_tI(cur) * 512 + pw * 4);
           o[0] = make_uint4(d[0], d[1], d[2], d[3]);
           o[1] = make_uint4(d[4], d[5], d[6], d[7]);
-          a.Ys[slot * a.ys_stride + tile_tI(cur) * 16 + (pw >> 3)] = (uint8_t)sb;
+          a.Ys[slot * a.ys_stride + tw.tile_tI(cur) * 16 + (pw >> 3)] = (uint8_t)sb;
         }
         }
       }
@@ -1172,7 +874,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     // the scale stages that the exchange buffer reaches into are written at the top of the next tile
     if constexpr (!ROW8) lds_barrier();
   } else {
-    const int64_t col0 = tile_h0(cur) + 64 * q + 4 * c_e;
+    const int64_t col0 = tw.tile_h0(cur) + 64 * q + 4 * c_e;
     float bd[4];
     {
       const float4 vb = *(const float4*)(s_bias[buf] + 64 * q + 4 * c_e);
@@ -1256,13 +958,13 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   // Everything in flight lands here: the next tile's first slices, this tile's stores (stores and loads share
   // the counter but complete in no fixed order between them, so the K loop's counting waits must not start
   // while stores are out), and the small loads issued ahead of the epilogue, which may be used from here on.
-  all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
   if (!have_next) break;
-  if (STAGE == 2) aff_put(nxt.e, buf ^ 1, aff_n);
-  rs_put(nxt.e, buf ^ 1, rs_n, aff_n);
-  bias_put(nxt, buf ^ 1, bias_n);
-  wsc_put(nxt, buf ^ 1, wsc_n);
-  if (have_nn) ids_put(buf, nn.nrows, ids_nn);  // the table of the tile that has just ended
+  if (STAGE == 2) tw.aff_put(nxt.e, buf ^ 1, aff_n);
+  tw.rs_put(nxt.e, buf ^ 1, rs_n, aff_n);
+  tw.bias_put(nxt, buf ^ 1, bias_n);
+  tw.wsc_put(nxt, buf ^ 1, wsc_n);
+  if (have_nn) tw.ids_put(buf, nn.nrows, ids_nn);  // the table of the tile that has just ended
   cur = nxt;
   L = Ln;
   Ln += Lstep;
@@ -1302,14 +1004,22 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int interleave = __builtin_amdgcn_readfirstlane(a.q_off[8 * (CHUNK_CLASSES + 1)]);
   int L = w;
   // classes in queue order (CHUNK_CLASS_TILES / CHUNK_CLASS_LAST in combine.hpp)
+  // (tiles of up to 64 rows stream their weights through registers, three slices ahead; 4-bit weights likewise)
+#define MX_TILES(TILES_) (WFMT != MX_WFMT_E2M1 && (TILES_) >= 8)
+#define MX_RUN_TILES(TILES_, LAST_)                                                                               \
+  if constexpr (MX_TILES(TILES_))                                                                                \
+    L = mx_gemm_tiles_wide<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \
+                                                           (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave); \
+  else                                                                                                           \
+    L = mx_gemm_tiles<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs,  \
+                                                      (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave);
 #define MX_RUN_CLASS(CLS_)                                                                                     \
   {                                                                                                            \
     const int startL = (__builtin_amdgcn_readfirstlane(qo[CLS_]) - qbase) * a.col_tiles;                       \
     const int endL = (__builtin_amdgcn_readfirstlane(qo[CLS_ + 1]) - qbase) * a.col_tiles;                     \
-    if (L < endL)                                                                                              \
-      L = mx_gemm_tiles<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT>(                         \
-          a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc, L, startL, endL,  \
-          W, qbase, interleave);                                                                               \
+    if (L < endL) {                                                                                            \
+      MX_RUN_TILES(CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_])                                              \
+    }                                                                                                          \
     __syncthreads();                                                                                           \
   }
   // The same for a run of neighbouring classes on one instance of the tile loop (whose row tiles cover the largest).
@@ -1319,9 +1029,9 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                   CHUNK_CLASS_LAST[C1_] == LAST_, "the instance covers the classes of the run");              \
     const int startL = (__builtin_amdgcn_readfirstlane(qo[C0_]) - qbase) * a.col_tiles;                        \
     const int endL = (__builtin_amdgcn_readfirstlane(qo[C1_ + 1]) - qbase) * a.col_tiles;                      \
-    if (L < endL)                                                                                              \
-      L = mx_gemm_tiles<STAGE, TILES_, LAST_, WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \
-                                                    (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave); \
+    if (L < endL) {                                                                                            \
+      MX_RUN_TILES(TILES_, LAST_)                                                                              \
+    }                                                                                                          \
     __syncthreads();                                                                                           \
   }
   static_assert(CHUNK_CLASSES == 12, "one MX_RUN_CLASS per class");
@@ -1352,6 +1062,8 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     MX_RUN_RANGE(11, 11, 4, true)
   }
 #undef MX_RUN_RANGE
+#undef MX_RUN_TILES
+#undef MX_TILES
 #undef MX_RUN_CLASS
   if (a.clk && blockIdx.x == 0 && threadIdx.x == 0) {
     a.clk[0] = clock64() - clk0;
@@ -1361,11 +1073,15 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 #define MX_CAT_(a, b, c, d) a##b##c##d
 #define MX_CAT(a, b, c, d) MX_CAT_(a, b, c, d)
+constexpr int MX_LDS_LAUNCH = MX_INST_WFMT == MX_WFMT_E2M1 ? MX_LDS
+                              : MX_INST_WFMT == MX_WFMT_ROW8 || MX_INST_WFMT == MX_WFMT_BF16
+                                  ? (MX_LDS > MX_WIDE_LDS_PLAIN ? MX_LDS : MX_WIDE_LDS_PLAIN)
+                                  : (MX_LDS > MX_WIDE_LDS_SCALED ? MX_LDS : MX_WIDE_LDS_SCALED);
 int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT)(const MxArgs& m, unsigned grid, hipStream_t s) {
   const hipError_t err = hipFuncSetAttribute((const void*)mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, MX_LDS);
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, MX_LDS_LAUNCH);
   if (err != hipSuccess) return MOE_E_LAUNCH;
-  hipLaunchKernelGGL((mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>), dim3(grid), dim3(MXT), MX_LDS, s, m);
+  hipLaunchKernelGGL((mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>), dim3(grid), dim3(MXT), MX_LDS_LAUNCH, s, m);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
