@@ -321,11 +321,16 @@ struct MxTileWalk {
   }
   // which stages fetch the affinities: down always; gate/up of the fp8-row kind, for PRE_SCALE
   static constexpr bool AFF_ROWS = STAGE == 2 || ROW8;
-  // what has been requested with the *_raw functions above may be used once this has passed
-  __device__ __forceinline__ auto all_loads_landed(int (&x)[2], int (&y)[2], int& z, int (&u)[2], int& v) const {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // what has been requested with the *_raw functions above may be used once this has passed (OUT: memory instructions
+  // issued behind them that may still be out)
+  template <int OUT>
+  __device__ __forceinline__ void loads_landed(int (&x)[2], int (&y)[2], int& z, int (&u)[2], int& v) const {
+    asm volatile("s_waitcnt vmcnt(%0)" : : "n"(OUT) : "memory");
     asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(y[0]), "+v"(y[1]), "+v"(z));
     if constexpr (ROW8) asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(v));
+  }
+  __device__ __forceinline__ void all_loads_landed(int (&x)[2], int (&y)[2], int& z, int (&u)[2], int& v) const {
+    loads_landed<0>(x, y, z, u, v);
   }
 };
 

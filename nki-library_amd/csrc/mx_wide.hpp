@@ -45,7 +45,13 @@ struct MxWideCfg {
   static constexpr int WSP = 256 + 16;
   static constexpr int WS = 4 * WSP;
   static constexpr int LDS_PLAIN = OFF_AS, LDS_SCALED = OFF_WS + 2 * WS;
+  // The epilogue's exchange, 4 KB per wave: behind the rest, or, where that fills the LDS, in the part of the second
+  // activation stage that is loaded by the next tile's first slice.
+  static constexpr int OFF_EX_BIG = SA + ((RT + 1) / 2) * 4096;
+  static_assert(NMT <= 16 || OFF_EX_BIG + 16384 <= 2 * SA, "the exchange fits the part of the stage that is free");
 };
+static_assert(MxWideCfg<16>::LDS_PLAIN + 16384 <= MxWideCfg<20>::LDS_PLAIN &&
+              MxWideCfg<16>::LDS_SCALED + 16384 <= MxWideCfg<20>::LDS_SCALED, "the exchange of the smaller tiles fits");
 constexpr int MX_WIDE_LDS_PLAIN = MxWideCfg<20>::LDS_PLAIN, MX_WIDE_LDS_SCALED = MxWideCfg<20>::LDS_SCALED;
 
 // One MFMA: weight fragment wf (first operand, element format WFMT) x activation fragment af into the fixed accumulators
@@ -380,7 +386,10 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
         }
         auto mul = [&](auto jj_, auto half_) {
           constexpr int jj = decltype(jj_)::value, half = decltype(half_)::value;
-          constexpr int xx = LASTG ? jj % 2 : jj / 8, cc = LASTG ? jj / 2 : jj % 8, rr = r0 + xx;
+          // (8-bit formats: there and back, so that every MFMA shares an operand with the one before: less switching, a
+          // clock 2 % higher in a loop of nothing but these MFMAs, 8 % against both operands changing every time)
+          constexpr int turn = BF16 ? 0 : LASTG ? (jj / 2) & 1 : (jj / 8) & 1;
+          constexpr int xx = LASTG ? (jj % 2) ^ turn : jj / 8, cc = LASTG ? jj / 2 : turn ? 7 - jj % 8 : jj % 8, rr = r0 + xx;
           if constexpr (rr < 8) mxw_mfma<(rr * 8 + cc) * 4, WFMT, half>(wf[cc], af[set][xx], wsc[cc], asc[rr]);
           else mxw_mfma_v<WFMT, half>(accv[rr - 8][cc], wf[cc], af[set][xx], wsc[cc], asc[rr]);
         };
@@ -459,22 +468,25 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   request_first(std::integral_constant<int, 0>{}, std::integral_constant<int, NFIRST>{});
   int Ln = L + Lstep;  // the item after the current one
   bool have_next = Ln < endL;
-  {
-    const MxTile nx = tw.tile_at(have_next ? Ln : L);
-    tw.ids_raw(nx, ids_nn);
-    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-    if (have_next) tw.ids_put(1, nx.nrows, ids_nn);  // published by the barrier below
-  }
+  MxTile nxt = tw.tile_at(have_next ? Ln : L);
+  tw.ids_raw(nxt, ids_nn);
+  tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  if (have_next) tw.ids_put(1, nxt.nrows, ids_nn);  // published by the barrier below
   int buf = 0;  // which of the two row tables belongs to the current tile
-
-  for (;;) {
+  auto zero_accumulators = [&]() {
     acc_fence();
     static_for<0, (RT < 8 ? RT : 8) * 32>([&](auto i_) { acc_zero<decltype(i_)::value>(); });
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 8; ++j) accv[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
-    // (the tile's first loads have landed: every wave has waited for its own)
+  };
+  zero_accumulators();
+  bool have_nn = Ln + Lstep < endL;
+  MxTile nn = tw.tile_at(have_nn ? Ln + Lstep : L);  // the tile after the next one
+
+  for (;;) {
+    // (what the tile's first slice needs has landed: every wave has waited for its own loads)
     lds_barrier();
     {
       typedef std::integral_constant<int, 0> S0;
@@ -501,12 +513,12 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
         for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(accv[i][j]));
     }
 
+    // (the exchange shares LDS with the loads past the end then: those of all waves have to be over)
+    if constexpr (BIG) asm volatile("s_barrier" ::: "memory");
+
     // ---- the next tile's first loads, and what the tile after it needs, go out around the epilogue ----------------
     // (Every wave is past B2 of the last slice: nothing in LDS that the epilogues of the others need is overwritten.  No
     // branch surrounds a load into registers, see bwmm_mx.hip: behind the last tile they are issued all the same.)
-    const bool have_nn = Ln + Lstep < endL;
-    const MxTile nxt = tw.tile_at(have_next ? Ln : L);
-    const MxTile nn = tw.tile_at(have_nn ? Ln + Lstep : L);
     const int nbuf = have_next ? buf ^ 1 : buf;
     tile_live = have_next ? -1 : 0;
     aim_loads_at(nxt, nbuf);
@@ -515,11 +527,26 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     tw.bias_raw(nxt, bias_n);
     tw.wsc_raw(nxt, wsc_n);
     tw.ids_raw(nn, ids_nn);
-    constexpr int STEPS = (STAGE == 1 && SCALED) ? RT : 2 * RT;  // of the epilogue; behind each a share of the first loads
+    // The epilogue's steps; behind each of the first half of them a share of the first loads.  (All at once they fill the
+    // CU's load queue, and this arithmetic, which could run meanwhile, waits behind the first that does not fit.)
+    constexpr int STEPS = (STAGE == 1 && ROW8) ? 2 * RT : RT, LSTEPS = (STEPS + 1) / 2;
+    constexpr int STORES = (STAGE == 2) ? 4 : (SCALED || !BF16) ? 2 : 1;  // at least, per step
+    auto loads_by = [](int i) constexpr { return i >= LSTEPS ? NFIRST : i * NFIRST / LSTEPS; };  // requested ahead of step i
     auto spread = [&](auto i_) {
       constexpr int i = decltype(i_)::value;
-      request_first(std::integral_constant<int, i * NFIRST / STEPS>{}, std::integral_constant<int, (i + 1) * NFIRST / STEPS>{});
+      request_first(std::integral_constant<int, loads_by(i)>{}, std::integral_constant<int, loads_by(i + 1)>{});
     };
+    // Loads and stores that may still be out when the next tile starts, those issued behind the last load that its first
+    // slice needs: slice 1's loads and the stores of the later steps (loads and stores complete in issue order; a store
+    // that is not counted here only makes the wait a longer one).
+    constexpr int NEED = 1 + NW + NAJ;
+    auto last_need_step = [=]() constexpr {
+      int i = 0;
+      while (loads_by(i + 1) < NEED) ++i;
+      return i;
+    };
+    constexpr int OUT = NFIRST - NEED + STORES * (STEPS - 1 - last_need_step());
+    static_assert(OUT < 64, "the counter of outstanding memory instructions");
 
     // ---- epilogue -------------------------------------------------------------------------------------------------
     // (lane-derived values are derived again from a copy the compiler cannot see through: they would otherwise be kept
@@ -542,18 +569,28 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const v2f_ p = {x, y};
       return __builtin_bit_cast(int, __builtin_convertvector(p, v2bf_));
     };
-    // Two pieces of a row's 128-byte line that the lane holds (16 bytes each: 64 bytes of a row per group of four lanes)
-    // become one piece of two rows: lanes c and c + 8 of a group exchange, so that the first store writes whole lines of
-    // rows 0 .. 7 of the row tile (lanes c < 8: first half, c >= 8: second half), the second one those of rows 8 .. 15.
-    auto whole_lines = [&](v4i& x, v4i& y) {
+    // A lane holds 16-byte pieces of one row and its neighbours pieces of other rows, which is what a store makes a request
+    // each of (64 per instruction instead of 8 or 16 whole lines: the epilogue of a 256 x 256 down tile took 15 k cycles,
+    // half of them in its stores).  So the wave's 16 rows go through 4 KB of LDS of its own: PIECES pieces per row, written
+    // by row, read back with a row's pieces in neighbouring lanes; pieces are swizzled with the row.
+    constexpr int PIECES = (STAGE == 2) ? 16 : (ROW8 && !BF16) ? 8 : 4, PITCH = PIECES * 16, NST = PIECES / 4;
+    constexpr int FOLD = PIECES == 16 ? 0 : PIECES == 8 ? 1 : 2;
+    constexpr int OFF_EX = BIG ? Cfg::OFF_EX_BIG : SCALED ? Cfg::LDS_SCALED : Cfg::LDS_PLAIN;
+    const int lane_e = tid_e & 63;
+    uint8_t* const ex = smem + OFF_EX + w * 4096;
+    uint8_t* const ex_w = ex + c_e * PITCH;
+    auto ex_put = [&](int piece, const v4i& o) { *(v4i*)(ex_w + ((piece ^ (c_e >> FOLD)) & (PIECES - 1)) * 16) = o; };
+    const int st_row = lane_e / PIECES, st_piece = lane_e % PIECES;  // of the first store; 64 / PIECES rows more per store
+    auto ex_get = [&](v4i (&o)[NST]) {
+      asm volatile("" ::: "memory");
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int lo = x[k], hi = y[k];
-        x[k] = __builtin_amdgcn_update_dpp(lo, hi, 0x128 /* row_ror:8 */, 0xf, 0xc, false);
-        y[k] = __builtin_amdgcn_update_dpp(hi, lo, 0x128 /* row_ror:8 */, 0xf, 0x3, false);
+      for (int k = 0; k < NST; ++k) {
+        const int row = k * (64 / PIECES) + st_row;
+        o[k] = *(const v4i*)(ex + row * PITCH + ((st_piece ^ (row >> FOLD)) & (PIECES - 1)) * 16);
       }
+      asm volatile("" ::: "memory");
     };
-    const int line_row0 = wm * RT * 16 + (c_e & 7), line_half = c_e >> 3;  // ... the lane's row and half then
+    const int st_row0 = wm * RT * 16 + st_row;
     if constexpr (STAGE == 1) {
       int cmask = a.clamp_mask;
       asm volatile("" : "+s"(cmask));
@@ -596,7 +633,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const v4i rdys = make_rsrc(SCALED ? (const void*)(a.Ys + (int64_t)cur.slot0 * ys_rowb) : (const void*)a.tp2id,
                                  SCALED ? (uint32_t)(cur.nrows * ys_rowb) : 0u);
       const int pl = p0 + 16 * wn + 4 * g_e;  // MX: the lane's first partition
-      const uint32_t yq_voff = (uint32_t)(row0 * y_rowb + tI * 512 + pl * 4);
+      const uint32_t yq_voff = (uint32_t)(st_row0 * y_rowb + tI * 512 + (p0 + 16 * wn) * 4 + st_piece * 16);
       // (the scale byte of a block is stored by the even one of its two lane groups; the other's store is out of range)
       const uint32_t ys_voff = (g_e & 1) ? 0xffffffffu : (uint32_t)(row0 * ys_rowb + tI * 16 + (pl >> 3));
       // dense kinds: natural column of the lane's first value of quarter 2 wn + j
@@ -629,6 +666,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
           if constexpr (!PLAIN)
 #pragma unroll
             for (int t = 0; t < 4; ++t) tab[t] = pair_tab(t);
+          v4i ex_o[NST];
           static_for<0, RT>([&](auto rt_) {
             constexpr int rt = decltype(rt_)::value;
             float y[4][4];
@@ -652,10 +690,14 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
 #pragma unroll
             for (int r = 0; r < 4; ++r)
               o[r] = (int)pack4_e4m3(clip448(y[0][r] * is), clip448(y[1][r] * is), clip448(y[2][r] * is), clip448(y[3][r] * is));
-            st_b128_plain(o, yq_voff, rdy, rt * 16 * y_rowb);
+            // (the rows before are stored while these values wait for theirs)
+            if constexpr (rt > 0) st_b128_plain(ex_o[0], yq_voff, rdy, (rt - 1) * 16 * y_rowb);
+            ex_put(g_e, o);
+            ex_get(ex_o);
             st_b8((int)sb, ys_voff, rdys, rt * 16 * ys_rowb);
             spread(rt_);
           });
+          st_b128_plain(ex_o[0], yq_voff, rdy, (RT - 1) * 16 * y_rowb);
         } else {
           static_for<0, 2>([&](auto j_) {  // quarter 2 wn + j: tile pairs 2 j and 2 j + 1
             constexpr int j = decltype(j_)::value;
@@ -666,8 +708,14 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
               const int n = (int)a.I_tab - (nat_col(j) + 2 * k);
               y_live[k] = n >= 2 ? -1 : n == 1 ? 0xffff : 0;
             }
-            const uint32_t y_voff = BF16 ? (uint32_t)(row0 * y_rowb + nat_col(j) * 2)
-                                         : (uint32_t)(line_row0 * y_rowb + (nat_col(j) + 16 * line_half) * 4);
+            constexpr int ES = BF16 ? 2 : 4;
+            const int col0 = tI * 512 + (2 * wn + j) * Pt + p0;  // the quarter's first column
+            const uint32_t y_voff = (uint32_t)(st_row0 * y_rowb + col0 * ES + st_piece * 16);
+            v4i ex_o[NST];
+            auto store = [&](int rt) {
+#pragma unroll
+              for (int k = 0; k < NST; ++k) st_b128(ex_o[k], y_voff, rdy, (rt * 16 + k * (64 / PIECES)) * y_rowb);
+            };
             static_for<0, RT>([&](auto rt_) {
               constexpr int rt = decltype(rt_)::value;
               const float rs = s_rs[buf][row0 + rt * 16];
@@ -681,7 +729,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
               if constexpr (BF16) {
                 const v4i o = {pack2(y[0][0], y[0][1]) & y_live[0], pack2(y[0][2], y[0][3]) & y_live[1],
                                pack2(y[1][0], y[1][1]) & y_live[2], pack2(y[1][2], y[1][3]) & y_live[3]};
-                st_b128(o, y_voff, rdy, rt * 16 * y_rowb);
+                if constexpr (rt > 0) store(rt - 1);
+                ex_put(g_e, o);
                 if (!PLAIN && a.ckpt != nullptr) {
                   // the checkpoint takes gate / up projections after scale, bias and clamp, transposed.  Neighbouring lanes
                   // hold neighbouring rows: where the block size is even (two rows then share a block and an aligned
@@ -691,9 +740,9 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
                   const bool pair = (ck_B & 1) == 0;
                   const int row = row0 + rt * 16 - (pair ? odd : 0);
                   const uint32_t slot = (uint32_t)(cur.slot0 + row), n = slot / ck_B, rr = slot - n * ck_B;
-                  const int col0 = nat_col(j) + (pair ? 4 * odd : 0);
-                  const int live = row < cur.nrows ? (int)a.ckpt_I - col0 : 0;  // columns from col0 on that exist
-                  const uint32_t off0 = (n - ck_n0) * 2u * ck_gu + ((uint32_t)col0 * ck_B + rr) * 2u;
+                  const int ccol0 = nat_col(j) + (pair ? 4 * odd : 0);
+                  const int live = row < cur.nrows ? (int)a.ckpt_I - ccol0 : 0;  // columns from ccol0 on that exist
+                  const uint32_t off0 = (n - ck_n0) * 2u * ck_gu + ((uint32_t)ccol0 * ck_B + rr) * 2u;
                   static_for<0, 2>([&](auto gu_) {
                     constexpr int gu = decltype(gu_)::value;
                     const float (&v)[2][4] = gu ? uu : gg;
@@ -713,17 +762,16 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
                   });
                 }
               } else {
-v4i o[2];
+                if constexpr (rt > 0) store(rt - 1);
 #pragma unroll
                 for (int h = 0; h < 2; ++h)
-                  o[h] = (v4i){__builtin_bit_cast(int, y[h][0]), __builtin_bit_cast(int, y[h][1]),
-                               __builtin_bit_cast(int, y[h][2]), __builtin_bit_cast(int, y[h][3])};
-                whole_lines(o[0], o[1]);
-                st_b128(o[0], y_voff, rdy, rt * 16 * y_rowb);
-                st_b128(o[1], y_voff, rdy, (rt * 16 + 8) * y_rowb);
+                  ex_put(4 * h + g_e, (v4i){__builtin_bit_cast(int, y[h][0]), __builtin_bit_cast(int, y[h][1]),
+                                            __builtin_bit_cast(int, y[h][2]), __builtin_bit_cast(int, y[h][3])});
               }
+              ex_get(ex_o);
               spread(std::integral_constant<int, j * RT + rt>{});
             });
+            store(RT - 1);
           });
         }
       };
@@ -746,86 +794,106 @@ v4i o[2];
       // rows past the chunk's last are dropped by the range check (rows of padding slots inside the chunk are written:
       // nothing reads them)
       const v4i rd = make_rsrc(a.D + (int64_t)cur.slot0 * a.H, (uint32_t)((int64_t)cur.nrows * a.H * 2));
-      // bf16 kind: the down checkpoint [N, B, H] = [slots, H] takes the same rows ahead of the affinity (a descriptor of
-      // zero records when there is none)
-      const v4i rdc = make_rsrc((BF16 && a.ckpt) ? a.ckpt + (int64_t)cur.slot0 * a.H : a.D,
-                                (BF16 && a.ckpt) ? (uint32_t)((int64_t)cur.nrows * a.H * 2) : 0u);
+      // bf16 kind: the down checkpoint [N, B, H] = [slots, H] takes the same rows ahead of the affinity
+      const v4i rdc = make_rsrc((BF16 ? a.ckpt : a.D) + (int64_t)cur.slot0 * a.H, (uint32_t)((int64_t)cur.nrows * a.H * 2));
       const int lcol = 128 * wn + 8 * g_e;  // the lane's first column of tile pair 0 within the tile
-      const uint32_t d_voff = (uint32_t)(line_row0 * rowb) + (uint32_t)(((int)tw.tile_h0(cur) + lcol + 32 * line_half) * 2);
+      const uint32_t d_voff = (uint32_t)(st_row0 * rowb) + (uint32_t)(((int)tw.tile_h0(cur) + 128 * wn) * 2 + st_piece * 16);
       float affs[RT], rss[RT];
 #pragma unroll
       for (int i = 0; i < RT; ++i) {
         affs[i] = post ? s_aff[buf][row0 + i * 16] : 1.f;
         if constexpr (ROW8) rss[i] = s_rs[buf][row0 + i * 16];
       }
-      // (PLAIN: no bias and, bf16, no scales and no checkpoint: what most layers are)
-      auto passes = [&](auto plain_) {
-      constexpr bool PLAIN = decltype(plain_)::value;
-      static_for<0, 2>([&](auto j_) {  // tile pairs 2 j and 2 j + 1: one 128-byte line of every row
-        constexpr int j = decltype(j_)::value;
-        float bd[2][8], sd[2][8];
+      // (PLAIN: no bias and, bf16, no scales, what most layers are; CKPT: the bf16 kind's checkpoint is written)
+      auto passes = [&](auto plain_, auto ckpt_) {
+        constexpr bool PLAIN = decltype(plain_)::value, CKPT = decltype(ckpt_)::value;
+        float bd[4][8], sd[4][8];
+        if constexpr (!PLAIN || (ROW8 && !BF16)) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+          for (int t = 0; t < 4; ++t)
 #pragma unroll
-          for (int k = 0; k < 8; k += 4) {
-            const float4 vb = *(const float4*)(s_bias[buf] + lcol + 32 * (2 * j + h) + k);
-            bd[h][k] = vb.x; bd[h][k + 1] = vb.y; bd[h][k + 2] = vb.z; bd[h][k + 3] = vb.w;
-            if constexpr (ROW8) {
-              const float4 vs = *(const float4*)(s_wsc[buf] + lcol + 32 * (2 * j + h) + k);
-              sd[h][k] = vs.x; sd[h][k + 1] = vs.y; sd[h][k + 2] = vs.z; sd[h][k + 3] = vs.w;
+            for (int k = 0; k < 8; k += 4) {
+              const float4 vb = *(const float4*)(s_bias[buf] + lcol + 32 * t + k);
+              bd[t][k] = vb.x; bd[t][k + 1] = vb.y; bd[t][k + 2] = vb.z; bd[t][k + 3] = vb.w;
+              if constexpr (ROW8) {
+                const float4 vs = *(const float4*)(s_wsc[buf] + lcol + 32 * t + k);
+                sd[t][k] = vs.x; sd[t][k + 1] = vs.y; sd[t][k + 2] = vs.z; sd[t][k + 3] = vs.w;
+              }
             }
-          }
+        }
+        v4i ex_o[NST];
+        auto store = [&](int rt, const v4i& d) {
+#pragma unroll
+          for (int k = 0; k < NST; ++k) st_b128(ex_o[k], d_voff, d, (rt * 16 + k * (64 / PIECES)) * rowb);
+        };
         static_for<0, RT>([&](auto rt_) {
           constexpr int rt = decltype(rt_)::value;
-          v4i o[2], oc[2];
-          static_for<0, 2>([&](auto h_) {
-            constexpr int h = decltype(h_)::value, t = 2 * j + h;
+          v4i o[4], oc[4];
+          static_for<0, 4>([&](auto t_) {
+            constexpr int t = decltype(t_)::value;
             float lo[4], hi[4], v[8];
             acc_of(rt_, std::integral_constant<int, 2 * t>{}, lo);
             acc_of(rt_, std::integral_constant<int, 2 * t + 1>{}, hi);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
               float x = k < 4 ? lo[k & 3] : hi[k & 3];
-              if constexpr (ROW8 && !(BF16 && PLAIN)) x = (x * sd[h][k]) * rss[rt];
-              v[k] = PLAIN ? x : x + bd[h][k];
+              if constexpr (ROW8 && !(BF16 && PLAIN)) x = (x * sd[t][k]) * rss[rt];
+              v[k] = PLAIN ? x : x + bd[t][k];
             }
-            if constexpr (BF16 && !PLAIN) oc[h] = (v4i){pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
-            o[h] = (v4i){pack2(v[0] * affs[rt], v[1] * affs[rt]), pack2(v[2] * affs[rt], v[3] * affs[rt]),
+            if constexpr (CKPT) oc[t] = (v4i){pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
+            o[t] = (v4i){pack2(v[0] * affs[rt], v[1] * affs[rt]), pack2(v[2] * affs[rt], v[3] * affs[rt]),
                          pack2(v[4] * affs[rt], v[5] * affs[rt]), pack2(v[6] * affs[rt], v[7] * affs[rt])};
           });
-          if constexpr (BF16 && !PLAIN) {
-            if (a.ckpt != nullptr) {
-              whole_lines(oc[0], oc[1]);
-              st_b128(oc[0], d_voff + 128 * j, rdc, rt * 16 * rowb);
-              st_b128(oc[1], d_voff + 128 * j, rdc, (rt * 16 + 8) * rowb);
-            }
+          // (the rows before are stored while these values wait for theirs)
+          if constexpr (rt > 0) store(rt - 1, rd);
+          if constexpr (CKPT) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t) ex_put(4 * t + g_e, oc[t]);
+            ex_get(ex_o);
+            store(rt, rdc);
           }
-          whole_lines(o[0], o[1]);
-          st_b128(o[0], d_voff + 128 * j, rd, rt * 16 * rowb);
-          st_b128(o[1], d_voff + 128 * j, rd, (rt * 16 + 8) * rowb);
-          spread(std::integral_constant<int, j * RT + rt>{});
+#pragma unroll
+          for (int t = 0; t < 4; ++t) ex_put(4 * t + g_e, o[t]);
+          ex_get(ex_o);
+          spread(rt_);
         });
-      });
+        store(RT - 1, rd);
       };
-      if (a.bias == nullptr && (!BF16 || (a.ckpt == nullptr && a.w_cscale == nullptr))) passes(std::true_type{});
-      else passes(std::false_type{});
+      const bool plain = a.bias == nullptr && (!BF16 || a.w_cscale == nullptr);
+      if constexpr (BF16) {
+        if (a.ckpt != nullptr) passes(std::false_type{}, std::true_type{});
+        else if (plain) passes(std::true_type{}, std::false_type{});
+        else passes(std::false_type{}, std::false_type{});
+      } else {
+        if (plain) passes(std::true_type{}, std::false_type{});
+        else passes(std::false_type{}, std::false_type{});
+      }
     }
     tile_live = -1;
 
     // ---- hand over to the next tile -----------------------------------------------------------------------------
-    // Everything in flight lands here: the next tile's first slices, this tile's stores and the small loads, which may
-    // be used from here on.
-    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-    if (!have_next) break;
+    // The loads of the next tile's first slice and the small loads land here (the latter may be used from here on); the
+    // stores drain under the next tile's first slice, whose B2 waits for all of them.
+    zero_accumulators();
+    if (!have_next) {
+      tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+      break;
+    }
+    const bool have_n3 = Ln + 2 * Lstep < endL;
+    const MxTile n3 = tw.tile_at(have_n3 ? Ln + 2 * Lstep : L);
+    tw.template loads_landed<OUT>(ids_nn, aff_n, bias_n, rs_n, wsc_n);
     if (STAGE == 2) tw.aff_put(nxt.e, buf ^ 1, aff_n);
     tw.rs_put(nxt.e, buf ^ 1, rs_n, aff_n);
     tw.bias_put(nxt, buf ^ 1, bias_n);
     tw.wsc_put(nxt, buf ^ 1, wsc_n);
     if (have_nn) tw.ids_put(buf, nn.nrows, ids_nn);  // the table of the tile that has just ended
     cur = nxt;
+    nxt = nn;
+    nn = n3;
     L = Ln;
     Ln += Lstep;
     have_next = have_nn;
+    have_nn = have_n3;
     buf ^= 1;
   }
   return Ln;
