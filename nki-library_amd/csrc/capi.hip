@@ -503,6 +503,9 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
            mx_rows_fits(stage, m.wfmt, RowsCall{n_real, a->H, a->E, a->N, a->B, (int64_t)gx, bk.max_chunks});
   };
   mark(2);
+  // the checkpoints' padding rows: with the combine where one call issues it all, behind their stage otherwise
+  constexpr unsigned LAYER = MOE_STAGE_GATE_UP | MOE_STAGE_DOWN | MOE_STAGE_COMBINE;
+  const bool ckpt_tail = mx_fast && (a->gate_up_activations_T || a->down_activations) && (stages & LAYER) == LAYER;
   // Checkpoints of blocks that never run stay zero: cleared ahead for the general kernel; behind the large-tile kernels
   // launch_ckpt_pad clears them with the copies of the padding rows.
   if (!mx_fast && a->gate_up_activations_T && (stages & MOE_STAGE_GATE_UP)) {
@@ -545,8 +548,8 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       rc = launch_gemm_stage(a->kind, 1, g1, gx1, gy, s);
     }
     if (rc != MOE_OK) return rc;
-    if (mx_fast && a->gate_up_activations_T) {
-      rc = launch_ckpt_pad(1, (uint16_t*)a->gate_up_activations_T, bk, a, s);
+    if (mx_fast && a->gate_up_activations_T && !ckpt_tail) {
+      rc = launch_ckpt_pad(1, bk, a, s);
       if (rc != MOE_OK) return rc;
     }
   }
@@ -590,14 +593,14 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       rc = launch_gemm_stage(a->kind, 2, g2, gx2, gy, s);
     }
     if (rc != MOE_OK) return rc;
-    if (mx_fast && a->down_activations) {
-      rc = launch_ckpt_pad(2, (uint16_t*)a->down_activations, bk, a, s);
+    if (mx_fast && a->down_activations && !ckpt_tail) {
+      rc = launch_ckpt_pad(2, bk, a, s);
       if (rc != MOE_OK) return rc;
     }
   }
   mark(5);
   if (stages & MOE_STAGE_COMBINE) {
-    rc = launch_combine(bk, a, ws + p.d, n_real, s);
+    rc = ckpt_tail ? launch_ckpt_tail(bk, a, ws + p.d, n_real, s) : launch_combine(bk, a, ws + p.d, n_real, s);
     if (rc != MOE_OK) return rc;
   }
   mark(6);

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(1024) void plan_chunks_kernel(
 // same results: the GEMMs compute the first of them (see build_chunks), and these kernels copy it to the rest of the
 // expert's blocks and clear the blocks that do not run.  A training-shaped call has as many padding rows as tokens:
 // T = 1024, top-4 of 8 experts of H = 3072, I = 2048, B = 512 lists 7680 rows for 4096 routed ones: the GEMMs over all of them
-// took 205 + 134 us and clearing both checkpoints beforehand 33; over the routed ones 125 + 82, and 15 + 9 for these copies.
+// took 205 + 134 us and clearing both checkpoints beforehand 33; over the routed ones 125 + 82, and 16 + 9 for these copies.
 
 // A block's run (the executed blocks of its expert around it): the slot of the row to copy, and the block's first row
 // behind it; rows 0 .. B of a block that does not run are to be cleared (src = -1).  Every thread of the workgroup gets it.
@@ -154,16 +154,16 @@ __device__ __forceinline__ CkptPad ckpt_pad_of(int64_t b, const int32_t* __restr
 }
 
 constexpr int CKPT_COLS = 64;  // columns of the gate_up checkpoint per workgroup
-__global__ __launch_bounds__(256) void ckpt_pad_gate_up_kernel(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
-                                                               const int32_t* __restrict__ n_active,
-                                                               const int32_t* __restrict__ valid_rows, int64_t B, int64_t E,
-                                                               int64_t cols) {
+// workgroup y of ny that share block b
+__device__ __forceinline__ void ckpt_pad_gate_up(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
+                                                 const int32_t* __restrict__ n_active,
+                                                 const int32_t* __restrict__ valid_rows, int64_t B, int64_t E, int64_t cols,
+                                                 int64_t b, int64_t y, int64_t ny) {
   __shared__ int s_w[3];
   __shared__ uint16_t s_v[CKPT_COLS];
-  const int64_t b = blockIdx.x;
   const CkptPad p = ckpt_pad_of(b, b2e, n_active, valid_rows, B, E, s_w);
   if (p.first >= B) return;
-  for (int64_t c0 = (int64_t)blockIdx.y * CKPT_COLS; c0 < cols; c0 += (int64_t)gridDim.y * CKPT_COLS) {
+  for (int64_t c0 = y * CKPT_COLS; c0 < cols; c0 += ny * CKPT_COLS) {
     __syncthreads();  // (s_v of the pass before)
     const int nc = (int)(cols - c0 < CKPT_COLS ? cols - c0 : CKPT_COLS);
     if ((int)threadIdx.x < nc) {
@@ -193,14 +193,12 @@ __global__ __launch_bounds__(256) void ckpt_pad_gate_up_kernel(uint16_t* __restr
 }
 
 constexpr int CKPT_ROWS = 16;  // rows of the down checkpoint per workgroup
-__global__ __launch_bounds__(256) void ckpt_pad_down_kernel(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
-                                                            const int32_t* __restrict__ n_active,
-                                                            const int32_t* __restrict__ valid_rows, int64_t B, int64_t E,
-                                                            int64_t H) {
+__device__ __forceinline__ void ckpt_pad_down(uint16_t* __restrict__ ck, const int32_t* __restrict__ b2e,
+                                              const int32_t* __restrict__ n_active, const int32_t* __restrict__ valid_rows,
+                                              int64_t B, int64_t E, int64_t H, int64_t b, int64_t y, int64_t ny) {
   __shared__ int s_w[3];
-  const int64_t b = blockIdx.x;
   const CkptPad p = ckpt_pad_of(b, b2e, n_active, valid_rows, B, E, s_w);
-  for (int64_t rb = (int64_t)blockIdx.y * CKPT_ROWS; rb < B; rb += (int64_t)gridDim.y * CKPT_ROWS) {
+  for (int64_t rb = y * CKPT_ROWS; rb < B; rb += ny * CKPT_ROWS) {
     const int64_t r0 = rb < p.first ? p.first : rb, r1 = rb + CKPT_ROWS < B ? rb + CKPT_ROWS : B;
     if (r0 >= r1) continue;
     if (H % 8 == 0 && ((uintptr_t)ck & 15) == 0) {
@@ -218,88 +216,90 @@ __global__ __launch_bounds__(256) void ckpt_pad_down_kernel(uint16_t* __restrict
   }
 }
 
-// The whole bookkeeping of a small problem (decode-sized: a few ten thousand slots) by ONE workgroup of 1024
-// threads in one launch: clear the per-token counts, find the active blocks and their valid rows, count the slots
-// per token, build the expert chunks and the work queues, scan the counts and fill the token -> slot lists.  The
-// four launches it replaces take longer to start than to run at such sizes.  Steps communicate through global
-// memory that this workgroup alone writes and reads, ordered by workgroup barriers.
+// up to this many slots, tokens and blocks the bookkeeping is one launch of one workgroup (prep_small_kernel)
+constexpr int64_t PREP_SMALL_SLOTS = 40960, PREP_SMALL_TOKENS = 4096, PREP_SMALL_BLOCKS = 2048;
+
+// The whole bookkeeping of a small problem (up to a few ten thousand slots) by ONE workgroup of 1024 threads in one
+// launch: find the active blocks and their valid rows, count the slots per token, build the expert chunks and the work
+// queues, scan the counts and fill the token -> slot lists.  The four launches it replaces take longer to start than to
+// run at such sizes.  It is a chain of steps, so what counts is the latency of each: the counts, the list positions and
+// the valid rows live in LDS, and the two passes over the slots deal units of 64 slots to all sixteen waves, four in
+// flight per wave (a wave per block with the counts behind global atomics left three quarters of the waves idle and took 27
+// us at 15 blocks of 512 slots over 1024 tokens; now 17).
 __global__ __launch_bounds__(1024) void prep_small_kernel(
     const int32_t* __restrict__ tp2id, const int32_t* __restrict__ b2e, const int32_t* __restrict__ conditions,
     int64_t n_conditions, int64_t N, int64_t B, int64_t E, int64_t n_real, int32_t* __restrict__ n_active,
-    int32_t* __restrict__ valid_rows, int32_t* __restrict__ cnt, int64_t clear_words, int32_t* __restrict__ n_chunks,
-    int32_t* __restrict__ chunk_slot, int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert,
-    int32_t* __restrict__ chunk_xcd, int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks,
-    int32_t* __restrict__ off, int32_t* __restrict__ cursor, int32_t* __restrict__ list, bool pad_row) {
+    int32_t* __restrict__ valid_rows, int32_t* __restrict__ n_chunks, int32_t* __restrict__ chunk_slot,
+    int32_t* __restrict__ chunk_rows, int32_t* __restrict__ chunk_expert, int32_t* __restrict__ chunk_xcd,
+    int32_t* __restrict__ q_chunk, int32_t* __restrict__ q_off, int64_t max_chunks, int32_t* __restrict__ off,
+    int32_t* __restrict__ list, bool pad_row) {
   __shared__ int s_ws[16];
   __shared__ int s_first_zero;
-  for (int64_t i = threadIdx.x; i < clear_words; i += blockDim.x) cnt[i] = 0;  // cnt and cursor are adjacent
-  for (int64_t b = threadIdx.x; b < N; b += blockDim.x) valid_rows[b] = 0;
-  if (threadIdx.x == 0) s_first_zero = (int)N;
-  __threadfence_block();
+  __shared__ int s_cnt[PREP_SMALL_TOKENS];    // slots per token, then the next free place of its list
+  __shared__ int s_valid[PREP_SMALL_BLOCKS];  // valid rows per block = 1 + last row with a real token
+  const int tid = threadIdx.x;
+  for (int i = tid; i < (int)n_real; i += 1024) s_cnt[i] = 0;
+  for (int b = tid; b < (int)N; b += 1024) s_valid[b] = 0;
+  if (tid == 0) s_first_zero = (int)N;
   __syncthreads();
   if (conditions) {
     const int64_t lim = n_conditions < N ? n_conditions : N;
-    for (int64_t i = threadIdx.x; i < lim; i += blockDim.x)
+    for (int64_t i = tid; i < lim; i += 1024)
       if (conditions[i] == 0) atomicMin(&s_first_zero, (int)i);
+    __syncthreads();
   }
-  __syncthreads();
-  const int na = s_first_zero;
-  if (threadIdx.x == 0) *n_active = na;
-  // A wave per active block, four blocks at a time so that a wave has their loads in flight together (blocks from
-  // the first zero condition on hold nothing: a decode-sized batch is mostly such blocks, and their valid rows
-  // were cleared above).  body(u, slot, row, id) runs for every slot that holds a token in a block with a valid
-  // expert; after(u, block) once per block.
+  const int na = s_first_zero;  // (blocks from the first zero condition on hold nothing)
+  if (tid == 0) *n_active = na;
+  // body(block, slot, row, id, live): 64 neighbouring slots of one block per call; live: a token in a block of an expert
   constexpr int U = 4;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-  const int iB = (int)B;
-  auto over_blocks = [&](auto&& body, auto&& after) {
-    for (int b0 = wave * U; b0 < na; b0 += nwaves * U) {
-      int e[U];
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int iB = (int)B, per = (iB + 63) / 64, units = na * per;
+  auto over_slots = [&](auto&& body) {
+    for (int u0 = wave; u0 < units; u0 += 16 * U) {
+      int e[U], id[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) e[u] = (b0 + u < na) ? b2e[b0 + u] : -1;
-      for (int r0 = 0; r0 < iB; r0 += 64) {
-        const int r = r0 + lane;
-        int id[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) id[u] = (b0 + u < na && r < iB) ? tp2id[(b0 + u) * iB + r] : -1;
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          if (e[u] >= 0 && e[u] < E && id[u] >= 0 && id[u] < n_real) body(u, (b0 + u) * iB + r, r, id[u]);
+      for (int u = 0; u < U; ++u) {
+        const int un = u0 + 16 * u, b = un / per, r = (un - b * per) * 64 + lane;
+        e[u] = un < units ? b2e[b] : -1;
+        id[u] = (un < units && r < iB) ? tp2id[b * iB + r] : -1;
       }
 #pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (b0 + u < na) after(u, b0 + u);
+      for (int u = 0; u < U; ++u) {
+        const int un = u0 + 16 * u, b = un / per, r = (un - b * per) * 64 + lane;
+        if (e[u] >= 0 && e[u] < E) body(b, b * iB + r, r, id[u], id[u] >= 0 && id[u] < n_real);
+      }
     }
   };
-  int v[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) v[u] = 0;
-  over_blocks(
-      [&](int u, int, int r, int id) {
-        v[u] = r + 1;  // rows ascend: the last one stays
-        atomicAdd(&cnt[id], 1);
-      },
-      [&](int u, int b) {
-        int m = v[u];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
-        if (lane == 0) valid_rows[b] = m;  // valid rows = 1 + last row with a real token
-        v[u] = 0;
-      });
+  over_slots([&](int b, int, int r, int id, bool live) {
+    if (live) atomicAdd(&s_cnt[id], 1);
+    const uint64_t m = __ballot(live);
+    if (m != 0 && lane == 0) atomicMax(&s_valid[b], r + 64 - __builtin_clzll(m));  // (lane 0: r is the unit's first row)
+  });
+  __syncthreads();
+  for (int b = tid; b < (int)N; b += 1024) valid_rows[b] = s_valid[b];
   __threadfence_block();
   __syncthreads();
   build_chunks(b2e, n_active, valid_rows, N, B, E, n_chunks, chunk_slot, chunk_rows, chunk_expert, chunk_xcd, q_chunk,
                q_off, max_chunks, s_ws, pad_row);
+  // counts -> list offsets: four consecutive tokens per thread
+  static_assert(PREP_SMALL_TOKENS == 4 * 1024, "one round of the workgroup");
+  {
+    const int i0 = 4 * tid;
+    int v[4], total;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (i0 + j < n_real) ? s_cnt[i0 + j] : 0;
+    int run = block_excl_scan(v[0] + v[1] + v[2] + v[3], s_ws, &total);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (i0 + j < n_real) off[i0 + j] = s_cnt[i0 + j] = run;
+      run += v[j];
+    }
+    if (tid == 0) off[n_real] = total;
+  }
   __syncthreads();
-  inv_scan(cnt, off, n_real, s_ws);
-  __threadfence_block();
-  __syncthreads();
-  over_blocks(
-      [&](int, int sl, int, int id) {
-        const int p = atomicAdd(&cursor[id], 1);
-        list[off[id] + p] = sl;
-      },
-      [&](int, int) {});
+  over_slots([&](int, int sl, int, int id, bool live) {
+    if (live) list[atomicAdd(&s_cnt[id], 1)] = sl;
+  });
 }
 
 __global__ __launch_bounds__(256) void inv_fill_kernel(const int32_t* __restrict__ tp2id,
@@ -319,14 +319,13 @@ __global__ __launch_bounds__(256) void inv_fill_kernel(const int32_t* __restrict
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// One workgroup per output row (a few, side by side along the row, when the rows are too few to fill the GPU:
-// gridDim.y).  D: bf16 [N*B, H] contributions.
-__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ D, const int32_t* __restrict__ off,
-                                                      const int32_t* __restrict__ list, uint16_t* __restrict__ out,
-                                                      uint16_t* __restrict__ out_shard1, int64_t out_row_stride,
-                                                      int64_t H, int64_t n_real) {
+// One workgroup per output row t (a few, side by side along the row, when the rows are too few to fill the GPU: y of
+// ny).  D: bf16 [N*B, H] contributions.
+__device__ __forceinline__ void combine_row(const uint16_t* __restrict__ D, const int32_t* __restrict__ off,
+                                            const int32_t* __restrict__ list, uint16_t* __restrict__ out,
+                                            uint16_t* __restrict__ out_shard1, int64_t out_row_stride, int64_t H,
+                                            int64_t n_real, int64_t t, int64_t y, int64_t ny) {
   __shared__ int s_sorted[COMBINE_MAX_K];
-  const int64_t t = blockIdx.x;
   int cnt = 0, base = 0;
   if (t < n_real) {
     base = off[t];
@@ -353,7 +352,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   uint16_t* zrow = out_shard1 ? out_shard1 + t * out_row_stride : nullptr;  // the other shard's row: zeros
   const bool vec = (H % 8 == 0) && ((out_row_stride % 8) == 0) && (((uintptr_t)out & 15) == 0) &&
                    (((uintptr_t)out_shard1 & 15) == 0);
-  const int64_t vt = (int64_t)blockIdx.y * blockDim.x + threadIdx.x, vstride = (int64_t)gridDim.y * blockDim.x;
+  const int64_t vt = y * blockDim.x + threadIdx.x, vstride = ny * blockDim.x;
   if (vec) {
     for (int64_t c = vt * 8; c < H; c += vstride * 8) {
       float acc[8];
@@ -397,6 +396,48 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
   }
 }
 
+__global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict__ D, const int32_t* __restrict__ off,
+                                                      const int32_t* __restrict__ list, uint16_t* __restrict__ out,
+                                                      uint16_t* __restrict__ out_shard1, int64_t out_row_stride,
+                                                      int64_t H, int64_t n_real) {
+  combine_row(D, off, list, out, out_shard1, out_row_stride, H, n_real, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// The checkpoints' padding rows and the combine of one layer in one launch: three jobs that share no data and are each too
+// short to fill the memory system from start to end.  Workgroups [0, n_gu) take the gate_up checkpoint (y_gu per block), the
+// next n_dn the down checkpoint, the rest the output rows.  T = 1024, top-4 of 8 experts of H = 3072, I = 2048, B = 512:
+// 16.5 + 9 + 10 us in three launches.
+struct CkptTail {
+  uint16_t *ck_gu, *ck_dn;
+  const int32_t *b2e, *n_active, *valid_rows;
+  int64_t B, E, cols, H;
+  int64_t n_gu, y_gu, n_dn, y_dn, y_c;
+};
+__global__ __launch_bounds__(256) void ckpt_tail_kernel(const CkptTail k, const uint16_t* __restrict__ D,
+                                                        const int32_t* __restrict__ off, const int32_t* __restrict__ list,
+                                                        uint16_t* __restrict__ out, uint16_t* __restrict__ out_shard1,
+                                                        int64_t out_row_stride, int64_t n_real) {
+  int64_t i = blockIdx.x;
+  if (i < k.n_gu) {
+    ckpt_pad_gate_up(k.ck_gu, k.b2e, k.n_active, k.valid_rows, k.B, k.E, k.cols, i / k.y_gu, i % k.y_gu, k.y_gu);
+    return;
+  }
+  i -= k.n_gu;
+  if (i < k.n_dn) {
+    ckpt_pad_down(k.ck_dn, k.b2e, k.n_active, k.valid_rows, k.B, k.E, k.H, i / k.y_dn, i % k.y_dn, k.y_dn);
+    return;
+  }
+  i -= k.n_dn;
+  combine_row(D, off, list, out, out_shard1, out_row_stride, k.H, n_real, i / k.y_c, i % k.y_c, k.y_c);
+}
+// (one stage of a layer that is issued stage by stage)
+__global__ __launch_bounds__(256) void ckpt_pad_kernel(const CkptTail k) {
+  if (k.n_gu)
+    ckpt_pad_gate_up(k.ck_gu, k.b2e, k.n_active, k.valid_rows, k.B, k.E, k.cols, blockIdx.x / k.y_gu, blockIdx.x % k.y_gu, k.y_gu);
+  else
+    ckpt_pad_down(k.ck_dn, k.b2e, k.n_active, k.valid_rows, k.B, k.E, k.H, blockIdx.x / k.y_dn, blockIdx.x % k.y_dn, k.y_dn);
+}
+
 // ---- host-side orchestration used by moe_blockwise() -------------------------------------
 
 size_t bookkeeping_bytes(int64_t T1, int64_t N, int64_t B) {
@@ -428,19 +469,16 @@ Bookkeeping carve_bookkeeping(void* base, int64_t T1, int64_t N, int64_t B) {
   return k;
 }
 
-// up to this many slots and tokens the bookkeeping is one launch of one workgroup (prep_small_kernel)
-constexpr int64_t PREP_SMALL_SLOTS = 40960, PREP_SMALL_TOKENS = 4096;
-
 int launch_prep(const Bookkeeping& k, const moe_bwmm_args* a, int64_t n_real, hipStream_t s) {
   const bool pad_row = a->gate_up_activations_T != nullptr || a->down_activations != nullptr;
   // cnt and cursor are adjacent: one clear covers both.  A fill kernel rather than a memset
   // node, so that the sequence stays safe to record into a HIP graph.
   const int64_t clear_words = (int64_t)((uint8_t*)k.off - (uint8_t*)k.cnt) / 4;
-  if (a->N * a->B <= PREP_SMALL_SLOTS && n_real <= PREP_SMALL_TOKENS) {
+  if (a->N * a->B <= PREP_SMALL_SLOTS && n_real <= PREP_SMALL_TOKENS && a->N <= PREP_SMALL_BLOCKS) {
     hipLaunchKernelGGL(prep_small_kernel, dim3(1), dim3(1024), 0, s, a->token_position_to_id, a->block_to_expert,
-                       a->conditions, a->n_conditions, a->N, a->B, a->E, n_real, k.n_active, k.valid_rows, k.cnt,
-                       clear_words, k.n_chunks, k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk,
-                       k.q_off, k.max_chunks, k.off, k.cursor, k.list, pad_row);
+                       a->conditions, a->n_conditions, a->N, a->B, a->E, n_real, k.n_active, k.valid_rows, k.n_chunks,
+                       k.chunk_slot, k.chunk_rows, k.chunk_expert, k.chunk_xcd, k.q_chunk, k.q_off, k.max_chunks, k.off,
+                       k.list, pad_row);
     MOE_CHECK_LAUNCH();
     return MOE_OK;
   }
@@ -472,31 +510,46 @@ int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int
   return MOE_OK;
 }
 
-int launch_ckpt_pad(int stage, uint16_t* ck, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s) {
-  const int64_t cols = 2 * a->I;
-  const int64_t gy = stage == 1 ? (cols + CKPT_COLS - 1) / CKPT_COLS : (a->B + CKPT_ROWS - 1) / CKPT_ROWS;
-  const dim3 grid((unsigned)a->N, (unsigned)(gy < 65535 ? gy : 65535));
-  if (stage == 1)
-    hipLaunchKernelGGL(ckpt_pad_gate_up_kernel, grid, dim3(256), 0, s, ck, a->block_to_expert, k.n_active, k.valid_rows, a->B,
-                       a->E, cols);
-  else
-    hipLaunchKernelGGL(ckpt_pad_down_kernel, grid, dim3(256), 0, s, ck, a->block_to_expert, k.n_active, k.valid_rows, a->B,
-                       a->E, a->H);
+static int64_t at_most(int64_t v, int64_t lim) { return v < lim ? v : lim; }
+// few rows (decode): up to 8 workgroups share a row of the result, 8 columns per thread each
+static int64_t combine_split(const moe_bwmm_args* a) {
+  return a->T1 <= 256 ? at_most((a->H + 256 * 8 - 1) / (256 * 8), 8) : 1;
+}
+static CkptTail ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, bool gate_up, bool down) {
+  CkptTail t;
+  t.ck_gu = (uint16_t*)a->gate_up_activations_T;
+  t.ck_dn = (uint16_t*)a->down_activations;
+  t.b2e = a->block_to_expert; t.n_active = k.n_active; t.valid_rows = k.valid_rows;
+  t.B = a->B; t.E = a->E; t.cols = 2 * a->I; t.H = a->H;
+  // (a grid below 2^31 workgroups: N * B is, and a workgroup per block and 64 columns or 16 rows at most)
+  t.y_gu = at_most((t.cols + CKPT_COLS - 1) / CKPT_COLS, at_most(65535, ((int64_t)1 << 29) / a->N + 1));
+  t.y_dn = at_most((a->B + CKPT_ROWS - 1) / CKPT_ROWS, at_most(65535, ((int64_t)1 << 29) / a->N + 1));
+  t.n_gu = gate_up ? a->N * t.y_gu : 0;
+  t.n_dn = down ? a->N * t.y_dn : 0;
+  t.y_c = combine_split(a);
+  return t;
+}
+
+int launch_ckpt_pad(int stage, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s) {
+  const CkptTail t = ckpt_tail(k, a, stage == 1, stage == 2);
+  hipLaunchKernelGGL(ckpt_pad_kernel, dim3((unsigned)(t.n_gu + t.n_dn)), dim3(256), 0, s, t);
+  MOE_CHECK_LAUNCH();
+  return MOE_OK;
+}
+
+int launch_ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s) {
+  const CkptTail t = ckpt_tail(k, a, a->gate_up_activations_T != nullptr, a->down_activations != nullptr);
+  const int64_t grid = t.n_gu + t.n_dn + a->T1 * t.y_c;
+  if (grid >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
+  hipLaunchKernelGGL(ckpt_tail_kernel, dim3((unsigned)grid), dim3(256), 0, s, t, (const uint16_t*)D, k.off, k.list,
+                     (uint16_t*)a->output, (uint16_t*)a->output_shard1, a->out_row_stride, n_real);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
 
 int launch_combine(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s) {
-  // few rows (decode): up to 8 workgroups share a row, 8 columns per thread each
-  unsigned split = 1;
-  if (a->T1 <= 256) {
-    const int64_t per_wg = 256 * 8;
-    split = (unsigned)((a->H + per_wg - 1) / per_wg);
-    if (split > 8) split = 8;
-    if (split < 1) split = 1;
-  }
-  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)a->T1, split), dim3(256), 0, s, (const uint16_t*)D, k.off, k.list,
-                     (uint16_t*)a->output, (uint16_t*)a->output_shard1, a->out_row_stride, a->H, n_real);
+  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)a->T1, (unsigned)combine_split(a)), dim3(256), 0, s, (const uint16_t*)D,
+                     k.off, k.list, (uint16_t*)a->output, (uint16_t*)a->output_shard1, a->out_row_stride, a->H, n_real);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }

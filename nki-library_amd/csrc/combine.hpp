@@ -66,7 +66,9 @@ int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int
                        hipStream_t s);
 // The padding rows and the blocks that do not run of the gate/up (stage 1) or down (2) checkpoint, after the large-tile
 // GEMM that wrote the other rows.
-int launch_ckpt_pad(int stage, uint16_t* ck, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s);
+int launch_ckpt_pad(int stage, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s);
+// Both and the combine in one launch (a layer issued in one call).
+int launch_ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s);
 int launch_combine(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s);
 // Zero `bytes` bytes at p (a multiple of 4, p 4-byte aligned) with a kernel, so that callers may capture it in a graph.
 int launch_fill_zero_bytes(void* p, size_t bytes, hipStream_t s);
