@@ -94,8 +94,7 @@ def build(verbose=True, jobs=None):
     jobs = jobs or min(len(cmds), os.cpu_count() or 4, 16)
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         errs = list(ex.map(_run, cmds))
-        # (4-bit weights run on the other tile loop, all of whose loads carry the longer wait)
-        list(ex.map(check_tile_code, [u[0] for u, (_, fmt) in zip(units, MX_INSTANCES) if fmt != 2]))
+        list(ex.map(check_tile_code, [u[0] for u in units[:len(MX_INSTANCES)]]))
     link = ["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", *[u[0] for u in units], "-o", OUT]
     if verbose:
         print(" ".join(link), flush=True)

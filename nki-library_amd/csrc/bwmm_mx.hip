@@ -1004,8 +1004,8 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int interleave = __builtin_amdgcn_readfirstlane(a.q_off[8 * (CHUNK_CLASSES + 1)]);
   int L = w;
   // classes in queue order (CHUNK_CLASS_TILES / CHUNK_CLASS_LAST in combine.hpp)
-  // (tiles of up to 64 rows stream their weights through registers, three slices ahead; 4-bit weights likewise)
-#define MX_TILES(TILES_) (WFMT != MX_WFMT_E2M1 && (TILES_) >= 8)
+  // (tiles of up to 64 rows stream their weights through registers, three slices ahead)
+#define MX_TILES(TILES_) ((TILES_) >= 8)
 #define MX_RUN_TILES(TILES_, LAST_)                                                                               \
   if constexpr (MX_TILES(TILES_))                                                                                \
     L = mx_gemm_tiles_wide<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \
@@ -1073,8 +1073,7 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 
 #define MX_CAT_(a, b, c, d) a##b##c##d
 #define MX_CAT(a, b, c, d) MX_CAT_(a, b, c, d)
-constexpr int MX_LDS_LAUNCH = MX_INST_WFMT == MX_WFMT_E2M1 ? MX_LDS
-                              : MX_INST_WFMT == MX_WFMT_ROW8 || MX_INST_WFMT == MX_WFMT_BF16
+constexpr int MX_LDS_LAUNCH = MX_INST_WFMT == MX_WFMT_ROW8 || MX_INST_WFMT == MX_WFMT_BF16
                                   ? (MX_LDS > MX_WIDE_LDS_PLAIN ? MX_LDS : MX_WIDE_LDS_PLAIN)
                                   : (MX_LDS > MX_WIDE_LDS_SCALED ? MX_LDS : MX_WIDE_LDS_SCALED);
 int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT)(const MxArgs& m, unsigned grid, hipStream_t s) {

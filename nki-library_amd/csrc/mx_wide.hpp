@@ -1,5 +1,4 @@
-// The tile loop of the large-tile expert GEMMs for tiles of 8 to 20 row tiles and 8-bit or bf16 weights: both operands
-// through LDS.
+// The tile loop of the large-tile expert GEMMs for tiles of 8 to 20 row tiles: both operands through LDS.
 //
 // A workgroup (4 waves, one per SIMD) multiplies up to 320 rows x 256 columns.  The waves stand in a 2 x 2 grid: wave
 // (wm, wn) owns half of the row tiles and 128 columns, so that a K slice of 128 bytes costs it 8 + 8 operand fragments for
@@ -59,9 +58,11 @@ constexpr int MX_WIDE_LDS_PLAIN = MxWideCfg<20>::LDS_PLAIN, MX_WIDE_LDS_SCALED =
 #define MXW_MFMA(FMT_)                                                                                          \
   asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 a[%0:%1], %2, %3, a[%0:%1], %4, %5 op_sel_hi:[0,0,0]" FMT_     \
                : : "n"(ACC), "n"(ACC + 3), "v"(wf), "v"(af), "v"(sw), "v"(sa))
-template <int ACC, int WFMT, int HALF>
-__device__ __forceinline__ void mxw_mfma(const v8i& wf, const v8i& af, int sw, int sa) {
-  if constexpr (WFMT == MX_WFMT_BF16) {
+template <int ACC, int WFMT, int HALF, class WFrag>
+__device__ __forceinline__ void mxw_mfma(const WFrag& wf, const v8i& af, int sw, int sa) {
+  if constexpr (WFMT == MX_WFMT_E2M1) {
+    MXW_MFMA(" cbsz:4");
+  } else if constexpr (WFMT == MX_WFMT_BF16) {
     const v4i w4 = HALF ? (v4i){wf[4], wf[5], wf[6], wf[7]} : (v4i){wf[0], wf[1], wf[2], wf[3]};
     const v4i a4 = HALF ? (v4i){af[4], af[5], af[6], af[7]} : (v4i){af[0], af[1], af[2], af[3]};
     asm volatile("v_mfma_f32_16x16x32_bf16 a[%0:%1], %2, %3, a[%0:%1]" : : "n"(ACC), "n"(ACC + 3), "v"(w4), "v"(a4));
@@ -76,9 +77,11 @@ __device__ __forceinline__ void mxw_mfma(const v8i& wf, const v8i& af, int sw, i
 #define MXW_MFMA(FMT_)                                                                                       \
   asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0]" FMT_              \
                : "+v"(acc) : "v"(wf), "v"(af), "v"(sw), "v"(sa))
-template <int WFMT, int HALF>
-__device__ __forceinline__ void mxw_mfma_v(v4f& acc, const v8i& wf, const v8i& af, int sw, int sa) {
-  if constexpr (WFMT == MX_WFMT_BF16) {
+template <int WFMT, int HALF, class WFrag>
+__device__ __forceinline__ void mxw_mfma_v(v4f& acc, const WFrag& wf, const v8i& af, int sw, int sa) {
+  if constexpr (WFMT == MX_WFMT_E2M1) {
+    MXW_MFMA(" cbsz:4");
+  } else if constexpr (WFMT == MX_WFMT_BF16) {
     const v4i w4 = HALF ? (v4i){wf[4], wf[5], wf[6], wf[7]} : (v4i){wf[0], wf[1], wf[2], wf[3]};
     const v4i a4 = HALF ? (v4i){af[4], af[5], af[6], af[7]} : (v4i){af[0], af[1], af[2], af[3]};
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w4), "v"(a4));
@@ -128,11 +131,13 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
                                                   float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L,
                                                   const int startL, const int endL, const int Lstep, const int qbase,
                                                   const int interleave) {
-  static_assert(NMT >= 8 && NMT % 2 == 0 && WFMT != MX_WFMT_E2M1, "8-bit and bf16 weights, at least four row tiles per wave");
+  static_assert(NMT >= 8 && NMT % 2 == 0, "at least four row tiles per wave");
   using Cfg = MxWideCfg<NMT>;
   constexpr bool BF16 = WFMT == MX_WFMT_BF16;
   constexpr bool ROW8 = WFMT == MX_WFMT_ROW8 || BF16;
   constexpr bool SCALED = !ROW8;
+  constexpr bool FP4 = WFMT == MX_WFMT_E2M1;
+  constexpr int ES = FP4 ? 2 : 4;  // bytes of a weight element (four K values of a column)
   constexpr int RT = Cfg::RT, SA = Cfg::SA, SW = Cfg::SW;
   constexpr bool BIG = NMT > 16;  // row tiles 8, 9 of a wave accumulate in ordinary registers
 
@@ -152,7 +157,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   //     MX: tile pair = quarter q, pieces = 4 of the 8 pieces (of 4 partitions) that wave wn owns of each quarter
   //     bf16: tile pairs 2j, 2j+1 = quarter 2 wn + j, a lane gets 8 neighbouring columns of the two pairs (16-byte stores)
   //     fp8-row: the same quarters, a lane 4 neighbouring columns of each pair (fp32 results, 16-byte stores)
-  //   down: tile pairs, a lane gets 8 neighbouring columns of a pair (bf16 results, 16-byte stores)
+  //   down: tile pairs, a lane gets 8 neighbouring columns of a pair (4-bit weights, whose DMA brings two pieces at a time:
+  //     twice 4)
   struct Piece {
     int q, gu, cl;  // gate/up: quarter, gate or up, piece of 4 partitions among the column tile's 8; down: cl alone
   };
@@ -161,7 +167,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     const int t = tt >> 1, odd = tt & 1;
     if (STAGE == 2) {
       p.q = 0; p.gu = 0;
-      p.cl = pwn * 32 + t * 8 + 2 * gq + odd;
+      p.cl = pwn * 32 + t * 8 + (FP4 ? 4 * odd + gq : 2 * gq + odd);
     } else if (SCALED) {
       p.q = t; p.gu = odd;
       p.cl = pwn * 4 + gq;
@@ -181,23 +187,25 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   const int64_t w_pstride = (STAGE == 1) ? 2 * (int64_t)nH * a.I : (int64_t)a.nI * a.H;  // elements between partitions
   const int64_t w_tstride = (STAGE == 1) ? a.I : a.H;                                     // ... between tiles of 512
   const bool pk = a.w_packed != 0;
-  constexpr int PK_LOAD = 1024, PK_WAVE = 8 * PK_LOAD, PK_SLICE = 4 * PK_WAVE;
+  constexpr int PK_LANE = FP4 ? 8 : 16, PK_LOAD = 64 * PK_LANE, PK_WAVE = 8 * PK_LOAD, PK_SLICE = 4 * PK_WAVE;
   const int64_t w_expert_bytes = pk ? (int64_t)a.col_tiles * nks * PK_SLICE
-                                    : (STAGE == 1 ? 128 : (int64_t)a.pI) * w_pstride * 4;
+                                    : (STAGE == 1 ? 128 : (int64_t)a.pI) * w_pstride * ES;
   const int64_t ws_expert_bytes = (STAGE == 1 ? 16 : ((int64_t)a.pI + 7) / 8) * w_pstride;
-  // a weight slice: wave w brings partitions 4 w .. 4 w + 3 and 16 + 4 w .. 16 + 4 w + 3; all of these have the swizzle w
-  const int w_step = uni(pk ? PK_LOAD : (int)(w_pstride * 4)), w_jump = uni(pk ? 4 * PK_LOAD : (int)(w_pstride * 64));
-  const int w_pb = uni(pk ? PK_SLICE : (int)(w_pstride * 128)), w_kt = uni(pk ? 4 * PK_SLICE : (int)(w_tstride * 4));
+  // a weight slice: wave w brings partitions 4 w .. 4 w + 3 and 16 + 4 w .. 16 + 4 w + 3, one per load, or (4-bit weights)
+  // 8 w .. 8 w + 7, two per load; all of these have the swizzle w
+  const int w_step = uni(pk ? 1024 : (int)(w_pstride * 4)), w_jump = uni(pk ? 4 * PK_LOAD : (int)(w_pstride * 64));
+  const int w_pb = uni(pk ? PK_SLICE : (int)(w_pstride * 32 * ES)), w_kt = uni(pk ? 4 * PK_SLICE : (int)(w_tstride * ES));
   const int ws_pb = uni((int)(w_pstride * 4)), ws_kt = uni((int)w_tstride);
-  const int lu = (lane >> 2) ^ w;  // logical 64-byte unit that belongs at the lane's place
-  const Piece lp = piece_at(lu >> 3, lu & 7, lane & 3);                    // ... its piece, for the weights
+  const int lu = FP4 ? ((lane & 31) >> 1) ^ w : (lane >> 2) ^ w;  // logical column tile that belongs at the lane's place
+  const Piece lp = piece_at(lu >> 3, lu & 7, FP4 ? 2 * (lane & 1) : lane & 3);  // ... its (first) piece, for the weights
   const Piece sp = piece_at(lane >> 5, (lane >> 2) & 7, lane & 3);         // the lane's piece of the weight scales (no swizzle)
 
   // ---- loads ----------------------------------------------------------------------------------------------------
   constexpr int NAJ = NMT / 2;            // activation loads of a slice per wave (8 rows x 128 bytes each)
   constexpr int NA1 = (NAJ + 1) / 2;      // ... of these behind B2, the others under the next slice's first MFMAs
   constexpr int NAS = SCALED ? (BIG ? 2 : 1) : 0;  // loads of the activation scales, one set for four slices
-  constexpr int NW = 8 + (SCALED ? 1 : 0);
+  constexpr int NWL = FP4 ? 4 : 8;        // weight loads of a slice per wave
+  constexpr int NW = NWL + (SCALED ? 1 : 0);
   constexpr int NAV = (STAGE == 1) ? NAJ : 1;
   const int arow0 = tid >> 3, ach = tid & 7;
   uint32_t a_voff[NAV], as_voff = 0, as_voff2 = 0, w_voff = 0, ws_voff = 0;
@@ -245,12 +253,14 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     auto piece_elem = [&](const Piece& p) {
       return (STAGE == 1) ? (uint32_t)(p.gu * nH) * (uint32_t)a.I + (uint32_t)(p.q * Pt + p.cl * 4) : (uint32_t)(p.cl * 4);
     };
+    // (4-bit weights: the upper half of the wave brings the second partition of a load)
     if (pk)
-      w_voff = (STAGE == 1) ? (uint32_t)(lp.q * PK_WAVE + (w * 16 + ((lp.cl >> 2) & 1) * 8 + lp.gu * 4 + (lp.cl & 3)) * 16)
-                            : (uint32_t)((lp.cl >> 4) * PK_WAVE + (w * 16 + (lp.cl & 15)) * 16);
+      w_voff = ((STAGE == 1) ? (uint32_t)(lp.q * PK_WAVE + (w * 16 + ((lp.cl >> 2) & 1) * 8 + lp.gu * 4 + (lp.cl & 3)) * PK_LANE)
+                             : (uint32_t)((lp.cl >> 4) * PK_WAVE + (w * 16 + (lp.cl & 15)) * PK_LANE)) +
+               (FP4 ? (uint32_t)((lane >> 5) * PK_LOAD) : 0u);
     else
-      w_voff = (uint32_t)(4 * w) * (uint32_t)(w_pstride * 4) + piece_elem(lp) * 4u;
-    w_base = uni(pk ? t.xt * nks * PK_SLICE : colu * 4);
+      w_voff = (uint32_t)(FP4 ? 8 * w + (lane >> 5) : 4 * w) * (uint32_t)(w_pstride * ES) + piece_elem(lp) * (uint32_t)ES;
+    w_base = uni(pk ? t.xt * nks * PK_SLICE : colu * ES);
     rw_ = make_rsrc((const uint8_t*)a.W + (int64_t)t.e * w_expert_bytes, (uint32_t)w_expert_bytes);
     rw_rec = rw_[2];
     if constexpr (SCALED) {
@@ -287,8 +297,9 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   auto load_w = [&](auto u_, auto i_, auto loop_) {
     constexpr int U = decltype(u_)::value, i = decltype(i_)::value;
     constexpr bool LOOP = decltype(loop_)::value;
-    if constexpr (i < 8)
-      dma_b128<U * SW + (i < 4 ? i : 12 + i) * 1024, LASTUSE, LOOP>(lds_w, w_voff, rw_, w_off + (i < 4 ? i * w_step : w_jump + (i - 4) * w_step));
+    if constexpr (i < NWL)
+      dma_b128<U * SW + (FP4 || i < 4 ? i : 12 + i) * 1024, LASTUSE, LOOP>(
+          lds_w, w_voff, rw_, w_off + (FP4 || i < 4 ? i * w_step : w_jump + (i - 4) * w_step));
     else
       dma_b32<U * Cfg::WS, LOOP>(lds_ws, ws_voff, rs_, ws_off);
   };
@@ -307,12 +318,18 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   const uint8_t* pa_lo = smem + (wm * RT * 16 + c) * MXROW + ((g ^ (c & 7)) * 16);
   const uint8_t* pa_hi = smem + (wm * RT * 16 + c) * MXROW + (((g + 4) ^ (c & 7)) * 16);
   // Column tile 4 x + b of the wave: 64-byte unit wn * 8 + 4 x + (b ^ g), dword c, of partitions 4 g + r and 16 + 4 g + r.
-  const uint8_t* pw[4];
+  // (4-bit weights: 32-byte units, a dword holds two columns, partitions 8 g + r)
+  const uint8_t* pw[FP4 ? 8 : 4];
 #pragma unroll
-  for (int b = 0; b < 4; ++b) pw[b] = smem + Cfg::OFF_W + 4 * g * 1024 + (wn * 8 + (b ^ g)) * 64 + c * 4;
+  for (int b = 0; b < (FP4 ? 8 : 4); ++b)
+    pw[b] = smem + Cfg::OFF_W + 4096 * g + (wn * 8 + ((b & 4) | ((b & 3) ^ g))) * (16 * ES) + (FP4 ? c >> 1 : c) * 4;
   const uint8_t* pas = smem + Cfg::OFF_AS + (wm * RT * 16 + c) * 16 + g;
   const uint8_t* pws = smem + Cfg::OFF_WS + g * Cfg::WSP + wn * 128 + c;
-  v8i wf[8], af[2][2];
+  typedef typename std::conditional<FP4, v4i, v8i>::type WFrag;
+  WFrag wf[8];
+  v8i af[2][2];
+  v8i wraw[4];  // 4-bit weights as read, column tile t in t & 3: two columns to a dword, see finish_w
+  const uint32_t half_sel = (c & 1) ? 0x07060302u : 0x05040100u;  // the lane's column of the two
   int wsc[8], asc[RT];
 #pragma unroll
   for (int i = 0; i < 8; ++i) wsc[i] = 0x7f;
@@ -320,12 +337,29 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   for (int i = 0; i < RT; ++i) asc[i] = 0x7f;
   auto read_w = [&](auto u_, auto t_) {
     constexpr int U = decltype(u_)::value, tt = decltype(t_)::value;
-    const uint8_t* p = pw[tt & 3] + U * SW + (tt >> 2) * 256;
-    v8i f;
+    if constexpr (FP4) {
+      const uint8_t* p = pw[tt] + U * SW;
 #pragma unroll
-    for (int r = 0; r < 8; ++r) f[r] = *(const int*)(p + (r < 4 ? r : 12 + r) * 1024);
-    wf[tt] = f;
+      for (int r = 0; r < 8; ++r) wraw[tt & 3][r] = *(const int*)(p + r * 512);
+    } else {
+      const uint8_t* p = pw[tt & 3] + U * SW + (tt >> 2) * 256;
+      v8i f;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) f[r] = *(const int*)(p + (r < 4 ? r : 12 + r) * 1024);
+      wf[tt] = f;
+    }
     if constexpr (SCALED) wsc[tt] = *(pws + U * Cfg::WS + tt * 16);
+  };
+  // 4-bit weights: two partitions of the lane's column to a register (and the distance that an MFMA needs behind a vector
+  // instruction that wrote its operand)
+  auto finish_w = [&](auto t_) {
+    constexpr int tt = decltype(t_)::value;
+    if constexpr (FP4) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        wf[tt][r] = (int)__builtin_amdgcn_perm((uint32_t)wraw[tt & 3][2 * r + 1], (uint32_t)wraw[tt & 3][2 * r], half_sel);
+      asm volatile("s_nop 1" : "+v"(wf[tt]));
+    }
   };
   auto read_a = [&](auto u_, auto i_, v8i& f) {
     constexpr int o = decltype(u_)::value * SA + decltype(i_)::value * 16 * MXROW;
@@ -398,6 +432,10 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
           mul(std::integral_constant<int, j - 1>{}, std::integral_constant<int, 1>{});
           mul(j_, std::integral_constant<int, 1>{});
         }
+        if constexpr (m == 3) {  // the last two column tiles that were read
+          finish_w(std::integral_constant<int, 6>{});
+          finish_w(std::integral_constant<int, 7>{});
+        }
         // loads, spread over the MFMAs between the barriers
         if constexpr (m < MB1) {
           constexpr int NA2 = NAJ - NA1;
@@ -407,7 +445,10 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
           static_for<n * NW / span, (n + 1) * NW / span>([&](auto i_) { load_w(UC{}, i_, loop_); });
         } else {
           constexpr int n = m - MB2;
-          if constexpr (n % 2 == 1) read_w(UN{}, std::integral_constant<int, n / 2>{});
+          if constexpr (n % 2 == 1) {
+            read_w(UN{}, std::integral_constant<int, n / 2>{});
+            if constexpr (n / 2 >= 2) finish_w(std::integral_constant<int, n / 2 - 2>{});
+          }
           static_for<n * NA1 / 16, (n + 1) * NA1 / 16>([&](auto i_) { load_a(UC{}, i_, loop_); });
           if constexpr (n % 2 == 1) asm volatile("" ::: "memory");
         }
@@ -494,6 +535,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       static_for<0, RT - 2>([&](auto i_) { read_as(i_, 0); });
       static_for<0, 8>([&](auto t_) {
         read_w(S0{}, t_);
+        if constexpr (decltype(t_)::value >= 2) finish_w(std::integral_constant<int, decltype(t_)::value - 2>{});
         asm volatile("" ::: "memory");  // (reads of two column tiles are not to be merged: their halves would need moves)
       });
     }
@@ -796,7 +838,17 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const v4i rd = make_rsrc(a.D + (int64_t)cur.slot0 * a.H, (uint32_t)((int64_t)cur.nrows * a.H * 2));
       // bf16 kind: the down checkpoint [N, B, H] = [slots, H] takes the same rows ahead of the affinity
       const v4i rdc = make_rsrc((BF16 ? a.ckpt : a.D) + (int64_t)cur.slot0 * a.H, (uint32_t)((int64_t)cur.nrows * a.H * 2));
-      const int lcol = 128 * wn + 8 * g_e;  // the lane's first column of tile pair 0 within the tile
+      const int lcol = 128 * wn + (FP4 ? 4 : 8) * g_e;  // the lane's first column of tile pair 0 within the tile
+      constexpr int HI = FP4 ? 16 : 4;                  // ... of the pair's second tile behind that of its first
+      auto put = [&](int t, const v4i& o) {
+        if constexpr (FP4) {
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            *(v2i*)(ex_w + (((4 * t + 2 * h + (g_e >> 1)) ^ c_e) & 15) * 16 + (g_e & 1) * 8) = (v2i){o[2 * h], o[2 * h + 1]};
+        } else {
+          ex_put(4 * t + g_e, o);
+        }
+      };
       const uint32_t d_voff = (uint32_t)(st_row0 * rowb) + (uint32_t)(((int)tw.tile_h0(cur) + 128 * wn) * 2 + st_piece * 16);
       float affs[RT], rss[RT];
 #pragma unroll
@@ -813,10 +865,10 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
           for (int t = 0; t < 4; ++t)
 #pragma unroll
             for (int k = 0; k < 8; k += 4) {
-              const float4 vb = *(const float4*)(s_bias[buf] + lcol + 32 * t + k);
+              const float4 vb = *(const float4*)(s_bias[buf] + lcol + 32 * t + (k ? HI : 0));
               bd[t][k] = vb.x; bd[t][k + 1] = vb.y; bd[t][k + 2] = vb.z; bd[t][k + 3] = vb.w;
               if constexpr (ROW8) {
-                const float4 vs = *(const float4*)(s_wsc[buf] + lcol + 32 * t + k);
+                const float4 vs = *(const float4*)(s_wsc[buf] + lcol + 32 * t + (k ? HI : 0));
                 sd[t][k] = vs.x; sd[t][k + 1] = vs.y; sd[t][k + 2] = vs.z; sd[t][k + 3] = vs.w;
               }
             }
@@ -848,12 +900,12 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
           if constexpr (rt > 0) store(rt - 1, rd);
           if constexpr (CKPT) {
 #pragma unroll
-            for (int t = 0; t < 4; ++t) ex_put(4 * t + g_e, oc[t]);
+            for (int t = 0; t < 4; ++t) put(t, oc[t]);
             ex_get(ex_o);
             store(rt, rdc);
           }
 #pragma unroll
-          for (int t = 0; t < 4; ++t) ex_put(4 * t + g_e, o[t]);
+          for (int t = 0; t < 4; ++t) put(t, o[t]);
           ex_get(ex_o);
           spread(rt_);
         });

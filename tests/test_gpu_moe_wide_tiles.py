@@ -24,7 +24,8 @@ def test_wide_mx(rows, I):
     _check(o[0, :rows], _golden_mx_options(c, 3, REF_MX_CLAMPS)[:rows], f"wide mx rows={rows} I={I}")
 
 
-@pytest.mark.parametrize("rows,fmt,copies", [(200, "e5m2", True), (300, "e5m2", False), (320, "e4m3", False), (193, "e4m3", False)])
+@pytest.mark.parametrize("rows,fmt,copies", [(200, "e5m2", True), (300, "e5m2", False), (320, "e4m3", False), (193, "e4m3", False),
+                                              (128, "e2m1", True), (256, "e2m1", False), (320, "e2m1", True), (577, "e2m1", False)])
 def test_wide_mx_formats_and_layouts(rows, fmt, copies):
     from nkilib.core.moe.moe_cte import _launch
 
