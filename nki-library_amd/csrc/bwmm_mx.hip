@@ -1,36 +1,25 @@
-// Blockwise expert GEMMs for gfx950, large-tile version: the launch, and the tile loop of 4-bit weights and of tiles of up
-// to 64 rows (all others: mx_wide.hpp, both operands through LDS).
+// Blockwise expert GEMMs for gfx950, large-tile version: the launch, the weight copies in read order, and the tile loop of
+// chunks of up to 64 rows.  (Chunks of more rows: mx_wide.hpp.)
 //
-// A 256-thread workgroup (4 waves, one per SIMD) owns an "expert chunk" of up to 320 consecutive
-// slots of one expert and 256 output columns:
+// A 256-thread workgroup (4 waves, one per SIMD) owns a chunk of consecutive slots of one expert and 256 output columns:
 //   gate/up: 32 intermediate partitions p x 4 q, for gate and for up; wave w owns q = w
 //   down:    256 hidden columns; wave w owns 64 of them
-// so every weight byte that enters the CU is used by all rows of the chunk, and both operands enter
-// the CU exactly once per workgroup (smaller or split tiles were measured: 128-row workgroups double
-// the traffic into the CU and, because sibling workgroups drift apart by more K slices than the L2
-// holds, the traffic over the fabric as well).  A wave accumulates rows x 64 columns: 16 x 4 MFMA
-// tiles in the 256 accumulation registers, plus 4 x 4 tiles in ordinary registers for chunks of
-// 257..320 rows.
-//
-// With one wave per SIMD nothing overlaps unless the instruction stream says so, so the K loop is
-// written as a fixed sequence of instructions (MFMAs, loads, waits) around which the compiler only
-// allocates registers:
-//   * the loads of slice ks+D (D = 3, or 2 for 320-row chunks) are issued one by one between the
-//     MFMAs of slice ks (a burst of loads blocks the wave at the issue stage while the matrix pipe
-//     drains);
-//   * expert weights (B operand) go global -> registers, never through LDS.  In the reference
-//     layout a weight column's K runs over partitions p (4 K values per x4 element), and lane
+// so every weight byte that enters the CU is used by all rows of the chunk, and both operands enter the CU exactly once per
+// workgroup.  What bounds a chunk of so few rows is the stream of its weights, so they go straight into registers, three
+// slices ahead (96 KB in flight per CU; 32 tokens over 256 MXFP8 experts of H = 7168, I = 2048: gate/up at 7.0 TB/s), and
+// the K loop is a fixed sequence of instructions (MFMAs, loads, waits) around which the compiler only allocates registers:
+//   * the loads of slice ks+3 are issued one by one between the MFMAs of slice ks;
+//   * in the reference layout a weight column's K runs over partitions p (4 K values per x4 element), and lane
 //     group g of v_mfma_scale_f32_16x16x128_f8f6f4 needs K bytes [16g,16g+16) and [64+16g,
 //     64+16g+16) of the 128-byte K slice, i.e. partitions 4g..4g+3 and 16+4g..16+4g+3 of the 32
 //     partitions of the slice (4-bit weights: K 32g..32g+31 = partitions 8g..8g+7): eight loads
 //     per lane, each fetching 4 adjacent columns = 4 MFMA column tiles at once.  The loads land in
-//     one of D "raw" register sets; a set is transposed into MFMA operand order at the top of the
+//     one of three "raw" register sets; a set is transposed into MFMA operand order at the top of the
 //     slice that uses it;
 //   * activations (A operand, rows gathered through token_position_to_id) go global -> LDS
-//     directly into a ring of D+1 stages of 256 (320) rows x 128 K-bytes, read by all four waves;
-//     the fragments of the next two row tiles are read while the current two multiply;
+//     directly into a ring of four stages, read by all four waves;
 //   * E8M0 scales ride along: A scales sit in LDS as [g][row%16][row/16] so that one 16-byte read
-//     gives a lane the scales of 16 row tiles (selected with op_sel); B scales are 4 bytes per lane
+//     gives a lane the scales of its row tiles (selected with op_sel); B scales are 4 bytes per lane
 //     per K slice straight from global.
 // The gate/up epilogue computes act(gate)*up in registers (a pair of lanes holds gate and up of the
 // same elements and exchanges them) and passes the products through LDS so that the MX
@@ -44,24 +33,20 @@
 namespace moe {
 
 constexpr int MX_EP = 128 + 8;  // epilogue exchange: floats per row ([q][32 partitions] + pad)
-// Per variant (NMT row tiles): how many slices the loads run ahead, the ring of activation stages, and
-// the bytes of one stage.  Chunks of up to 256 rows: 3 slices ahead, 4 stages of 256 rows.  Chunks of
-// 257..320 rows (an expert's usual load plus a small excess, which would otherwise cost a second pass
-// over the expert's weights): 2 slices ahead, 3 stages of 320 rows -- the 64 extra accumulators
-// live in ordinary registers, which leaves room for two raw weight sets, not three.
+// Tiles of up to four row tiles: how many slices the loads run ahead, the ring of activation stages, and a stage's bytes.
 template <int NMT>
 struct MxCfg {
-  static constexpr int D = NMT > 16 ? 2 : 3;          // slices between a load and its use
-  static constexpr int RING = D + 1;                  // activation stages
-  static constexpr int ROWS = NMT > 16 ? 320 : 256;   // rows of a stage
-  static constexpr int SA = ROWS * MXROW;             // bytes of a stage's rows
-  static constexpr int SSP = NMT > 16 ? 32 : 16;      // scale bytes per (K block, row within tile): one per row tile
-  static constexpr int SS = 64 * SSP;                 // bytes of a stage's scales, [g][c][mt]
+  static_assert(NMT % 2 == 0 && NMT <= 4, "a thread looks after one row of scales, a group of two row tiles is multiplied at a time");
+  static constexpr int D = 3;              // slices between a load and its use
+  static constexpr int RING = D + 1;       // activation stages
+  static constexpr int ROWS = 256;         // rows of a stage
+  static constexpr int SA = ROWS * MXROW;  // bytes of a stage's rows
+  static constexpr int SSP = 16;           // scale bytes per (K block, row within tile): one per row tile
+  static constexpr int SS = 64 * SSP;      // bytes of a stage's scales, [g][c][mt]
   static constexpr int LDS = RING * (SA + SS);
 };
-constexpr int MX_LDS_LOOP = MxCfg<16>::LDS > MxCfg<20>::LDS ? MxCfg<16>::LDS : MxCfg<20>::LDS;
 constexpr int MX_LDS_EPI = 64 * MX_EP * 4;
-constexpr int MX_LDS = MX_LDS_EPI > MX_LDS_LOOP ? MX_LDS_EPI : MX_LDS_LOOP;
+constexpr int MX_LDS = MX_LDS_EPI > MxCfg<4>::LDS ? MX_LDS_EPI : MxCfg<4>::LDS;
 
 
 template <class Operand>
@@ -128,43 +113,6 @@ __device__ __forceinline__ void mfma_asm(const v8i& af, const BOp& bf, int sa, i
 }
 #undef MX_MFMA_CASE
 #undef MX_MFMA_ASM
-// The same with the accumulator tile in ordinary registers (row tiles 16..19 of a 320-row chunk).
-#define MX_MFMA_ASM(FMT_, SEL_, SELHI_)                                                                        \
-  asm volatile("v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:" SEL_ " op_sel_hi:" SELHI_ FMT_ \
-               : "+v"(c) : "v"(af), "v"(bf), "v"(sa), "v"(sb))
-#define MX_MFMA_CASE(OA_, OB_, SEL_, SELHI_)               \
-  if constexpr (OA == OA_ && OB == OB_) {                  \
-    if constexpr (WFMT == 0) MX_MFMA_ASM("", SEL_, SELHI_); \
-    else if constexpr (WFMT == 1) MX_MFMA_ASM(" blgp:1", SEL_, SELHI_); \
-    else MX_MFMA_ASM(" blgp:4", SEL_, SELHI_);             \
-  }
-template <int OA, int OB, int WFMT, class BOp>
-__device__ __forceinline__ void mfma_asm_v(v4f& c, const v8i& af, const BOp& bf, int sa, int sb) {
-  if constexpr (WFMT == MX_WFMT_BF16) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0\n\tv_mfma_f32_16x16x32_bf16 %0, %3, %4, %0"
-                 : "+v"(c) : "v"(lo4(af)), "v"(lo4(bf)), "v"(hi4(af)), "v"(hi4(bf)));
-  } else {
-  MX_MFMA_CASE(0, 0, "[0,0,0]", "[0,0,0]");
-  MX_MFMA_CASE(1, 0, "[1,0,0]", "[0,0,0]");
-  MX_MFMA_CASE(2, 0, "[0,0,0]", "[1,0,0]");
-  MX_MFMA_CASE(3, 0, "[1,0,0]", "[1,0,0]");
-  MX_MFMA_CASE(0, 1, "[0,1,0]", "[0,0,0]");
-  MX_MFMA_CASE(1, 1, "[1,1,0]", "[0,0,0]");
-  MX_MFMA_CASE(2, 1, "[0,1,0]", "[1,0,0]");
-  MX_MFMA_CASE(3, 1, "[1,1,0]", "[1,0,0]");
-  MX_MFMA_CASE(0, 2, "[0,0,0]", "[0,1,0]");
-  MX_MFMA_CASE(1, 2, "[1,0,0]", "[0,1,0]");
-  MX_MFMA_CASE(2, 2, "[0,0,0]", "[1,1,0]");
-  MX_MFMA_CASE(3, 2, "[1,0,0]", "[1,1,0]");
-  MX_MFMA_CASE(0, 3, "[0,1,0]", "[0,1,0]");
-  MX_MFMA_CASE(1, 3, "[1,1,0]", "[0,1,0]");
-  MX_MFMA_CASE(2, 3, "[0,1,0]", "[1,1,0]");
-  MX_MFMA_CASE(3, 3, "[1,1,0]", "[1,1,0]");
-  }
-}
-#undef MX_MFMA_CASE
-#undef MX_MFMA_ASM
-
 // NMT = number of 16-row tiles this instantiation multiplies (the chunks it takes have at most NMT*16 rows).
 // Keeping it a compile-time constant keeps the K loop free of branches around the MFMAs.
 // LASTUSE: the chunks are the last ones of their experts, so their weights are streamed past the L2 (which
@@ -195,11 +143,10 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   constexpr bool ROW8 = WFMT == MX_WFMT_ROW8 || BF16;
   constexpr int MFMT = BF16 ? MX_WFMT_BF16 : ROW8 ? MX_WFMT_E4M3 : WFMT;  // element format of the MFMA's B operand
   constexpr int D = Cfg::D, RING = Cfg::RING, SA = Cfg::SA, SS = Cfg::SS, SSP = Cfg::SSP;
-  constexpr bool BIG = NMT > 16;  // row tiles 16.. accumulate in ordinary registers
   uint8_t* sA = smem;
   uint8_t* sS = smem + RING * SA;
   // ring arithmetic: x in [0, 2 RING)
-  auto wrapst = [](int x) { return (RING == 4) ? (x & 3) : ((x >= RING) ? x - RING : x); };
+  auto wrapst = [](int x) { return x & (RING - 1); };
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -226,12 +173,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   // check of the descriptor returns zeros)
   constexpr int NAV = (STAGE == 1) ? NAJ : 1;
   uint32_t a_voff[NAV];
-  // A scales: thread covers row tid (and, in a chunk of more than 256 rows, row 256 + tid % 64: every
-  // wave issues that load so that all waves count the same loads, the first wave's is used)
-  uint32_t as_voff = 0, as_voff2 = 0;
-  // where the scales of row 256 + tid go: the other waves' copies land in a row tile that does not
-  // exist (no branch inside the K loop: values that cross one stop being known as uniform)
-  const int row_hi = (tid < 64) ? 256 + tid : 31 * 16 + (tid & 15);
+  uint32_t as_voff = 0;  // A scales: thread covers row tid
 
   // ---- K schedule -----------------------------------------------------------------------------------
   // stage 1: ks -> (H tile ks>>2, partition group ks&3), all slices full.
@@ -296,11 +238,11 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   constexpr bool SCALED = !ROW8;
   constexpr int UNIT_SCALES = 0x7f7f7f7f;
   constexpr int NBL = 8;
-  constexpr int NSC = SCALED ? (BIG ? 2 : 1) : 0;
+  constexpr int NSC = SCALED ? 1 : 0;
   constexpr int NLB = NBL + (SCALED ? 1 : 0);  // weight loads of a slice
   constexpr int N1 = NAJ + NLB;             // loads of a slice that carries no activation scales
   constexpr int N0 = N1 + NSC;              // loads of one that does
-  typedef typename std::conditional<D == 3, v3i, v2i>::type ScaleRegs;
+  typedef v3i ScaleRegs;
   typedef typename std::conditional<FP4, v2i, v4i>::type RawLoad;
   typedef typename std::conditional<FP4, v4i, v8i>::type BOperand;
   struct BRaw {
@@ -343,7 +285,6 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       return (uint32_t)(t.slot0 + ((row < t.nrows) ? row : (t.nrows - 1))) * (uint32_t)a.a_scale_stride;
     };
     as_voff = scale_row_off(tid);
-    as_voff2 = BIG ? scale_row_off(256 + (tid & 63)) : 0u;
     int64_t colu;
     if (STAGE == 1) {
       colu = (int64_t)tw.tile_tI(t) * 512 + (int64_t)q * tw.tile_Pt(t) + tw.tile_p0(t);
@@ -390,7 +331,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     r.s_off = uni((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride);
     return r;
   };
-  auto issue_load = [&](auto idx_, const SliceAddr& sa, BRaw& b, ScaleRegs& sc0, ScaleRegs& sc1, auto with_scales_) {
+  auto issue_load = [&](auto idx_, const SliceAddr& sa, BRaw& b, ScaleRegs& sc0, auto with_scales_) {
     constexpr int idx = decltype(idx_)::value;
     if constexpr (idx < NAJ) {
       // the wave's 64 lanes fill 8 rows x 128 bytes = 1 KB of the ring stage, in lane order
@@ -403,8 +344,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       // dwords sit in different cache lines, so this load costs the memory pipeline as many
       // requests as all the activation rows of a slice together -- hence one in D slices
       if constexpr (decltype(with_scales_)::value) {
-        if constexpr (idx == NAJ) ld_dwords(sc0, as_voff, ras_, sa.as_off);
-        else ld_dwords(sc1, as_voff2, ras_, sa.as_off);
+        ld_dwords(sc0, as_voff, ras_, sa.as_off);
       }
     } else if constexpr (idx < NAJ + NSC + NBL) {
       constexpr int i = idx - NAJ - NSC;
@@ -425,8 +365,6 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     for (int gg = 0; gg < 4; ++gg) sd[(gg * 16 + cc) * SSP + mt] = (uint8_t)((raw >> (8 * gg)) & 0xffu);
   };
 
-  v4f accv[4][4];  // row tiles 16..19
-
   // ---- K loop ---------------------------------------------------------------------------------------
   // Loads run D slices ahead of the MFMAs (what the memory system delivers is the amount in flight
   // divided by its latency, and one wave per SIMD has nobody to take over while it waits): during
@@ -443,7 +381,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const int rd_lo = c * MXROW + ((g ^ (c & 7)) * 16), rd_hi = c * MXROW + (((g + 4) ^ (c & 7)) * 16);
   constexpr int NG = NMT / 2;
   BRaw br[D];
-  ScaleRegs asr = 0, asr2 = 0;  // activation scales as loaded: row tid, row 256 + tid % 64
+  ScaleRegs asr = 0;  // activation scales as loaded: row tid
   static_for<0, D>([&](auto u_) {
     constexpr int u = decltype(u_)::value;
 #pragma unroll
@@ -457,21 +395,14 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     const uint8_t* plo = sA + st * SA + rd_lo;
     const uint8_t* phi = sA + st * SA + rd_hi;
     v4i asc = (v4i){UNIT_SCALES, UNIT_SCALES, UNIT_SCALES, UNIT_SCALES};
-    int asc_hi = UNIT_SCALES;
-    if constexpr (SCALED) {
-      asc = *(const v4i*)(sS + st * SS + (g * 16 + c) * SSP);
-      if constexpr (BIG) asc_hi = *(const int*)(sS + st * SS + (g * 16 + c) * SSP + 16);
-    }
+    if constexpr (SCALED) asc = *(const v4i*)(sS + st * SS + (g * 16 + c) * SSP);
     // first fragments of this slice: in flight while the weights are transposed
     v8i af[2][2];
     af[0][0] = frag_from_lds(plo, phi);
     af[0][1] = frag_from_lds(plo + 16 * MXROW, phi + 16 * MXROW);
     asm volatile("" ::: "memory");
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NLB + (D - 2) * N1) : "memory");
-    if constexpr (SCALED && U == D - 1) {  // activation scales of slices ks+1 .. ks+D
-      asm volatile("" : "+v"(asr));
-      if constexpr (BIG) asm volatile("" : "+v"(asr2));
-    }
+    if constexpr (SCALED && U == D - 1) asm volatile("" : "+v"(asr));  // activation scales of slices ks+1 .. ks+D
     // (the wait names no register: an in/out operand may be copied into place ahead of its
     // statement, i.e. read while its load is still in flight; the registers are tied to this point
     // by statements of their own)
@@ -520,10 +451,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
         constexpr int j = decltype(j_)::value;
         constexpr int mt = 2 * gi + j / 4, nt = j % 4;
         constexpr int m = gi * 8 + j;  // MFMA number within the slice
-        if constexpr (mt < 16)
-          mfma_asm<16 * mt + 4 * nt, mt % 4, nt, MFMT>(af[cur][j / 4], b.f[nt], asc[mt / 4], b.sc);
-        else
-          mfma_asm_v<mt % 4, nt, MFMT>(accv[mt - 16][nt], af[cur][j / 4], b.f[nt], asc_hi, b.sc);
+        mfma_asm<16 * mt + 4 * nt, mt % 4, nt, MFMT>(af[cur][j / 4], b.f[nt], asc[mt / 4], b.sc);
         if constexpr (m == 0) {
           // the scalar arithmetic for the addresses of slice ks+D starts here, behind the first
           // MFMA, instead of ahead of it
@@ -533,33 +461,24 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
         }
         if constexpr (SCALED && U == D - 1 && m >= 3 && m < 3 + D) {
           scales_to_operand_order(wrapst(st + m - 2), (uint32_t)asr[m - 3], tid);
-          if constexpr (BIG) scales_to_operand_order(wrapst(st + m - 2), (uint32_t)asr2[m - 3], row_hi);
         }
         static_for<m * N0 / (8 * NG), (m + 1) * N0 / (8 * NG)>(
-            [&](auto i_) { issue_load(i_, sad, braw, asr, asr2, std::integral_constant<bool, U == 0>{}); });
+            [&](auto i_) { issue_load(i_, sad, braw, asr, std::integral_constant<bool, U == 0>{}); });
       });
     });
-    // (accumulators in ordinary registers are C++ values: should the compiler copy one where paths
-    // join, the MFMA that wrote it has left the pipe)
-    if constexpr (BIG) asm volatile("s_nop 15");
     acc_fence();
     __syncthreads();
   };
 
   // The first D slices of a tile are requested at once (for the first tile before anything else, for every later
   // one ahead of the epilogue of the tile before it).
-  // (numbered 0 .. D * N0 - 1 in issue order, slice after slice, so that a part of them can be asked for at a time)
-  constexpr int NFIRST = D * N0;
-  SliceAddr sa_first;  // of the slice whose loads are being issued
-  auto request_first = [&](auto n0_, auto n1_) {
-    static_for<decltype(n0_)::value, (decltype(n1_)::value < NFIRST ? decltype(n1_)::value : NFIRST)>([&](auto n_) {
-      constexpr int n = decltype(n_)::value;
-      constexpr int u = n / N0, i = n % N0;
-      if constexpr (i == 0) sa_first = slice_addr(u, u);
-      issue_load(std::integral_constant<int, i>{}, sa_first, br[u], asr, asr2, std::integral_constant<bool, u == 0>{});
+  auto request_first_slices = [&]() {
+    static_for<0, D>([&](auto u_) {
+      constexpr int u = decltype(u_)::value;
+      const SliceAddr sa = slice_addr(u, u);
+      static_for<0, N0>([&](auto i_) { issue_load(i_, sa, br[u], asr, std::integral_constant<bool, u == 0>{}); });
     });
   };
-  auto request_first_slices = [&]() { request_first(std::integral_constant<int, 0>{}, std::integral_constant<int, NFIRST>{}); };
 
   // ---- first tile: nothing is in flight yet, so plain loads and waits do ----------------------------------
   MxTile cur = tw.tile_at(L);
@@ -595,21 +514,13 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
 
   for (;;) {
   acc_fence();
-  static_for<0, (BIG ? 16 : NMT) * 16>([&](auto i_) { acc_zero<decltype(i_)::value>(); });
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) accv[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
+  static_for<0, NMT * 16>([&](auto i_) { acc_zero<decltype(i_)::value>(); });
   // (the activation rows of slice 0, and the activation scales of the first D slices, are in)
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(NLB + (D - 1) * N1) : "memory");
   if constexpr (SCALED) {
     asm volatile("" : "+v"(asr));
-    if constexpr (BIG) asm volatile("" : "+v"(asr2));
 #pragma unroll
-    for (int j = 0; j < D; ++j) {
-      scales_to_operand_order(j, (uint32_t)asr[j], tid);
-      if constexpr (BIG) scales_to_operand_order(j, (uint32_t)asr2[j], row_hi);
-    }
+    for (int j = 0; j < D; ++j) scales_to_operand_order(j, (uint32_t)asr[j], tid);
   }
   __syncthreads();
   int st = 0;
@@ -633,7 +544,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     for (int j = 0; j < NBL; ++j) asm volatile("" : : "v"(br[u].d[j]));
     asm volatile("" : : "v"(br[u].sc));
   }
-  asm volatile("" : : "v"(asr), "v"(asr2));
+  asm volatile("" : : "v"(asr));
 
   // ---- the next tile's first loads, and what the tile after it needs, go out ahead of the epilogue ---------
   // The loads of the next tile's first D slices are in flight from here until the wait that follows the epilogue
@@ -649,11 +560,9 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const int nbuf = have_next ? buf ^ 1 : buf;  // (behind the last tile: its own row table, which holds valid ids)
   tile_live = have_next ? -1 : 0;
   aim_loads_at(nxt, nbuf);
-  // (down stage: they go out a few at a time between the row tiles of the epilogue, see there; not for the smallest
-  // tiles, whose launches do little but stream weights: there every load asked for later is time lost, 2 % of the
-  // down launch at decode sizes)
-  constexpr bool SPREAD_FIRST = STAGE == 2 && NMT >= 8;
-  if constexpr (!SPREAD_FIRST) request_first_slices();
+  // (all at once: launches of such tiles do little but stream weights, and every load asked for later is time lost, 2 % of
+  // the down launch at decode sizes when they went out between the row tiles of the epilogue)
+  request_first_slices();
   if (TW::AFF_ROWS) tw.aff_raw(nxt, nbuf, aff_n);
   tw.rs_raw(nxt, nbuf, rs_n);
   tw.bias_raw(nxt, bias_n);
@@ -743,8 +652,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
           float av[4][4];  // [column tile][row]
           static_for<0, 16>([&](auto i_) {
             constexpr int i = decltype(i_)::value;
-            if constexpr (mt < 16) av[i / 4][i % 4] = acc_get<16 * mt + i>();
-            else av[i / 4][i % 4] = accv[mt - 16][i / 4][i % 4];
+            av[i / 4][i % 4] = acc_get<16 * mt + i>();
           });
           float y[2][4];
           float ckg[4][2], cku[4][2];  // bf16 kind: gate / up ahead of the activation, for the checkpoint
@@ -916,8 +824,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       float av[4][4];  // [column tile][row]
       static_for<0, 16>([&](auto i_) {
         constexpr int i = decltype(i_)::value;
-        if constexpr (mt < 16) av[i / 4][i % 4] = acc_get<16 * mt + i>();
-        else av[i / 4][i % 4] = accv[mt - 16][i / 4][i % 4];
+        av[i / 4][i % 4] = acc_get<16 * mt + i>();
       });
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -944,12 +851,6 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
         }
         st_b64(o, d_voff, rd, (mt * 16 + r) * rowb);
       }
-      // The next tile's first slices, a share behind every row tile: asked for all at once ahead of the epilogue
-      // they fill the CU's load queue, the wave stands at the first instruction that does not fit until the memory
-      // system has worked the queue down, and this arithmetic and these stores, which could run meanwhile, wait
-      // behind it.
-      constexpr int PER = (NFIRST + NMT - 1) / NMT;
-      if constexpr (SPREAD_FIRST) request_first(std::integral_constant<int, mt * PER>{}, std::integral_constant<int, (mt + 1) * PER>{});
     });
   }
   tile_live = -1;
@@ -1004,10 +905,8 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int interleave = __builtin_amdgcn_readfirstlane(a.q_off[8 * (CHUNK_CLASSES + 1)]);
   int L = w;
   // classes in queue order (CHUNK_CLASS_TILES / CHUNK_CLASS_LAST in combine.hpp)
-  // (tiles of up to 64 rows stream their weights through registers, three slices ahead)
-#define MX_TILES(TILES_) ((TILES_) >= 8)
 #define MX_RUN_TILES(TILES_, LAST_)                                                                               \
-  if constexpr (MX_TILES(TILES_))                                                                                \
+  if constexpr ((TILES_) >= 8)                                                                                   \
     L = mx_gemm_tiles_wide<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \
                                                            (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave); \
   else                                                                                                           \
@@ -1063,7 +962,6 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 #undef MX_RUN_RANGE
 #undef MX_RUN_TILES
-#undef MX_TILES
 #undef MX_RUN_CLASS
   if (a.clk && blockIdx.x == 0 && threadIdx.x == 0) {
     a.clk[0] = clock64() - clk0;

@@ -54,8 +54,8 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
           if (v > 0) last_end = j * B + v;
         }
         // (pad_row: activation checkpoints hold every row of every executed block, padding rows included.  Those behind
-        // the last token are all alike, so the chunks take one of them along, which ckpt_pad_gate_up_kernel /
-        // ckpt_pad_down_kernel then copy to the others)
+        // the last token are all alike, so the chunks take one of them along, which ckpt_pad_gate_up /
+        // ckpt_pad_down (csrc/combine.hip) then copy to the others)
         if (pad_row) last_end = last_end < 0 ? b * B + 1 : last_end < j * B ? last_end + 1 : last_end;
         // chunks of CHUNK_ROWS rows; the last one absorbs a remainder of up to CHUNK_ROWS_MAX - CHUNK_ROWS
         // rows, which saves the pass over the expert's weights that a small chunk of its own would cost
