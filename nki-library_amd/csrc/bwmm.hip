@@ -870,6 +870,21 @@ int launch_gemm_stage(int kind, int stage, const GemmArgs& g, unsigned gx, unsig
   return stage == 1 ? launch_gemm<MOE_KIND_MXFP8, 1>(g, gx, gy, s) : launch_gemm<MOE_KIND_MXFP8, 2>(g, gx, gy, s);
 }
 
+// One workgroup per record: H codes to their aligned row, the fp32 behind them to the scales.  (Records are 4-byte aligned.)
+__global__ __launch_bounds__(256) void split_rows_kernel(const uint8_t* __restrict__ rec, uint8_t* __restrict__ codes,
+                                                         float* __restrict__ scales, int64_t H) {
+  const uint32_t* r = (const uint32_t*)(rec + (int64_t)blockIdx.x * (H + 4));
+  uint32_t* o = (uint32_t*)(codes + (int64_t)blockIdx.x * H);
+  const int words = (int)(H / 4);
+  for (int i = threadIdx.x; i < words; i += 256) o[i] = r[i];
+  if (threadIdx.x == 0) scales[blockIdx.x] = __uint_as_float(r[words]);
+}
+int launch_split_rows(const uint8_t* rec, uint8_t* codes, float* scales, int64_t rows, int64_t H, hipStream_t s) {
+  hipLaunchKernelGGL(split_rows_kernel, dim3((unsigned)rows), dim3(256), 0, s, rec, codes, scales, H);
+  MOE_CHECK_LAUNCH();
+  return MOE_OK;
+}
+
 int launch_row_requant(const float* Y, uint8_t* Yq, float* ys, const Bookkeeping& k, int64_t N, int64_t B, int64_t I,
                        int64_t y_stride, int64_t Iw, hipStream_t s) {
   hipLaunchKernelGGL(row_requant_kernel, dim3((unsigned)(N * B)), dim3(256), 0, s, Y, Yq, ys, k.n_active, k.valid_rows,

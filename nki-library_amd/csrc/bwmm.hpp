@@ -76,8 +76,8 @@ struct MxArgs {
   const float* w_cscale;   // [cscale_experts][2*I] (gate/up: gate then up) or [cscale_experts][H] (down)
   int32_t cscale_experts;  // E or 1
   int32_t w_scale_shared;  // 1: W_scale holds one expert's worth of block scales that serves every expert
-  const float* a_rscale;   // stage 2: row scale of the re-quantised intermediate, [N*B]; stage 1: null, a row's scale
-                           // is the fp32 behind its H codes (the RMSNorm-Quant ROW record)
+  const float* a_rscale;   // stage 2: row scale of the re-quantised intermediate, [N*B]; stage 1: the token rows' scales,
+                           // or null: a row's scale is the fp32 behind its H codes (the RMSNorm-Quant ROW record)
   int64_t a_scale_bytes;   // size of the A_scale table when it is not a_rows * a_scale_stride (stride 0: one row
                            // of constants for every row)
   float* Y32;              // stage 1 output of this format: fp32 [N*B, y32_stride], columns in natural order
@@ -149,6 +149,8 @@ int launch_relayout_x4(const uint8_t* gate_up, const uint8_t* down, uint8_t* dst
 // 2H / 2I bytes.
 int launch_relayout_x4_bf16(const void* gate_up, const void* down, int w8, uint8_t* dst, int which, int64_t E, int64_t H,
                             int64_t I, int64_t I_pad, hipStream_t s);
+// ROW records [rows, H + 4] -> codes [rows, H] and scales [rows] (see split_rows in capi.hip).
+int launch_split_rows(const uint8_t* rec, uint8_t* codes, float* scales, int64_t rows, int64_t H, hipStream_t s);
 int launch_fill_bytes(void* p, size_t bytes, uint8_t value, hipStream_t s);
 int launch_row_requant(const float* Y, uint8_t* Yq, float* ys, const Bookkeeping& k, int64_t N, int64_t B, int64_t I,
                        int64_t y_stride, int64_t Iw, hipStream_t s);

@@ -288,14 +288,15 @@ struct MxTileWalk {
     if constexpr (ROW8) {
       // (bf16: nothing to fetch; the load stays, from an address that is valid, so that every format issues the
       // same loads)
-      const v4i rd = make_rsrc((STAGE == 1 || BF16) ? (const void*)a.A : (const void*)a.a_rscale, 0xffffffffu);
+      const v4i rd = make_rsrc((BF16 || (STAGE == 1 && !a.a_rscale)) ? (const void*)a.A : (const void*)a.a_rscale, 0xffffffffu);
 #pragma unroll
       for (int j = 0; j < (ROWS2 ? 2 : 1); ++j) {
         const int r = tid + 256 * j;
         uint32_t off;
         if (STAGE == 1) {
           const int id = s_tok[buf][(r < NMT * 16) ? r : 0];
-          off = (uint32_t)((id >= 0) ? id : 0) * (uint32_t)a.a_stride + (BF16 ? 0u : (uint32_t)a.H);
+          off = (uint32_t)((id >= 0) ? id : 0) * (a.a_rscale ? 4u : (uint32_t)a.a_stride) +
+                ((BF16 || a.a_rscale) ? 0u : (uint32_t)a.H);
         } else {
           off = (uint32_t)(t.slot0 + ((r < t.nrows) ? r : t.nrows - 1)) << 2;
         }
