@@ -37,7 +37,7 @@ PEAK_HBM_GBS = 8000.0
 # that holds the runs it comes from, and only while the kernel sources still hash to what that summary was taken
 # from: a kernel changed since then has no measured traffic until it is profiled again.
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "mx_gemm_c4_moe_layer.md")
-TRAFFIC_SOURCES = ("nki-library_amd/csrc/bwmm_mx.hip", "nki-library_amd/csrc/bwmm.hpp")
+TRAFFIC_SOURCES = tuple(f"nki-library_amd/csrc/{f}" for f in ("bwmm_mx.hip", "mx_wide.hpp", "mx_tile.hpp", "bwmm.hpp"))
 
 
 def profiled_traffic(workload, routing):

@@ -225,7 +225,7 @@ constexpr int64_t PREP_SMALL_SLOTS = 40960, PREP_SMALL_TOKENS = 4096, PREP_SMALL
 // run at such sizes.  It is a chain of steps, so what counts is the latency of each: the counts, the list positions and
 // the valid rows live in LDS, and the two passes over the slots deal units of 64 slots to all sixteen waves, four in
 // flight per wave (a wave per block with the counts behind global atomics left three quarters of the waves idle and took 27
-// us at 15 blocks of 512 slots over 1024 tokens; now 17).
+// us at 15 blocks of 512 slots over 1024 tokens; now 15).
 __global__ __launch_bounds__(1024) void prep_small_kernel(
     const int32_t* __restrict__ tp2id, const int32_t* __restrict__ b2e, const int32_t* __restrict__ conditions,
     int64_t n_conditions, int64_t N, int64_t B, int64_t E, int64_t n_real, int32_t* __restrict__ n_active,
@@ -406,7 +406,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t* __restrict
 // The checkpoints' padding rows and the combine of one layer in one launch: three jobs that share no data and are each too
 // short to fill the memory system from start to end.  Workgroups [0, n_gu) take the gate_up checkpoint (y_gu per block), the
 // next n_dn the down checkpoint, the rest the output rows.  T = 1024, top-4 of 8 experts of H = 3072, I = 2048, B = 512:
-// 16.5 + 9 + 10 us in three launches.
+// 16.5 + 9 + 10 us in three launches, 21 in this one.
 struct CkptTail {
   uint16_t *ck_gu, *ck_dn;
   const int32_t *b2e, *n_active, *valid_rows;

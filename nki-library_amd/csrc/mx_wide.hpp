@@ -20,12 +20,12 @@
 //     landed; the loads of the activations two slices ahead go out, and under the last 16 MFMAs the fragments of the next
 //     slice are read: a weight fragment is read into the registers of the one whose last MFMA has just been issued.
 //     No slice begins with a wait for LDS.
-// What bounds it: the matrix pipes, at the clock that the part holds.  A bf16 slice of 16 row tiles takes 2690 cycles, its
-// MFMAs alone 2480 (128 of 16 x 16 x 32, one in 19.35 cycles); an MXFP8 slice with the weights from HBM 3100 of 2048 (half
-// of HBM's rate).  Against the register-weight loop, which took some 4000: layer of 4096 tokens, top-2 of 8 bf16 experts of
-// H = 2048, I = 4096 414 -> 378 us (gate/up 258 -> 226); fp8-row, 4096 tokens over 8 experts of H = 4096, I = 14336
-// 1418 -> 1361 us; MXFP8, 8192 tokens over 256 experts of H = 7168, I = 2048 3155 -> 3045 us (back to back, where the part
-// answers shorter waits with a lower clock; the gate/up launch by itself 1.89 -> 1.63 ms).
+// What bounds it: the matrix pipes, at the clock that the part's power leaves them.  A bf16 slice of 16 row tiles takes 2690
+// cycles, its MFMAs alone 2480 (128 of 16 x 16 x 32, one in 19.35 cycles); an fp8-row slice 2540 and an MXFP8 slice with the
+// weights from HBM 3050 cycles of 2048.  Layers back to back, against the loop before (weights through registers, one wave
+// across all rows, some 4000 cycles per slice): 8192 tokens over 256 MXFP8 experts of H = 7168, I = 2048 3155 -> 3010 us;
+// 4096 tokens, top-2 of 8 bf16 experts of H = 2048, I = 4096 440 -> 409; 8192 tokens, top-8 of 128 MXFP8 experts of H = 2048,
+// I = 768 539 -> 502; 1999 tokens, top-4 of 32 MXFP4 experts of H = 3072, I = 1536 203 -> 196.
 #pragma once
 
 #include "mx_tile.hpp"
