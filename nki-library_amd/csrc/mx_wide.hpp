@@ -680,10 +680,10 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const uint32_t ys_voff = (g_e & 1) ? 0xffffffffu : (uint32_t)(row0 * ys_rowb + tI * 16 + (pl >> 3));
       // dense kinds: natural column of the lane's first value of quarter 2 wn + j
       auto nat_col = [&](int j) { return tI * 512 + (2 * wn + j) * Pt + p0 + (BF16 ? 8 : 4) * g_e; };
-      // activation checkpoint [N, 2, I, B] (bwmm_shard_on_I.py:160-176): offsets from the chunk's first block on
-      const uint32_t ck_B = BF16 ? (uint32_t)a.ckpt_B : 1u, ck_n0 = (uint32_t)cur.slot0 / ck_B;
-      const uint32_t ck_gu = BF16 ? (uint32_t)a.ckpt_I * ck_B * 2u : 0u;  // bytes from gate to up
-      uint8_t* ck_base = (uint8_t*)a.ckpt + (int64_t)ck_n0 * 2 * ck_gu;
+      // activation checkpoint [N, 2, I, B] (bwmm_shard_on_I.py:160-176): a block's gate or up half is less than 4 GiB (the
+      // call's intermediate rows are), so 32 bits hold an offset inside a half, and which half is a matter of 64 bits
+      const uint32_t ck_B = BF16 ? (uint32_t)a.ckpt_B : 1u;
+      const uint32_t ck_half = BF16 ? (uint32_t)a.ckpt_I * ck_B * 2u : 0u;  // bytes
       auto passes = [&](auto act_, auto plain_) {
         constexpr int ACT = decltype(act_)::value;
         constexpr bool PLAIN = decltype(plain_)::value;
@@ -784,22 +784,24 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
                   const uint32_t slot = (uint32_t)(cur.slot0 + row), n = slot / ck_B, rr = slot - n * ck_B;
                   const int ccol0 = nat_col(j) + (pair ? 4 * odd : 0);
                   const int live = row < cur.nrows ? (int)a.ckpt_I - ccol0 : 0;  // columns from ccol0 on that exist
-                  const uint32_t off0 = (n - ck_n0) * 2u * ck_gu + ((uint32_t)ccol0 * ck_B + rr) * 2u;
+                  uint8_t* const ck_gate = (uint8_t*)a.ckpt + (uint64_t)(2u * n) * ck_half;
+                  const uint32_t off0 = ((uint32_t)ccol0 * ck_B + rr) * 2u;
                   static_for<0, 2>([&](auto gu_) {
                     constexpr int gu = decltype(gu_)::value;
                     const float (&v)[2][4] = gu ? uu : gg;
+                    uint8_t* const ck = gu ? ck_gate + ck_half : ck_gate;
                     if (pair) {
 #pragma unroll
                       for (int k = 0; k < 4; ++k) {
                         const float own = odd ? v[1][k] : v[0][k], give = odd ? v[0][k] : v[1][k];
                         const float got = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true));
                         const uint32_t word = odd ? pack2_bf16(got, own) : pack2_bf16(own, got);
-                        if (k < live) *(uint32_t*)(ck_base + (off0 + gu * ck_gu + k * ck_B * 2u)) = word;
+                        if (k < live) *(uint32_t*)(ck + (off0 + k * ck_B * 2u)) = word;
                       }
                     } else {
 #pragma unroll
                       for (int k = 0; k < 8; ++k)
-                        if (k < live) *(uint16_t*)(ck_base + (off0 + gu * ck_gu + k * ck_B * 2u)) = (uint16_t)pack2_bf16(v[k >> 2][k & 3], 0.f);
+                        if (k < live) *(uint16_t*)(ck + (off0 + k * ck_B * 2u)) = (uint16_t)pack2_bf16(v[k >> 2][k & 3], 0.f);
                     }
                   });
                 }

@@ -98,3 +98,48 @@ def test_checkpoints_follow_the_tables():
         graph.replay()
         torch.cuda.synchronize()
         assert same(outs, n), n
+
+
+@pytest.mark.parametrize("N,B,first", [
+    (1, 131200, 0),     # a block of the gate_up checkpoint of more than 4 GiB, two rows to a store
+    (1, 131201, 0),     # the same, row by row
+    (2, 65600, 65500),  # blocks of 2 GiB, a chunk that goes on into the second one
+])
+def test_gate_up_checkpoint_past_4_gib(N, B, first):
+    """One expert, 200 tokens from slot `first` on, every other slot padding: each token's column equals that of the same
+    tokens in a block of 256 rows (which the tests above compare with the oracle), each other slot's the padding row's."""
+    import torch
+    from nkilib.core.moe.moe_cte import SkipMode
+    from nkilib.core.moe.moe_cte.bwmm_shard_on_block import run_dense_variant
+
+    dev = torch.device("cuda:0")
+    T, H, I = 200, 256, 8192
+    g = torch.Generator(device=dev)
+    g.manual_seed(43)
+
+    def bf16(*shape, std=0.1):
+        return (torch.randn(shape, generator=g, device=dev) * std).to(torch.bfloat16)
+
+    x = bf16(T + 1, H, std=1.0)
+    x[T] = 0
+    aff = torch.ones((T + 1, 1), dtype=torch.bfloat16, device=dev)
+    gu, dw, gu_b, d_b = bf16(1, H, 2, I), bf16(1, I, H), bf16(1, 2, I, std=0.5), bf16(1, H)
+
+    def layer(n, b, at):
+        tp = torch.full((n * b,), T, dtype=torch.int32, device=dev)
+        tp[at:at + T] = torch.arange(T, dtype=torch.int32, device=dev)
+        return run_dense_variant(x, aff, gu, dw, b, tp, torch.zeros(n, dtype=torch.int32, device=dev), "TH",
+                                 gate_and_up_proj_bias=gu_b, down_proj_bias=d_b, skip_dma=SkipMode(False, False),
+                                 checkpoint_gate_up=True)
+
+    out0, want = layer(1, 256, 0)
+    out, ck = layer(N, B, first)
+    assert torch.equal(out.view(torch.int16), out0.view(torch.int16))
+    want = want[0].view(torch.int16)                                             # [2, I, 256]
+    for n in range(N):
+        lo, hi = max(first - n * B, 0), min(first + T - n * B, B)                # the block's rows with tokens
+        for gu_ in range(2):
+            rows, w = ck[n, gu_].view(torch.int16), want[gu_]
+            t0 = n * B + lo - first
+            assert torch.equal(rows[:, lo:hi], w[:, t0:t0 + hi - lo]), (n, gu_, "tokens")
+            assert bool((rows[:, :lo] == w[:, T:T + 1]).all()) and bool((rows[:, hi:] == w[:, T:T + 1]).all()), (n, gu_, "padding")
