@@ -515,17 +515,27 @@ static int64_t at_most(int64_t v, int64_t lim) { return v < lim ? v : lim; }
 static int64_t combine_split(const moe_bwmm_args* a) {
   return a->T1 <= 256 ? at_most((a->H + 256 * 8 - 1) / (256 * 8), 8) : 1;
 }
+// A launch holds fewer than 2^32 threads along x (hipLaunchKernel refuses more).
+constexpr int64_t MAX_WORKGROUPS = (((int64_t)1 << 32) - 1) / 256;
+// A workgroup per block and 64 columns (16 rows), or, beyond a million of them, as many per block as stay below that: every
+// further one would only search the blocks' table again.
+CkptGrid ckpt_grid(int64_t N, int64_t B, int64_t cols, bool gate_up, bool down) {
+  const int64_t per_block = N < ((int64_t)1 << 20) ? ((int64_t)1 << 20) / N : 1;
+  CkptGrid g;
+  g.y_gu = at_most((cols + CKPT_COLS - 1) / CKPT_COLS, per_block);
+  g.y_dn = at_most((B + CKPT_ROWS - 1) / CKPT_ROWS, per_block);
+  g.n_gu = gate_up ? N * g.y_gu : 0;
+  g.n_dn = down ? N * g.y_dn : 0;
+  return g;
+}
 static CkptTail ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, bool gate_up, bool down) {
   CkptTail t;
   t.ck_gu = (uint16_t*)a->gate_up_activations_T;
   t.ck_dn = (uint16_t*)a->down_activations;
   t.b2e = a->block_to_expert; t.n_active = k.n_active; t.valid_rows = k.valid_rows;
   t.B = a->B; t.E = a->E; t.cols = 2 * a->I; t.H = a->H;
-  // (a grid below 2^31 workgroups: N * B is, and a workgroup per block and 64 columns or 16 rows at most)
-  t.y_gu = at_most((t.cols + CKPT_COLS - 1) / CKPT_COLS, at_most(65535, ((int64_t)1 << 29) / a->N + 1));
-  t.y_dn = at_most((a->B + CKPT_ROWS - 1) / CKPT_ROWS, at_most(65535, ((int64_t)1 << 29) / a->N + 1));
-  t.n_gu = gate_up ? a->N * t.y_gu : 0;
-  t.n_dn = down ? a->N * t.y_dn : 0;
+  const CkptGrid g = ckpt_grid(a->N, a->B, t.cols, gate_up, down);
+  t.n_gu = g.n_gu; t.y_gu = g.y_gu; t.n_dn = g.n_dn; t.y_dn = g.y_dn;
   t.y_c = combine_split(a);
   return t;
 }
@@ -540,7 +550,13 @@ int launch_ckpt_pad(int stage, const Bookkeeping& k, const moe_bwmm_args* a, hip
 int launch_ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s) {
   const CkptTail t = ckpt_tail(k, a, a->gate_up_activations_T != nullptr, a->down_activations != nullptr);
   const int64_t grid = t.n_gu + t.n_dn + a->T1 * t.y_c;
-  if (grid >= (int64_t)1 << 31) return MOE_E_BAD_SHAPE;
+  if (grid > MAX_WORKGROUPS) {  // (millions of blocks or tokens: each of the three fits a launch of its own)
+    for (int stage = 1; stage <= 2; ++stage) {
+      const int rc = (stage == 1 ? t.n_gu : t.n_dn) > 0 ? launch_ckpt_pad(stage, k, a, s) : MOE_OK;
+      if (rc != MOE_OK) return rc;
+    }
+    return launch_combine(k, a, D, n_real, s);
+  }
   hipLaunchKernelGGL(ckpt_tail_kernel, dim3((unsigned)grid), dim3(256), 0, s, t, (const uint16_t*)D, k.off, k.list,
                      (uint16_t*)a->output, (uint16_t*)a->output_shard1, a->out_row_stride, n_real);
   MOE_CHECK_LAUNCH();

@@ -66,6 +66,11 @@ int launch_plan_chunks(const Bookkeeping& k, const int32_t* block_to_expert, int
                        hipStream_t s);
 // The padding rows and the blocks that do not run of the gate/up (stage 1) or down (2) checkpoint, after the large-tile
 // GEMM that wrote the other rows.
+// ckpt_grid: their workgroups, n of each of the two = y for every one of the N blocks (cols: 2 I).
+struct CkptGrid {
+  int64_t n_gu, y_gu, n_dn, y_dn;
+};
+CkptGrid ckpt_grid(int64_t N, int64_t B, int64_t cols, bool gate_up, bool down);
 int launch_ckpt_pad(int stage, const Bookkeeping& k, const moe_bwmm_args* a, hipStream_t s);
 // Both and the combine in one launch (a layer issued in one call).
 int launch_ckpt_tail(const Bookkeeping& k, const moe_bwmm_args* a, const void* D, int64_t n_real, hipStream_t s);

@@ -143,3 +143,37 @@ def test_gate_up_checkpoint_past_4_gib(N, B, first):
             t0 = n * B + lo - first
             assert torch.equal(rows[:, lo:hi], w[:, t0:t0 + hi - lo]), (n, gu_, "tokens")
             assert bool((rows[:, :lo] == w[:, T:T + 1]).all()) and bool((rows[:, hi:] == w[:, T:T + 1]).all()), (n, gu_, "padding")
+
+
+@pytest.mark.parametrize("N,B,I", [
+    (1 << 18, 2, 2048),  # 2^24 pieces of 64 columns
+    (1 << 23, 1, 8),     # so many blocks that the copies of the two checkpoints need a launch each
+])
+def test_checkpoints_of_very_many_blocks(N, B, I):
+    """The first blocks hold 200 tokens, the others do not run: the same values as in one block of 256 rows, and zeros."""
+    import torch
+    from nkilib.core.moe.moe_cte import SkipMode
+    from nkilib.core.moe.moe_cte.bwmm_shard_on_block import run_dense_variant
+
+    dev = torch.device("cuda:0")
+    T, H = 200, 256
+    g = torch.Generator(device=dev)
+    g.manual_seed(44)
+    x, gu, dw = [(torch.randn(s, generator=g, device=dev) * 0.1).to(torch.bfloat16) for s in ((T + 1, H), (1, H, 2, I), (1, I, H))]
+    x[T] = 0
+    aff = torch.ones((T + 1, 1), dtype=torch.bfloat16, device=dev)
+
+    def layer(n, b, active):
+        tp = torch.full((n * b,), T, dtype=torch.int32, device=dev)
+        tp[:T] = torch.arange(T, dtype=torch.int32, device=dev)
+        cond = (torch.arange(n + 1, device=dev) < active).to(torch.int32)
+        return run_dense_variant(x, aff, gu, dw, b, tp, torch.zeros(n, dtype=torch.int32, device=dev), "TH", conditions=cond,
+                                 skip_dma=SkipMode(False, False), checkpoint_gate_up=True, checkpoint_down=True)
+
+    out0, gu0, d0 = layer(1, 256, 1)
+    out, gu1, d1 = layer(N, B, T // B)
+    na = T // B
+    assert torch.equal(out.view(torch.int16), out0.view(torch.int16))
+    assert torch.equal(gu1[:na].permute(1, 2, 0, 3).reshape(2, I, T).view(torch.int16), gu0[0, :, :, :T].contiguous().view(torch.int16))
+    assert torch.equal(d1[:na].reshape(T, H).view(torch.int16), d0[0, :T].view(torch.int16))
+    assert not bool(gu1[na:].any()) and not bool(d1[na:].any())

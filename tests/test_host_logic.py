@@ -190,3 +190,25 @@ def _rows_fit(stage, fmt, H, I, E, N, B, rows):
     tiles = (I + 127) // 128 if stage == 1 else H // 256
     c = RowsCall(rows, H, E, N, B, tiles, N * ((B + 255) // 256))
     return bool(f(stage, ("e4m3", "e5m2", "e2m1", "row8", "bf16").index(fmt), ctypes.byref(c)))
+
+
+@pytest.mark.parametrize("N,B,I,per_block", [
+    (15, 512, 2048, (64, 32)), (2000, 128, 14336, (448, 8)),  # a workgroup per 64 columns, per 16 rows
+    (1 << 18, 2, 2048, (4, 1)), (37500, 4, 14336, (27, 1)),   # past a million of them
+    ((1 << 24) - 1, 1, 8, (1, 1)),
+])
+def test_checkpoint_padding_grids_fit_a_launch(N, B, I, per_block):
+    """ckpt_grid (csrc/combine.hip): each of the two launches stays below 2^32 threads of 256 to a workgroup."""
+    import ctypes
+
+    from nkilib import _native as nv
+
+    class CkptGrid(ctypes.Structure):
+        _fields_ = [(n, ctypes.c_int64) for n in ("n_gu", "y_gu", "n_dn", "y_dn")]
+
+    f = nv.lib()._ZN3moe9ckpt_gridElllbb
+    f.restype, f.argtypes = CkptGrid, [ctypes.c_int64] * 3 + [ctypes.c_bool] * 2
+    g = f(N, B, 2 * I, True, True)
+    assert (g.y_gu, g.y_dn) == per_block and (g.n_gu, g.n_dn) == (N * g.y_gu, N * g.y_dn)
+    assert max(g.n_gu, g.n_dn) * 256 < 1 << 32
+    assert (f(N, B, 2 * I, False, True).n_gu, f(N, B, 2 * I, True, False).n_dn) == (0, 0)
