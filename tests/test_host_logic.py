@@ -212,3 +212,47 @@ def test_checkpoint_padding_grids_fit_a_launch(N, B, I, per_block):
     assert (g.y_gu, g.y_dn) == per_block and (g.n_gu, g.n_dn) == (N * g.y_gu, N * g.y_dn)
     assert max(g.n_gu, g.n_dn) * 256 < 1 << 32
     assert (f(N, B, 2 * I, False, True).n_gu, f(N, B, 2 * I, True, False).n_dn) == (0, 0)
+
+
+def _build_module():
+    import importlib.util
+    import os
+
+    path = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "nki-library_amd", "build.py")
+    spec = importlib.util.spec_from_file_location("moe_build", path)
+    build = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(build)
+    return build
+
+
+_LOAD = ["s_add_u32 m0, s33, 0xf000", "s_nop 0", "buffer_load_dwordx4 v186, s[60:63], s10 offen lds"]
+_MFMA = "v_mfma_f32_16x16x32_bf16 a[0:3], v[8:11], v[12:15], a[0:3]"
+
+
+@pytest.mark.parametrize("code,ok", [
+    (["v_accvgpr_write_b32 a0, 0", "v_accvgpr_read_b32 v5, a3", _MFMA, *_LOAD], True),
+    (["v_accvgpr_write_b32 a0, v7", *_LOAD], False),             # a spill into an accumulation register
+    (["ds_read_b64 a[4:5], v7", *_LOAD], False),                 # a load into one
+    (["v_readfirstlane_b32 s10, v3", "s_nop 1", *_LOAD], False),
+    (["v_add_co_u32_e64 v3, s[10:11], v4, v5", *_LOAD], False),
+    (["v_readfirstlane_b32 s10, v3", "s_nop 0", "s_nop 0", "s_nop 0", "s_nop 0", "s_nop 0", *_LOAD], True),
+    (["v_perm_b32 v9, v3, v4, v5", _MFMA, *_LOAD], False),       # its operand, just written
+    (["v_perm_b32 v16, v3, v4, v5", _MFMA, *_LOAD], True),
+    (["v_perm_b32 v9, v3, v4, v5", "s_nop 1", _MFMA, *_LOAD], True),
+    ([_MFMA], False),                                            # no load of the K loop at all
+])
+def test_check_of_the_compiled_tile_loops(code, ok):
+    """build.check_tile_lines on listings that keep and break what the tile loops rely on."""
+    build = _build_module()
+    if ok:
+        build.check_tile_lines(code, "listing")
+    else:
+        with pytest.raises(RuntimeError):
+            build.check_tile_lines(code, "listing")
+
+
+def test_build_without_the_listing_tools(tmp_path, monkeypatch):
+    """Where LLVM's binary tools are absent the build goes on and says so."""
+    monkeypatch.setenv("ROCM_PATH", str(tmp_path))
+    build = _build_module()
+    assert "not checked" in build.check_tile_code("x.o")
