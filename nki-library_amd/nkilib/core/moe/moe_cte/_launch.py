@@ -16,7 +16,8 @@ from .moe_cte_utils import SkipMode
 
 # Profiling hook: when set to a callable, the pipeline is issued one stage per C-ABI call and
 # ``stage_callback(name)`` runs after each stage has been enqueued (bench.py records a HIP event
-# there).  The kernels and their order are identical to the single-call path.
+# there).  The kernels and their order are those of the single-call path, except that a layer with activation
+# checkpoints copies their padding rows behind each GEMM instead of together with the combine (the same values).
 stage_callback = None
 
 _STAGES = (

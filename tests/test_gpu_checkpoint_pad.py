@@ -1,6 +1,7 @@
-"""Activation checkpoints behind an expert's last token and in blocks that do not run (ckpt_pad_*_kernel): every row against
-the oracle's, and the same bits whether the tables are the block build's own or copies of them; calls with checkpoints
-follow tables that change.  Tolerances are those of test_gpu_moe.py."""
+"""Activation checkpoints (csrc/combine.hip: ckpt_tail_kernel, and ckpt_pad_kernel for a layer issued stage by stage): the
+rows of tokens, those behind an expert's last token and the blocks that do not run, every row against the oracle's; the same
+bits whether the tables are the block build's own or copies of them, and from one call and from a call per stage; calls with
+checkpoints follow tables that change.  Tolerances are those of test_gpu_moe.py."""
 
 import numpy as np
 import pytest
@@ -18,12 +19,16 @@ pytestmark = pytest.mark.gpu
     (300, 512, 256, 4, 2, 512, False, True),   # the same with conditions: the blocks past the experts stay zero
     (40, 512, 128, 8, 2, 64, True, False),     # short blocks, pieces of eight rows with rows to keep
     (100, 256, 64, 4, 1, 33, False, True),     # odd blocks: element by element; I shorter than a column tile
+    (300, 256, 160, 2, 1, 33, False, True),    # odd blocks in chunks of 150 rows, which go through five blocks each
+    (600, 256, 128, 2, 1, 131, False, False),  # ... of 300 rows
+    (700, 256, 128, 2, 1, 131, True, False),   # ... and a second chunk that begins within a block
+    (700, 256, 128, 2, 1, 130, False, False),  # the same with even blocks, two rows to a store
     (256, 256, 96, 2, 1, 128, False, False),   # full blocks: the last run's only padding is whole blocks
     (9, 256, 128, 16, 1, 128, True, False),    # experts without a token
 ])
-def test_checkpoint_padding(T, H, I, E, k, B, skip, cond):
+def test_checkpoint_padding(T, H, I, E, k, B, skip, cond, monkeypatch):
     import torch
-    from nkilib.core.moe.moe_cte import SkipMode, build_token_blocks
+    from nkilib.core.moe.moe_cte import SkipMode, _launch, build_token_blocks
     from nkilib.core.moe.moe_cte.bwmm_shard_on_block import run_dense_variant
 
     dev = torch.device("cuda:0")
@@ -31,19 +36,21 @@ def test_checkpoint_padding(T, H, I, E, k, B, skip, cond):
     ids = i32_tensor(ob.router_with_controlled_distribution(T, k, E).astype(np.int32), dev)
     args = (bf16_tensor(c["hidden"], dev), bf16_tensor(c["aff"].reshape(-1, 1), dev), bf16_tensor(c["gate_up_w"], dev),
             bf16_tensor(c["down_w"], dev))
-    outs = []
-    for planned in (False, True):
+    outs, stages = [], []
+    for planned, by_stage in ((False, False), (True, False), (True, True)):
         tp, b2e, co = build_token_blocks(ids, E, B, c["N"], skip_token=skip)
         assert np.array_equal(tp.cpu().numpy(), c["tp2id"])
         if not planned:  # (copies: not the tables that the plan belongs to)
             tp, b2e, co = tp.clone(), b2e.clone(), co.clone()
         junk = [torch.full((c["N"] * B * max(2 * I, H),), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2)]
         del junk  # the checkpoints are allocated over it
+        monkeypatch.setattr(_launch, "stage_callback", stages.append if by_stage else None)
         outs.append(run_dense_variant(*args, B, tp, b2e, "TH", conditions=co if cond else None,
                                       gate_and_up_proj_bias=bf16_tensor(c["gate_up_bias"], dev),
                                       down_proj_bias=bf16_tensor(c["down_bias"], dev), skip_dma=SkipMode(skip, False),
                                       checkpoint_gate_up=True, checkpoint_down=True))
     torch.cuda.synchronize()
+    assert stages == ["prep", "gate_up", "down", "combine"]
     g_out, g_gu, g_d = omoe.moe_blockwise_ref(
         c["hidden"], c["aff"], c["gate_up_w"], c["down_w"], c["tp2id"], c["b2e"], B,
         conditions=c["cond"] if cond else None, gate_up_proj_bias=c["gate_up_bias"], down_proj_bias=c["down_bias"],
@@ -52,8 +59,8 @@ def test_checkpoint_padding(T, H, I, E, k, B, skip, cond):
         _check(from_bf16_tensor(out)[:T], g_out[:T], "output")
         _check(from_bf16_tensor(gu), g_gu, "gate_up_activations_T")
         _check(from_bf16_tensor(d), g_d, "down_activations")
-    for x, y in zip(*outs):
-        assert torch.equal(x.view(torch.int16), y.view(torch.int16))
+    for x, y, z in zip(*outs):
+        assert torch.equal(x.view(torch.int16), y.view(torch.int16)) and torch.equal(x.view(torch.int16), z.view(torch.int16))
 
 
 def test_checkpoints_follow_the_tables():
