@@ -856,9 +856,10 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   tile_live = -1;
 
   // ---- hand over to the next tile ------------------------------------------------------------------------
-  // Everything in flight lands here: the next tile's first slices, this tile's stores (stores and loads share
-  // the counter but complete in no fixed order between them, so the K loop's counting waits must not start
-  // while stores are out), and the small loads issued ahead of the epilogue, which may be used from here on.
+  // Everything in flight lands here: the next tile's first slices, this tile's stores, and the small loads issued ahead of
+  // the epilogue, which may be used from here on.  (The K loop's waits count from nothing outstanding.  Loads and stores
+  // share one counter, which counts down in issue order, so a wait that leaves stores out would do, as in mx_wide.hpp; the
+  // stores of so few rows are not worth one.)
   tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
   if (!have_next) break;
   if (STAGE == 2) tw.aff_put(nxt.e, buf ^ 1, aff_n);
@@ -905,6 +906,11 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int interleave = __builtin_amdgcn_readfirstlane(a.q_off[8 * (CHUNK_CLASSES + 1)]);
   int L = w;
   // classes in queue order (CHUNK_CLASS_TILES / CHUNK_CLASS_LAST in combine.hpp)
+  // (Chunks of up to 64 rows are a stream of weights, for which three slices ahead in registers beat two stages in LDS.
+  // mx_gemm_tiles on 4 row tiles | mx_gemm_tiles_wide on 8, gate/up + down, us: MXFP8, 256 experts of H = 7168, I = 2048 with
+  // 16 rows each 1123 + 637 | 1155 + 663, with 64 1216 + 685 | 1236 + 697; 128 of 2048, 768 with 64 rows 85 + 56 | 90 + 59;
+  // MXFP4, 64 of 7168, 2048 with 16 rows 170 + 103 | 215 + 133, with 64 214 + 109 | 232 + 137; bf16, 64 of 4096, 2048 with
+  // 64 rows 390 + 189 | 397 + 192; fp8-row, the same 206 + 104 | 209 + 110.)
 #define MX_RUN_TILES(TILES_, LAST_)                                                                               \
   if constexpr ((TILES_) >= 8)                                                                                   \
     L = mx_gemm_tiles_wide<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \

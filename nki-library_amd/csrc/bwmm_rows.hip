@@ -111,8 +111,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   // MX gate/up: neighbouring items (column groups of one expert) share the lines that hold the block scales, 16 bytes of a
   // line each, so every XCD takes a contiguous eighth of the items (workgroup ids go round the XCDs; the grid is a multiple
   // of 8): dealt round-robin, every XCD fetched nearly every such line (one token on 8 experts of H = 7168, I = 2048: 294
-  // MB where 242 are needed, the layer 91 us; now 85).  Elsewhere nothing is shared and the round-robin order is the better
-  // one by a per cent (20 tokens on 128 bf16 experts: 167 | 168 us): it spreads an expert's weights over the memory.
+  // MB where 242 are needed, the layer 91 us; now 84).  Elsewhere nothing is shared, and round-robin | by XCD came out the
+  // same within the spread of the runs (20 tokens on 128 bf16 experts of H = 2048, I = 768, gate/up + down: 95 + 49.7 |
+  // 96 + 50.1 us; 16 on 64 fp8-row experts of 4096, 768: 48.2 + 30.1 | 48.6 + 29.4) but for the smallest: 256 tokens on 8 bf16
+  // experts of 512, 1024: 17.4 + 18.2 | 16.7 + 19.4.  Those keep the order that deals neighbouring items to all XCDs.
   constexpr bool BY_XCD = STAGE == 1 && SCALED;
   const int xcd = blockIdx.x & 7;
   const int item0 = BY_XCD ? (int)((int64_t)n_items * xcd / 8) + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
@@ -457,8 +459,13 @@ static int launch_rows(const MxArgs& m, int64_t rows, int64_t max_chunks, int cu
 //     80 | 70); 4-bit ones there while the tiles are few (48 rows: 119 of 4096, 2048: 115 | 131; 59 of 2048, 6400: 81 | 104;
 //     32 of 3072, 1536: 31 | 28).
 //   bf16 beyond 64 rows, one pass of 64 on average, while the large-tile kernel has a tile for half of the CUs or less: 256
-//     tokens over 8 experts, two of them each, of H = 512, I = 1024: gate/up 23 | 17, down 27 | 18; of H = 4096, I = 1024:
-//     72 | 61 and 28 | 33; 384 tokens of the former: 23 | 20 and 27 | 21, not taken: a pass more per expert and falling.
+//     tokens over 8 experts, two of them each, of H = 512, I = 1024: gate/up 19 | 17, down 23 | 18; of H = 4096, I = 1024:
+//     70 | 61 and 27 | 33; 384 tokens of the former: 21 | 20 and 25 | 21, not taken: a pass more per expert and falling.
+//   (Every time with chunks of more than 64 rows, i.e. this paragraph and the table below, is of the present loop of
+//     mx_wide.hpp.  Over 260 random shapes of up to 64 tokens, bf16 up to 256, on that build: gate/up 1.049 and down 1.016
+//     times the better kernel's time, the large-tile kernels alone 1.67 and 1.72, this one alone 1.007 and 1.002.  What the
+//     rule leaves is small launches that it still gives to the large tiles, MX kinds with 33 to 64 tokens over four experts
+//     above all: 46 tokens of H = 2048, I = 512: 37 | 15 and 21 | 9.)
 bool mx_rows_fits(int stage, int wfmt, const RowsCall& c) {
   const bool fp4 = wfmt == MX_WFMT_E2M1, bf16 = wfmt == MX_WFMT_BF16, mx = !bf16 && wfmt != MX_WFMT_ROW8;
   if (stage == 1 && mx) {
@@ -478,8 +485,8 @@ bool mx_rows_fits(int stage, int wfmt, const RowsCall& c) {
   if (!bf16 || c.rows > 256 || c.col_tiles * c.max_chunks > 128) return false;
   // A table of N blocks is made for about (N - (E - 1)) * B routed rows.  One with fewer blocks than experts was cut by the
   // caller to what it holds, which may be whole blocks: several passes, worth it while the large-tile kernel has a chunk
-  // for an XCD or less (gate/up, 7 blocks of 128 rows over H = 2048, I = 1024: 76 | 44; 4 of 256: 114 | 74; 16 of 256 over
-  // H = 4096: 112 | 275).
+  // for an XCD or less (gate/up, 7 blocks of 128 rows over H = 2048, I = 1024: 72 | 43; 4 of 256: 95 | 75; 16 of 256 over
+  // H = 4096: 100 | 273).
   if (c.N < c.E) return c.max_chunks <= 8 || (c.B < c.rows ? c.B : c.rows) <= 64;
   return (c.N - (c.E - 1)) * c.B / c.E <= 64;
 }

@@ -124,8 +124,13 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
     if (in_lds) s_cx[i] = v;
     else chunk_xcd[i] = v;
   };
-  // (what a chunk costs per K slice is its loads, the same for every chunk, plus its MFMAs: measured over the
-  // row-tile classes 1.16 us + 0.055 us per row tile, i.e. 21 row tiles' worth of fixed cost)
+  // (what a chunk costs per K slice is its loads, the same for every chunk, plus its MFMAs.  CHUNK_FIXED_COST_TILES, the
+  // fixed part in row tiles, was set by the loop that ran every tile with the weights in registers: 21.  Launches with
+  // equal chunks of 8 to 16 row tiles on the present loop put it at 36 (gate/up, MXFP8, 256 experts of H = 7168, I = 2048:
+  // 1377 us at 8 row tiles, 1626 at 16), 17 (its down stage: 745, 989), 29 and 18 (128 experts of H = 2048, I = 768: 93 and
+  // 113, 63 and 83); past 16 a row tile costs 1.1 to 2.3 times as much (1912 and 1124, 128 and 98 at 20).  No one number
+  // fits both stages of a layer, whose chunks are the same, and this one lies between them.  Formats other than e4m3 run
+  // 10 to 14 row tiles on the instance of 16, which is not counted here.)
   auto work_of = [&](int i) { return chunk_row_tiles(rows_of(i), true) + CHUNK_FIXED_COST_TILES; };
   int wcarry = 0;
   for (int i0 = 0; i0 < n; i0 += (int)blockDim.x) {

@@ -52,7 +52,7 @@ __host__ __device__ inline int chunk_class(int rows, bool last) {
 }
 
 constexpr int CHUNK_ROWS = 256;      // rows of every chunk of a run but the last
-constexpr int CHUNK_FIXED_COST_TILES = 20;  // a chunk's loads per K slice, in row tiles of MFMA time (XCD balance)
+constexpr int CHUNK_FIXED_COST_TILES = 20;  // a chunk's loads per K slice, in row tiles of MFMA time (XCD balance, chunks.hpp)
 constexpr int CHUNK_ROWS_MAX = 320;  // the last chunk of a run takes up to this many
 inline int64_t max_chunks_for(int64_t N, int64_t B) { return N * ((B + CHUNK_ROWS - 1) / CHUNK_ROWS); }
 

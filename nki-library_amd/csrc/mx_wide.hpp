@@ -26,6 +26,8 @@
 // across all rows, some 4000 cycles per slice): 8192 tokens over 256 MXFP8 experts of H = 7168, I = 2048 3155 -> 3010 us;
 // 4096 tokens, top-2 of 8 bf16 experts of H = 2048, I = 4096 440 -> 409; 8192 tokens, top-8 of 128 MXFP8 experts of H = 2048,
 // I = 768 539 -> 502; 1999 tokens, top-4 of 32 MXFP4 experts of H = 3072, I = 1536 203 -> 196.
+// (Dense kinds: no vector ALU instruction in the K loop; MX: one per slice, the address of the activation scales, and with
+// 4-bit weights the 32 that pick a column's halves.)
 #pragma once
 
 #include "mx_tile.hpp"
@@ -303,7 +305,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     else
       dma_b32<U * Cfg::WS, LOOP>(lds_ws, ws_voff, rs_, ws_off);
   };
-  // Activation scales of the four slices from ks0 (a multiple of four) on.
+  // Activation scales of the four slices from ks0 (a multiple of four) on.  (The loop requests them in every second slice:
+  // ahead of a group's first slice the group, and once more from within it, the same bytes to the same places.)
   auto load_as = [&](int ks0, auto loop_) {
     constexpr bool LOOP = decltype(loop_)::value;
     if constexpr (SCALED) {
@@ -579,8 +582,9 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       request_first(std::integral_constant<int, loads_by(i)>{}, std::integral_constant<int, loads_by(i + 1)>{});
     };
     // Loads and stores that may still be out when the next tile starts, those issued behind the last load that its first
-    // slice needs: slice 1's loads and the stores of the later steps (loads and stores complete in issue order; a store
-    // that is not counted here only makes the wait a longer one).
+    // slice needs: slice 1's loads and the stores of the later steps (vector loads and stores share one counter on this
+    // target, which counts down in issue order: the compiler relies on it as well and waits for vmcnt(2) ahead of the use
+    // of a load with two stores behind it; a store that is not counted here only makes the wait a longer one).
     constexpr int NEED = 1 + NW + NAJ;
     auto last_need_step = [=]() constexpr {
       int i = 0;
