@@ -462,7 +462,7 @@ static int launch_rows(const MxArgs& m, int64_t rows, int64_t max_chunks, int cu
 //     tokens over 8 experts, two of them each, of H = 512, I = 1024: gate/up 19 | 17, down 23 | 18; of H = 4096, I = 1024:
 //     70 | 61 and 27 | 33; 384 tokens of the former: 21 | 20 and 25 | 21, not taken: a pass more per expert and falling.
 //   (Every time with chunks of more than 64 rows, i.e. this paragraph and the table below, is of the present loop of
-//     mx_wide.hpp.  Over 260 random shapes of up to 64 tokens, bf16 up to 256, on that build: gate/up 1.049 and down 1.016
+//     mx_wide.hpp.  Over 260 random shapes of up to 64 tokens, bf16 up to 256: gate/up 1.049 and down 1.016
 //     times the better kernel's time, the large-tile kernels alone 1.67 and 1.72, this one alone 1.007 and 1.002.  What the
 //     rule leaves is small launches that it still gives to the large tiles, MX kinds with 33 to 64 tokens over four experts
 //     above all: 46 tokens of H = 2048, I = 512: 37 | 15 and 21 | 9.)

@@ -20,9 +20,9 @@
 //     landed; the loads of the activations two slices ahead go out, and under the last 16 MFMAs the fragments of the next
 //     slice are read: a weight fragment is read into the registers of the one whose last MFMA has just been issued.
 //     No slice begins with a wait for LDS.
-// What bounds it: the matrix pipes, at the clock that the part's power leaves them.  A bf16 slice of 16 row tiles takes 2690
-// cycles, its MFMAs alone 2480 (128 of 16 x 16 x 32, one in 19.35 cycles); an fp8-row slice 2540 and an MXFP8 slice with the
-// weights from HBM 3050 cycles of 2048.  Layers back to back, against the loop before (weights through registers, one wave
+// What bounds it: the matrix pipes with bf16 (a slice of 16 row tiles takes 2690 cycles, its MFMAs alone 2480: 128 of
+// 16 x 16 x 32, one in 19.35 cycles); with 8 bits, where the MFMAs take 2048, the DMA's latency (fp8-row 2540 cycles, MXFP8 with
+// the weights from HBM 3050); all of them at the clock that the part's power leaves, 1.7 to 2.1 GHz.  Layers back to back, against the loop before (weights through registers, one wave
 // across all rows, some 4000 cycles per slice): 8192 tokens over 256 MXFP8 experts of H = 7168, I = 2048 3155 -> 3010 us;
 // 4096 tokens, top-2 of 8 bf16 experts of H = 2048, I = 4096 440 -> 409; 8192 tokens, top-8 of 128 MXFP8 experts of H = 2048,
 // I = 768 539 -> 502; 1999 tokens, top-4 of 32 MXFP4 experts of H = 3072, I = 1536 203 -> 196.
