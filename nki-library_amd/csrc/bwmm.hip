@@ -6,7 +6,7 @@
 //   MXFP8    v_mfma_scale_f32_16x16x128_f8f6f4, E8M0 block scales of both operands applied by
 //            the matrix core
 // This file holds the general tiled kernel, for the shapes the large-tile kernels (bwmm_mx.hip) do not take (H % 256,
-// % 512 for the fp8 kinds; I % 128 for MXFP8): a 256-thread workgroup owns 128 rows of one block
+// % 512 for the fp8 kinds; MXFP8: what mx_fast, csrc/capi.hip, turns down): a 256-thread workgroup owns 128 rows of one block
 // (one expert) and 128 output columns (256 in stage 1: gate and up), stages one 128-byte
 // K-slice of both operands in LDS in K-contiguous order and lets each of the four waves run
 // 2 x (8|16) MFMA tiles over it.  Rows are gathered through token_position_to_id while the A

@@ -183,8 +183,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   if (STAGE == 1) {
     nks = (int)(a.H / 128);
   } else {
-    const int64_t tail = a.I % 512;
-    nks = (int)((a.I / 512) * 4 + (tail / 128));
+    nks = (int)mx_col_tiles(a.I);
   }
 
   // ---- B operand addressing ---------------------------------------------------------------------------
@@ -222,6 +221,16 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
                                                         : (uint32_t)((GROWS * g * w_pstride + 4 * c) * ES));
   const uint32_t s_voff = (STAGE == 1) ? (uint32_t)(g * w_pstride + hcol * nH * a.I + 4 * cl)
                                        : (uint32_t)(g * w_pstride + 4 * c);
+  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // 8).  Loads of partitions past that are aimed past the end of the expert's weights and scales, both smaller than 2^31
+  // bytes, and return zeros: the lane's offsets in the slice that slice_addr was last called for.
+  constexpr bool KTAIL = STAGE == 2 && !ROW8;
+  const int nP = (int)(a.I >> 2);
+  constexpr uint32_t PAST_END = 0x80000000u;
+  // (Where even the first partition of a load does not exist, its scalar offset alone may lie past the end: such loads go
+  // through a descriptor of zero records.)
+  uint32_t w_lo = w_voff, w_hi = w_voff, s_lo = s_voff;  // partitions GROWS g ..; 16 + 4 g .. (8-bit); the scales of block g
+  int rw_hi = 0;
   // bytes of one expert's weights: the reference layout's, or col_tiles x nks runs of 32 KB
   const int64_t w_expert_bytes = pk * ((int64_t)a.col_tiles * nks * PK_SLICE) +
                                  npk * ((STAGE == 1) ? 128 * w_pstride * ES : (int64_t)a.pI * w_pstride * ES);
@@ -329,6 +338,14 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
     r.as_off = ks * 4;
     r.w_off = uni(pk * (ks * PK_SLICE) + npk * (int)(((int64_t)(pb * 32) * w_pstride + (int64_t)kt * w_tstride) * ES));
     r.s_off = uni((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride);
+    if constexpr (KTAIL) {
+      w_lo = (ks * 32 + GROWS * g < nP) ? w_voff : PAST_END;
+      if constexpr (!FP4) {
+        w_hi = (ks * 32 + 16 + GROWS * g < nP) ? w_voff : PAST_END;
+        rw_hi = uni(rw_rec & (ks * 32 + 16 < nP ? tile_live : 0));
+      }
+      s_lo = (ks * 32 + 8 * g < nP) ? s_voff : PAST_END;
+    }
     return r;
   };
   auto issue_load = [&](auto idx_, const SliceAddr& sa, BRaw& b, ScaleRegs& sc0, auto with_scales_) {
@@ -348,11 +365,12 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
       }
     } else if constexpr (idx < NAJ + NSC + NBL) {
       constexpr int i = idx - NAJ - NSC;
-      if constexpr (FP4) ld_b64<LASTUSE>(b.d[i], w_voff, rw_, w_soff[i] + sa.w_off);
-      else ld_b128<LASTUSE>(b.d[i], w_voff, rw_, w_soff[i] + sa.w_off);
+      if constexpr (KTAIL && !FP4 && i == 4) rw_[2] = rw_hi;
+      if constexpr (FP4) ld_b64<LASTUSE>(b.d[i], w_lo, rw_, w_soff[i] + sa.w_off);
+      else ld_b128<LASTUSE>(b.d[i], i < 4 ? w_lo : w_hi, rw_, w_soff[i] + sa.w_off);
     } else {
       static_assert(SCALED || idx < NAJ + NSC + NBL, "no scale load without scales");
-      if constexpr (SCALED) ld_b32(b.sc, s_voff, rs_, s_soff + sa.s_off);
+      if constexpr (SCALED) ld_b32(b.sc, s_lo, rs_, s_soff + sa.s_off);
     }
   };
   // The MFMA wants a lane's scale byte to be that of row 16*mt + c and K block g, one byte per row
@@ -759,10 +777,13 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
             d[k] = pack4_e4m3(clip448(yv[0][k] * is), clip448(yv[1][k] * is), clip448(yv[2][k] * is), clip448(yv[3][k] * is));
           const int64_t slot = cur.slot0 + row;
           const int pw = tw.tile_p0(cur) + 8 * j;  // first partition of the block within the intermediate tile
+          const uint32_t p_live = pw < tw.tile_Pt(cur) ? ~0u : 0u;  // past the last of a short tile: zeros, whatever the columns hold
+#pragma unroll
+          for (int k = 0; k < 8; ++k) d[k] &= p_live;
           uint4* o = (uint4*)(a.Yq + slot * a.y_stride + tw.tile_tI(cur) * 512 + pw * 4);
           o[0] = make_uint4(d[0], d[1], d[2], d[3]);
           o[1] = make_uint4(d[4], d[5], d[6], d[7]);
-          a.Ys[slot * a.ys_stride + tw.tile_tI(cur) * 16 + (pw >> 3)] = (uint8_t)sb;
+          a.Ys[slot * a.ys_stride + tw.tile_tI(cur) * 16 + (pw >> 3)] = (uint8_t)(sb & p_live);
         }
         }
       }
@@ -1007,6 +1028,7 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
   const int g = lane >> 4, c = lane & 15;
   const int64_t pr = FP4 ? i : ((i < 4) ? i : (16 + i - 4)), kt = ks >> 2, pb = ks & 3;
   int64_t elem, expert_elems;
+  bool live;  // (a short last tile's padding: zeros)
   if (stage == 1) {
     const int64_t nH = H / 512, pstride = 2 * nH * I;
     const int64_t tI = xt >> 2, p0 = (xt & 3) * 32;
@@ -1014,19 +1036,21 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
     const int64_t colu = tI * 512 + q * (rows_t / 4) + p0;
     elem = (GROWS * g + pr + pb * 32) * pstride + (c >> 3) * nH * I + 4 * (c & 7) + colu + kt * I;
     expert_elems = 128 * pstride;
+    live = p0 + 4 * (c & 7) < rows_t / 4;
   } else {
     const int64_t nI = (I + 511) / 512, pI = I > 512 ? 128 : I / 4, pstride = nI * H;
     elem = (GROWS * g + pr + pb * 32) * pstride + 4 * c + xt * 256 + 64 * q + kt * H;
     expert_elems = pI * pstride;
+    live = ks * 32 + GROWS * g + pr < I / 4;
   }
   const uint8_t* src = W + (e * expert_elems + elem) * ES;
   const int64_t o = (d & ~(int64_t)63) + (stage == 1 ? mx_pack_lane(lane) : lane);
-  if constexpr (FP4) *(uint2*)(dst + o * LB) = *(const uint2*)src;
-  else *(uint4*)(dst + o * LB) = *(const uint4*)src;
+  if constexpr (FP4) *(uint2*)(dst + o * LB) = live ? *(const uint2*)src : make_uint2(0, 0);
+  else *(uint4*)(dst + o * LB) = live ? *(const uint4*)src : make_uint4(0, 0, 0, 0);
 }
 
 static void mx_pack_geometry(int stage, int64_t H, int64_t I, int64_t* col_tiles, int64_t* nks) {
-  const int64_t over_i = (I / 512) * 4 + (I % 512) / 128;
+  const int64_t over_i = mx_col_tiles(I);
   *col_tiles = stage == 1 ? over_i : H / 256;
   *nks = stage == 1 ? H / 128 : over_i;
 }

@@ -84,7 +84,13 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
 
   int nks;
   if (STAGE == 1) nks = (int)(a.H / 128);
-  else nks = (int)((a.I / 512) * 4 + (a.I % 512) / 128);
+  else nks = (int)mx_col_tiles(a.I);
+  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // 8); a load of partitions past that is aimed past the end of the expert's weights (less than 2^31 bytes) and returns zeros
+  // (where even the first partition of a load does not exist: through a descriptor of zero records)
+  constexpr bool KTAIL = STAGE == 2 && SCALED;
+  constexpr uint32_t PAST_END = 0x80000000u;
+  const int nP = (int)(a.I >> 2);
 
   // weight addressing: as in mx_gemm_tiles (same layouts, one wave per 64 columns)
   constexpr int ES = FP4 ? 2 : 4, GROWS = FP4 ? 8 : 4;
@@ -197,15 +203,18 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
         const int kt = ks >> 2, pb = ks & 3;
         const rsrc_t rw = rsrc_of(Wp, live ? (uint32_t)w_expert_bytes : 0u);
         const int w_off = w_base + uni32(pk ? ks * PK_SLICE : (int)(((int64_t)(pb * 32) * w_pstride + (int64_t)kt * w_tstride) * ES));
+        const uint32_t w_lo = (!KTAIL || ks * 32 + GROWS * g < nP) ? w_voff : PAST_END;
+        const uint32_t w_hi = (!KTAIL || ks * 32 + 16 + GROWS * g < nP) ? w_voff : PAST_END;
+        const rsrc_t rw_hi = (KTAIL && !FP4) ? rsrc_of(Wp, ks * 32 + 16 < nP ? (uint32_t)w_expert_bytes : 0u) : rw;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int soff = w_off + (FP4 ? i : (i < 4) ? i : w_jump + i - 4) * w_step;
-          if constexpr (FP4) s.b[i] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rw, w_voff, soff, AUX_NT));
-          else s.b[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, w_voff, soff, AUX_NT));
+          if constexpr (FP4) s.b[i] = __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(rw, w_lo, soff, AUX_NT));
+          else s.b[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(i < 4 ? rw : rw_hi, i < 4 ? w_lo : w_hi, soff, AUX_NT));
         }
         if constexpr (SCALED) {
           const rsrc_t rs = rsrc_of(Sp, live ? (uint32_t)ws_expert : 0u);
-          s.bs = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, s_voff, s_base + uni32((int)((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride)), 0);
+          s.bs = (int)__builtin_amdgcn_raw_buffer_load_b32(rs, (!KTAIL || ks * 32 + 8 * g < nP) ? s_voff : PAST_END, s_base + uni32((int)((int64_t)(pb * 4) * w_pstride + (int64_t)kt * w_tstride)), 0);
         }
       };
       auto load_a = [&](ASlice& s, int ks) {
@@ -320,7 +329,7 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
 #pragma unroll
           for (int qq = 0; qq < 4; ++qq) {
             float gv = part(r, qq * 32 + pp), uv = part(r, qq * 32 + 16 + pp);
-            if (a.bias) {
+            if (a.bias && p < Pt) {
               const int64_t b0 = ((((int64_t)e * a.pI + p) * 2) * a.nI + tI) * 4 + qq;
               gv += bias_at(b0);
               uv += bias_at(b0 + (int64_t)a.nI * 4);
@@ -334,9 +343,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
           const uint32_t sb = mx_scale_byte(am);
           const float is = mx_inv_scale(sb);
           const int64_t slot = slot0 + row0 + r;
+          const uint32_t p_live = p < Pt ? ~0u : 0u;  // past the last partition of a short tile: zeros, whatever the columns hold
           *(uint32_t*)(a.Yq + slot * a.y_stride + tI * 512 + p * 4) =
-              pack4_e4m3(clip448(y[0] * is), clip448(y[1] * is), clip448(y[2] * is), clip448(y[3] * is));
-          if ((pp & 7) == 0) a.Ys[slot * a.ys_stride + tI * 16 + (p >> 3)] = (uint8_t)sb;
+              pack4_e4m3(clip448(y[0] * is), clip448(y[1] * is), clip448(y[2] * is), clip448(y[3] * is)) & p_live;
+          if ((pp & 7) == 0) a.Ys[slot * a.ys_stride + tI * 16 + (p >> 3)] = (uint8_t)(sb & p_live);
         }
       } else if constexpr (STAGE == 1) {
         // thread = (row, two neighbouring columns)

@@ -2,6 +2,8 @@
 // device check, workspace planning and the blockwise-MoE driver.
 #include <string.h>
 
+#include <initializer_list>
+
 #include "bwmm.hpp"
 
 using namespace moe;
@@ -45,6 +47,36 @@ struct Plan {
   int64_t Iw;      // padded intermediate width (elements) of the stage-2 A operand
   int64_t pI, nI;  // MXFP8
 };
+
+// MX kinds on the large-tile and few-rows kernels (csrc/bwmm_mx.hip, csrc/bwmm_rows.hip).  mx_shape: the expert shape and
+// weight type, which alone decide whether there are copies of the weights in those kernels' order; mx_fast: the call as well.
+// Byte offsets (row * row stride, added to a 64-bit base) and buffer descriptors of at most 2^32 - 1 bytes for the
+// activations, the intermediate and their scales; signed 32-bit byte offsets inside one expert's weights (of which the
+// copies hold whole column tiles and K slices); the row tables (token ids, affinities, bias) through 32-bit byte offsets.
+// Where I is no multiple of 128 the general kernel takes what they do not: activations past those offsets, and tensors that
+// lie closer than the 16 (tables: 4) bytes their loads are aligned to.
+constexpr int64_t LIM32 = (int64_t)1 << 32, LIM31 = (int64_t)1 << 31;
+bool aligned(std::initializer_list<const void*> ptrs, uintptr_t n) {
+  for (const void* p : ptrs)
+    if ((uintptr_t)p % n != 0) return false;
+  return true;
+}
+bool mx_shape(const moe_bwmm_args* a) {
+  if (a->kind != MOE_KIND_MXFP8 || !mx_fast_path_ok(a->H, a->I)) return false;
+  if (a->I % 128 != 0 && !aligned({a->gate_up_proj_weight, a->down_proj_weight}, 16)) return false;
+  const int64_t es = a->weight_dtype == MOE_DT_FP4_E2M1 ? 2 : 4;  // bytes of an x4 weight element
+  const int64_t pI = a->I > 512 ? 128 : (mx_col_tiles(a->I) * 32), nI = (a->I + 511) / 512;
+  return 128 * 2 * (a->H / 512) * (mx_col_tiles(a->I) * 128) * es < LIM31 && pI * nI * a->H * es < LIM31 &&
+         a->E * pI * 2 * nI * 4 * 4 < LIM32 && a->E * a->H * 4 < LIM32;
+}
+bool mx_fast(const moe_bwmm_args* a) {
+  const int64_t slots = a->N * a->B, Iw = (a->I + 511) / 512 * 512;
+  if (a->I % 128 != 0 && !(aligned({a->hidden_states, a->hidden_states_scale}, 16) &&
+                           aligned({a->gate_up_proj_scale, a->down_proj_scale, a->gate_and_up_proj_bias, a->down_proj_bias,
+                                    a->expert_affinities_masked}, 4)))
+    return false;
+  return mx_shape(a) && a->T1 * a->H < LIM32 && slots * Iw < LIM32 && slots * 4 < LIM32 && a->T1 * a->E * 4 < LIM32;
+}
 
 int validate(const moe_bwmm_args* a) {
   if (!a || !a->hidden_states || !a->gate_up_proj_weight || !a->down_proj_weight || !a->token_position_to_id ||
@@ -97,20 +129,9 @@ int validate(const moe_bwmm_args* a) {
   // offsets reach would read wrong rows without any error, so it is refused here (the reference states its
   // own size limits the same way, bwmm_shard_on_block_mx.py:586-633).
   const int64_t slots = a->N * a->B;
-  if (a->kind == MOE_KIND_MXFP8 && mx_fast_path_ok(a->H, a->I)) {
-    // large-tile kernels: byte offsets (row * row stride, added to a 64-bit base) and buffer descriptors of at most
-    // 2^32 - 1 bytes for the activations, the intermediate and their scales; signed 32-bit byte offsets inside one
-    // expert's weights
-    const int64_t lim32 = (int64_t)1 << 32, lim31 = (int64_t)1 << 31;
-    const int64_t Iw = (a->I + 511) / 512 * 512;
-    const int64_t es = a->weight_dtype == MOE_DT_FP4_E2M1 ? 2 : 4;  // bytes of an x4 weight element
-    const int64_t pI = a->I > 512 ? 128 : a->I / 4, nI = (a->I + 511) / 512;
-    if (a->T1 * a->H >= lim32 || slots * Iw >= lim32) return MOE_E_BAD_SHAPE;
-    if (128 * 2 * (a->H / 512) * a->I * es >= lim31 || pI * nI * a->H * es >= lim31) return MOE_E_BAD_SHAPE;
-    // the row tables (token ids, affinities, bias) are fetched through 32-bit byte offsets as well
-    if (slots * 4 >= lim32 || a->T1 * a->E * 4 >= lim32 || a->E * pI * 2 * nI * 4 * 4 >= lim32 ||
-        a->E * a->H * 4 >= lim32)
-      return MOE_E_BAD_SHAPE;
+  if (a->kind == MOE_KIND_MXFP8) {
+    // (an I that is no multiple of 128: past these limits the general kernel takes the call)
+    if (a->I % 128 == 0 && !mx_fast(a)) return MOE_E_BAD_SHAPE;
   } else if (a->kind != MOE_KIND_MXFP8) {
     // general tiled kernel, dense kinds: row offsets are kept in units of 4 bytes in 32 bits (the value ~0 is
     // reserved for "no such row"), i.e. each A operand must stay below 2^34 - 4 bytes = 16 GiB
@@ -303,7 +324,7 @@ int kmajor_copy(const moe_bwmm_args* a, const Plan& p, int which, void* dst, hip
 // for every format, of the down weights for 4-bit ones (whose pieces in the reference layout are 512 bytes; the
 // 8-bit ones' 1 KB pieces were measured no slower than a copy).
 static bool mx_packable(const moe_bwmm_args* a, int which) {
-  if (a->kind != MOE_KIND_MXFP8 || !mx_fast_path_ok(a->H, a->I)) return false;
+  if (!mx_shape(a)) return false;
   return which == 0 || a->weight_dtype == MOE_DT_FP4_E2M1;
 }
 
@@ -472,7 +493,7 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
 
   const bool bf_fast = bf16_fast(a);
   const bool r8_fast = row8_fast(a) || bf_fast;  // (what the two share: x4 copies with unit scale tables)
-  const bool mx_fast = (a->kind == MOE_KIND_MXFP8 && mx_fast_path_ok(a->H, a->I)) || r8_fast;
+  const bool mx_fast = ::mx_fast(a) || r8_fast;
   MxArgs m;
   memset(&m, 0, sizeof(m));
   if (mx_fast) {
@@ -559,7 +580,7 @@ extern "C" int moe_blockwise_stages(const moe_bwmm_args* a, unsigned stages, voi
       m1.clk = a->gemm_clocks;
 
       // column tiles of 32 partitions x 4 q, gate and up: 4 per full intermediate tile + those of a short last one
-      const unsigned gx = (unsigned)((m1.I / 512) * 4 + (m1.I % 512) / 128);
+      const unsigned gx = (unsigned)mx_col_tiles(m1.I);
       const bool few = few_rows(1, gx);
       if (!few && split_rows(a)) {
         rc = launch_split_rows(m1.A, ws + p.xq, (float*)(ws + p.xs), a->T1, a->H, s);

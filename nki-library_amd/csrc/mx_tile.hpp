@@ -177,7 +177,7 @@ struct MxTileWalk {
     return t;
   }
   // gate/up: column tiles are numbered over the existing ones, 4 per full intermediate tile, then those of a
-  // short last tile (whose partitions per q are a multiple of 32 on this path): intermediate tile, first
+  // short last tile (the last of them may hold fewer than 32 partitions per q): intermediate tile, first
   // partition, partitions per q.  down: first hidden column.
   __device__ __forceinline__ auto tile_tI(const MxTile& t) const { return t.xt >> 2; }
   __device__ __forceinline__ auto tile_p0(const MxTile& t) const { return (t.xt & 3) * 32; }
@@ -259,7 +259,9 @@ struct MxTileWalk {
   __device__ __forceinline__ auto bias_index(const MxTile& t) const {
     if (ROW8) return (uint32_t)t.e * ncols() + natural_col(t);
     if (STAGE == 1) {
-      const uint32_t p = (uint32_t)(tile_p0(t) + (tid & 31));
+      // (partitions that a short last tile does not have: the table may end with the last one that exists)
+      const int p_ = tile_p0(t) + (tid & 31), Pt = tile_Pt(t);
+      const uint32_t p = (uint32_t)(p_ < Pt ? p_ : Pt - 1);
       return ((((uint32_t)t.e * (uint32_t)a.pI + p) * 2u + (uint32_t)(tid >> 7)) * (uint32_t)a.nI + (uint32_t)tile_tI(t)) * 4u +
              (uint32_t)((tid >> 5) & 3);
     }

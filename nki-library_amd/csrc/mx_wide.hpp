@@ -183,7 +183,11 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   // ---- K schedule (slice ks: tile of 512 ks >> 2, partition group ks & 3; see bwmm_mx.hip) ------------------------
   int nks;
   if (STAGE == 1) nks = (int)(a.H / 128);
-  else nks = (int)((a.I / 512) * 4 + (a.I % 512) / 128);
+  else nks = (int)mx_col_tiles(a.I);
+  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // 8); weights and scales past that are not read (see aim_w)
+  constexpr bool KTAIL = STAGE == 2 && SCALED;
+  const int nP = uni((int)(a.I >> 2));
 
   // ---- operand addressing -----------------------------------------------------------------------------------
   const int64_t w_pstride = (STAGE == 1) ? 2 * (int64_t)nH * a.I : (int64_t)a.nI * a.H;  // elements between partitions
@@ -286,19 +290,22 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     else dma_b128<U * SA + j * 4096, false, LOOP>(lds_a, a_voff[0], ra_, a_off + j * a_group_bytes);
   };
   // Weights and their scales: load i of NW.
-  int w_off = 0, ws_off = 0;
+  int w_off = 0, ws_off = 0, rw_hi = 0;
   auto aim_w = [&](int ks) {
     const int kt = ks >> 2, pb = ks & 3, live = (ks < nks) ? tile_live : 0;
     w_off = w_base + pb * w_pb + kt * w_kt;
-    rw_[2] = uni(rw_rec & live);
+    // (KTAIL: the wave's first partitions, 4-bit weights all of them, and those of its second half; its scales' block)
+    rw_[2] = uni(rw_rec & (KTAIL ? (ks * 32 + (FP4 ? 8 : 4) * w < nP ? tile_live : 0) : live));
+    if constexpr (KTAIL && !FP4) rw_hi = uni(rw_rec & (ks * 32 + 16 + 4 * w < nP ? tile_live : 0));
     if constexpr (SCALED) {
       ws_off = ws_base + pb * ws_pb + kt * ws_kt;
-      rs_[2] = uni(rs_rec & live);
+      rs_[2] = uni(rs_rec & (KTAIL ? (ks * 32 + 8 * w < nP ? tile_live : 0) : live));
     }
   };
   auto load_w = [&](auto u_, auto i_, auto loop_) {
     constexpr int U = decltype(u_)::value, i = decltype(i_)::value;
     constexpr bool LOOP = decltype(loop_)::value;
+    if constexpr (KTAIL && !FP4 && i == 4) rw_[2] = rw_hi;
     if constexpr (i < NWL)
       dma_b128<U * SW + (FP4 || i < 4 ? i : 12 + i) * 1024, LASTUSE, LOOP>(
           lds_w, w_voff, rw_, w_off + (FP4 || i < 4 ? i * w_step : w_jump + (i - 4) * w_step));
@@ -679,6 +686,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const v4i rdys = make_rsrc(SCALED ? (const void*)(a.Ys + (int64_t)cur.slot0 * ys_rowb) : (const void*)a.tp2id,
                                  SCALED ? (uint32_t)(cur.nrows * ys_rowb) : 0u);
       const int pl = p0 + 16 * wn + 4 * g_e;  // MX: the lane's first partition
+      const int p_live = pl < Pt ? -1 : 0;    // ... past the last one of a short tile: zeros, whatever the columns hold
       const uint32_t yq_voff = (uint32_t)(st_row0 * y_rowb + tI * 512 + (p0 + 16 * wn) * 4 + st_piece * 16);
       // (the scale byte of a block is stored by the even one of its two lane groups; the other's store is out of range)
       const uint32_t ys_voff = (g_e & 1) ? 0xffffffffu : (uint32_t)(row0 * ys_rowb + tI * 16 + (pl >> 3));
@@ -735,12 +743,12 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
             v4i o;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-              o[r] = (int)pack4_e4m3(clip448(y[0][r] * is), clip448(y[1][r] * is), clip448(y[2][r] * is), clip448(y[3][r] * is));
+              o[r] = (int)pack4_e4m3(clip448(y[0][r] * is), clip448(y[1][r] * is), clip448(y[2][r] * is), clip448(y[3][r] * is)) & p_live;
             // (the rows before are stored while these values wait for theirs)
             if constexpr (rt > 0) st_b128_plain(ex_o[0], yq_voff, rdy, (rt - 1) * 16 * y_rowb);
             ex_put(g_e, o);
             ex_get(ex_o);
-            st_b8((int)sb, ys_voff, rdys, rt * 16 * ys_rowb);
+            st_b8((int)sb & p_live, ys_voff, rdys, rt * 16 * ys_rowb);
             spread(rt_);
           });
           st_b128_plain(ex_o[0], yq_voff, rdy, (RT - 1) * 16 * y_rowb);

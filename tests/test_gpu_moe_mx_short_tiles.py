@@ -1,0 +1,58 @@
+"""GPU parity of the MX kinds where the last intermediate tile holds no multiple of 32 partitions (I % 128 != 0): the last
+column tile of the gate/up stage and the last K slice of the down stage are 8, 16 or 24 partitions of their 32, in the
+few-rows kernel and both tile loops of the large-tile kernels, with the weights' copies and in place.  Tolerances are those of
+test_gpu_moe.py."""
+
+import numpy as np
+import pytest
+
+from helpers import from_bf16_tensor, mx_case
+from test_gpu_moe import REF_MX_CLAMPS, _check, _golden_mx_options, _run_mx_options
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,H,I,E,k,fmt", [
+    (1, 512, 32, 4, 2, "e4m3"),       # few rows; 8 partitions in all, one K slice
+    (20, 512, 480, 4, 2, "e4m3"),     # two row tiles; a full slice grid but 8 partitions
+    (7, 1024, 608, 4, 2, "e2m1"),     # 4-bit weights; 24 partitions behind a full intermediate tile
+    (40, 512, 192, 4, 1, "e4m3"),     # chunks of up to 64 rows: weights through registers
+    (40, 512, 160, 3, 1, "e2m1"),
+    (300, 1024, 96, 4, 2, "e4m3"),    # chunks past 64 rows: both operands through LDS
+    (600, 512, 1120, 2, 1, "e4m3"),   # ... of more than 256 rows
+    (500, 512, 544, 2, 1, "e2m1"),
+    (300, 512, 832, 4, 2, "e5m2"),
+])
+@pytest.mark.parametrize("copies", [True, False])
+def test_short_tiles(T, H, I, E, k, fmt, copies):
+    from nkilib.core.moe.moe_cte import _launch
+
+    # (Another seed for the smallest: with 32 intermediate values in all, one that an exponential's last bit moves across the
+    # tie between two e4m3 codes changes by 1/16, and a row of outputs by up to that share of its largest term.  Seed 51 has
+    # such a value, 3.2e-2 off against the oracle in this kernel and in the general kernel alike.)
+    c = mx_case(T, H, I, E, k, 128, seed=61 if I == 32 else 51, bias=True, weight_format=fmt, random_codes=True)
+    want = _golden_mx_options(c, 3, REF_MX_CLAMPS)[:T]
+    was = _launch.mx_weight_copies
+    try:
+        _launch.mx_weight_copies = copies
+        o = from_bf16_tensor(_run_mx_options(c, 3, REF_MX_CLAMPS, False))
+        _check(o[0, :T], want, f"mx short tiles {fmt} T={T} I={I} copies={copies}")
+        if I > 512 and fmt != "e2m1":
+            # what stands in the down weights past the last partition is nothing's input: the bits do not change with it
+            nan = 0x7f  # not a number in both 8-bit formats; a scale of 255 is none either
+            c["down_q"][:, I % 512 // 4:, I // 512] = nan
+            c["down_s"][:, I % 512 // 32:, I // 512] = 255
+            assert np.array_equal(from_bf16_tensor(_run_mx_options(c, 3, REF_MX_CLAMPS, False)), o)
+    finally:
+        _launch.mx_weight_copies = was
+
+
+@pytest.mark.parametrize("T", [20, 300])  # the few-rows and the large-tile kernels
+def test_infinite_rows_with_a_short_tile(T):
+    """A row whose activations overflow reaches the columns that the last tile does not have as well: its own outputs may be
+    anything, every other row keeps its bits."""
+    c = mx_case(T, 512, 96, 4, 2, 128, seed=52, weight_format="e4m3")
+    want = from_bf16_tensor(_run_mx_options(c, 0, None, False))
+    c["hidden"][0] = 3e38
+    o = from_bf16_tensor(_run_mx_options(c, 0, None, False))
+    assert np.array_equal(o[0, 1:T], want[0, 1:T])
