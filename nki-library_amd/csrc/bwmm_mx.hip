@@ -129,8 +129,7 @@ __device__ __forceinline__ void mfma_asm(const v8i& af, const BOp& bf, int sa, i
 template <int STAGE, int NMT, bool LASTUSE, int WFMT>
 __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int (*s_tok)[MX_ROWS_MAX],
                                              float (*s_aff)[MX_ROWS_MAX], float (*s_bias)[MXT],
-                                             float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L, const int startL,
-                                             const int endL, const int Lstep, const int qbase, const int interleave) {
+                                             float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L, int& step, const MxRun& run) {
   using Cfg = MxCfg<NMT>;
   // ROW8: the fp8-row kind.  Same K loop on e4m3 operands with block scales of 2^0; what differs is the epilogue
   // (per-channel weight scale x per-row activation scale ahead of the bias, bias and scales indexed by natural
@@ -156,8 +155,7 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   const int q = w;
 
   typedef MxTileWalk<STAGE, NMT, WFMT> TW;
-  const TW tw{a, s_tok, s_aff, s_bias, s_rs, s_wsc, tid, startL, qbase, interleave, startL / a.col_tiles,
-              (endL - startL) / a.col_tiles};
+  const TW tw{a, s_tok, s_aff, s_bias, s_rs, s_wsc, tid, run};
   const int hcol = (STAGE == 1) ? (c >> 3) : 0, cl = (STAGE == 1) ? (c & 7) : c;
 
   // A staging: thread covers rows (tid>>3) + 32 j; its load goes straight to LDS slot tid&7 of that
@@ -519,8 +517,8 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   }
   aim_loads_at(cur, 0);
   request_first_slices();
-  int Ln = L + Lstep;  // the item after the current one
-  bool have_next = Ln < endL;
+  int Ln = L + step;  // the item after the current one
+  bool have_next = Ln < run.end;
   {
     // (the wait in here also waits for the first slices: once per workgroup and class)
     const MxTile nx = tw.tile_at(have_next ? Ln : L);
@@ -572,9 +570,9 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   // No branch surrounds any of these loads (see above): after the last tile of the list they are issued all the
   // same, the slices through descriptors of zero records (no traffic), the rest from the addresses of the last
   // tile.
-  const bool have_nn = Ln + Lstep < endL;
+  const bool have_nn = L + run.W2 < run.end;
   const MxTile nxt = tw.tile_at(have_next ? Ln : L);
-  const MxTile nn = tw.tile_at(have_nn ? Ln + Lstep : L);
+  const MxTile nn = tw.tile_at(have_nn ? L + run.W2 : L);
   const int nbuf = have_next ? buf ^ 1 : buf;  // (behind the last tile: its own row table, which holds valid ids)
   tile_live = have_next ? -1 : 0;
   aim_loads_at(nxt, nbuf);
@@ -890,10 +888,12 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
   if (have_nn) tw.ids_put(buf, nn.nrows, ids_nn);  // the table of the tile that has just ended
   cur = nxt;
   L = Ln;
-  Ln += Lstep;
+  step = run.W2 - step;
+  Ln += step;
   have_next = have_nn;
   buf ^= 1;
   }
+  step = run.W2 - step;
   return Ln;
 }
 
@@ -922,46 +922,92 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   const int xcd = blockIdx.x & 7, w = blockIdx.x >> 3, W = gridDim.x >> 3;
   // (for a caller that wants to know the clock the part held under this launch, see MxArgs::clk)
   const long long clk0 = a.clk ? clock64() : 0, tick0 = a.clk ? wall_clock64() : 0;
-  const int32_t* qo = a.q_off + xcd * (CHUNK_CLASSES + 1);
-  const int qbase = __builtin_amdgcn_readfirstlane(qo[0]);
-  const int interleave = __builtin_amdgcn_readfirstlane(a.q_off[8 * (CHUNK_CLASSES + 1)]);
-  int L = w;
-  // classes in queue order (CHUNK_CLASS_TILES / CHUNK_CLASS_LAST in combine.hpp)
+  // (The queue's offsets, one to a lane of every wave, and kept in LDS, where each wave writes the same values and needs no
+  // barrier to read its own: a round trip to memory per class, nearly all of which hold nothing for a workgroup, made a
+  // launch of one tile per workgroup 113 -> 130 us.)
+  __shared__ int s_q[CHUNK_CLASSES + 2], s_tail;
+  const int lane = threadIdx.x & 63;
+  int q_lane = 0;  // lane c: where class c begins; lane CHUNK_CLASSES: the end; the lane behind: the interleave
+  if (lane <= CHUNK_CLASSES + 1) {
+    q_lane = a.q_off[lane <= CHUNK_CLASSES ? xcd * (CHUNK_CLASSES + 1) + lane : 8 * (CHUNK_CLASSES + 1)];
+    s_q[lane] = q_lane;
+  }
+  MxRun run;
+  run.qbase = __builtin_amdgcn_readlane(q_lane, 0);
+  run.interleave = __builtin_amdgcn_readlane(q_lane, CHUNK_CLASSES + 1);
+  run.W2 = 2 * W;
+  // A last round of at most half of the workgroups: its tiles are cut by rows into two or four pieces, each for a workgroup of its
+  // own (tiles of more than 128 rows, pieces of at least 64: a shorter one takes as long).  Half the rows are 0.65 to 0.75 of a
+  // tile's time, whose loads of weights stay.  (Not with interleaved chunks, whose items' order follows from the class.)  A layer
+  // before | with this and the instances below, us: 1999 tokens, top-4 of 32 MXFP4 experts of H = 3072, I = 1536, 384 tiles for
+  // 256 workgroups 198 | 181; 447, top-5 of 8 bf16 experts of 6144, 256 197 | 143; 377, top-3 of 4 MXFP4 experts of 5120, 640
+  // 126 | 96; 222, top-4 of 4 bf16 experts of 6144, 128 179 | 119.
+  const int total = (__builtin_amdgcn_readlane(q_lane, CHUNK_CLASSES) - run.qbase) * a.col_tiles;
+  const int round = total / W, rest = total - round * W;
+  const int shift = (run.interleave > 1 || rest == 0 || 2 * rest > W) ? 0 : 4 * rest > W ? 1 : 2;
+  const int whole = shift ? round * W : total;
+  run.cut = whole << 2 | shift;
+  int L = w, step = 2 * (W - 1 - w) + 1;
+  constexpr int NO_CLASS = CHUNK_CLASSES;
   // (Chunks of up to 64 rows are a stream of weights, for which three slices ahead in registers beat two stages in LDS.
   // mx_gemm_tiles on 4 row tiles | mx_gemm_tiles_wide on 8, gate/up + down, us: MXFP8, 256 experts of H = 7168, I = 2048 with
   // 16 rows each 1123 + 637 | 1155 + 663, with 64 1216 + 685 | 1236 + 697; 128 of 2048, 768 with 64 rows 85 + 56 | 90 + 59;
   // MXFP4, 64 of 7168, 2048 with 16 rows 170 + 103 | 215 + 133, with 64 214 + 109 | 232 + 137; bf16, 64 of 4096, 2048 with
   // 64 rows 390 + 189 | 397 + 192; fp8-row, the same 206 + 104 | 209 + 110.)
-#define MX_RUN_TILES(TILES_, LAST_)                                                                               \
-  if constexpr ((TILES_) >= 8)                                                                                   \
-    L = mx_gemm_tiles_wide<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, \
-                                                           (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave); \
-  else                                                                                                           \
-    L = mx_gemm_tiles<STAGE, (TILES_), (LAST_), WFMT>(a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs,  \
-                                                      (float(*)[MXT])s_wsc, L, startL, endL, W, qbase, interleave);
-#define MX_RUN_CLASS(CLS_)                                                                                     \
-  {                                                                                                            \
-    const int startL = (__builtin_amdgcn_readfirstlane(qo[CLS_]) - qbase) * a.col_tiles;                       \
-    const int endL = (__builtin_amdgcn_readfirstlane(qo[CLS_ + 1]) - qbase) * a.col_tiles;                     \
-    if (L < endL) {                                                                                            \
-      MX_RUN_TILES(CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_])                                              \
-    }                                                                                                          \
-    __syncthreads();                                                                                           \
+  auto aim_at_class_of = [&](int l) {
+    const int ln = threadIdx.x & 63;
+    const int q = s_q[ln <= CHUNK_CLASSES ? ln : 0];
+    const int c = __builtin_popcountll(__ballot(ln >= 1 && ln < CHUNK_CLASSES && l >= (q - run.qbase) * a.col_tiles));
+    run.pos0 = __builtin_amdgcn_readlane(q, c) - run.qbase;
+    run.npos = __builtin_amdgcn_readlane(q, c + 1) - run.qbase - run.pos0;
+    return c;
+  };
+  // the instance that the workgroup's piece of the last round takes, one of the smallest three: none ahead of its tile's class
+  {
+    int inst = NO_CLASS;
+    const int p = (round & 1) ? W - 1 - w : w;
+    if (shift && p < rest << shift) {
+      run.pos0 = run.npos = 0;
+      const int rows = MxTileWalk<STAGE, 8, WFMT>{a, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc,
+                                                  (int)threadIdx.x, run}.tile_at(whole + p).nrows;
+      if (rows > 0) inst = chunk_class(rows, true);
+    }
+    s_tail = inst;  // (every wave the same)
   }
-  // The same for a run of neighbouring classes on one instance of the tile loop (whose row tiles cover the largest).
-#define MX_RUN_RANGE(C0_, C1_, TILES_, LAST_)                                                                  \
-  {                                                                                                            \
-    static_assert(CHUNK_CLASS_TILES[C0_] <= TILES_ && CHUNK_CLASS_LAST[C0_] == LAST_ &&                        \
-                  CHUNK_CLASS_LAST[C1_] == LAST_, "the instance covers the classes of the run");              \
-    const int startL = (__builtin_amdgcn_readfirstlane(qo[C0_]) - qbase) * a.col_tiles;                        \
-    const int endL = (__builtin_amdgcn_readfirstlane(qo[C1_ + 1]) - qbase) * a.col_tiles;                      \
-    if (L < endL) {                                                                                            \
-      MX_RUN_TILES(TILES_, LAST_)                                                                              \
-    }                                                                                                          \
-    __syncthreads();                                                                                           \
-  }
-  static_assert(CHUNK_CLASSES == 12, "one MX_RUN_CLASS per class");
-  if constexpr (WFMT == MX_WFMT_E4M3) {
+  // What the workgroup runs next: its items of the class that holds item L, and its piece as well where the same instance takes
+  // it, or the piece alone; NO_CLASS at the end.
+  auto next_run = [&]() {
+    const int tail = __builtin_amdgcn_readfirstlane(s_tail);
+    const int whole = run.cut >> 2;
+    if (L < whole) {
+      const int c = aim_at_class_of(L);
+      // (the piece lies behind the workgroup's last whole item, in whose class or a later one its tile is)
+      const int end = (run.pos0 + run.npos) * a.col_tiles;
+      run.end = c == tail ? whole + W : end < whole ? end : whole;
+      return c;
+    }
+    run.end = whole + W;
+    return L < run.end ? tail : NO_CLASS;
+  };
+  // The instances one behind the other (in a loop over them the compiler keeps values of one in registers through all the
+  // others), entered at the first that the workgroup needs and left behind its last: every one that is only stepped over
+  // costs a fetch of code.
+  int next = next_run();
+#define MX_RUN_CLASS(CLS_)                                                                                             \
+  case CLS_:                                                                                                           \
+    if (next == CLS_) {                                                                                                \
+      if constexpr (CHUNK_CLASS_TILES[CLS_] >= 8)                                                                      \
+        L = mx_gemm_tiles_wide<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT>(                          \
+            a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc, L, step, run);           \
+      else                                                                                                             \
+        L = mx_gemm_tiles<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT>(                               \
+            a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc, L, step, run);           \
+      __syncthreads();                                                                                                 \
+      next = next_run();                                                                                               \
+    }                                                                                                                  \
+    if (next == NO_CLASS) break;                                                                                       \
+    [[fallthrough]];
+  switch (next) {
     MX_RUN_CLASS(0)
     MX_RUN_CLASS(1)
     MX_RUN_CLASS(2)
@@ -974,21 +1020,9 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     MX_RUN_CLASS(9)
     MX_RUN_CLASS(10)
     MX_RUN_CLASS(11)
-  } else {
-    // Every other format runs the last chunks of 10 .. 18 row tiles on the instances of 16 and 20: the finer
-    // classes pay where experts hold a router's ragged 256 +- 15 rows (the e4m3 workloads that are timed), and
-    // each instance costs this file a twelfth of its compile time.
-    MX_RUN_RANGE(0, 0, 20, false)
-    MX_RUN_RANGE(1, 2, 20, true)
-    MX_RUN_RANGE(3, 3, 16, false)
-    MX_RUN_RANGE(4, 7, 16, true)
-    MX_RUN_RANGE(8, 8, 8, false)
-    MX_RUN_RANGE(9, 9, 8, true)
-    MX_RUN_RANGE(10, 10, 4, false)
-    MX_RUN_RANGE(11, 11, 4, true)
+    default: break;
   }
-#undef MX_RUN_RANGE
-#undef MX_RUN_TILES
+  static_assert(CHUNK_CLASSES == 12, "one MX_RUN_CLASS per class");
 #undef MX_RUN_CLASS
   if (a.clk && blockIdx.x == 0 && threadIdx.x == 0) {
     a.clk[0] = clock64() - clk0;
@@ -1098,7 +1132,7 @@ int launch_mx_gemm(int stage, const MxArgs& m0, unsigned gx, unsigned gy, hipStr
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
     return MOE_E_LAUNCH;
-  const uint64_t tiles = (uint64_t)gx * gy;
+  const uint64_t tiles = 4 * (uint64_t)gx * gy;  // (or pieces of them, see mx_gemm_kernel)
   unsigned per_xcd = (unsigned)cus / 8u;
   if ((tiles + 7u) / 8u < per_xcd) per_xcd = (unsigned)((tiles + 7u) / 8u);
   const unsigned grid = 8u * per_xcd;

@@ -129,9 +129,8 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
   // equal chunks of 8 to 16 row tiles on the present loop put it at 36 (gate/up, MXFP8, 256 experts of H = 7168, I = 2048:
   // 1377 us at 8 row tiles, 1626 at 16), 17 (its down stage: 745, 989), 29 and 18 (128 experts of H = 2048, I = 768: 93 and
   // 113, 63 and 83); past 16 a row tile costs 1.1 to 2.3 times as much (1912 and 1124, 128 and 98 at 20).  No one number
-  // fits both stages of a layer, whose chunks are the same, and this one lies between them.  Formats other than e4m3 run
-  // 10 to 14 row tiles on the instance of 16, which is not counted here.)
-  auto work_of = [&](int i) { return chunk_row_tiles(rows_of(i), true) + CHUNK_FIXED_COST_TILES; };
+  // fits both stages of a layer, whose chunks are the same, and this one lies between them.)
+  auto work_of = [&](int i) { return chunk_row_tiles(rows_of(i)) + CHUNK_FIXED_COST_TILES; };
   int wcarry = 0;
   for (int i0 = 0; i0 < n; i0 += (int)blockDim.x) {
     const int i = i0 + threadIdx.x;
@@ -149,11 +148,15 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
   }
   __threadfence_block();
   __syncthreads();
-  // (interleaved chunks share their weight tiles through the L2: none of them streams the weights past it, so
-  // "last chunk of its expert" is no class of its own then)
+  // (interleaved chunks share their weight tiles through the L2: none of them streams the weights past it, whether last of
+  // its expert or not)
   auto key_of = [&](int i) {
     const bool last = interleave == 1 && ((i + 1 >= n) || (chunk_expert_of(i + 1) != chunk_expert_of(i)));
-    return xcd_of(i) * CHUNK_CLASSES + chunk_class(rows_of(i), last);
+    // (with checkpoints, i.e. pad_row, chunks of 18 row tiles run on the instance of 20: its waves' shares of the checkpoint's
+    // columns end at multiples of 64 bytes, and the gate/up launch of T = 1024, top-4 of 8 bf16 experts of H = 3072, I = 2048
+    // takes 117 us instead of 127)
+    const int cls = chunk_class(rows_of(i), last);
+    return xcd_of(i) * CHUNK_CLASSES + (pad_row && CHUNK_CLASS_TILES[cls] == 18 ? cls - 2 : cls);
   };
   __shared__ uint8_t s_key[KEYS_IN_LDS];  // the chunks' keys, for the rank loop below
   for (int i = threadIdx.x; i < n; i += blockDim.x) {

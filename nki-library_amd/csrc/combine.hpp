@@ -31,27 +31,29 @@ struct Bookkeeping {
 };
 
 // Classes of chunks = instances of the large-tile kernels' tile loop: how many 16-row tiles the instance multiplies
-// (at least the chunk's rows / 16) and whether the chunk is the last one of its expert (its weights are then
-// streamed past the L2).  Last chunks, which carry an expert's ragged remainder, choose among eight row-tile counts,
-// so that at most one or two tiles of a chunk multiply padding (a router's 256 +- 15 rows per expert made one MFMA in
-// eight multiply padding with the counts 4 / 8 / 16 / 20 alone); chunks that are not the last of their expert hold
-// exactly CHUNK_ROWS rows unless chunks are interleaved (see build_chunks), and choose among four.  Queue order =
-// class order: largest tiles first, so that a launch ends on its small ones.
+// (at least the chunk's rows / 16) and whether it streams the weights past the L2, as nobody asks for them again: the last
+// chunk of an expert.  It carries the expert's ragged remainder and chooses among eight row-tile counts, so that at most one
+// or two tiles of a chunk multiply padding (a router's 256 +- 15 rows per expert made one MFMA in eight multiply padding with the
+// counts 4 / 8 / 16 / 20 alone); the others hold exactly CHUNK_ROWS rows.  (What streaming is worth, a layer without it | with it |
+// with it for every chunk: 8192 tokens, top-8 of 128 MXFP8 experts of H = 2048, I = 768, popular and unpopular ones 529 |
+// 503 | 511 us; 3191, one of 64 of 6656, 1536 499 | 462 | 489; 10240, top-4 of 128 bf16 experts of 3072, 192 427 | 393 | 396.
+// Where several chunks of an expert work on the same weight tile at a time (interleaved, see build_chunks) none of them streams:
+// with streaming ones among them the down launch of 3740 tokens, top-8 of 16 fp8-row experts of H = 4608, I = 256 took 117 us
+// instead of 98.  Such runs have fewer sizes to choose from.)
+// Queue order = class order: largest tiles first, so that a launch ends on its small ones.
 constexpr int CHUNK_CLASSES = 12;
-constexpr int CHUNK_CLASS_TILES[CHUNK_CLASSES] = {20, 20, 18, 16, 16, 14, 12, 10, 8, 8, 4, 4};
-constexpr bool CHUNK_CLASS_LAST[CHUNK_CLASSES] = {false, true, true, false, true, true, true, true, false, true, false, true};
+constexpr int CHUNK_CLASS_TILES[CHUNK_CLASSES] = {20, 20, 18, 18, 16, 16, 14, 12, 10, 8, 8, 4};
+constexpr bool CHUNK_CLASS_LAST[CHUNK_CLASSES] = {false, true, false, true, false, true, true, true, true, false, true, true};
+constexpr int CHUNK_ROWS = 256;      // rows of every chunk of a run but the last
 // 16-row tiles of the instance that runs a chunk of `rows` rows
-__host__ __device__ inline int chunk_row_tiles(int rows, bool last) {
-  if (!last) return rows <= 64 ? 4 : rows <= 128 ? 8 : rows <= 256 ? 16 : 20;
-  return rows <= 64 ? 4 : rows <= 128 ? 8 : 2 * ((rows + 31) / 32);
-}
-__host__ __device__ inline int chunk_class(int rows, bool last) {
-  const int t = chunk_row_tiles(rows, last);
-  if (!last) return t == 20 ? 0 : t == 16 ? 3 : t == 8 ? 8 : 10;
-  return t == 20 ? 1 : t == 18 ? 2 : t == 16 ? 4 : t == 14 ? 5 : t == 12 ? 6 : t == 10 ? 7 : t == 8 ? 9 : 11;
+__host__ __device__ inline int chunk_row_tiles(int rows) { return rows <= 64 ? 4 : rows <= 128 ? 8 : 2 * ((rows + 31) / 32); }
+// (`stream`: false for a chunk whose weights another chunk will ask for)
+__host__ __device__ inline int chunk_class(int rows, bool stream) {
+  const int t = chunk_row_tiles(rows);
+  if (!stream) return t == 20 ? 0 : t == 18 ? 2 : t >= 10 ? 4 : 9;
+  return t == 20 ? 1 : t == 18 ? 3 : t == 16 ? 5 : t == 14 ? 6 : t == 12 ? 7 : t == 10 ? 8 : t == 8 ? 10 : 11;
 }
 
-constexpr int CHUNK_ROWS = 256;      // rows of every chunk of a run but the last
 constexpr int CHUNK_FIXED_COST_TILES = 20;  // a chunk's loads per K slice, in row tiles of MFMA time (XCD balance, chunks.hpp)
 constexpr int CHUNK_ROWS_MAX = 320;  // the last chunk of a run takes up to this many
 inline int64_t max_chunks_for(int64_t N, int64_t B) { return N * ((B + CHUNK_ROWS - 1) / CHUNK_ROWS); }

@@ -126,7 +126,25 @@ struct MxTile {
   int nrows, e, slot0, xt;
 };
 
-// One class of a launch's tiles: items startL .. endL of the XCD's queue.
+// A run of a workgroup's items on one instance of a tile loop.  The items of an XCD's queue go to its W workgroups in rounds of W,
+// every other round in reverse: of a queue in order of falling size the workgroup with the largest of one round gets the
+// smallest of the next (in the same order every round, the first workgroups got the largest of all of them.  A layer with the same
+// order every round | in turns, us: 540 tokens, top-3 of 32 bf16 experts of H = 4096, I = 4096 735 | 692; 83, top-5 of 64 of 6144,
+// 1024 427 | 390; 8192, top-8 of 128 MXFP8 experts of 2048, 768 518 | 513; 3191, one of 64 of 6656, 1536 493 | 497).
+// (Few words: they are live in scalar registers through the tile loops, whose epilogues have none to spare.)
+struct MxRun {
+  int end;  // the run ends ahead of this item
+  int W2;   // 2 W: from an item of the workgroup's to the one after the next
+  int qbase, interleave;
+  int pos0, npos;  // the chunks of the class: first place in the queue, number
+  int cut;  // whole << 2 | shift: items from `whole` on are pieces, 1 << shift of a tile, equal parts of its chunk's rows
+  __device__ __forceinline__ static int rows_per_piece(int rows, int shift) {
+    const int per = (((rows + (1 << shift) - 1) >> shift) + 31) & ~31;
+    return rows <= 128 ? rows : per < 64 ? 64 : per;
+  }
+};
+
+// The tiles of a run.
 template <int STAGE, int NMT, int WFMT>
 struct MxTileWalk {
   // ROW8: the fp8-row kind (and the bf16 kind): per-channel weight scale x per-row activation scale ahead of the bias,
@@ -140,7 +158,8 @@ struct MxTileWalk {
   float (*s_bias)[MXT];
   float (*s_rs)[MX_ROWS_MAX];  // (token entries for the MX formats)
   float (*s_wsc)[MXT];
-  int tid, startL, qbase, interleave, pos0, npos;
+  int tid;
+  const MxRun& run;
 
   // ---- tiles ------------------------------------------------------------------------------------
   // Everything that says which tile: uniform values, kept in scalar registers.  A tile's queue entry (two words)
@@ -151,28 +170,32 @@ struct MxTileWalk {
   // group of G queue positions the chunk varies fastest, so that workgroups with neighbouring items work on the
   // same column tile of different chunks (of one expert: they share the weight tile); G = 1 is column tiles
   // innermost.  The last group of a class may hold fewer than G chunks.
-  // (items are numbered through the XCD's whole queue; the class's own run from startL to endL)
-  __device__ __forceinline__ auto tile_at(int l) const {
+  // (items are numbered through the XCD's whole queue)
+  __device__ __forceinline__ auto tile_at(int l0) const {
     int pos, xt;
-    if (interleave == 1) {
+    const int whole = run.cut >> 2, shift = run.cut & 3, over = l0 - whole;
+    const int l = over < 0 ? l0 : whole + (over >> shift);
+    if (run.interleave == 1) {
       pos = l / a.col_tiles;
       xt = l - pos * a.col_tiles;
     } else {
-      const int per_group = interleave * a.col_tiles;
-      const int lr = l - startL;
+      const int per_group = run.interleave * a.col_tiles;
+      const int lr = l - run.pos0 * a.col_tiles;
       const int grp = lr / per_group, j = lr - grp * per_group;
-      const int base = grp * interleave;
-      const int G = (npos - base < interleave) ? npos - base : interleave;
+      const int base = grp * run.interleave;
+      const int G = (run.npos - base < run.interleave) ? run.npos - base : run.interleave;
       xt = j / G;
-      pos = pos0 + base + (j - xt * G);
+      pos = run.pos0 + base + (j - xt * G);
     }
     v2i raw;
     asm volatile(MX_SGPR_WAIT "s_load_dwordx2 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)"
-                 : "=s"(raw) : "s"(a.q_chunk), "s"((qbase + pos) * 8) : "memory");
+                 : "=s"(raw) : "s"(a.q_chunk), "s"((run.qbase + pos) * 8) : "memory");
     MxTile t;
     t.xt = xt;
-    t.slot0 = raw[0];
-    t.nrows = raw[1] & 0xffff;
+    const int rows = raw[1] & 0xffff, per = over < 0 ? rows : MxRun::rows_per_piece(rows, shift);
+    const int row0 = over < 0 ? 0 : (over & ((1 << shift) - 1)) * per;
+    t.slot0 = raw[0] + row0;
+    t.nrows = rows - row0 < per ? rows - row0 : per;
     t.e = raw[1] >> 16;
     return t;
   }

@@ -130,9 +130,7 @@ __device__ __forceinline__ void st_b128_plain(const v4i& d, uint32_t voff, const
 template <int STAGE, int NMT, bool LASTUSE, int WFMT>
 __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem, int (*s_tok)[MX_ROWS_MAX],
                                                   float (*s_aff)[MX_ROWS_MAX], float (*s_bias)[MXT],
-                                                  float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L,
-                                                  const int startL, const int endL, const int Lstep, const int qbase,
-                                                  const int interleave) {
+                                                  float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L, int& step, const MxRun& run) {
   static_assert(NMT >= 8 && NMT % 2 == 0, "at least four row tiles per wave");
   using Cfg = MxWideCfg<NMT>;
   constexpr bool BF16 = WFMT == MX_WFMT_BF16;
@@ -149,8 +147,7 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   const int wm = w >> 1, wn = w & 1;
   const int nH = (int)(a.H / 512);
   typedef MxTileWalk<STAGE, NMT, WFMT> TW;
-  const TW tw{a, s_tok, s_aff, s_bias, s_rs, s_wsc, tid, startL, qbase, interleave, startL / a.col_tiles,
-              (endL - startL) / a.col_tiles};
+  const TW tw{a, s_tok, s_aff, s_bias, s_rs, s_wsc, tid, run};
 
   // ---- columns ------------------------------------------------------------------------------------------------
   // Position Q = (wn, column tile tt, piece gq) of a 4-column piece among the workgroup's 64; a lane of group g ends up
@@ -471,6 +468,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   // The loads a tile starts on, numbered in issue order (so that a part of them can be asked for at a time): scales of the
   // first four slices, slices 0 and 1 (the second part of slice 1's activations is requested by slice 0).
   constexpr int NFIRST = 1 + NW + NAJ + NW + NA1;
+  constexpr int NFIRST_LOADS = NFIRST - 1 + NAS;  // instructions (the scales are none, one or two)
+  static_assert(NFIRST_LOADS < 64, "the counter of outstanding memory instructions");
   auto request_first = [&](auto n0_, auto n1_) {
     static_for<decltype(n0_)::value, (decltype(n1_)::value < NFIRST ? decltype(n1_)::value : NFIRST)>([&](auto n_) {
       constexpr int n = decltype(n_)::value;
@@ -497,31 +496,42 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   };
 
   // ---- first tile: nothing is in flight yet, so plain waits do --------------------------------------------------
+  // (every round trip to memory is a microsecond of the launch: what does not depend on the token ids goes out with them, in the
+  // down stage the first slices, whose rows are slots)
   MxTile cur = tw.tile_at(L);
   int ids_nn[2] = {0, 0}, aff_n[2] = {0, 0}, bias_n = 0;  // requested ahead of an epilogue, put in place after it
   int rs_n[2] = {0, 0}, wsc_n = 0;                          // (fp8-row and bf16 kinds only)
+  auto first_slices = [&]() {
+    aim_loads_at(cur, 0);
+    request_first(std::integral_constant<int, 0>{}, std::integral_constant<int, NFIRST>{});
+  };
   tw.ids_raw(cur, ids_nn);
   tw.bias_raw(cur, bias_n);
   tw.wsc_raw(cur, wsc_n);
-  tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  if constexpr (STAGE == 2) {
+    first_slices();
+    tw.template loads_landed<NFIRST_LOADS>(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  } else {
+    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  }
   tw.ids_put(0, cur.nrows, ids_nn);
   tw.bias_put(cur, 0, bias_n);
   tw.wsc_put(cur, 0, wsc_n);
-  __syncthreads();
+  lds_barrier();
   if (TW::AFF_ROWS) {
     tw.aff_raw(cur, 0, aff_n);
     tw.rs_raw(cur, 0, rs_n);
-    tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
-    if (STAGE == 2) tw.aff_put(cur.e, 0, aff_n);
-    tw.rs_put(cur.e, 0, rs_n, aff_n);
   }
-  aim_loads_at(cur, 0);
-  request_first(std::integral_constant<int, 0>{}, std::integral_constant<int, NFIRST>{});
-  int Ln = L + Lstep;  // the item after the current one
-  bool have_next = Ln < endL;
+  if constexpr (STAGE == 1) first_slices();
+  int Ln = L + step;  // the item after the current one
+  bool have_next = Ln < run.end;
   MxTile nxt = tw.tile_at(have_next ? Ln : L);
   tw.ids_raw(nxt, ids_nn);
   tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
+  if (TW::AFF_ROWS) {
+    if (STAGE == 2) tw.aff_put(cur.e, 0, aff_n);
+    tw.rs_put(cur.e, 0, rs_n, aff_n);
+  }
   if (have_next) tw.ids_put(1, nxt.nrows, ids_nn);  // published by the barrier below
   int buf = 0;  // which of the two row tables belongs to the current tile
   auto zero_accumulators = [&]() {
@@ -533,8 +543,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       for (int j = 0; j < 8; ++j) accv[i][j] = (v4f){0.f, 0.f, 0.f, 0.f};
   };
   zero_accumulators();
-  bool have_nn = Ln + Lstep < endL;
-  MxTile nn = tw.tile_at(have_nn ? Ln + Lstep : L);  // the tile after the next one
+  bool have_nn = L + run.W2 < run.end;
+  MxTile nn = tw.tile_at(have_nn ? L + run.W2 : L);  // the tile after the next one
 
   for (;;) {
     // (what the tile's first slice needs has landed: every wave has waited for its own loads)
@@ -692,10 +702,87 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       const uint32_t ys_voff = (g_e & 1) ? 0xffffffffu : (uint32_t)(row0 * ys_rowb + tI * 16 + (pl >> 3));
       // dense kinds: natural column of the lane's first value of quarter 2 wn + j
       auto nat_col = [&](int j) { return tI * 512 + (2 * wn + j) * Pt + p0 + (BF16 ? 8 : 4) * g_e; };
-      // activation checkpoint [N, 2, I, B] (bwmm_shard_on_I.py:160-176): a block's gate or up half is less than 4 GiB (the
-      // call's intermediate rows are), so 32 bits hold an offset inside a half, and which half is a matter of 64 bits
-      const uint32_t ck_B = BF16 ? (uint32_t)a.ckpt_B : 1u;
-      const uint32_t ck_half = BF16 ? (uint32_t)a.ckpt_I * ck_B * 2u : 0u;  // bytes
+      // Activation checkpoint [N, 2, I, B] (bwmm_shard_on_I.py:160-176), bf16 kind: gate / up projections after scale, bias and
+      // clamp, transposed, ahead of the results' pass.  Up to 64 of the wave's rows x a quarter's 32 columns at a time go through
+      // its 4 KB of LDS, column by column, and leave as 16-byte pieces of 8 rows, eight of them side by side (in blocks of a
+      // multiple of 8 rows; row by row otherwise).  (Stored from the registers 4 bytes at a time, in every activation's copy of
+      // the results' pass: a layer of 1024 tokens, top-4 of 8 experts of H = 3072, I = 2048 243 us, now 241, and half of this
+      // file's compile time; without streaming stores 247.)  A block's gate or up half is less than 4 GiB (the call's
+      // intermediate rows are), so 32 bits hold an offset inside a half, and which half is a matter of 64 bits.
+      auto ckpt_pass = [&]() {
+        if constexpr (BF16) {
+          const uint32_t ck_B = (uint32_t)a.ckpt_B, ck_half = (uint32_t)a.ckpt_I * ck_B * 2u;  // bytes
+          const bool whole = (ck_B & 7) == 0 && (uni((int)(uintptr_t)a.ckpt) & 15) == 0;
+          static_for<0, 2>([&](auto j_) {
+            constexpr int j = decltype(j_)::value;
+            const PairTab tab[2] = {pair_tab(2 * j), pair_tab(2 * j + 1)};
+            const int col0 = tI * 512 + (2 * wn + j) * Pt + p0;  // the quarter's first column
+            static_for<0, (RT + 3) / 4>([&](auto grp_) {
+              constexpr int r0 = 4 * decltype(grp_)::value, nr = RT - r0 < 4 ? RT - r0 : 4;
+              if ((wm * RT + r0) * 16 >= cur.nrows) return;
+              // the lane's piece when they leave: column 8 k + lane / 8, rows 8 (lane % 8) ..
+              const int unit = lane_e & 7, row = (wm * RT + r0) * 16 + 8 * unit;
+              const uint32_t slot = (uint32_t)(cur.slot0 + row);
+              const int rows = unit < 2 * nr ? cur.nrows - row : 0;  // of the piece, rows that exist (8 and more: all)
+              static_for<0, 2>([&](auto gu_) {
+                constexpr int gu = decltype(gu_)::value;
+                const float lo = gu ? u_lo : g_lo, hi = gu ? u_hi : g_hi;
+                static_for<0, nr>([&](auto i_) {
+                  constexpr int i = decltype(i_)::value;
+                  const float rs = s_rs[buf][row0 + (r0 + i) * 16];
+                  float v[8];  // columns 8 g_e .. 8 g_e + 7 of the quarter
+                  static_for<0, 2>([&](auto h_) {
+                    constexpr int h = decltype(h_)::value;
+                    float x[4];
+                    acc_of(std::integral_constant<int, r0 + i>{}, std::integral_constant<int, 2 * (2 * j + h) + gu>{}, x);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                      v[4 * h + r] = __builtin_amdgcn_fmed3f((x[r] * (gu ? tab[h].su : tab[h].sg)[r]) * rs + (gu ? tab[h].bu : tab[h].bg)[r], lo, hi);
+                  });
+                  // neighbouring lanes hold neighbouring rows: the even one takes the first four columns for both, the odd one
+                  // the last four
+                  const int odd = c_e & 1;
+#pragma unroll
+                  for (int k = 0; k < 4; ++k) {
+                    const float own = odd ? v[4 + k] : v[k], give = odd ? v[k] : v[4 + k];
+                    const float got = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true));
+                    const int col = 8 * g_e + 4 * odd + k, u = (2 * i + (c_e >> 3)) ^ (2 * g_e + odd);
+                    *(uint32_t*)(ex + col * 128 + u * 16 + ((c_e >> 1) & 3) * 4) = odd ? pack2_bf16(got, own) : pack2_bf16(own, got);
+                  }
+                });
+                asm volatile("" ::: "memory");
+                v4i d[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                  const int col = 8 * k + (lane_e >> 3);
+                  d[k] = *(const v4i*)(ex + col * 128 + (unit ^ (col >> 2)) * 16);
+                }
+                const int ccol = col0 + (lane_e >> 3);
+                if (whole && rows >= 8) {
+                  const uint32_t n = slot / ck_B, rr = slot - n * ck_B;
+                  uint8_t* const at = (uint8_t*)a.ckpt + (uint64_t)(2u * n + gu) * ck_half + ((uint32_t)ccol * ck_B + rr) * 2u;
+#pragma unroll
+                  for (int k = 0; k < 4; ++k)
+                    if (ccol + 8 * k < (int)a.ckpt_I) __builtin_nontemporal_store(d[k], (v4i*)(at + (uint32_t)(8 * k) * ck_B * 2u));
+                } else {
+#pragma clang loop unroll(disable)
+                  for (int r = 0; r < (rows < 8 ? rows : 8); ++r) {
+                    const uint32_t n = (slot + r) / ck_B, rr = slot + r - n * ck_B;
+                    uint8_t* const at = (uint8_t*)a.ckpt + (uint64_t)(2u * n + gu) * ck_half + ((uint32_t)ccol * ck_B + rr) * 2u;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                      const int w01 = (r & 2) ? d[k][1] : d[k][0], w23 = (r & 2) ? d[k][3] : d[k][2];
+                      const uint32_t word = (uint32_t)((r & 4) ? w23 : w01) >> (16 * (r & 1));
+                      if (ccol + 8 * k < (int)a.ckpt_I) *(uint16_t*)(at + (uint32_t)(8 * k) * ck_B * 2u) = (uint16_t)word;
+                    }
+                  }
+                }
+                asm volatile("" ::: "memory");
+              });
+            });
+          });
+        }
+      };
       auto passes = [&](auto act_, auto plain_) {
         constexpr int ACT = decltype(act_)::value;
         constexpr bool PLAIN = decltype(plain_)::value;
@@ -785,38 +872,6 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
                                pack2(y[1][0], y[1][1]) & y_live[2], pack2(y[1][2], y[1][3]) & y_live[3]};
                 if constexpr (rt > 0) store(rt - 1);
                 ex_put(g_e, o);
-                if (!PLAIN && a.ckpt != nullptr) {
-                  // the checkpoint takes gate / up projections after scale, bias and clamp, transposed.  Neighbouring lanes
-                  // hold neighbouring rows: where the block size is even (two rows then share a block and an aligned
-                  // word) the even lane takes the first four of the eight columns for both rows, the odd one the last
-                  // four; otherwise every lane stores its own row
-                  const int odd = c_e & 1;
-                  const bool pair = (ck_B & 1) == 0;
-                  const int row = row0 + rt * 16 - (pair ? odd : 0);
-                  const uint32_t slot = (uint32_t)(cur.slot0 + row), n = slot / ck_B, rr = slot - n * ck_B;
-                  const int ccol0 = nat_col(j) + (pair ? 4 * odd : 0);
-                  const int live = row < cur.nrows ? (int)a.ckpt_I - ccol0 : 0;  // columns from ccol0 on that exist
-                  uint8_t* const ck_gate = (uint8_t*)a.ckpt + (uint64_t)(2u * n) * ck_half;
-                  const uint32_t off0 = ((uint32_t)ccol0 * ck_B + rr) * 2u;
-                  static_for<0, 2>([&](auto gu_) {
-                    constexpr int gu = decltype(gu_)::value;
-                    const float (&v)[2][4] = gu ? uu : gg;
-                    uint8_t* const ck = gu ? ck_gate + ck_half : ck_gate;
-                    if (pair) {
-#pragma unroll
-                      for (int k = 0; k < 4; ++k) {
-                        const float own = odd ? v[1][k] : v[0][k], give = odd ? v[0][k] : v[1][k];
-                        const float got = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, give), 0xb1 /* quad_perm 1 0 3 2 */, 0xf, 0xf, true));
-                        const uint32_t word = odd ? pack2_bf16(got, own) : pack2_bf16(own, got);
-                        if (k < live) *(uint32_t*)(ck + (off0 + k * ck_B * 2u)) = word;
-                      }
-                    } else {
-#pragma unroll
-                      for (int k = 0; k < 8; ++k)
-                        if (k < live) *(uint16_t*)(ck + (off0 + k * ck_B * 2u)) = (uint16_t)pack2_bf16(v[k >> 2][k & 3], 0.f);
-                    }
-                  });
-                }
               } else {
                 if constexpr (rt > 0) store(rt - 1);
 #pragma unroll
@@ -834,7 +889,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       // (the plain form, without bias and clamps, exists for SiLU alone: every instance of this code lengthens the build)
       // (bf16: nor scales; a row without a token is zeros then as it is)
       const bool pre = a.scaling_mode == MOE_SCALE_PRE || a.scaling_mode == MOE_SCALE_PRE_DELAYED;
-      const bool plain = cmask == 0 && a.bias == nullptr && (!BF16 || (a.ckpt == nullptr && a.w_cscale == nullptr && !pre));
+      const bool plain = cmask == 0 && a.bias == nullptr && (!BF16 || (a.w_cscale == nullptr && !pre));
+      if (BF16 && a.ckpt != nullptr) ckpt_pass();
       switch (a.act_fn) {
         case MOE_ACT_SILU:
           if (plain) passes(std::integral_constant<int, MOE_ACT_SILU>{}, std::true_type{});
@@ -945,8 +1001,8 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
       tw.all_loads_landed(ids_nn, aff_n, bias_n, rs_n, wsc_n);
       break;
     }
-    const bool have_n3 = Ln + 2 * Lstep < endL;
-    const MxTile n3 = tw.tile_at(have_n3 ? Ln + 2 * Lstep : L);
+    const bool have_n3 = Ln + run.W2 < run.end;
+    const MxTile n3 = tw.tile_at(have_n3 ? Ln + run.W2 : L);
     tw.template loads_landed<OUT>(ids_nn, aff_n, bias_n, rs_n, wsc_n);
     if (STAGE == 2) tw.aff_put(nxt.e, buf ^ 1, aff_n);
     tw.rs_put(nxt.e, buf ^ 1, rs_n, aff_n);
@@ -957,11 +1013,13 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
     nxt = nn;
     nn = n3;
     L = Ln;
-    Ln += Lstep;
+    step = run.W2 - step;
+    Ln += step;
     have_next = have_nn;
     have_nn = have_n3;
     buf ^= 1;
   }
+  step = run.W2 - step;
   return Ln;
 }
 
