@@ -1036,9 +1036,7 @@ constexpr int MX_LDS_LAUNCH = MX_INST_WFMT == MX_WFMT_ROW8 || MX_INST_WFMT == MX
                                   ? (MX_LDS > MX_WIDE_LDS_PLAIN ? MX_LDS : MX_WIDE_LDS_PLAIN)
                                   : (MX_LDS > MX_WIDE_LDS_SCALED ? MX_LDS : MX_WIDE_LDS_SCALED);
 int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT)(const MxArgs& m, unsigned grid, hipStream_t s) {
-  const hipError_t err = hipFuncSetAttribute((const void*)mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, MX_LDS_LAUNCH);
-  if (err != hipSuccess) return MOE_E_LAUNCH;
+  if (allow_lds<&mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>>(MX_LDS_LAUNCH) != hipSuccess) return MOE_E_LAUNCH;
   hipLaunchKernelGGL((mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>), dim3(grid), dim3(MXT), MX_LDS_LAUNCH, s, m);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
@@ -1128,10 +1126,8 @@ int launch_mx_gemm(int stage, const MxArgs& m0, unsigned gx, unsigned gy, hipStr
   m.col_tiles = (int32_t)gx;
   // one workgroup per CU (a workgroup fills a CU's registers and most of its LDS, and walks its share of the
   // tiles itself); fewer when there cannot be that many tiles (gy = upper bound on the number of chunks)
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-    return MOE_E_LAUNCH;
+  const int cus = device_cus();
+  if (cus < 8) return MOE_E_LAUNCH;
   const uint64_t tiles = 4 * (uint64_t)gx * gy;  // (or pieces of them, see mx_gemm_kernel)
   unsigned per_xcd = (unsigned)cus / 8u;
   if ((tiles + 7u) / 8u < per_xcd) per_xcd = (unsigned)((tiles + 7u) / 8u);

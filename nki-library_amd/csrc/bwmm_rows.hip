@@ -416,9 +416,7 @@ static int launch_one(const MxArgs& m, int64_t max_chunks, int cus, hipStream_t 
   const int64_t items = max_chunks * m.col_tiles * (4 / Cfg::CG);
   const int64_t resident = (int64_t)cus * (8 / Cfg::NW);
   const unsigned grid = ((unsigned)(items < resident ? items : resident) + 7u) & ~7u;
-  const hipError_t err = hipFuncSetAttribute((const void*)mx_rows_kernel<STAGE, WFMT, MT, CGT, KP>,
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS);
-  if (err != hipSuccess) return MOE_E_LAUNCH;
+  if (allow_lds<&mx_rows_kernel<STAGE, WFMT, MT, CGT, KP>>(Cfg::LDS) != hipSuccess) return MOE_E_LAUNCH;
   hipLaunchKernelGGL((mx_rows_kernel<STAGE, WFMT, MT, CGT, KP>), dim3(grid), dim3(64 * Cfg::NW), Cfg::LDS, s, m);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
@@ -505,10 +503,8 @@ int launch_mx_rows(int stage, const MxArgs& m0, unsigned gx, int64_t max_chunks,
   if (gx == 0 || max_chunks == 0) return MOE_OK;
   MxArgs m = m0;
   m.col_tiles = (int32_t)gx;
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8)
-    return MOE_E_LAUNCH;
+  const int cus = device_cus();
+  if (cus < 8) return MOE_E_LAUNCH;
   switch (m.wfmt) {
     case MX_WFMT_E4M3: return stage == 1 ? launch_rows<1, MX_WFMT_E4M3>(m, rows, max_chunks, cus, s) : launch_rows<2, MX_WFMT_E4M3>(m, rows, max_chunks, cus, s);
     case MX_WFMT_E5M2: return stage == 1 ? launch_rows<1, MX_WFMT_E5M2>(m, rows, max_chunks, cus, s) : launch_rows<2, MX_WFMT_E5M2>(m, rows, max_chunks, cus, s);

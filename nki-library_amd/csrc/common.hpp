@@ -1,6 +1,7 @@
 // Shared device/host helpers for the gfx950 MoE kernels.
 #pragma once
 
+#include <atomic>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -198,5 +199,29 @@ __device__ __forceinline__ float clip448(float v) { return fminf(fmaxf(v, -448.0
 
 // csrc/build_blocks.hip: address of the current device's built-in scratch, looked up once per device
 int build_blocks_static_setup();
+
+// What a launch asks of the runtime and gets the same answer to each time, asked once per device: the dynamic LDS that a kernel may
+// use, the number of CUs.  (The first 64 devices; any further one asks every time.)
+template <auto KERNEL>
+inline hipError_t allow_lds(int bytes) {
+  static std::atomic<uint64_t> done{0};
+  int dev = 0;
+  const hipError_t err = hipGetDevice(&dev);
+  if (err != hipSuccess) return err;
+  const uint64_t bit = dev < 64 ? (uint64_t)1 << dev : 0;
+  if (done.load(std::memory_order_acquire) & bit) return hipSuccess;
+  const hipError_t set = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+  if (set == hipSuccess) done.fetch_or(bit, std::memory_order_release);
+  return set;
+}
+inline int device_cus() {  // 0: unknown
+  static std::atomic<int> known[64];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev < 64) known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
+}
 
 }  // namespace moe

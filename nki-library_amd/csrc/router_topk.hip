@@ -429,8 +429,7 @@ template <int NT, int MT, bool PIPE>
 static int launch_router(const RouterArgs& a, hipStream_t s) {
   const unsigned grid = (unsigned)((a.T + 64 * MT - 1) / (64 * MT));
   const size_t lds = PIPE ? (size_t)3 * 16 * NT * 128 : (size_t)16 * NT * RT_PITCH * 2;
-  hipError_t err = hipFuncSetAttribute((const void*)router_kernel<NT, MT, PIPE>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (err != hipSuccess) return MOE_E_LAUNCH;
+  if (allow_lds<&router_kernel<NT, MT, PIPE>>((int)lds) != hipSuccess) return MOE_E_LAUNCH;
   hipLaunchKernelGGL((router_kernel<NT, MT, PIPE>), dim3(grid), dim3(RT_THREADS), lds, s, a);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
@@ -746,8 +745,7 @@ template <int EG, int TW, int RING>
 static int launch_router_split(const RouterSplitArgs& a, int64_t tiles, hipStream_t s) {
   constexpr int M = 16 * TW * (8 / EG);
   const size_t lds = (size_t)RING * (M + 64 * EG) * 128;
-  hipError_t err = hipFuncSetAttribute((const void*)router_split_kernel<EG, TW, RING>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (err != hipSuccess) return MOE_E_LAUNCH;
+  if (allow_lds<&router_split_kernel<EG, TW, RING>>((int)lds) != hipSuccess) return MOE_E_LAUNCH;
   hipLaunchKernelGGL((router_split_kernel<EG, TW, RING>), dim3((unsigned)(tiles * a.nsplit)), dim3(512), lds, s, a);
   MOE_CHECK_LAUNCH();
   return MOE_OK;

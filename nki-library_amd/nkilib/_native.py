@@ -216,7 +216,8 @@ _DT = {torch.bfloat16: DT_BF16, torch.float16: DT_FP16, torch.float32: DT_FP32}
 
 
 def dtype_code(t, what):
-    kernel_assert(t.dtype in _DT, f"{what} must be bfloat16, float16 or float32 but got {t.dtype}")
+    if not (t.dtype in _DT):
+        kernel_assert(False, f"{what} must be bfloat16, float16 or float32 but got {t.dtype}")
     return _DT[t.dtype]
 
 
@@ -224,12 +225,14 @@ def index_dtype_code(t, what):
     """Element type code for the index operators, which also take int32."""
     if t.dtype == torch.int32:
         return DT_INT32
-    kernel_assert(t.dtype in _DT, f"{what} must be int32, bfloat16, float16 or float32 but got {t.dtype}")
+    if not (t.dtype in _DT):
+        kernel_assert(False, f"{what} must be int32, bfloat16, float16 or float32 but got {t.dtype}")
     return _DT[t.dtype]
 
 
 def require_device_tensor(t, what):
-    kernel_assert(isinstance(t, torch.Tensor), f"{what} must be a torch.Tensor")
+    if not (isinstance(t, torch.Tensor)):
+        kernel_assert(False, f"{what} must be a torch.Tensor")
     if not t.is_cuda:
         raise NativeLibraryError(
             f"{what} lives on {t.device}: these kernels run on an MI355X (ROCm) device only; there is no CPU path"

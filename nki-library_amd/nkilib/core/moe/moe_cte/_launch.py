@@ -132,26 +132,33 @@ def run_blockwise(
     T1, H, I, E = dims["T1"], dims["H"], dims["I"], dims["E"]
     B = int(block_size)
     dev = hidden_states.device
-    kernel_assert(B > 0, f"block_size must be positive, got {B}")
+    if not (B > 0):
+        kernel_assert(False, f"block_size must be positive, got {B}")
 
     tp2id = nv.require_device_tensor(token_position_to_id, "token_position_to_id").reshape(-1)
-    kernel_assert(tp2id.dtype == torch.int32, f"token_position_to_id must be int32 but got {tp2id.dtype}")
-    kernel_assert(tp2id.numel() % B == 0, f"token_position_to_id length {tp2id.numel()} is not a multiple of B={B}")
+    if not (tp2id.dtype == torch.int32):
+        kernel_assert(False, f"token_position_to_id must be int32 but got {tp2id.dtype}")
+    if not (tp2id.numel() % B == 0):
+        kernel_assert(False, f"token_position_to_id length {tp2id.numel()} is not a multiple of B={B}")
     N = tp2id.numel() // B
     b2e = nv.require_device_tensor(block_to_expert, "block_to_expert").reshape(-1)
-    kernel_assert(b2e.dtype == torch.int32, f"block_to_expert must be int32 but got {b2e.dtype}")
-    kernel_assert(b2e.numel() == N, f"block_to_expert must have N={N} entries but got {b2e.numel()}")
+    if not (b2e.dtype == torch.int32):
+        kernel_assert(False, f"block_to_expert must be int32 but got {b2e.dtype}")
+    if not (b2e.numel() == N):
+        kernel_assert(False, f"block_to_expert must have N={N} entries but got {b2e.numel()}")
     cond = None
     if conditions is not None:
         cond = nv.require_device_tensor(conditions, "conditions").reshape(-1)
-        kernel_assert(cond.dtype == torch.int32, f"conditions must be int32 but got {cond.dtype}")
+        if not (cond.dtype == torch.int32):
+            kernel_assert(False, f"conditions must be int32 but got {cond.dtype}")
 
     aff = None
     if expert_affinities_scaling_mode != ExpertAffinityScaleMode.NO_SCALE:
         aff = nv.require_device_tensor(expert_affinities_masked, "expert_affinities_masked")
-        kernel_assert(aff.numel() == T1 * E, f"expert_affinities_masked must hold (T+1)*E={T1 * E} values, got {aff.numel()}")
-        kernel_assert(aff.dtype in (torch.bfloat16, torch.float32),
-                      f"expert_affinities_masked must be bfloat16 or float32 but got {aff.dtype}")
+        if not (aff.numel() == T1 * E):
+            kernel_assert(False, f"expert_affinities_masked must hold (T+1)*E={T1 * E} values, got {aff.numel()}")
+        if not (aff.dtype in (torch.bfloat16, torch.float32)):
+            kernel_assert(False, f"expert_affinities_masked must be bfloat16 or float32 but got {aff.dtype}")
     bias_dt = nv.DT_BF16
     gub = db = None
     if gate_and_up_proj_bias is not None or down_proj_bias is not None:
@@ -162,7 +169,8 @@ def run_blockwise(
         kernel_assert(gub.dtype == db.dtype and gub.dtype in (torch.bfloat16, torch.float32),
                       "bias tensors must both be bfloat16 or both float32")
         bias_dt = nv.DT_BF16 if gub.dtype == torch.bfloat16 else nv.DT_FP32
-        kernel_assert(db.numel() == E * H, f"down_proj_bias must be [E, H] but got {tuple(db.shape)}")
+        if not (db.numel() == E * H):
+            kernel_assert(False, f"down_proj_bias must be [E, H] but got {tuple(db.shape)}")
 
     # the combine stage writes every row of the result (zeros where a token has no contribution) and, through
     # output_shard1, zeros into the second shard slot, which the reference leaves zero after its reduction

@@ -86,7 +86,8 @@ def _blockwise_mm_shard_intermediate_dropping(
         expert_affinities_scaling_mode = ExpertAffinityScaleMode.PRE_SCALE  # bwmm_shard_on_I.py:2084-2085
     E = gate_up_proj_weight.shape[0]
     N = token_position_to_id.numel() // int(block_size)
-    kernel_assert(N == E, f"the dropping layer has one block per expert: N ({N}) must equal E ({E})")
+    if not (N == E):
+        kernel_assert(False, f"the dropping layer has one block per expert: N ({N}) must equal E ({E})")
     own_expert = torch.arange(N, dtype=torch.int32, device=hidden_states.device)
     return run_dense_variant(
         hidden_states, expert_affinities_masked, gate_up_proj_weight, down_proj_weight, block_size,

@@ -33,7 +33,8 @@ def _run(conditions, hidden_states, expert_affinities_masked, gate_up_proj_weigh
     kernel_assert(not (skip_dma or SkipMode()).skip_weight, "DMA weight skipping not supported for MXFP4/MXFP8 kernel")
     if conditions is not None:
         N = token_position_to_id.numel() // block_size
-        kernel_assert(conditions.numel() >= N, f"conditions must hold one entry per block ({N}), got {conditions.numel()}")
+        if not (conditions.numel() >= N):
+            kernel_assert(False, f"conditions must hold one entry per block ({N}), got {conditions.numel()}")
     return _bwmm_shard_on_block_mx(
         hidden_states, expert_affinities_masked, gate_up_proj_weight, down_proj_weight, token_position_to_id,
         block_to_expert, conditions=conditions, gate_and_up_proj_bias=gate_and_up_proj_bias,

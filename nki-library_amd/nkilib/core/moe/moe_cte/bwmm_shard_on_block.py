@@ -25,14 +25,17 @@ def _expand_scale(scale, E, width, what):
     per tensor [1,1,2] / [E,1,2] (gate, up) or [.,1,1], and per channel [.,1,2I] / [.,1,H].
     """
     s = scale.to(torch.float32)
-    kernel_assert(s.dim() == 3 and s.shape[1] == 1, f"{what} must be [E or 1, 1, n] but got {tuple(s.shape)}")
-    kernel_assert(s.shape[0] in (1, E), f"{what} first dimension must be 1 or E={E} but got {s.shape[0]}")
+    if not (s.dim() == 3 and s.shape[1] == 1):
+        kernel_assert(False, f"{what} must be [E or 1, 1, n] but got {tuple(s.shape)}")
+    if not (s.shape[0] in (1, E)):
+        kernel_assert(False, f"{what} first dimension must be 1 or E={E} but got {s.shape[0]}")
     n = s.shape[2]
     if n == width:
         return s.reshape(s.shape[0], width).contiguous()
     if n == 1:
         return s.reshape(s.shape[0], 1).expand(s.shape[0], width).contiguous()
-    kernel_assert(n == 2 and width % 2 == 0, f"{what} last dimension must be 1, 2 or {width} but got {n}")
+    if not (n == 2 and width % 2 == 0):
+        kernel_assert(False, f"{what} last dimension must be 1, 2 or {width} but got {n}")
     return s.reshape(s.shape[0], 2, 1).expand(s.shape[0], 2, width // 2).reshape(s.shape[0], width).contiguous()
 
 
@@ -48,12 +51,13 @@ def run_dense_variant(
     hidden_states = nv.require_device_tensor(hidden_states, "hidden_states")
     guw = nv.require_device_tensor(gate_up_proj_weight, "gate_up_proj_weight")
     dw = nv.require_device_tensor(down_proj_weight, "down_proj_weight")
-    kernel_assert(hidden_states.dim() == 2, f"hidden_states must be [T+1, H] but got {tuple(hidden_states.shape)}")
-    kernel_assert(guw.dim() == 4 and guw.shape[2] == 2,
-                  f"gate_up_proj_weight must be [E, H, 2, I] but got {tuple(guw.shape)}")
+    if not (hidden_states.dim() == 2):
+        kernel_assert(False, f"hidden_states must be [T+1, H] but got {tuple(hidden_states.shape)}")
+    if not (guw.dim() == 4 and guw.shape[2] == 2):
+        kernel_assert(False, f"gate_up_proj_weight must be [E, H, 2, I] but got {tuple(guw.shape)}")
     E, H, _, I = guw.shape
-    kernel_assert(dw.dim() == 3 and dw.shape[0] == E and dw.shape[2] == H and dw.shape[1] >= I,
-                  f"down_proj_weight must be [E, I_padded, H] = [{E}, >={I}, {H}] but got {tuple(dw.shape)}")
+    if not (dw.dim() == 3 and dw.shape[0] == E and dw.shape[2] == H and dw.shape[1] >= I):
+        kernel_assert(False, f"down_proj_weight must be [E, I_padded, H] = [{E}, >={I}, {H}] but got {tuple(dw.shape)}")
     kernel_assert(expert_affinities_scaling_mode != ExpertAffinityScaleMode.PRE_SCALE_DELAYED,
                   "Currently ExpertAffinityScaleMode PRE_SCALE_DELAYED is not support ")
     T1 = hidden_states.shape[0]
@@ -72,26 +76,31 @@ def run_dense_variant(
         kernel_assert(gus.shape[0] == ds.shape[0], "weight scales must agree on their expert dimension")
         scale_experts = gus.shape[0]
     if gate_and_up_proj_bias is not None:
-        kernel_assert(tuple(gate_and_up_proj_bias.shape) == (E, 2, I),
-                      f"gate_and_up_proj_bias must be [E, 2, I] but got {tuple(gate_and_up_proj_bias.shape)}")
+        if not (tuple(gate_and_up_proj_bias.shape) == (E, 2, I)):
+            kernel_assert(
+                False,
+                f"gate_and_up_proj_bias must be [E, 2, I] but got {tuple(gate_and_up_proj_bias.shape)}",
+            )
 
     fp8_act = hidden_states.dtype in (torch.float8_e4m3fn, torch.uint8)
     if fp8_act:
         # RMSNorm-Quant ROW records: [T+1, H+4] (rmsnorm_quant.py:149-156)
-        kernel_assert(hidden_states.shape[1] == H + 4,
-                      f"fp8 hidden_states must be rmsnorm_quant ROW records [T+1, H+4={H + 4}] but got "
-                      f"{tuple(hidden_states.shape)}")
+        if not (hidden_states.shape[1] == H + 4):
+            kernel_assert(False, f"fp8 hidden_states must be rmsnorm_quant ROW records [T+1, H+4={H + 4}] but got "
+                                 f"{tuple(hidden_states.shape)}")
         kernel_assert(fp8_w and gus is not None, "fp8 activations need fp8 weights with per-channel scales")
         kind, wdt = nv.KIND_FP8_ROW, nv.DT_FP8
     else:
-        kernel_assert(hidden_states.dtype == torch.bfloat16,
-                      f"hidden_states must be bfloat16 (or fp8 ROW records) but got {hidden_states.dtype}")
-        kernel_assert(hidden_states.shape[1] == H, f"hidden_states must be [T+1, {H}] but got {tuple(hidden_states.shape)}")
+        if not (hidden_states.dtype == torch.bfloat16):
+            kernel_assert(False, f"hidden_states must be bfloat16 (or fp8 ROW records) but got {hidden_states.dtype}")
+        if not (hidden_states.shape[1] == H):
+            kernel_assert(False, f"hidden_states must be [T+1, {H}] but got {tuple(hidden_states.shape)}")
         if fp8_w:
             kernel_assert(gus is not None, "fp8 weights need gate_up_proj_scale / down_proj_scale")
             kind, wdt = nv.KIND_BF16, nv.DT_FP8
         else:
-            kernel_assert(guw.dtype == torch.bfloat16, f"weights must be bfloat16 or fp8 but got {guw.dtype}")
+            if not (guw.dtype == torch.bfloat16):
+                kernel_assert(False, f"weights must be bfloat16 or fp8 but got {guw.dtype}")
             kind, wdt = nv.KIND_BF16, nv.DT_BF16
     return run_blockwise(
         kind, hidden_states, expert_affinities_masked, guw, dw, token_position_to_id, block_to_expert, block_size,

@@ -84,33 +84,47 @@ def _bwmm_shard_on_block_mx(
     wdt = nv.DT_FP4_E2M1 if "float4" in wd else (nv.DT_FP8_E5M2 if "e5m2" in wd else nv.DT_FP8)
     wbytes = 2 if wdt == nv.DT_FP4_E2M1 else 4  # bytes of an x4 element
     hidden_states = nv.require_device_tensor(hidden_states, "hidden_states")
-    kernel_assert(hidden_states.dim() == 2, f"hidden_states must be [T+1, H] but got {tuple(hidden_states.shape)}")
+    if not (hidden_states.dim() == 2):
+        kernel_assert(False, f"hidden_states must be [T+1, H] but got {tuple(hidden_states.shape)}")
     T1, H = hidden_states.shape
     kernel_assert(block_size % 128 == 0, "Blocksize must be a multiple of 128")
-    kernel_assert(H % 512 == 0, f"Hidden dim size must be multiples of 512, found {H} ")
-    kernel_assert(512 <= H <= 16384, f"Hidden dims must be between 512 and 16384, found {H}")
+    if not (H % 512 == 0):
+        kernel_assert(False, f"Hidden dim size must be multiples of 512, found {H} ")
+    if not (512 <= H <= 16384):
+        kernel_assert(False, f"Hidden dims must be between 512 and 16384, found {H}")
     guw = _as_bytes(gate_up_proj_weight, "gate_up_proj_weight")
     dw = _as_bytes(down_proj_weight, "down_proj_weight")
     gus = nv.require_device_tensor(gate_up_proj_scale, "gate_up_proj_scale")
     ds = nv.require_device_tensor(down_proj_scale, "down_proj_scale")
     kernel_assert(gus.dtype == torch.uint8 and ds.dtype == torch.uint8, "MX scales must be uint8 (E8M0)")
-    kernel_assert(gus.dim() == 5 and gus.shape[1] == 16 and gus.shape[2] == 2 and gus.shape[3] == H // 512,
-                  f"gate_up_proj_scale must be [E, 16, 2, H/512, I] but got {tuple(gus.shape)}")
+    if not (gus.dim() == 5 and gus.shape[1] == 16 and gus.shape[2] == 2 and gus.shape[3] == H // 512):
+        kernel_assert(False, f"gate_up_proj_scale must be [E, 16, 2, H/512, I] but got {tuple(gus.shape)}")
     E, I = gus.shape[0], gus.shape[4]
     nI = (I + 511) // 512
     pI = 128 if I > 512 else I // 4
-    kernel_assert(I % 16 == 0, f"down_proj_weight I must be divisible by 16, found {I} . Please pad it")
-    kernel_assert(I % 512 == 0 or (I % 512) % 32 == 0, f"I tail must be a multiple of 32, found {I}")
-    kernel_assert(guw.numel() == E * 128 * 2 * (H // 512) * I * wbytes,
-                  f"gate_up_proj_weight must be x4 [E={E}, 128, 2, {H // 512}, {I}] of {wbytes}-byte elements "
-                  f"but holds {guw.numel()} bytes")
-    kernel_assert(dw.numel() == E * pI * nI * H * wbytes,
-                  f"down_proj_weight must be x4 [E={E}, {pI}, {nI}, {H}] of {wbytes}-byte elements but holds {dw.numel()} bytes")
-    kernel_assert(tuple(ds.shape) == (E, (pI + 7) // 8, nI, H),
-                  f"down_proj_scale must be [{E}, {(pI + 7) // 8}, {nI}, {H}] but got {tuple(ds.shape)}")
+    if not (I % 16 == 0):
+        kernel_assert(False, f"down_proj_weight I must be divisible by 16, found {I} . Please pad it")
+    if not (I % 512 == 0 or (I % 512) % 32 == 0):
+        kernel_assert(False, f"I tail must be a multiple of 32, found {I}")
+    if not (guw.numel() == E * 128 * 2 * (H // 512) * I * wbytes):
+        kernel_assert(
+            False,
+            f"gate_up_proj_weight must be x4 [E={E}, 128, 2, {H // 512}, {I}] of {wbytes}-byte elements "
+            f"but holds {guw.numel()} bytes",
+        )
+    if not (dw.numel() == E * pI * nI * H * wbytes):
+        kernel_assert(
+            False,
+            f"down_proj_weight must be x4 [E={E}, {pI}, {nI}, {H}] of {wbytes}-byte elements but holds {dw.numel()} bytes",
+        )
+    if not (tuple(ds.shape) == (E, (pI + 7) // 8, nI, H)):
+        kernel_assert(False, f"down_proj_scale must be [{E}, {(pI + 7) // 8}, {nI}, {H}] but got {tuple(ds.shape)}")
     if gate_and_up_proj_bias is not None:
-        kernel_assert(tuple(gate_and_up_proj_bias.shape) == (E, pI, 2, nI, 4),
-                      f"gate_and_up_proj_bias must be [{E}, {pI}, 2, {nI}, 4] but got {tuple(gate_and_up_proj_bias.shape)}")
+        if not (tuple(gate_and_up_proj_bias.shape) == (E, pI, 2, nI, 4)):
+            kernel_assert(
+                False,
+                f"gate_and_up_proj_bias must be [{E}, {pI}, 2, {nI}, 4] but got {tuple(gate_and_up_proj_bias.shape)}",
+            )
     kernel_assert(is_tensor_update_accumulating, "Only support topK > 1 at the moment.")
     kernel_assert(expert_affinities_scaling_mode in (ExpertAffinityScaleMode.POST_SCALE, ExpertAffinityScaleMode.NO_SCALE),
                   "MX blockwise MoE supports POST_SCALE / NO_SCALE only")
@@ -119,15 +133,21 @@ def _bwmm_shard_on_block_mx(
         xs = nv.require_device_tensor(hidden_states_scale, "hidden_states_scale")
         kernel_assert(hidden_states.dtype in (torch.uint8, torch.float8_e4m3fn),
                       "pre-quantised hidden_states must be uint8 / float8_e4m3fn codes")
-        kernel_assert(xs.dtype == torch.uint8 and tuple(xs.shape) == (T1, H // 32),
-                      f"hidden_states_scale must be uint8 [{T1}, {H // 32}] but got {tuple(xs.shape)}")
+        if not (xs.dtype == torch.uint8 and tuple(xs.shape) == (T1, H // 32)):
+            kernel_assert(False, f"hidden_states_scale must be uint8 [{T1}, {H // 32}] but got {tuple(xs.shape)}")
     else:
-        kernel_assert(hidden_states.dtype == torch.bfloat16,
-                      f"hidden_states must be bfloat16 (or MXFP8 codes with hidden_states_scale) but got {hidden_states.dtype}")
+        if not (hidden_states.dtype == torch.bfloat16):
+            kernel_assert(
+                False,
+                f"hidden_states must be bfloat16 (or MXFP8 codes with hidden_states_scale) but got {hidden_states.dtype}",
+            )
     if conditions is not None and _out_shape_kind == "2TH":
         N = token_position_to_id.numel() // block_size
-        kernel_assert(conditions.numel() == N + 2,
-                      f"condition vector must have exactly N+2 elements, got {conditions.numel()} != N + 2 ({N} + 2)")
+        if not (conditions.numel() == N + 2):
+            kernel_assert(
+                False,
+                f"condition vector must have exactly N+2 elements, got {conditions.numel()} != N + 2 ({N} + 2)",
+            )
     dims = {"T1": T1, "H": H, "I": I, "E": E}
     return run_blockwise(
         nv.KIND_MXFP8, hidden_states, expert_affinities_masked, guw, dw, token_position_to_id, block_to_expert,

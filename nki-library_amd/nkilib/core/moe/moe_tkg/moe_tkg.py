@@ -56,7 +56,8 @@ def _moe_tkg(
     x = nv.require_device_tensor(hidden_input, "hidden_input")
     guw = nv.require_device_tensor(expert_gate_up_weights, "expert_gate_up_weights")
     dw = nv.require_device_tensor(expert_down_weights, "expert_down_weights")
-    kernel_assert(x.dim() == 2, f"{_PREFIX} hidden_input must be [T, H] but got {tuple(x.shape)}")
+    if not (x.dim() == 2):
+        kernel_assert(False, f"{_PREFIX} hidden_input must be [T, H] but got {tuple(x.shape)}")
     T, H = x.shape
     E_L = guw.shape[0]
     mode = ExpertAffinityScaleMode(expert_affinities_scaling_mode)
@@ -64,24 +65,30 @@ def _moe_tkg(
     is_mx = _is_mx(guw, expert_gate_up_weights_scale)
     # moe_tkg.py:316-402
     if is_mx:
-        kernel_assert(expert_gate_up_weights_scale is not None and expert_down_weights_scale is not None,
-                      f"{_PREFIX} Scales must be set when using MX weights")
+        if not (expert_gate_up_weights_scale is not None and expert_down_weights_scale is not None):
+            kernel_assert(False, f"{_PREFIX} Scales must be set when using MX weights")
     if is_all_expert_dynamic:
-        kernel_assert(is_all_expert, f"{_PREFIX} is_all_expert_dynamic=True requires is_all_expert=True, but got "
-                                     f"{is_all_expert=}")
-        kernel_assert(block_size is not None, f"{_PREFIX} is_all_expert_dynamic=True requires block_size != None, "
-                                              f"but got {block_size=}")
-    kernel_assert(hidden_input_scale is None,
-                  f"{_PREFIX} hidden_input_scale describes a pre-quantised input in SBUF, which has no counterpart on "
-                  "gfx950; pass bfloat16 hidden_input")
-    kernel_assert(mode != ExpertAffinityScaleMode.PRE_SCALE_DELAYED,
-                  f"{_PREFIX} PRE_SCALE_DELAYED option is only applicable in CTE expert_mlp case")
-    kernel_assert(mode != ExpertAffinityScaleMode.PRE_SCALE, f"{_PREFIX} Kernel does not support pre-scale mode")
-    kernel_assert(gate_up_input_scale is None and down_input_scale is None,
-                  f"{_PREFIX} Static quantization is not supported in MoE TKG kernel")
+        if not is_all_expert:
+            kernel_assert(False, f"{_PREFIX} is_all_expert_dynamic=True requires is_all_expert=True, but got "
+                                 f"{is_all_expert=}")
+        if not (block_size is not None):
+            kernel_assert(False, f"{_PREFIX} is_all_expert_dynamic=True requires block_size != None, "
+                                 f"but got {block_size=}")
+    if not (hidden_input_scale is None):
+        kernel_assert(
+            False,
+            f"{_PREFIX} hidden_input_scale describes a pre-quantised input in SBUF, which has no counterpart on "
+            "gfx950; pass bfloat16 hidden_input",
+        )
+    if not (mode != ExpertAffinityScaleMode.PRE_SCALE_DELAYED):
+        kernel_assert(False, f"{_PREFIX} PRE_SCALE_DELAYED option is only applicable in CTE expert_mlp case")
+    if not (mode != ExpertAffinityScaleMode.PRE_SCALE):
+        kernel_assert(False, f"{_PREFIX} Kernel does not support pre-scale mode")
+    if not (gate_up_input_scale is None and down_input_scale is None):
+        kernel_assert(False, f"{_PREFIX} Static quantization is not supported in MoE TKG kernel")
     if is_all_expert:
-        kernel_assert(expert_affinities_eager is None,
-                      f"{_PREFIX} expert_affinities eager mode not supported with is_all_expert=True")
+        if not (expert_affinities_eager is None):
+            kernel_assert(False, f"{_PREFIX} expert_affinities eager mode not supported with is_all_expert=True")
     dev = x.device
     B = _BLOCK
     scaled = mode != ExpertAffinityScaleMode.NO_SCALE
@@ -94,10 +101,11 @@ def _moe_tkg(
         b2e = torch.arange(E_L, dtype=torch.int32, device=dev).repeat_interleave(nb)
         table = None
         if scaled:
-            kernel_assert(rank_id is not None,
-                          f"{_PREFIX} rank_id is required for all-expert mode with affinity scaling")
+            if not (rank_id is not None):
+                kernel_assert(False, f"{_PREFIX} rank_id is required for all-expert mode with affinity scaling")
             aff = nv.require_device_tensor(expert_affinities, "expert_affinities")
-            kernel_assert(aff.dim() == 2 and aff.shape[0] == T, f"{_PREFIX} expert_affinities must be [T, E]")
+            if not (aff.dim() == 2 and aff.shape[0] == T):
+                kernel_assert(False, f"{_PREFIX} expert_affinities must be [T, E]")
             rank = nv.require_device_tensor(rank_id, "rank_id").reshape(-1)[:1].to(torch.int64)
             cols = rank * E_L + torch.arange(E_L, dtype=torch.int64, device=dev)  # moe_tkg_affinity_masking.py:81-89
             table = aff.index_select(1, cols)
@@ -109,7 +117,8 @@ def _moe_tkg(
             table = table.contiguous()
     else:
         idx = nv.require_device_tensor(expert_index, "expert_index")
-        kernel_assert(idx.dim() == 2 and idx.shape[0] == T, f"{_PREFIX} expert_index must be [T, K]")
+        if not (idx.dim() == 2 and idx.shape[0] == T):
+            kernel_assert(False, f"{_PREFIX} expert_index must be [T, K]")
         K = idx.shape[1]
         ids = idx.to(torch.int32).contiguous()
         N = get_n_blocks(T, K, E_L, B)
@@ -118,13 +127,17 @@ def _moe_tkg(
         if scaled:
             if expert_affinities_eager is not None:
                 eager = nv.require_device_tensor(expert_affinities_eager, "expert_affinities_eager")
-                kernel_assert(tuple(eager.shape) == (T, K), f"{_PREFIX} expert_affinities_eager must be [T, K]")
+                if not (tuple(eager.shape) == (T, K)):
+                    kernel_assert(False, f"{_PREFIX} expert_affinities_eager must be [T, K]")
                 table = torch.zeros((T, E_L), dtype=eager.dtype, device=dev)
                 table.scatter_(1, idx.to(torch.int64), eager)
             else:
                 table = nv.require_device_tensor(expert_affinities, "expert_affinities")
-                kernel_assert(tuple(table.shape) == (T, E_L),
-                              f"{_PREFIX} expert_affinities must be [T, E] = [{T}, {E_L}] but got {tuple(table.shape)}")
+                if not (tuple(table.shape) == (T, E_L)):
+                    kernel_assert(
+                        False,
+                        f"{_PREFIX} expert_affinities must be [T, E] = [{T}, {E_L}] but got {tuple(table.shape)}",
+                    )
     if table is not None and table.dtype not in (torch.bfloat16, torch.float32):
         table = table.to(torch.float32)
 
@@ -141,14 +154,17 @@ def _moe_tkg(
     else:
         gus = ds = None
         if expert_gate_up_weights_scale is not None or expert_down_weights_scale is not None:
-            kernel_assert(expert_gate_up_weights_scale is not None and expert_down_weights_scale is not None,
-                          f"{_PREFIX} gate/up and down weight scales must be given together")
+            if not (expert_gate_up_weights_scale is not None and expert_down_weights_scale is not None):
+                kernel_assert(False, f"{_PREFIX} gate/up and down weight scales must be given together")
             I = guw.shape[-1]
             gus = nv.require_device_tensor(expert_gate_up_weights_scale, "expert_gate_up_weights_scale")
             ds = nv.require_device_tensor(expert_down_weights_scale, "expert_down_weights_scale")
-            kernel_assert(tuple(gus.shape) == (E_L, 2, I) and tuple(ds.shape) == (E_L, H),
-                          f"{_PREFIX} row scales must be [E_L, 2, I] and [E_L, H] but got {tuple(gus.shape)}, "
-                          f"{tuple(ds.shape)}")
+            if not (tuple(gus.shape) == (E_L, 2, I) and tuple(ds.shape) == (E_L, H)):
+                kernel_assert(
+                    False,
+                    f"{_PREFIX} row scales must be [E_L, 2, I] and [E_L, H] but got {tuple(gus.shape)}, "
+                    f"{tuple(ds.shape)}",
+                )
             gus, ds = gus.reshape(E_L, 1, 2 * I), ds.reshape(E_L, 1, H)
         out = run_dense_variant(
             x, table, guw, dw, B, tp2id, b2e, "TH", gate_and_up_proj_bias=expert_gate_up_bias,

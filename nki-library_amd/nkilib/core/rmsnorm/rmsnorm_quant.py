@@ -31,16 +31,14 @@ class RmsNormQuantKernelArgs:
     eps: float = 1e-6
 
     def __post_init__(self):
-        kernel_assert(
-            self.quantization_type in (QuantizationType.ROW, QuantizationType.STATIC),
-            f"{self.quantization_type.name} quantization is not supported",
-        )
-        kernel_assert(
-            self.norm_type == NormType.NO_NORM or self.norm_type == NormType.RMS_NORM,
-            f"{self.norm_type.name} normalization is not supported",
-        )
-        kernel_assert(self.lower_bound >= 0, f"Lower bound must be positive but got {self.lower_bound}")
-        kernel_assert(self.eps >= 0, f"Epsilon must be positive but got {self.eps}")
+        if not (self.quantization_type in (QuantizationType.ROW, QuantizationType.STATIC)):
+            kernel_assert(False, f"{self.quantization_type.name} quantization is not supported")
+        if not (self.norm_type == NormType.NO_NORM or self.norm_type == NormType.RMS_NORM):
+            kernel_assert(False, f"{self.norm_type.name} normalization is not supported")
+        if not (self.lower_bound >= 0):
+            kernel_assert(False, f"Lower bound must be positive but got {self.lower_bound}")
+        if not (self.eps >= 0):
+            kernel_assert(False, f"Epsilon must be positive but got {self.eps}")
 
     def needs_rms_normalization(self) -> bool:
         return self.norm_type == NormType.RMS_NORM
@@ -57,30 +55,37 @@ class RmsNormQuantKernelArgs:
 
 def _validate(hidden, ln_w, input_sc, kargs):
     """Shape checks of the reference (_validate_kernel_input, rmsnorm_quant.py:174-262)."""
-    kernel_assert(len(hidden.shape) >= 2, f"Rank of hidden must be at least 2 but got {len(hidden.shape)}")
+    if not (len(hidden.shape) >= 2):
+        kernel_assert(False, f"Rank of hidden must be at least 2 but got {len(hidden.shape)}")
     H = hidden.shape[-1]
     if kargs.is_static_quant():
         kernel_assert(input_sc is not None, "input_dequant_scale must be provided for static quantization")
-        kernel_assert(
-            tuple(input_sc.shape) == (128, 1),
-            f"static input dequant scale shape must be broadcasted to (128, 1) but got {tuple(input_sc.shape)}",
-        )
+        if not (tuple(input_sc.shape) == (128, 1)):
+            kernel_assert(
+                False,
+                f"static input dequant scale shape must be broadcasted to (128, 1) but got {tuple(input_sc.shape)}",
+            )
     if kargs.needs_rms_normalization():
         kernel_assert(ln_w is not None, "ln_w must be provided for RMS normalization")
-        kernel_assert(len(ln_w.shape) in (1, 2), f"Rank of ln_w must be 1 or 2 but got {len(ln_w.shape)}")
-        kernel_assert(ln_w.shape[-1] == H, f"ln_w vector length must equal {H} but got {ln_w.shape[-1]}")
+        if not (len(ln_w.shape) in (1, 2)):
+            kernel_assert(False, f"Rank of ln_w must be 1 or 2 but got {len(ln_w.shape)}")
+        if not (ln_w.shape[-1] == H):
+            kernel_assert(False, f"ln_w vector length must equal {H} but got {ln_w.shape[-1]}")
         if len(ln_w.shape) == 2:
-            kernel_assert(ln_w.shape[0] <= 1, f"ln_w first dimension {ln_w.shape[0]} must be at most 1")
+            if not (ln_w.shape[0] <= 1):
+                kernel_assert(False, f"ln_w first dimension {ln_w.shape[0]} must be at most 1")
     if len(hidden.shape) >= 3:
-        kernel_assert(hidden.shape[0] <= MAX_B, f"Batch dimension {hidden.shape[0]} exceeds maximum {MAX_B}")
-        kernel_assert(hidden.shape[1] <= MAX_S, f"Sequence length {hidden.shape[1]} exceeds maximum {MAX_S}")
-        kernel_assert(hidden.shape[2] <= MAX_H, f"Hidden dimension {hidden.shape[2]} exceeds maximum {MAX_H}")
+        if not (hidden.shape[0] <= MAX_B):
+            kernel_assert(False, f"Batch dimension {hidden.shape[0]} exceeds maximum {MAX_B}")
+        if not (hidden.shape[1] <= MAX_S):
+            kernel_assert(False, f"Sequence length {hidden.shape[1]} exceeds maximum {MAX_S}")
+        if not (hidden.shape[2] <= MAX_H):
+            kernel_assert(False, f"Hidden dimension {hidden.shape[2]} exceeds maximum {MAX_H}")
     else:
-        kernel_assert(H <= MAX_H, f"Processing dimension {H} exceeds maximum {MAX_H}")
-        kernel_assert(
-            hidden.shape[0] <= MAX_B * MAX_S,
-            f"Outer dimension {hidden.shape[0]} exceeds maximum {MAX_B * MAX_S} (MAX_B * MAX_S)",
-        )
+        if not (H <= MAX_H):
+            kernel_assert(False, f"Processing dimension {H} exceeds maximum {MAX_H}")
+        if not (hidden.shape[0] <= MAX_B * MAX_S):
+            kernel_assert(False, f"Outer dimension {hidden.shape[0]} exceeds maximum {MAX_B * MAX_S} (MAX_B * MAX_S)")
 
 
 def _rmsnorm_quant_kernel(

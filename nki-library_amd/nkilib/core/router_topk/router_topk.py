@@ -33,17 +33,22 @@ def _router_topk(x, w, w_bias, router_logits, expert_affinities, expert_index, a
     if int(x_hbm_layout) == 0:
         x = x.t().contiguous()  # [H, T] -> [T, H]: the GEMM reads token rows
     T, H = x.shape
-    kernel_assert(w.shape[0] == H, f"w must be [H, E] with H = {H} but got {tuple(w.shape)}")
+    if not (w.shape[0] == H):
+        kernel_assert(False, f"w must be [H, E] with H = {H} but got {tuple(w.shape)}")
     E = w.shape[1]
-    kernel_assert(1 <= int(k) <= 8 and int(k) <= E, f"k must be in [1, min(8, E)] but got {k}")
-    kernel_assert(E <= 512, f"E must be <= 512 but got {E}")
-    kernel_assert(H % 128 == 0, f"H must be a multiple of 128 but got {H}")
+    if not (1 <= int(k) <= 8 and int(k) <= E):
+        kernel_assert(False, f"k must be in [1, min(8, E)] but got {k}")
+    if not (E <= 512):
+        kernel_assert(False, f"E must be <= 512 but got {E}")
+    if not (H % 128 == 0):
+        kernel_assert(False, f"H must be a multiple of 128 but got {H}")
     act = RouterActFnType(act_fn) if not isinstance(act_fn, RouterActFnType) else act_fn
     dev = x.device
     bias = None
     if w_bias is not None:
         bias = nv.require_device_tensor(w_bias, "w_bias").reshape(-1)
-        kernel_assert(bias.numel() == E, f"w_bias must hold E = {E} values")
+        if not (bias.numel() == E):
+            kernel_assert(False, f"w_bias must hold E = {E} values")
     rows = T + (1 if _pad_row else 0)
     if expert_affinities is None:
         expert_affinities = torch.empty((rows, E), dtype=torch.bfloat16, device=dev)

@@ -37,7 +37,8 @@ def rmsnorm_mx_quantize_tkg(
     """
     # the reference has no other layout either (validate_shapes_quantize_mx, norm_tkg_utils.py:467)
     kernel_assert(hidden_dim_tp, "Only hidden_dim_tp=True is supported")
-    kernel_assert(len(input.shape) == 3, f"input must be [B, S, H] but got {tuple(input.shape)}")
+    if not (len(input.shape) == 3):
+        kernel_assert(False, f"input must be [B, S, H] but got {tuple(input.shape)}")
     B, S, H = input.shape
     BxS = B * S
     if residual is not None:
@@ -45,26 +46,30 @@ def rmsnorm_mx_quantize_tkg(
         # tensor engine and have no counterpart here)
         kernel_assert(tuple(input.shape) == tuple(residual.shape), "input and residual shapes must match")
         kernel_assert(output_residual is not None, "output_residual required when residual provided")
-        kernel_assert(tuple(output_residual.shape) == (BxS, H), f"expected output_residual shape (B*S, H)={(BxS, H)}")
+        if not (tuple(output_residual.shape) == (BxS, H)):
+            kernel_assert(False, f"expected output_residual shape (B*S, H)={(BxS, H)}")
         kernel_assert(residual.dtype == input.dtype and output_residual.dtype == input.dtype,
                       "residual and output_residual must have the input's dtype")
     else:
         kernel_assert(output_residual is None, "output_residual given without residual")
-    kernel_assert(H % 512 == 0, f"H must be divisible by 512, got {H}")
-    kernel_assert(gamma.shape[-1] == H, f"gamma length must equal {H} but got {gamma.shape[-1]}")
+    if not (H % 512 == 0):
+        kernel_assert(False, f"H must be divisible by 512, got {H}")
+    if not (gamma.shape[-1] == H):
+        kernel_assert(False, f"gamma length must equal {H} but got {gamma.shape[-1]}")
     nT = H // 512
-    kernel_assert(output_quant.numel() * output_quant.element_size() == 128 * nT * BxS * 4,
-                  f"output_quant must hold [128, {nT}, {BxS}] x4 elements")
+    if not (output_quant.numel() * output_quant.element_size() == 128 * nT * BxS * 4):
+        kernel_assert(False, f"output_quant must hold [128, {nT}, {BxS}] x4 elements")
     kernel_assert(output_scale.dtype == torch.uint8, "output_scale must be uint8")
     if output_scale.shape[0] == 16:
         layout = nv.MX_REF_DENSE
     else:
         kernel_assert(output_scale.shape[0] == 128, "output_scale first dimension must be 16 or 128")
         layout = nv.MX_REF_STRIDED
-    kernel_assert(tuple(output_scale.shape[1:]) == (nT, BxS), f"output_scale must be [*, {nT}, {BxS}]")
+    if not (tuple(output_scale.shape[1:]) == (nT, BxS)):
+        kernel_assert(False, f"output_scale must be [*, {nT}, {BxS}]")
     if output is not None:
-        kernel_assert(tuple(output.shape) == (128, BxS, H // 128) and output.dtype == torch.bfloat16,
-                      f"output must be bf16 [128, {BxS}, {H // 128}]")
+        if not (tuple(output.shape) == (128, BxS, H // 128) and output.dtype == torch.bfloat16):
+            kernel_assert(False, f"output must be bf16 [128, {BxS}, {H // 128}]")
     L = nv.lib()
     x = nv.require_device_tensor(input, "input")
     g = nv.require_device_tensor(gamma, "gamma")
@@ -72,7 +77,8 @@ def rmsnorm_mx_quantize_tkg(
     for t, n in ((output, "output"), (output_quant, "output_quant"), (output_scale, "output_scale"),
                  (output_residual, "output_residual")):
         if t is not None:
-            kernel_assert(t.is_cuda and t.is_contiguous(), f"{n} must be a contiguous device tensor")
+            if not (t.is_cuda and t.is_contiguous()):
+                kernel_assert(False, f"{n} must be a contiguous device tensor")
     with nv.on_device(x.device):
         rc = L.moe_rmsnorm_quant_mxfp8(nv.ptr(x), nv.dtype_code(x, "input"), nv.ptr(r), nv.ptr(output_residual), nv.ptr(g),
                                        nv.dtype_code(g, "gamma"), nv.ptr(output_quant), nv.ptr(output_scale),
@@ -93,9 +99,11 @@ def rmsnorm_mx_quantize(hidden: torch.Tensor, gamma: Optional[torch.Tensor], eps
     With ``residual`` ([T, H], hidden's dtype) the row ``hidden + residual`` (rounded to that dtype) is what is
     normalised and quantised, and it is returned as a third result: the layer's new residual stream.
     """
-    kernel_assert(len(hidden.shape) == 2, f"hidden must be [T, H] but got {tuple(hidden.shape)}")
+    if not (len(hidden.shape) == 2):
+        kernel_assert(False, f"hidden must be [T, H] but got {tuple(hidden.shape)}")
     T, H = hidden.shape
-    kernel_assert(H % 512 == 0, f"H must be divisible by 512, got {H}")
+    if not (H % 512 == 0):
+        kernel_assert(False, f"H must be divisible by 512, got {H}")
     L = nv.lib()
     x = nv.require_device_tensor(hidden, "hidden")
     g = nv.require_device_tensor(gamma, "gamma") if do_norm else None
