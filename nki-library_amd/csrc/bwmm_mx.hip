@@ -944,9 +944,6 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // 126 | 96; 222, top-4 of 4 bf16 experts of 6144, 128 179 | 119.
   const int total = (__builtin_amdgcn_readlane(q_lane, CHUNK_CLASSES) - run.qbase) * a.col_tiles;
   const int round = total / W, rest = total - round * W;
-  const int shift = (run.interleave > 1 || rest == 0 || 2 * rest > W) ? 0 : 4 * rest > W ? 1 : 2;
-  const int whole = shift ? round * W : total;
-  run.cut = whole << 2 | shift;
   int L = w, step = 2 * (W - 1 - w) + 1;
   constexpr int NO_CLASS = CHUNK_CLASSES;
   // (Chunks of up to 64 rows are a stream of weights, for which three slices ahead in registers beat two stages in LDS.
@@ -962,6 +959,12 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     run.npos = __builtin_amdgcn_readlane(q, c + 1) - run.qbase - run.pos0;
     return c;
   };
+  // (tiles of at most 128 rows, by the class of the round's first, its largest, are not cut)
+  int shift = (run.interleave > 1 || rest == 0 || 2 * rest > W) ? 0 : 4 * rest > W ? 1 : 2;
+  if (shift && aim_at_class_of(round * W) > 8) shift = 0;
+  static_assert(CHUNK_CLASS_TILES[8] == 10 && CHUNK_CLASS_TILES[9] == 8, "the last class of more than 128 rows");
+  const int whole = shift ? round * W : total;
+  run.cut = whole << 2 | shift;
   // the instance that the workgroup's piece of the last round takes, one of the smallest three: none ahead of its tile's class
   {
     int inst = NO_CLASS;

@@ -57,7 +57,9 @@ struct RowsCfg {
   static constexpr int LDS = KP * ROWS * PITCH * 4;
 };
 
-template <int STAGE, int WFMT, int MT, int CGT, int KP>
+// KTAIL: MX down stage whose K may end inside the last slice (an instance of its own: the offsets that it needs per slice
+// cost the one-token launch half a microsecond)
+template <int STAGE, int WFMT, int MT, int CGT, int KP, bool KTAIL>
 __global__ __launch_bounds__(64 * (RowsCfg<STAGE, WFMT, MT, CGT, KP>::NW))
 __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   using Cfg = RowsCfg<STAGE, WFMT, MT, CGT, KP>;
@@ -85,10 +87,10 @@ __attribute__((amdgpu_waves_per_eu(2, 8))) void mx_rows_kernel(const MxArgs a) {
   int nks;
   if (STAGE == 1) nks = (int)(a.H / 128);
   else nks = (int)mx_col_tiles(a.I);
-  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // K ends behind partition nP - 1 counted through all slices (whole MX blocks of
   // 8); a load of partitions past that is aimed past the end of the expert's weights (less than 2^31 bytes) and returns zeros
   // (where even the first partition of a load does not exist: through a descriptor of zero records)
-  constexpr bool KTAIL = STAGE == 2 && SCALED;
+  static_assert(!KTAIL || (STAGE == 2 && SCALED), "the other stages' K are whole slices");
   constexpr uint32_t PAST_END = 0x80000000u;
   const int nP = (int)(a.I >> 2);
 
@@ -410,16 +412,22 @@ constexpr bool ROWS_MT4 = WFMT == MX_WFMT_BF16 || (STAGE == 2 && (WFMT == MX_WFM
 
 // One workgroup per item, as many as the GPU holds at a time (the waves per SIMD that mx_rows_kernel is compiled for);
 // workgroups beyond the items end at once.
-template <int STAGE, int WFMT, int MT, int CGT, int KP>
-static int launch_one(const MxArgs& m, int64_t max_chunks, int cus, hipStream_t s) {
+template <int STAGE, int WFMT, int MT, int CGT, int KP, bool KTAIL>
+static int launch_instance(const MxArgs& m, int64_t max_chunks, int cus, hipStream_t s) {
   using Cfg = RowsCfg<STAGE, WFMT, MT, CGT, KP>;
   const int64_t items = max_chunks * m.col_tiles * (4 / Cfg::CG);
   const int64_t resident = (int64_t)cus * (8 / Cfg::NW);
   const unsigned grid = ((unsigned)(items < resident ? items : resident) + 7u) & ~7u;
-  if (allow_lds<&mx_rows_kernel<STAGE, WFMT, MT, CGT, KP>>(Cfg::LDS) != hipSuccess) return MOE_E_LAUNCH;
-  hipLaunchKernelGGL((mx_rows_kernel<STAGE, WFMT, MT, CGT, KP>), dim3(grid), dim3(64 * Cfg::NW), Cfg::LDS, s, m);
+  if (allow_lds<&mx_rows_kernel<STAGE, WFMT, MT, CGT, KP, KTAIL>>(Cfg::LDS) != hipSuccess) return MOE_E_LAUNCH;
+  hipLaunchKernelGGL((mx_rows_kernel<STAGE, WFMT, MT, CGT, KP, KTAIL>), dim3(grid), dim3(64 * Cfg::NW), Cfg::LDS, s, m);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
+}
+template <int STAGE, int WFMT, int MT, int CGT, int KP>
+static int launch_one(const MxArgs& m, int64_t max_chunks, int cus, hipStream_t s) {
+  if constexpr (STAGE == 2 && !RowsCfg<STAGE, WFMT, MT, CGT, KP>::ROW8)
+    if (m.I % 128 != 0) return launch_instance<STAGE, WFMT, MT, CGT, KP, true>(m, max_chunks, cus, s);
+  return launch_instance<STAGE, WFMT, MT, CGT, KP, false>(m, max_chunks, cus, s);
 }
 
 // Columns per workgroup.  64 (four waves on a quarter of K each) unless that leaves a second, partly filled round of
