@@ -4,7 +4,7 @@ Usage: ``python nki-library_amd/build.py``.  The library is written in-tree to
 ``nki-library_amd/nkilib/_lib/libmoe_gfx950.so`` where ``nkilib._native`` loads it.
 hipcc cross-compiles, so no GPU is needed to build.  Translation units are compiled in
 parallel into ``nki-library_amd/build/`` and linked; the MXFP8 large-tile GEMM
-(``csrc/bwmm_mx.hip``) is compiled once per (stage, weight format) plus once as the dispatcher.
+(``csrc/bwmm_mx.hip``) is compiled once per instance (``MX_INSTANCES``) plus once as the dispatcher.
 """
 
 import os
@@ -21,8 +21,9 @@ OBJ_DIR = os.path.join(HERE, "build")
 OUT_DIR = os.path.join(HERE, "nkilib", "_lib")
 OUT = os.path.join(OUT_DIR, "libmoe_gfx950.so")
 SOURCES = ["rmsnorm_quant.hip", "build_blocks.hip", "combine.hip", "bwmm.hip", "bwmm_mx.hip", "bwmm_rows.hip", "router_topk.hip", "index_ops.hip", "capi.hip"]
-# (stage, weight format) instances of the large-tile MX GEMM; formats as MX_WFMT_* in csrc/bwmm.hpp
-MX_INSTANCES = [(1, 0), (2, 0), (1, 1), (2, 1), (1, 2), (2, 2), (1, 3), (2, 3), (1, 4), (2, 4)]
+# (stage, weight format, K that ends inside a slice) instances of the large-tile MX GEMM; formats as MX_WFMT_* in csrc/bwmm.hpp
+MX_INSTANCES = [(1, 4, 0), (1, 3, 0), (1, 0, 0), (1, 1, 0), (1, 2, 0), (2, 4, 0), (2, 3, 0), (2, 0, 0), (2, 1, 0), (2, 2, 0),
+                (2, 0, 1), (2, 1, 1), (2, 2, 1)]
 FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -122,9 +123,10 @@ def build(verbose=True, jobs=None):
     os.makedirs(OBJ_DIR, exist_ok=True)
     inc = ["-I", os.path.join(ROOT, "include"), "-I", CSRC]
     units = []  # (object path, extra defines, source); the long-running instances of the large-tile GEMM go first
-    for stage, fmt in MX_INSTANCES:
-        units.append((os.path.join(OBJ_DIR, f"bwmm_mx_s{stage}_f{fmt}.o"),
-                      [*MX_FLAGS, f"-DMX_INST_STAGE={stage}", f"-DMX_INST_WFMT={fmt}"], os.path.join(CSRC, "bwmm_mx.hip")))
+    for stage, fmt, ktail in MX_INSTANCES:
+        units.append((os.path.join(OBJ_DIR, f"bwmm_mx_s{stage}_f{fmt}_t{ktail}.o"),
+                      [*MX_FLAGS, f"-DMX_INST_STAGE={stage}", f"-DMX_INST_WFMT={fmt}", f"-DMX_INST_KTAIL={ktail}"],
+                      os.path.join(CSRC, "bwmm_mx.hip")))
     for s in SOURCES:
         units.append((os.path.join(OBJ_DIR, s.replace(".hip", ".o")), MX_FLAGS if s in M0_CLOBBER_SOURCES else [],
                       os.path.join(CSRC, s)))

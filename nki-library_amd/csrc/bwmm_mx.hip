@@ -126,7 +126,7 @@ __device__ __forceinline__ void mfma_asm(const v8i& af, const BOp& bf, int sa, i
 // loads while the epilogue computes, and the next K loop starts on data that has arrived.  What the next tile
 // needs before its loads can be issued (token ids, affinities, bias) is read one tile earlier the same way:
 // requested before an epilogue, put in place after it.
-template <int STAGE, int NMT, bool LASTUSE, int WFMT>
+template <int STAGE, int NMT, bool LASTUSE, int WFMT, bool KTAIL>
 __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int (*s_tok)[MX_ROWS_MAX],
                                              float (*s_aff)[MX_ROWS_MAX], float (*s_bias)[MXT],
                                              float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L, int& step, const MxRun& run) {
@@ -219,10 +219,10 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
                                                         : (uint32_t)((GROWS * g * w_pstride + 4 * c) * ES));
   const uint32_t s_voff = (STAGE == 1) ? (uint32_t)(g * w_pstride + hcol * nH * a.I + 4 * cl)
                                        : (uint32_t)(g * w_pstride + 4 * c);
-  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // KTAIL: K ends inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
   // 8).  Loads of partitions past that are aimed past the end of the expert's weights and scales, both smaller than 2^31
   // bytes, and return zeros: the lane's offsets in the slice that slice_addr was last called for.
-  constexpr bool KTAIL = STAGE == 2 && !ROW8;
+  static_assert(!KTAIL || (STAGE == 2 && !ROW8), "the other stages' K are whole slices");
   const int nP = (int)(a.I >> 2);
   constexpr uint32_t PAST_END = 0x80000000u;
   // (Where even the first partition of a load does not exist, its scalar offset alone may lie past the end: such loads go
@@ -898,10 +898,13 @@ __device__ __forceinline__ int mx_gemm_tiles(const MxArgs& a, uint8_t* smem, int
 }
 
 
-// One translation unit per (stage, weight format): the build compiles this file once for each with
-// MX_INST_STAGE / MX_INST_WFMT defined, and once without them for the dispatcher below.
+// One translation unit per (stage, weight format, KTAIL): the build compiles this file once for each with
+// MX_INST_STAGE / MX_INST_WFMT / MX_INST_KTAIL defined, and once without them for the dispatcher below.
 #if defined(MX_INST_STAGE)
-template <int STAGE, int WFMT>
+// KTAIL: MX down stage whose K ends inside the last slice, a kernel of its own (without | with what its loads need per slice, down
+// launch where I is a multiple of 128, us: 3839 tokens, top-5 of 16 MXFP8 experts of H = 4608, I = 128 55.4 | 57.3; 4109, top-4 of
+// 16 of 3072, 2304 138.0 | 139.7; the same in MXFP4 123.6 | 127.1; 8192, top-2 of 64 of 7168, 2048 285.3 | 287.9)
+template <int STAGE, int WFMT, bool KTAIL>
 __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) void mx_gemm_kernel(const MxArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   __shared__ int s_tok[2][MX_ROWS_MAX];
@@ -1000,10 +1003,10 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   case CLS_:                                                                                                           \
     if (next == CLS_) {                                                                                                \
       if constexpr (CHUNK_CLASS_TILES[CLS_] >= 8)                                                                      \
-        L = mx_gemm_tiles_wide<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT>(                          \
+        L = mx_gemm_tiles_wide<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT, KTAIL>(                   \
             a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc, L, step, run);           \
       else                                                                                                             \
-        L = mx_gemm_tiles<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT>(                               \
+        L = mx_gemm_tiles<STAGE, CHUNK_CLASS_TILES[CLS_], CHUNK_CLASS_LAST[CLS_], WFMT, KTAIL>(                        \
             a, smem, s_tok, s_aff, s_bias, (float(*)[MX_ROWS_MAX])s_rs, (float(*)[MXT])s_wsc, L, step, run);           \
       __syncthreads();                                                                                                 \
       next = next_run();                                                                                               \
@@ -1033,14 +1036,15 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
-#define MX_CAT_(a, b, c, d) a##b##c##d
-#define MX_CAT(a, b, c, d) MX_CAT_(a, b, c, d)
+#define MX_CAT_(a, b, c, d, e, f) a##b##c##d##e##f
+#define MX_CAT(a, b, c, d, e, f) MX_CAT_(a, b, c, d, e, f)
 constexpr int MX_LDS_LAUNCH = MX_INST_WFMT == MX_WFMT_ROW8 || MX_INST_WFMT == MX_WFMT_BF16
                                   ? (MX_LDS > MX_WIDE_LDS_PLAIN ? MX_LDS : MX_WIDE_LDS_PLAIN)
                                   : (MX_LDS > MX_WIDE_LDS_SCALED ? MX_LDS : MX_WIDE_LDS_SCALED);
-int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT)(const MxArgs& m, unsigned grid, hipStream_t s) {
-  if (allow_lds<&mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>>(MX_LDS_LAUNCH) != hipSuccess) return MOE_E_LAUNCH;
-  hipLaunchKernelGGL((mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT>), dim3(grid), dim3(MXT), MX_LDS_LAUNCH, s, m);
+int MX_CAT(launch_mx_gemm_s, MX_INST_STAGE, _f, MX_INST_WFMT, _t, MX_INST_KTAIL)(const MxArgs& m, unsigned grid, hipStream_t s) {
+  constexpr auto kernel = &mx_gemm_kernel<MX_INST_STAGE, MX_INST_WFMT, MX_INST_KTAIL != 0>;
+  if (allow_lds<kernel>(MX_LDS_LAUNCH) != hipSuccess) return MOE_E_LAUNCH;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(MXT), MX_LDS_LAUNCH, s, m);
   MOE_CHECK_LAUNCH();
   return MOE_OK;
 }
@@ -1112,16 +1116,19 @@ int launch_mx_pack_weights(int stage, int fp4, const void* W, void* dst, int64_t
   return MOE_OK;
 }
 
-int launch_mx_gemm_s1_f0(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s2_f0(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s1_f1(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s2_f1(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s1_f2(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s2_f2(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s1_f3(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s2_f3(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s1_f4(const MxArgs& m, unsigned grid, hipStream_t s);
-int launch_mx_gemm_s2_f4(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s1_f0_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f0_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f0_t1(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s1_f1_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f1_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f1_t1(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s1_f2_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f2_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f2_t1(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s1_f3_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f3_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s1_f4_t0(const MxArgs& m, unsigned grid, hipStream_t s);
+int launch_mx_gemm_s2_f4_t0(const MxArgs& m, unsigned grid, hipStream_t s);
 
 int launch_mx_gemm(int stage, const MxArgs& m0, unsigned gx, unsigned gy, hipStream_t s) {
   if (gx == 0 || gy == 0) return MOE_OK;
@@ -1135,12 +1142,17 @@ int launch_mx_gemm(int stage, const MxArgs& m0, unsigned gx, unsigned gy, hipStr
   unsigned per_xcd = (unsigned)cus / 8u;
   if ((tiles + 7u) / 8u < per_xcd) per_xcd = (unsigned)((tiles + 7u) / 8u);
   const unsigned grid = 8u * per_xcd;
+  // (a K slice is 128 intermediate columns of the MX kinds; the dense kinds' K is padded to whole ones)
+  const bool ktail = stage == 2 && m.I % 128 != 0;
   switch (m.wfmt) {
-    case MX_WFMT_E4M3: return stage == 1 ? launch_mx_gemm_s1_f0(m, grid, s) : launch_mx_gemm_s2_f0(m, grid, s);
-    case MX_WFMT_E5M2: return stage == 1 ? launch_mx_gemm_s1_f1(m, grid, s) : launch_mx_gemm_s2_f1(m, grid, s);
-    case MX_WFMT_E2M1: return stage == 1 ? launch_mx_gemm_s1_f2(m, grid, s) : launch_mx_gemm_s2_f2(m, grid, s);
-    case MX_WFMT_ROW8: return stage == 1 ? launch_mx_gemm_s1_f3(m, grid, s) : launch_mx_gemm_s2_f3(m, grid, s);
-    case MX_WFMT_BF16: return stage == 1 ? launch_mx_gemm_s1_f4(m, grid, s) : launch_mx_gemm_s2_f4(m, grid, s);
+    case MX_WFMT_E4M3:
+      return stage == 1 ? launch_mx_gemm_s1_f0_t0(m, grid, s) : ktail ? launch_mx_gemm_s2_f0_t1(m, grid, s) : launch_mx_gemm_s2_f0_t0(m, grid, s);
+    case MX_WFMT_E5M2:
+      return stage == 1 ? launch_mx_gemm_s1_f1_t0(m, grid, s) : ktail ? launch_mx_gemm_s2_f1_t1(m, grid, s) : launch_mx_gemm_s2_f1_t0(m, grid, s);
+    case MX_WFMT_E2M1:
+      return stage == 1 ? launch_mx_gemm_s1_f2_t0(m, grid, s) : ktail ? launch_mx_gemm_s2_f2_t1(m, grid, s) : launch_mx_gemm_s2_f2_t0(m, grid, s);
+    case MX_WFMT_ROW8: return stage == 1 ? launch_mx_gemm_s1_f3_t0(m, grid, s) : launch_mx_gemm_s2_f3_t0(m, grid, s);
+    case MX_WFMT_BF16: return stage == 1 ? launch_mx_gemm_s1_f4_t0(m, grid, s) : launch_mx_gemm_s2_f4_t0(m, grid, s);
     default: return MOE_E_BAD_ARG;
   }
 }

@@ -127,7 +127,7 @@ __device__ __forceinline__ void st_b128_plain(const v4i& d, uint32_t voff, const
 
 // One class of tiles (see mx_gemm_tiles in bwmm_mx.hip for the walk over the queue, LASTUSE and the order of requests
 // around the epilogue).
-template <int STAGE, int NMT, bool LASTUSE, int WFMT>
+template <int STAGE, int NMT, bool LASTUSE, int WFMT, bool KTAIL>
 __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem, int (*s_tok)[MX_ROWS_MAX],
                                                   float (*s_aff)[MX_ROWS_MAX], float (*s_bias)[MXT],
                                                   float (*s_rs)[MX_ROWS_MAX], float (*s_wsc)[MXT], int L, int& step, const MxRun& run) {
@@ -181,9 +181,9 @@ __device__ __forceinline__ int mx_gemm_tiles_wide(const MxArgs& a, uint8_t* smem
   int nks;
   if (STAGE == 1) nks = (int)(a.H / 128);
   else nks = (int)mx_col_tiles(a.I);
-  // MX down stage: K may end inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
+  // KTAIL: K ends inside the last slice, behind partition nP - 1 counted through all slices (whole MX blocks of
   // 8); weights and scales past that are not read (see aim_w)
-  constexpr bool KTAIL = STAGE == 2 && SCALED;
+  static_assert(!KTAIL || (STAGE == 2 && SCALED), "the other stages' K are whole slices");
   const int nP = uni((int)(a.I >> 2));
 
   // ---- operand addressing -----------------------------------------------------------------------------------
