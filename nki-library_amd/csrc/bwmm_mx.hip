@@ -119,8 +119,8 @@ __device__ __forceinline__ void mfma_asm(const v8i& af, const BOp& bf, int sa, i
 // then keeps the activation tiles that the sibling workgroups share); an earlier chunk loads them
 // normally, for the chunk after it to find.
 //
-// A workgroup stays on its CU and walks a list of tiles of one class (items L, L + Lstep, ... below endL of its
-// XCD's queue; an item is a chunk and one of its column tiles).  Between two tiles nothing is left to the
+// A workgroup stays on its CU and walks a list of tiles of one class (its items of the XCD's queue from L on, in rounds of
+// alternating direction, ahead of run.end, see MxRun; an item is a chunk and one of its column tiles).  Between two tiles nothing is left to the
 // hardware's workgroup dispatch: as soon as the K loop of a tile has ended, the loads of the first D slices of the
 // next tile are issued, and only then does the tile's epilogue run -- the memory pipeline works through those
 // loads while the epilogue computes, and the next K loop starts on data that has arrived.  What the next tile
@@ -917,8 +917,8 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   // index, and each XCD has its own L2.  XCD x therefore takes the x-th of eight contiguous parts of the chunk
   // list (chunks are ordered by expert; the parts hold about equal work), as a queue of items (chunk, column
   // tile) with the chunks grouped by class and, inside a class, the column tiles innermost (or alternating between
-  // a few chunks of one expert, see tile_at); its workgroups take the items w, w + W, w + 2W, ... (W workgroups on
-  // the XCD).  The workgroups that share an activation tile, and the chunks that share an expert's weights, then run
+  // a few chunks of one expert, see tile_at); its W workgroups take the items in rounds of W, every other round in
+  // reverse (see MxRun).  The workgroups that share an activation tile, and the chunks that share an expert's weights, then run
   // at the same time behind the same L2, so each operand crosses the fabric about once; and a workgroup's
   // consecutive items are of one class, i.e. one instance of the code below, which carries its loads from tile
   // to tile.
@@ -980,20 +980,19 @@ __global__ __launch_bounds__(MXT) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     s_tail = inst;  // (every wave the same)
   }
-  // What the workgroup runs next: its items of the class that holds item L, and its piece as well where the same instance takes
-  // it, or the piece alone; NO_CLASS at the end.
+  // What the workgroup runs next: its whole items of the class that holds item L, or its piece; NO_CLASS at the end.  A piece's
+  // instance comes behind those of all whole items: these are ahead of the piece's tile in the queue, in its class or an earlier
+  // one, and half of a tile's rows (or less) are of a later class than the tile, which has more than 128.
   auto next_run = [&]() {
-    const int tail = __builtin_amdgcn_readfirstlane(s_tail);
     const int whole = run.cut >> 2;
     if (L < whole) {
       const int c = aim_at_class_of(L);
-      // (the piece lies behind the workgroup's last whole item, in whose class or a later one its tile is)
       const int end = (run.pos0 + run.npos) * a.col_tiles;
-      run.end = c == tail ? whole + W : end < whole ? end : whole;
+      run.end = end < whole ? end : whole;
       return c;
     }
     run.end = whole + W;
-    return L < run.end ? tail : NO_CLASS;
+    return L < run.end ? __builtin_amdgcn_readfirstlane(s_tail) : NO_CLASS;
   };
   // The instances one behind the other (in a loop over them the compiler keeps values of one in registers through all the
   // others), entered at the first that the workgroup needs and left behind its last: every one that is only stepped over
