@@ -286,7 +286,7 @@ typedef struct moe_bwmm_args {
    * weights with H % 256 == 0, and fp8-row weights with H % 512 == 0, the order
    * the large-tile kernels read, otherwise K-contiguous rows -- so one pair serves every call with those weights,
    * activation checkpoints included.)  MXFP8 kind: the x4 layouts are K-major already and are read in place when both are NULL;
-   * the same two calls make a copy of the gate/up weights in the
+   * where I % 128 == 0 the same two calls make a copy of the gate/up weights in the
    * order the kernel reads them (each workgroup then reads its weights as contiguous 32 KB runs: the gate/up GEMM
    * is 5 % faster at H = 7168, I = 2048 with 8-bit weights, for a second copy of those weights in memory); used
    * when gate_up_proj_weight_kmajor is set.  The block scales are no part of a copy: every call reads the tables it

@@ -109,9 +109,9 @@ inline int64_t dense_k_bytes(int64_t I, bool bf16) { return bf16 ? (I + 63) / 64
 // of the down stage may hold 8, 16 or 24 partitions of their 32: what lies past them in the weights and their tables is
 // read but never stored (gate/up, whose columns do not mix: the intermediate rows get zeros there), or not read (down:
 // loads out of range, zeros).  Measured on the general kernel (which still takes what mx_fast, csrc/capi.hip,
-// turns down) | here, us a layer: 7163 tokens, top-7 of 64 MXFP8 experts of H = 7168, I = 192 7935 | 674; 664, top-8 of 128 of
-// 6656, 832 14755 | 486; 1105, top-6 of 60 MXFP4 experts of 3072, 832 903 | 160; 5, top-8 of 32 MXFP8 experts of 4096, 960
-// 673 | 81; 43, one of 32 of 1536, 960 230 | 65.
+// turns down) | here, us a layer: 7163 tokens, top-7 of 64 MXFP8 experts of H = 7168, I = 192 7277 | 672; 664, top-8 of 128 of
+// 6656, 832 4454 | 526; 1105, top-6 of 60 MXFP4 experts of 3072, 832 897 | 152; 5, top-8 of 32 MXFP8 experts of 4096, 960
+// 685 | 91; 43, one of 32 of 1536, 960 225 | 61.
 inline bool mx_fast_path_ok(int64_t H, int64_t I) { return H % 512 == 0 && I % 32 == 0; }
 // column tiles of the gate/up stage = K slices of the down stage (I in columns; dense kinds: padded, or K bytes)
 __host__ __device__ inline int64_t mx_col_tiles(int64_t I) { return (I / 512) * 4 + (I % 512 + 127) / 128; }

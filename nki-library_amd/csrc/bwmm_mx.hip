@@ -1066,7 +1066,6 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
   const int g = lane >> 4, c = lane & 15;
   const int64_t pr = FP4 ? i : ((i < 4) ? i : (16 + i - 4)), kt = ks >> 2, pb = ks & 3;
   int64_t elem, expert_elems;
-  bool live;  // (a short last tile's padding: zeros)
   if (stage == 1) {
     const int64_t nH = H / 512, pstride = 2 * nH * I;
     const int64_t tI = xt >> 2, p0 = (xt & 3) * 32;
@@ -1074,17 +1073,15 @@ __global__ __launch_bounds__(256) void mx_pack_weights_kernel(int stage, const u
     const int64_t colu = tI * 512 + q * (rows_t / 4) + p0;
     elem = (GROWS * g + pr + pb * 32) * pstride + (c >> 3) * nH * I + 4 * (c & 7) + colu + kt * I;
     expert_elems = 128 * pstride;
-    live = p0 + 4 * (c & 7) < rows_t / 4;
   } else {
     const int64_t nI = (I + 511) / 512, pI = I > 512 ? 128 : I / 4, pstride = nI * H;
     elem = (GROWS * g + pr + pb * 32) * pstride + 4 * c + xt * 256 + 64 * q + kt * H;
     expert_elems = pI * pstride;
-    live = ks * 32 + GROWS * g + pr < I / 4;
   }
   const uint8_t* src = W + (e * expert_elems + elem) * ES;
   const int64_t o = (d & ~(int64_t)63) + (stage == 1 ? mx_pack_lane(lane) : lane);
-  if constexpr (FP4) *(uint2*)(dst + o * LB) = live ? *(const uint2*)src : make_uint2(0, 0);
-  else *(uint4*)(dst + o * LB) = live ? *(const uint4*)src : make_uint4(0, 0, 0, 0);
+  if constexpr (FP4) *(uint2*)(dst + o * LB) = *(const uint2*)src;
+  else *(uint4*)(dst + o * LB) = *(const uint4*)src;
 }
 
 static void mx_pack_geometry(int stage, int64_t H, int64_t I, int64_t* col_tiles, int64_t* nks) {
@@ -1099,7 +1096,7 @@ size_t mx_packed_weights_bytes(int stage, int fp4, int64_t E, int64_t H, int64_t
 }
 int launch_mx_pack_weights(int stage, int fp4, const void* W, void* dst, int64_t E, int64_t H, int64_t I,
                            hipStream_t s) {
-  if (!mx_fast_path_ok(H, I) || (((uintptr_t)W) & 15) != 0 || (((uintptr_t)dst) & 15) != 0) return MOE_E_BAD_ARG;
+  if (!mx_fast_path_ok(H, I) || I % 128 != 0 || (((uintptr_t)W) & 15) != 0 || (((uintptr_t)dst) & 15) != 0) return MOE_E_BAD_ARG;
   int64_t ct, nks;
   mx_pack_geometry(stage, H, I, &ct, &nks);
   const int64_t pieces = E * ct * nks * 2048;

@@ -51,8 +51,7 @@ struct Plan {
 // MX kinds on the large-tile and few-rows kernels (csrc/bwmm_mx.hip, csrc/bwmm_rows.hip).  mx_shape: the expert shape and
 // weight type, which alone decide whether there are copies of the weights in those kernels' order; mx_fast: the call as well.
 // Byte offsets (row * row stride, added to a 64-bit base) and buffer descriptors of at most 2^32 - 1 bytes for the
-// activations, the intermediate and their scales; signed 32-bit byte offsets inside one expert's weights (of which the
-// copies hold whole column tiles and K slices); the row tables (token ids, affinities, bias) through 32-bit byte offsets.
+// activations, the intermediate and their scales; signed 32-bit byte offsets inside one expert's weights; the row tables (token ids, affinities, bias) through 32-bit byte offsets.
 // Where I is no multiple of 128 the general kernel takes what they do not: activations past those offsets, and tensors that
 // lie closer than the 16 (tables: 4) bytes their loads are aligned to.
 constexpr int64_t LIM32 = (int64_t)1 << 32, LIM31 = (int64_t)1 << 31;
@@ -65,8 +64,8 @@ bool mx_shape(const moe_bwmm_args* a) {
   if (a->kind != MOE_KIND_MXFP8 || !mx_fast_path_ok(a->H, a->I)) return false;
   if (a->I % 128 != 0 && !aligned({a->gate_up_proj_weight, a->down_proj_weight}, 16)) return false;
   const int64_t es = a->weight_dtype == MOE_DT_FP4_E2M1 ? 2 : 4;  // bytes of an x4 weight element
-  const int64_t pI = a->I > 512 ? 128 : (mx_col_tiles(a->I) * 32), nI = (a->I + 511) / 512;
-  return 128 * 2 * (a->H / 512) * (mx_col_tiles(a->I) * 128) * es < LIM31 && pI * nI * a->H * es < LIM31 &&
+  const int64_t pI = a->I > 512 ? 128 : a->I / 4, nI = (a->I + 511) / 512;
+  return 128 * 2 * (a->H / 512) * a->I * es < LIM31 && pI * nI * a->H * es < LIM31 &&
          a->E * pI * 2 * nI * 4 * 4 < LIM32 && a->E * a->H * 4 < LIM32;
 }
 bool mx_fast(const moe_bwmm_args* a) {
@@ -322,9 +321,13 @@ int kmajor_copy(const moe_bwmm_args* a, const Plan& p, int which, void* dst, hip
 
 // MXFP8 kind: copies of the weights in the kernels' read order exist on the large-tile path: of the gate/up weights
 // for every format, of the down weights for 4-bit ones (whose pieces in the reference layout are 512 bytes; the
-// 8-bit ones' 1 KB pieces were measured no slower than a copy).
+// 8-bit ones' 1 KB pieces were measured no slower than a copy).  Where I is no multiple of 128 the weights are read in place:
+// those shapes never had copies, and their callers may write weights in ways that a kept copy does not see.  What that costs, with
+// copies | in place, us a layer: 300 tokens, top-4 of 32 MXFP4 experts of H = 5120, I = 2880 198 | 237; 4, top-8 of 64 of 5120,
+// 1440 105 | 123; 8192, top-4 of 32 of 2560, 2880 785 | 792; 664, top-8 of 128 MXFP8 experts of 6656, 832 476 | 526; 2000, top-8
+// of 64 of 4096, 704 265 | 280; 7163, top-7 of 64 of 7168, 192 656 | 672; 4096, top-4 of 32 of 3072, 2880 537 | 539.
 static bool mx_packable(const moe_bwmm_args* a, int which) {
-  if (!mx_shape(a)) return false;
+  if (a->I % 128 != 0 || !mx_shape(a)) return false;
   return which == 0 || a->weight_dtype == MOE_DT_FP4_E2M1;
 }
 

@@ -1,7 +1,6 @@
 """GPU parity of the MX kinds where the last intermediate tile holds no multiple of 32 partitions (I % 128 != 0): the last
 column tile of the gate/up stage and the last K slice of the down stage are 8, 16 or 24 partitions of their 32, in the
-few-rows kernel and both tile loops of the large-tile kernels, with the weights' copies and in place.  Tolerances are those of
-test_gpu_moe.py."""
+few-rows kernel and both tile loops of the large-tile kernels.  Tolerances are those of test_gpu_moe.py."""
 
 import numpy as np
 import pytest
@@ -56,3 +55,38 @@ def test_infinite_rows_with_a_short_tile(T):
     c["hidden"][0] = 3e38
     o = from_bf16_tensor(_run_mx_options(c, 0, None, False))
     assert np.array_equal(o[0, 1:T], want[0, 1:T])
+
+
+@pytest.mark.parametrize("fmt", ["e4m3", "e2m1"])
+@pytest.mark.parametrize("T", [20, 300])  # the few-rows and the large-tile kernels
+def test_weights_are_read_as_they_are(T, fmt):
+    """A weight loader writes through ``param.data``, which torch's version counter does not see.  Where I is no multiple of
+    128 the MX kinds keep nothing of the weights: the next call multiplies with what stands there now, and a call that is
+    recorded as the first with its weights leaves nothing behind."""
+    import torch
+    from nkilib.core.moe.moe_cte import _launch
+    from nkilib.core.moe.moe_cte.bwmm_shard_on_block_mx import bwmm_shard_on_block_mx
+    from helpers import bf16_tensor, i32_tensor, u8_tensor
+    from oracle.numerics import pack_e2m1_x4
+
+    dev = torch.device("cuda:0")
+    c, d = (mx_case(T, 512, 96, 4, 2, 128, seed=s, weight_format=fmt, random_codes=True) for s in (53, 54))
+
+    def weights(case):
+        if fmt == "e2m1":
+            return [torch.from_numpy(pack_e2m1_x4(case[w]).view(np.int16)).to(dev) for w in ("gate_up_q", "down_q")]
+        return [u8_tensor(case[w], dev).view(torch.float8_e4m3fn) for w in ("gate_up_q", "down_q")]
+
+    args = [bf16_tensor(c["hidden"], dev), bf16_tensor(c["aff"].reshape(-1, 1), dev)]
+    tables = [i32_tensor(c["tp2id"], dev), i32_tensor(c["b2e"], dev)]
+    kw = dict(gate_up_proj_scale=u8_tensor(c["gate_up_s"], dev), down_proj_scale=u8_tensor(c["down_s"], dev), block_size=128)
+    run = lambda w: bwmm_shard_on_block_mx[2](*args, *w, *tables, **kw)
+    kept = len(_launch._kmajor)
+    w, other = weights(c), weights(d)
+    first, second = run(w), run(other)
+    assert not torch.equal(first, second)
+    for t, o in zip(w, other):
+        raw = torch.uint8 if t.element_size() == 1 else torch.int16
+        t.data.view(raw).copy_(o.view(raw))
+    assert torch.equal(run(w), second)
+    assert len(_launch._kmajor) == kept
