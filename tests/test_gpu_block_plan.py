@@ -8,6 +8,7 @@ without a plan, and that a plan is used only with the tables it was made for.
 import numpy as np
 import pytest
 
+import large_tile_queues as lq
 from helpers import i32_tensor
 from oracle import blocks as ob
 
@@ -153,6 +154,13 @@ def test_plan_says_what_the_tables_say(T, k, E, B, skip, split, alpha, spoil):
     qo = p["q_off"][: 8 * (CLASSES + 1)].reshape(8, CLASSES + 1)
     assert qo[0, 0] == 0 and qo[7, CLASSES] == n and (np.diff(qo.reshape(-1)) >= 0).all()
     assert 1 <= int(p["q_off"][8 * (CLASSES + 1)]) <= 8
+    # ... in the XCD and class that the host's restatement gives it
+    interleave, queues = lq.queues_of(chunks) if chunks else (1, [[]] * 8)
+    assert int(p["q_off"][8 * (CLASSES + 1)]) == interleave
+    for x, queue in enumerate(queues):
+        for cls in range(CLASSES):
+            there = sorted((int(s), int(w) & 0xffff, int(w) >> 16) for s, w in q[qo[x, cls]: qo[x, cls + 1]])
+            assert there == sorted(ch for c_, ch in queue if c_ == cls), (x, cls)
 
 
 @pytest.mark.parametrize("T,k,E,B,spoil", [
@@ -218,7 +226,7 @@ def _dense_case(T, H, I, E, k, B, dev, seed=4, impl="shard_on_block"):
 @pytest.mark.parametrize("kind,T,H,I,E,k,B", [
     ("mx", 1500, 1024, 512, 8, 2, 128),      # large-tile MX kernels, several chunks per expert
     ("mx", 3, 1024, 512, 16, 4, 128),        # decode-sized
-    ("mx", 600, 1024, 96, 4, 2, 128),        # general tiled kernel (I % 128 != 0)
+    ("mx", 600, 1024, 96, 4, 2, 128),        # ... with a short last tile (I % 128 != 0)
     ("bf16", 900, 512, 256, 4, 2, 256),      # large-tile bf16 kernels
     ("bf16", 500, 320, 80, 4, 2, 64),        # general tiled kernel
 ])
