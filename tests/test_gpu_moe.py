@@ -350,7 +350,7 @@ def _run_fp8_row(c, gamma, mode=1, clamps=None, act=0, shared_scales=False):
 
 @pytest.mark.parametrize("T,H,I,E,k,B", [(256, 512, 512, 4, 2, 128), (384, 1024, 896, 8, 2, 128),
                                          (300, 512, 640, 2, 2, 128), (768, 1024, 896, 2, 2, 128),  # 256-row chunk tiles
-                                         # shapes outside the large-tile kernels: the general tiled kernel
+                                         # columns padded to a whole tile; H % 512 != 0: the general tiled kernel
                                          (256, 512, 448, 4, 2, 128), (300, 768, 512, 4, 2, 128)])
 def test_fp8_row_pipeline(T, H, I, E, k, B):
     """RMSNorm-Quant ROW -> fp8 x fp8 blockwise MoE with per-row / per-channel scales (BASELINE config 2 shape family)."""
@@ -369,7 +369,7 @@ def test_fp8_row_pipeline(T, H, I, E, k, B):
 
 @pytest.mark.parametrize("mode,clamp,act,I,shared", [(2, False, 0, 896, False), (1, True, 3, 896, True),
                                                      (2, True, 1, 896, False), (0, False, 0, 896, False),
-                                                     (2, True, 3, 448, True)])  # I = 448: the general tiled kernel
+                                                     (2, True, 3, 448, True)])  # I = 448: padded to a whole tile
 def test_fp8_row_scale_modes_and_clamps(mode, clamp, act, I, shared):
     """PRE_SCALE (the affinity scales the token's row, i.e. its dequantisation scale), NO_SCALE and the four clamps on
     the fp8-row kind.  The reference has no kernel with fp8 activations on this path: the rule is the dense
@@ -635,17 +635,17 @@ def test_mx_reference_table(H, T, I, E, B, k, act, fmt, skip, dynamic, uint):
 @pytest.mark.parametrize("I,B,uint", [(96, 128, False), (544, 256, True), (160, 128, True), (1056, 128, False)])
 def test_mx_weight_formats_outside_the_large_tile_shapes(fmt, I, B, uint):
     """e5m2 and MXFP4 weights where I is not a multiple of 128 (the reference takes any I % 16 == 0 whose tail past a
-    multiple of 512 is a multiple of 32, bwmm_shard_on_block_mx.py:620-633): the general tiled kernel, with the
-    reference table's options (Swish, bias, clamps)."""
+    multiple of 512 is a multiple of 32, bwmm_shard_on_block_mx.py:620-633), with the reference table's options (Swish,
+    bias, clamps).  (The kernels whose last tile is short; the general tiled kernel: test_gpu_moe_mx_general.py.)"""
     T, H, E, k = 256, 1024, 8, 2
     c = mx_case(T, H, I, E, k, B, seed=41, bias=True, weight_format=fmt, random_codes=True)
     out = _run_mx_options(c, 3, REF_MX_CLAMPS, uint)
     o = from_bf16_tensor(out)
     assert o.shape[0] == 2 and not o[1].any() and not o[0, T].any()
-    _check(o[0, :T], _golden_mx_options(c, 3, REF_MX_CLAMPS)[:T], f"mx general kernel I={I} B={B} {fmt}")
+    _check(o[0, :T], _golden_mx_options(c, 3, REF_MX_CLAMPS)[:T], f"mx short tile I={I} B={B} {fmt}")
 
 
-@pytest.mark.parametrize("I", [512, 96, 544])  # large-tile kernels; general tiled kernel (I % 128 != 0), with a tail tile
+@pytest.mark.parametrize("I", [512, 96, 544])  # whole tiles; short ones (I % 128 != 0), one behind a whole one
 @pytest.mark.parametrize(
     "act,clamps",
     [
@@ -659,7 +659,7 @@ def test_mx_weight_formats_outside_the_large_tile_shapes(fmt, I, B, uint):
 )
 def test_mx_activation_and_clamp_options(I, act, clamps):
     """Every ActFnType and every clamp limit on its own (limits small enough to cut a large share of the values)
-    through both MX code paths, with bias."""
+    with whole and short tiles, with bias."""
     T, H, E, k, B = 256, 512, 8, 2, 128
     c = mx_case(T, H, I, E, k, B, seed=31, bias=True, weight_std=0.05)
     out = _run_mx_options(c, act, clamps, uint_containers=False, prequant=(act == 2))
