@@ -131,7 +131,7 @@ int validate(const moe_bwmm_args* a) {
   if (a->kind == MOE_KIND_MXFP8) {
     // (an I that is no multiple of 128: past these limits the general kernel takes the call)
     if (a->I % 128 == 0 && !mx_fast(a)) return MOE_E_BAD_SHAPE;
-  } else if (a->kind != MOE_KIND_MXFP8) {
+  } else {
     // general tiled kernel, dense kinds: row offsets are kept in units of 4 bytes in 32 bits (the value ~0 is
     // reserved for "no such row"), i.e. each A operand must stay below 2^34 - 4 bytes = 16 GiB
     const int64_t lim34 = ((int64_t)1 << 34) - 4;

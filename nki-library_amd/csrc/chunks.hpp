@@ -153,8 +153,9 @@ __device__ __forceinline__ void build_chunks(const int32_t* __restrict__ b2e, co
   auto key_of = [&](int i) {
     const bool last = interleave == 1 && ((i + 1 >= n) || (chunk_expert_of(i + 1) != chunk_expert_of(i)));
     // (with checkpoints, i.e. pad_row, chunks of 18 row tiles run on the instance of 20: its waves' shares of the checkpoint's
-    // columns end at multiples of 64 bytes, and the gate/up launch of T = 1024, top-4 of 8 bf16 experts of H = 3072, I = 2048
-    // takes 117 us instead of 127)
+    // columns end at multiples of 64 bytes.  A layer with experts of 257 to 288 rows on 18 | on 20, us: 1024 tokens, top-4 of 8 of
+    // H = 3072, I = 2048 246 | 233; 741, top-6 of 16 of 3072, 4352 536 | 522; 2160, top-2 of 16 of 4096, 4480 625 | 614; 534, top-4 of 4 of
+    // 4608, 512 160 | 162; 270, top-8 of 8 of 512, 2560 142 | 144; over 29 such layers 20 takes 0.997 times as long.)
     const int cls = chunk_class(rows_of(i), last);
     return xcd_of(i) * CHUNK_CLASSES + (pad_row && CHUNK_CLASS_TILES[cls] == 18 ? cls - 2 : cls);
   };
