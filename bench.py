@@ -57,7 +57,7 @@ def profiled_traffic(workload, routing):
     if h.hexdigest() != sha.group(1):
         return None
     # the clock the part held during the profiled gate/up launches (GRBM_GUI_ACTIVE over the launch time)
-    ghz = re.search(r"`mx_gemm_kernel<1, 0>` \|[^\n]*\| ([0-9.]+) GHz \|", text)
+    ghz = re.search(r"`mx_gemm_kernel<1, 0, false>` \|[^\n]*\| ([0-9.]+) GHz \|", text)
     return int(val.group(1)), (float(ghz.group(1)) if ghz else None)
 
 
@@ -296,9 +296,9 @@ def bench_fp8_row(args):
     peak = PEAK_BF16_TFLOPS if bf16 else PEAK_FP8_TFLOPS
     roofline = {"bound": "mfma", "achieved": round(gu_tflops, 2), "peak": peak, "unit": "TFLOP/s",
                 "frac": round(gu_tflops / peak, 4), "traffic": None,
-                "kernel": ("moe::mx_gemm_kernel<1, 4> (gate/up blockwise GEMM of the bf16 kind on the large-tile kernels with "
+                "kernel": ("moe::mx_gemm_kernel<1, 4, false> (gate/up blockwise GEMM of the bf16 kind on the large-tile kernels with "
                            "fused act*up, on the x4-ordered weight copies kept from the first call)" if bf16 else
-                           "moe::mx_gemm_kernel<1, 3> (gate/up blockwise GEMM of the fp8-row kind on the large-tile "
+                           "moe::mx_gemm_kernel<1, 3, false> (gate/up blockwise GEMM of the fp8-row kind on the large-tile "
                            "kernels with fused scales and act*up, on the x4-ordered weight copies kept from the first "
                            "call)"),
                 "algorithmic_bytes": int(gu_bytes), "algorithmic_flops": int(flops_gu),
