@@ -37,10 +37,10 @@ _STAGES = (
 # of the bf16 kind, which are widened); ``kmajor_weight_cache = False`` makes every call build its copies in the
 # workspace instead.
 kmajor_weight_cache = True
-# The same mechanism for 8-bit MXFP8 weights on the large-tile shapes: copies in the order the kernels read them
+# The same mechanism for the MX kinds where I is a multiple of 128: copies in the order the kernels read them
 # (contiguous 32 KB runs per workgroup and K slice instead of 128-byte pieces of the reference layout), of the
-# gate/up weights only: that GEMM is 5 % faster at DeepSeek-V3's expert shape, the down GEMM was not.  A second
-# copy of the gate/up weights in HBM, made on the first call with a weight tensor pair; ``mx_weight_copies =
+# gate/up weights (that GEMM is 5 % faster at DeepSeek-V3's expert shape, the down GEMM was not) and of 4-bit down
+# weights.  A second copy of those weights in HBM, made on the first call with a weight tensor pair; ``mx_weight_copies =
 # False`` reads the reference layout in place.
 mx_weight_copies = True
 # Measurement hook: an int64 device tensor of 4 elements that the GEMMs (not the general kernel) fill with the shader cycles and
